@@ -393,7 +393,8 @@ __global__ __launch_bounds__(256) void k_copy_back_maps(
 // local; a root gets a slot per image (order irrelevant: positions are
 // written to the next buffer from values of the current one).
 __device__ __forceinline__ void k_img_build_body(int *__restrict__ counters, const int *__restrict__ sync_src,
-                                                   int *__restrict__ img_cnt, int *__restrict__ img_slot, int cap) {
+                                                   const int *__restrict__ sync_mult, int *__restrict__ img_cnt,
+                                                   int4 *__restrict__ img_tab, int cap) {
     if (counters[C_OVF]) return;
     const int nlocal = counters[C_NLOCAL], ng = counters[C_NGHOST];
     for (int q = blockIdx.x * 256 + threadIdx.x; q < ng; q += gridDim.x * 256) {
@@ -401,14 +402,19 @@ __device__ __forceinline__ void k_img_build_body(int *__restrict__ counters, con
         for (int hop = 0; root >= nlocal && hop < 64; hop++) root = sync_src[root - nlocal];
         if (root >= nlocal) { atomicMax(&counters[C_IMG_OVF], 1); continue; }
         const int k = atomicAdd(&img_cnt[root], 1);
-        if (k < IMG_MAX) img_slot[(size_t) k * cap + root] = q;
+        if (k < IMG_MAX) {
+            const int src = sync_src[q];
+            const int m = (sync_mult[3 * q] + 1) | (sync_mult[3 * q + 1] + 1) << 2 | (sync_mult[3 * q + 2] + 1) << 4;
+            img_tab[(size_t) k * cap + root] = make_int4(q, src == root ? -1 : src, m, 0);
+        }
         else atomicMax(&counters[C_IMG_OVF], 1);
     }
 }
 
 __global__ __launch_bounds__(256) void k_img_build(int *__restrict__ counters, const int *__restrict__ sync_src,
-                                                   int *__restrict__ img_cnt, int *__restrict__ img_slot, int cap) {
-    k_img_build_body(counters, sync_src, img_cnt, img_slot, cap);
+                                                   const int *__restrict__ sync_mult, int *__restrict__ img_cnt,
+                                                   int4 *__restrict__ img_tab, int cap) {
+    k_img_build_body(counters, sync_src, sync_mult, img_cnt, img_tab, cap);
 }
 
 
@@ -811,7 +817,7 @@ __device__ __forceinline__ void lj_wave(const LJArgs &A, int wv) {
         // counts past the list rows (a build never writes them) are clamped,
         // so no list load leaves the allocation
         const int n = moves ? min(numneighs[ii], A.ncap) : 0;
-        const int nmax = __builtin_amdgcn_readfirstlane(wave_max(n));
+        const int nmax = wave_max_uniform(n);
         const double xi = X[ii], yi = Y[ii], zi = Z[ii];
         const int ti = NT != 1 ? type[ii] : 0;
         const double eps0 = tab.eps[0], sig0 = tab.sig6[0];
@@ -853,8 +859,8 @@ __device__ __forceinline__ void lj_wave(const LJArgs &A, int wv) {
         };
         walk(0, n, nmax, false, t0, t1, t2);
         if (HALF) {
-            const int nr = moves ? min(A.nrev[ii], A.ncap) : 0;
-            const int nrmax = __builtin_amdgcn_readfirstlane(wave_max(nr));
+            const int nr = moves ? min(A.nrev[ii], A.rev0) : 0;
+            const int nrmax = wave_max_uniform(nr);
             walk(A.rev0, nr, nrmax, true, r0, r1, r2);
         }
         if (live) {
@@ -887,8 +893,9 @@ __device__ __forceinline__ void lj_wave(const LJArgs &A, int wv) {
                     }
                     if (do_vv1) {
                         Xn[i] = px; Yn[i] = py; Zn[i] = pz;
-                        if (A.Pn) A.Pn[i] = make_double4(px, py, pz, 0.0);
-                        if (im.on) write_images(im, i, nlocal, px, py, pz, X, Y, Z, Xn, Yn, Zn, A.g, A.Pn);
+                        const double tw = type_w(type[i]);
+                        if (A.Pn) A.Pn[i] = make_double4(px, py, pz, tw);
+                        if (im.on) write_images(im, i, nlocal, px, py, pz, X, Y, Z, Xn, Yn, Zn, A.g, A.Pn, tw);
                     }
                 }
             }
@@ -930,6 +937,11 @@ __device__ __forceinline__ double pair_swap(double v) {
     return __longlong_as_double(((long long) hi << 32) | (unsigned int) lo);
 }
 
+// the type word of a packed record's (z, type) half, from the other lane of the pair
+__device__ __forceinline__ int pair_swap_type(double w) {
+    return __builtin_amdgcn_mov_dpp((int) __double_as_longlong(w), 0xB1, 0xF, 0xF, true);
+}
+
 // The force kernel of the timestep (MODE 0: forces; MODE 1: fused with
 // final/initial integrate and the next positions) on TWO lanes per local: a
 // wave takes 32 consecutive cell-sorted locals, lane 2p + h of local p
@@ -945,14 +957,12 @@ __device__ __forceinline__ double pair_swap(double v) {
 // (z, 0), the next has lane 2p read record o's (z, 0) and lane 2p + 1 record
 // o's (x, y), and the z halves are swapped by DPP, so a record is touched by
 // one load instruction (one cache-line lookup) instead of two.
-// HALF: the own part (rows [0, n)) into T and the mirror part (rows
-// [rev0, rev0 + nrev)) into R, force = R + T, as lj_wave.
+// Full lists (half lists: lj_multi).
 // RED: kinetic energy of the locals (lane 2p) and energy / virial of every
-// lane's pairs (full lists: weight 1/2; half lists: 1 for local pairs and 1/2
-// for local-ghost pairs, own part only) into one partial per wave; the sums
+// lane's pairs (weight 1/2) into one partial per wave; the sums
 // over a wave's lanes are taken in lane order, so these totals may differ
 // from lj_wave's in the last bits.
-template <int NT, int MODE, bool RED, bool HALF, bool UNIT>
+template <int NT, int MODE, bool RED, bool UNIT>
 __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
     constexpr int U = 2;  // entries per lane per step (4 per local)
     const int lane = threadIdx.x & 63, h = lane & 1;
@@ -983,37 +993,37 @@ __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
         const int nt = tab.nt;
         const int stride = A.nl_stride;
         double u = 0.0, w = 0.0;
-        struct Pos { double2 a[U], b[U]; int t[U]; uint32_t j[U]; };
+        struct Pos { double2 a[U], b[U]; };
         // j[2q] / j[2q + 1]: the even / odd entry of pair q (both lanes)
         auto gather = [&](const uint32_t (&j)[2 * U], Pos &p) {
 #pragma unroll
             for (int q = 0; q < U; q++) {
                 p.a[q] = *(const double2 *) (P + (j[2 * q] << 5) + (h << 4));
                 p.b[q] = *(const double2 *) (P + (j[2 * q + 1] << 5) + ((h ^ 1) << 4));
-                const uint32_t jo = h ? j[2 * q + 1] : j[2 * q];
-                if (NT != 1) p.t[q] = type[jo];
-                p.j[q] = jo;
             }
         };
-        // one list part, rows [row0, row0 + cnt), summed in order into (a0, a1, a2) of lane 2p
-        auto walk = [&](int row0, int cnt, bool mirror, double &a0, double &a1, double &a2) {
-            const int nmax = __builtin_amdgcn_readfirstlane(wave_max(cnt));
+        // the list, summed in order into (a0, a1, a2) of lane 2p
+        auto walk = [&](int cnt, double &a0, double &a1, double &a2) {
+            const int nmax = wave_max_uniform(cnt);
             const int nst = (nmax + 2 * U - 1) / (2 * U);
             if (nst <= 0) return;  // wave-uniform
-            const uint4 *lp = (const uint4 *) A.nl + (size_t) (row0 >> 2) * stride + ii;
+            const uint4 *lp = (const uint4 *) A.nl + ii;
             const int gl = max((cnt + 3) / 4 - 1, 0);
             auto ldl = [&](int st, uint32_t (&j)[2 * U]) {
                 const uint4 g = lp[(size_t) min(st, gl) * stride];
                 j[0] = min(g.x, jmax);
-                j[1] = min(g.y, jmax);
-                j[2] = min(g.z, jmax);
+                j[2] = min(g.y, jmax);  // (a group holds its entries as 0, 2, 1, 3)
+                j[1] = min(g.z, jmax);
                 j[3] = min(g.w, jmax);
             };
             auto compute = [&](int st, const Pos &p) {
 #pragma unroll
                 for (int q = 0; q < U; q++) {
                     double sg6 = sig0, ep = eps0;
-                    if (NT != 1) { const int kt = ti * nt + p.t[q]; sg6 = s_sig6[kt]; ep = s_eps[kt]; }
+                    if (NT != 1) {
+                        const int kt = ti * nt + (pair_swap_type(h ? p.a[q].y : p.b[q].y) & 3);
+                        sg6 = s_sig6[kt]; ep = s_eps[kt];
+                    }
                     double g0, g1, g2, uu, ww;
                     const double2 xy = h ? p.b[q] : p.a[q];
                     const double zj = pair_swap(h ? p.a[q].x : p.b[q].x);
@@ -1022,11 +1032,7 @@ __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
                     // lane 2p: entry 4s + 2q (its own), then 4s + 2q + 1 (lane 2p + 1's)
                     a0 = a0 + g0; a1 = a1 + g1; a2 = a2 + g2;
                     a0 = a0 + odd_lane(g0); a1 = a1 + odd_lane(g1); a2 = a2 + odd_lane(g2);
-                    if (RED && !HALF) { u += uu; w += ww; }
-                    if (RED && HALF && !mirror) {
-                        const double wt = p.j[q] < (uint32_t) nlocal ? 2.0 : 1.0;
-                        u += wt * uu; w += wt * ww;
-                    }
+                    if (RED) { u += uu; w += ww; }
                 }
             };
             uint32_t LA[2 * U], LB[2 * U];
@@ -1044,13 +1050,12 @@ __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
                 compute(st + 1, PB);
             }
         };
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0;
+        double t0 = 0.0, t1 = 0.0, t2 = 0.0;
         // counts past the list rows (a build never writes them) are clamped
-        walk(0, moves ? min(A.numneighs[ii], A.ncap) : 0, false, t0, t1, t2);
-        if (HALF) walk(A.rev0, moves ? min(A.nrev[ii], A.ncap) : 0, true, r0, r1, r2);
+        walk(moves ? min(A.numneighs[ii], A.ncap) : 0, t0, t1, t2);
         if (RED) { pe = 0.5 * u; vir = 0.5 * w; }
         if (live && h == 0) {
-            const double f0 = r0 + t0, f1 = r1 + t1, f2 = r2 + t2;
+            const double f0 = 0.0 + t0, f1 = 0.0 + t1, f2 = 0.0 + t2;  // reset_volatile_properties, then += the sum
             A.fx[i] = f0; A.fy[i] = f1; A.fz[i] = f2;
             if (MODE == 1) {
                 const double m = A.mass[i];
@@ -1073,8 +1078,9 @@ __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
                 }
                 if (A.do_vv1) {
                     A.Xn[i] = px; A.Yn[i] = py; A.Zn[i] = pz;
-                    if (A.Pn) A.Pn[i] = make_double4(px, py, pz, 0.0);
-                    if (A.im.on) write_images(A.im, i, nlocal, px, py, pz, X, Y, Z, A.Xn, A.Yn, A.Zn, A.g, A.Pn);
+                    const double tw = NT != 1 ? type_w(ti) : 0.0;
+                    if (A.Pn) A.Pn[i] = make_double4(px, py, pz, tw);
+                    if (A.im.on) write_images(A.im, i, nlocal, px, py, pz, X, Y, Z, A.Xn, A.Yn, A.Zn, A.g, A.Pn, tw);
                 }
             }
         }
@@ -1090,9 +1096,239 @@ __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
     }
 }
 
-template <int NT, int MODE, bool RED, bool HALF, bool UNIT>
+template <int NT, int MODE, bool RED, bool UNIT>
 __global__ __launch_bounds__(64) void k_lj2(LJArgs A) {
-    lj_wave2<NT, MODE, RED, HALF, UNIT>(A, xcd_block(blockIdx.x, gridDim.x));
+    lj_wave2<NT, MODE, RED, UNIT>(A, xcd_block(blockIdx.x, gridDim.x));
+}
+
+// LDS operations of one wave complete in order, so what a wave hands from
+// lane to lane needs no wait, only an order the compiler keeps
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The force kernel of the timestep on L = 4 .. 32 lanes per local (M = 64 / L
+// consecutive cell-sorted locals per wave); MODE, RED and HALF as lj_wave2.
+// What bounds it: a system of a few thousand atoms fills few waves, so a step
+// is one chain of dependent loads and sums.  Lane h of local p evaluates
+// entry L r + eh of round r, all terms of a round at once; they go through LDS
+// (LDS operations of one wave complete in order: no barrier), and lane
+// (c, ps) adds component c of local ps in list order, so every sum is the
+// reference's, bit for bit.  The same lane then integrates its component, and
+// lane (k, ps) writes image k, so nothing after the sum is serial in the
+// components or the images.  Loads that need no other load -- the first two
+// list rounds, counts, velocities, the image table -- are issued before the
+// walk.  The lane pair of entries (e, e') gathers each 32-byte record with one
+// instruction (x, y on one lane, z and the type on the other, swapped by DPP);
+// the two pairs of a list group take entries 0, 2 and 1, 3, so that one
+// instruction touches consecutive entries (13.0 -> 10.1 M cache-line lookups
+// per launch at 131072 atoms).  A padded entry reads the last particle's
+// record, one line for all lanes.
+// Measured (100 steps with 5 rebuilds, one lane pair per local -> this):
+// 256 atoms 2.67 -> 1.61 ms, 2048 2.63 -> 1.74, 19652 2.81 -> 2.28, 55296
+// 3.82 -> 3.39; half lists 55296 5.21 -> 4.74, 131072 (400 steps) 32.5 -> 30.9.
+// HALF: the own part (rows [0, n)) into ft and the mirror part (rows
+// [rev0, rev0 + nrev)) into fr, force = fr + ft, as lj_wave; energy and virial
+// weigh a local pair 1 and a local-ghost pair 1/2, own part only.
+template <int L, int NT, int MODE, bool RED, bool HALF, bool UNIT>
+__device__ __forceinline__ void lj_multi(const LJArgs &A, int wv) {
+    constexpr int M = 64 / L;      // locals per wave
+    constexpr int S = L + 2;       // row stride of the term buffer (doubles)
+    __shared__ __align__(16) double s_term[2 * 3 * M * S];
+    const int lane = threadIdx.x & 63, p = lane / L, h = lane & (L - 1), odd = lane & 1;
+    const int eh = (h & ~3) | list_pos(h);  // the entry of a round this lane evaluates
+    const int nlocal = A.nlocal;
+    const uint32_t jmax = (uint32_t) max(nlocal + A.counters[C_NGHOST] - 1, 0);
+    const char *__restrict__ P = (const char *) A.P;
+    const double rc2 = A.rc2;
+    const LJTab &tab = A.tab;
+    __shared__ double s_eps[16], s_sig6[16];
+    if (NT != 1) {
+        if (lane < 16) { s_eps[lane] = tab.eps[lane]; s_sig6[lane] = tab.sig6[lane]; }
+        __syncthreads();
+    }
+    const int i0 = wv * M;
+    double ke = 0.0, pe = 0.0, vir = 0.0;
+    if (i0 < nlocal) {  // wave-uniform
+        const int ii = min(i0 + p, nlocal - 1);
+        const bool moves = !(A.flags[ii] & FLAG_FIXED);
+        const double xi = A.X[ii], yi = A.Y[ii], zi = A.Z[ii];
+        const double eps0 = tab.eps[0], sig0 = tab.sig6[0];
+        const int tn = NT != 1 ? A.type[ii] * tab.nt : 0;
+        const int stride = A.nl_stride;
+        double u = 0.0, w = 0.0;
+        const bool live = i0 + p < nlocal;
+        const int cnt = live ? min(A.numneighs[ii], A.ncap) : 0;
+        const int cnt_r = HALF && live ? min(A.nrev[ii], A.rows) : 0;
+        struct Pos { double2 a, b; };
+        // the component this lane sums: c of local ps
+        const int c = lane / M, ps = lane & (M - 1);
+        const double *row = s_term + (min(c, 2) * M + ps) * S;
+        double *out = s_term + p * S + eh;
+        constexpr int BUF = 3 * M * S;
+        const uint32_t off_e = odd ? 16u : 0u, off_o = odd ? 0u : 16u;
+        // half of list group h / 4 of the round, read by both lanes of a pair: entries 0, 2 or 1, 3
+        const uint32_t loff = ((uint32_t) (h >> 2) * (uint32_t) stride + (uint32_t) ii) * 16u + (h & 2) * 4u;
+        const int rounds = A.rows / L;  // rounds the allocated rows hold
+        auto ldl = [&](int row0, int r, int R) {
+            return *(const uint2 *) ((const char *) (A.nl + (size_t) row0 * stride) +
+                                     (size_t) min(r, R - 1) * ((size_t) stride * (L * 4)) + loff);
+        };
+        // JA, JB: rounds 0 and 1, loaded before the counts are known
+        auto walk = [&](int row0, int cnt, bool mirror, uint2 JA, uint2 JB, double &acc) {
+            const int nmax = wave_max_uniform(cnt);
+            const int R = (nmax + L - 1) / L;  // rounds of L entries
+            if (R <= 0) return;  // wave-uniform
+            const int cnt_h = cnt - eh, cnt_e = cnt - (eh & ~2);
+            auto gather = [&](int r, uint2 j, Pos &q) {
+                const bool some = cnt_e > r * L;
+                const uint32_t je = some ? min(j.x, jmax) : jmax;
+                const uint32_t jo = some ? min(j.y, jmax) : jmax;
+                q.a = *(const double2 *) (P + ((je << 5) + off_e));
+                q.b = *(const double2 *) (P + ((jo << 5) + off_o));
+            };
+            auto compute = [&](int r, uint2 j, const Pos &q, double *o) {
+                const double2 xy = odd ? q.b : q.a;
+                const double zj = pair_swap(odd ? q.a.x : q.b.x);
+                double sg6 = sig0, ep = eps0;
+                if (NT != 1) {
+                    const int tj = pair_swap_type(odd ? q.a.y : q.b.y);
+                    const int kt = tn + (tj & 3);
+                    sg6 = s_sig6[kt]; ep = s_eps[kt];
+                }
+                double g0, g1, g2, uu, ww;
+                lj_pair<RED, false, UNIT>(xi, yi, zi, xy.x, xy.y, zj, cnt_h > r * L, rc2, sg6, ep, g0, g1, g2, uu, ww);
+                o[0] = g0;
+                o[M * S] = g1;
+                o[2 * M * S] = g2;
+                if (RED && !HALF) { u += uu; w += ww; }
+                if (RED && HALF && !mirror) {
+                    const double wt = (odd ? j.y : j.x) < (uint32_t) nlocal ? 2.0 : 1.0;
+                    u += wt * uu; w += wt * ww;
+                }
+                wave_lds_sync();
+            };
+            auto sum = [&](const double *t) {
+#pragma unroll
+                for (int e = 0; e < L; e += 2) {
+                    const double2 v = *(const double2 *) (t + e);
+                    acc = acc + v.x;
+                    acc = acc + v.y;
+                }
+                wave_lds_sync();
+            };
+            Pos QA, QB;
+            gather(0, JA, QA);
+            for (int r = 0;;) {
+                gather(r + 1, JB, QB);
+                uint2 JC = ldl(row0, r + 2, R);
+                compute(r, JA, QA, out);
+                JA = JC;
+                if (r > 0) sum(row + BUF);
+                if (++r >= R) { sum(row); break; }
+                gather(r + 1, JA, QA);
+                JC = ldl(row0, r + 2, R);
+                compute(r, JB, QB, out + BUF);
+                JB = JC;
+                sum(row);
+                if (++r >= R) { sum(row + BUF); break; }
+            }
+        };
+        const uint2 J0 = ldl(0, 0, rounds), J1 = ldl(0, 1, rounds);
+        uint2 M0 = {0, 0}, M1 = {0, 0};
+        if (HALF) { M0 = ldl(A.rev0, 0, rounds); M1 = ldl(A.rev0, 1, rounds); }
+        // component c of local ps, and its image k = c: what follows the walk
+        // needs, loaded before it
+        const int i = min(i0 + ps, nlocal - 1);
+        const bool here = i0 + ps < nlocal, mine = c < 3 && here;
+        double *__restrict__ vp = c == 0 ? A.vx : c == 1 ? A.vy : A.vz;
+        double v = 0.0, x = 0.0, m = 1.0, bx = 0.0, by = 0.0, bz = 0.0;
+        int nimg = 0;
+        int4 im0 = {0, -1, 0, 0};
+        bool mv = false;
+        if (MODE == 1) {
+            v = vp[i];
+            x = (c == 0 ? A.X : c == 1 ? A.Y : A.Z)[i];
+            m = A.mass[i];
+            mv = !(A.flags[i] & FLAG_FIXED);
+            if (A.im.on) {
+                nimg = here ? min(A.im.cnt[i], IMG_MAX) : 0;
+                im0 = A.im.tab[(size_t) min(c, IMG_MAX - 1) * A.im.cap + i];
+                if (c >= nimg) im0.y = -1;
+                if (im0.y >= 0) { bx = A.X[im0.y]; by = A.Y[im0.y]; bz = A.Z[im0.y]; }
+            }
+        }
+        double ft = 0.0, fr = 0.0;
+        walk(0, moves ? cnt : 0, false, J0, J1, ft);
+        if (HALF) walk(A.rev0, moves ? cnt_r : 0, true, M0, M1, fr);
+        if (RED) { pe = 0.5 * u; vir = 0.5 * w; }
+        const double f = fr + ft;
+        if (mine) {
+            (c == 0 ? A.fx : c == 1 ? A.fy : A.fz)[i] = f;
+            if (MODE == 1) {
+                const double dt = A.dt;
+                if (mv) {
+                    double b = A.hdt * f;
+                    b = b / m;
+                    if (A.do_vv2) v = v + b;  // final_integrate(ts)
+                    if (RED) ke = v * v;
+                    if (A.do_vv1) {           // initial_integrate(ts+1)
+                        v = v + b;
+                        x = x + dt * v;
+                    }
+                    vp[i] = v;
+                } else if (RED) {
+                    ke = v * v;
+                }
+                if (A.do_vv1) (c == 0 ? A.Xn : c == 1 ? A.Yn : A.Zn)[i] = x;
+            }
+        }
+        if (MODE == 1 && A.do_vv1) {  // (wave-uniform)
+            // lane (c, ps): the packed record (c = 0) and images c, c + L of local ps
+            const double px = __shfl(x, ps, 64), py = __shfl(x, ps + M, 64), pz = __shfl(x, ps + 2 * M, 64);
+            const double tw = NT != 1 ? type_w(A.type[i]) : 0.0;
+            if (A.Pn && here && c == 0) A.Pn[i] = make_double4(px, py, pz, tw);
+            auto image = [&](const int4 &t, double b0, double b1, double b2) {
+                const bool own = t.y < 0;
+                const double gx = (own ? px : b0) + (double) ((t.z & 3) - 1) * A.g.len[0];
+                const double gy = (own ? py : b1) + (double) (((t.z >> 2) & 3) - 1) * A.g.len[1];
+                const double gz = (own ? pz : b2) + (double) (((t.z >> 4) & 3) - 1) * A.g.len[2];
+                const int s = nlocal + t.x;
+                A.Xn[s] = gx; A.Yn[s] = gy; A.Zn[s] = gz;
+                if (A.Pn) A.Pn[s] = make_double4(gx, gy, gz, tw);
+            };
+            if (c < nimg) image(im0, bx, by, bz);
+            if (L < IMG_MAX) {
+                for (int k = c + L; k < nimg; k += L) {
+                    const int4 t = A.im.tab[(size_t) k * A.im.cap + i];
+                    double b0 = 0.0, b1 = 0.0, b2 = 0.0;
+                    if (t.y >= 0) { b0 = A.X[t.y]; b1 = A.Y[t.y]; b2 = A.Z[t.y]; }
+                    image(t, b0, b1, b2);
+                }
+            }
+        }
+        if (RED && MODE == 1) {
+            // m (vx^2 + vy^2 + vz^2) of local ps on lane ps
+            const double k1 = __shfl(ke, ps + M, 64), k2 = __shfl(ke, ps + 2 * M, 64);
+            ke = (c == 0 && mine) ? m * (ke + k1 + k2) : 0.0;
+        }
+    }
+    if (RED) {
+        // one partial per wave (kinetic row from the fused kernel only)
+        const double a = wave_sum(ke), bb = wave_sum(pe), cc = wave_sum(vir);
+        if (lane == 0) {
+            if (MODE == 1) A.partials[wv] = a;
+            A.partials[(size_t) A.pstride + wv] = bb;
+            A.partials[(size_t) 2 * A.pstride + wv] = cc;
+        }
+    }
+}
+
+template <int L, int NT, int MODE, bool RED, bool HALF, bool UNIT>
+__global__ __launch_bounds__(64) void k_ljm(LJArgs A) {
+    lj_multi<L, NT, MODE, RED, HALF, UNIT>(A, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // the waves of many independent systems in one persistent launch: the grid
@@ -1147,12 +1383,13 @@ void launch_lj_older(hipStream_t s, const DevState &d, const Geom &g, const LJPa
     else hipLaunchKernelGGL((k_lj<0, 0, false, false, true>), grid, dim3(64), 0, s, A);
 }
 
-// the packed (x, y, z, 0) copy the force kernels gather from
+// the packed (x, y, z, type) copy the force kernels gather from
 __global__ __launch_bounds__(256) void k_pack_p(const int *__restrict__ counters, const double *__restrict__ X,
                                                 const double *__restrict__ Y, const double *__restrict__ Z,
-                                                double4 *__restrict__ P) {
+                                                const int *__restrict__ type, double4 *__restrict__ P) {
     const int n = counters[C_NLOCAL] + counters[C_NGHOST];
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) P[i] = make_double4(X[i], Y[i], Z[i], 0.0);
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+        P[i] = make_double4(X[i], Y[i], Z[i], type_w(type[i]));
 }
 
 // ---------------------------------------------------------------- integration
@@ -1186,7 +1423,7 @@ __global__ __launch_bounds__(256) void k_vv_post(const double *__restrict__ X, c
                                                  const double *__restrict__ mass, const int *__restrict__ flags,
                                                  int nlocal, double dt, double hdt, int do_vv2, int do_vv1,
                                                  double *__restrict__ partials, Images im, Geom g,
-                                                 double4 *__restrict__ Pn) {
+                                                 const int *__restrict__ type, double4 *__restrict__ Pn) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     double ke = 0.0;
     if (i < nlocal) {
@@ -1214,8 +1451,9 @@ __global__ __launch_bounds__(256) void k_vv_post(const double *__restrict__ X, c
         }
         if (do_vv1) {
             Xn[i] = px; Yn[i] = py; Zn[i] = pz;
-            if (Pn) Pn[i] = make_double4(px, py, pz, 0.0);
-            if (im.on) write_images(im, i, nlocal, px, py, pz, X, Y, Z, Xn, Yn, Zn, g, Pn);
+            const double tw = Pn ? type_w(type[i]) : 0.0;
+            if (Pn) Pn[i] = make_double4(px, py, pz, tw);
+            if (im.on) write_images(im, i, nlocal, px, py, pz, X, Y, Z, Xn, Yn, Zn, g, Pn, tw);
         }
     }
     if (RED) {
@@ -1598,7 +1836,7 @@ __global__ __launch_bounds__(256) void k_sync_pp(double *__restrict__ Xc, double
                                                  const double *__restrict__ Yp, const double *__restrict__ Zp,
                                                  const int *__restrict__ counters, const int *__restrict__ sync_src,
                                                  const int *__restrict__ sync_mult, Geom g,
-                                                 double4 *__restrict__ Pc) {
+                                                 const int *__restrict__ type, double4 *__restrict__ Pc) {
     const int n = counters[C_NSEND_ALL];
     const int nlocal = counters[C_NLOCAL];
     for (int q = blockIdx.x * 256 + threadIdx.x; q < n; q += gridDim.x * 256) {
@@ -1613,7 +1851,7 @@ __global__ __launch_bounds__(256) void k_sync_pp(double *__restrict__ Xc, double
         Xc[nlocal + q] = xg;
         Yc[nlocal + q] = yg;
         Zc[nlocal + q] = zg;
-        Pc[nlocal + q] = make_double4(xg, yg, zg, 0.0);
+        Pc[nlocal + q] = make_double4(xg, yg, zg, type_w(type[nlocal + q]));
     }
 }
 
@@ -1702,7 +1940,8 @@ void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g) {
                        d.alt_mass, d.alt_type, d.alt_flags, d.alt_uid, d.alt_shape, d.alt_ref, d.alt_cell, d.vx,
                        d.vy, d.vz, d.mass, d.type, d.flags, d.uid, d.shape, d.ref, d.particle_cell, d.phys,
                        d.send_map, d.send_mult, d.sync_src, d.sync_mult, d.img_cnt);
-    hipLaunchKernelGGL(k_img_build, dim3(grid), dim3(256), 0, s, d.counters, d.sync_src, d.img_cnt, d.img_slot, d.cap);
+    hipLaunchKernelGGL(k_img_build, dim3(grid), dim3(256), 0, s, d.counters, d.sync_src, d.sync_mult, d.img_cnt, d.img_tab,
+                       d.cap);
 }
 
 // ---------------------------------------------------------------- batched cell phase
@@ -1804,7 +2043,7 @@ __global__ __launch_bounds__(256) void k_copy_back_maps_batch(const RepDesc *__r
 
 __global__ __launch_bounds__(256) void k_img_build_batch(const RepDesc *__restrict__ D) {
     REP_ARGS;
-    k_img_build_body(d.counters, d.sync_src, d.img_cnt, d.img_slot, d.cap);
+    k_img_build_body(d.counters, d.sync_src, d.sync_mult, d.img_cnt, d.img_tab, d.cap);
 }
 
 #undef REP_ARGS
@@ -1932,7 +2171,7 @@ void launch_borders(hipStream_t s, const DevState &d, const Geom &g, const int *
 
 void launch_sync_pp(hipStream_t s, const DevState &d, const Geom &g, int cur, int prev, int grid) {
     hipLaunchKernelGGL(k_sync_pp, dim3(grid), dim3(256), 0, s, d.X[cur], d.Y[cur], d.Z[cur], d.X[prev], d.Y[prev],
-                       d.Z[prev], d.counters, d.sync_src, d.sync_mult, g, d.P[cur]);
+                       d.Z[prev], d.counters, d.sync_src, d.sync_mult, g, d.type, d.P[cur]);
 }
 
 void launch_sync_inplace(hipStream_t s, const DevState &d, const Geom &g, int grid, int with_vel) {
@@ -1955,13 +2194,33 @@ static LJTab make_tab(const LJParams &prm) {
 }
 
 int force_waves(const DevState &d) { return (d.nlocal + 63) / 64; }
-int lj_waves(const DevState &d) { return (d.nlocal + 31) / 32; }
+// Lanes per local of the timestep's force kernel.  More lanes shorten the
+// chain of a step while waves are few; past about 8000 waves the extra work
+// per lane (padding to whole rounds, the sums through LDS) costs more than the
+// latency it hides.  Full lists, 100 steps in ms on 32 / 16 / 8 / 4 / 2 lanes:
+// 2048 atoms 1.74 / 1.76 / 1.86 / 2.21 / 2.6, 8788 2.02 / 1.92 / 1.95 / 2.21 /
+// 2.6, 19652 2.78 / 2.37 / 2.28 / 2.48 / 2.8, 55296 4.93 / 3.90 / 3.48 / 3.39 /
+// 3.73, 131072 (400 steps) - / - / 21.9 / 21.0 / 20.6.  Half lists walk two
+// parts, so their waves are worth splitting longer: 131072 (400 steps) 30.2 on
+// 8, 30.9 on 4, 32.6 on 2; 256000 (60 steps) 11.1 / 10.6 / 10.9; 1048576 (20
+// steps) 27.2 / 26.3 / 26.6.
+static int lj_lanes(const DevState &d) {
+    const int n = d.nlocal;
+    if (n < 4096) return 32;
+    if (n < 12288) return 16;
+    if (n < 40000) return 8;
+    return n < 100000 || d.rev0 > 0 ? 4 : 2;
+}
+int lj_waves(const DevState &d) {
+    const int per = 64 / lj_lanes(d);
+    return (d.nlocal + per - 1) / per;
+}
 
 // image refresh only when the kernel writes next positions into the other
 // buffer and every local's images fit the table
 Images images_of(const DevState &d, bool writes_next) {
     Images im;
-    im.cnt = d.img_cnt; im.slot = d.img_slot; im.src = d.sync_src; im.mult = d.sync_mult;
+    im.cnt = d.img_cnt; im.tab = d.img_tab;
     im.cap = d.cap;
     im.on = (writes_next && d.img_on) ? 1 : 0;
     return im;
@@ -1971,6 +2230,8 @@ LJArgs lj_args(const DevState &d, const Geom &g, const LJParams &prm, int cur, i
                int fused, double *eatom, bool packed) {
     LJArgs A;
     A.counters = d.counters;
+    A.nlocal = d.nlocal;
+    A.rows = list_rows(d.ncap);
     A.g = g;
     A.lstart = d.lstart; A.gstart = d.gstart;
     A.X = d.X[cur]; A.Y = d.Y[cur]; A.Z = d.Z[cur];
@@ -1995,10 +2256,21 @@ static void lj_launch(hipStream_t s, const DevState &d, const Geom &g, const LJP
         const dim3 grid(force_waves(d));
         if (d.rev0 > 0) hipLaunchKernelGGL((k_lj<NT, MODE, RED, true, false, UNIT>), grid, dim3(64), 0, s, A);
         else hipLaunchKernelGGL((k_lj<NT, MODE, RED, false, false, UNIT>), grid, dim3(64), 0, s, A);
-    } else {
+    } else if constexpr (MODE != 2) {
         const dim3 grid(lj_waves(d));
-        if (d.rev0 > 0) hipLaunchKernelGGL((k_lj2<NT, MODE, RED, true, UNIT>), grid, dim3(64), 0, s, A);
-        else hipLaunchKernelGGL((k_lj2<NT, MODE, RED, false, UNIT>), grid, dim3(64), 0, s, A);
+#define LJM(L)                                                                                            \
+    do {                                                                                                  \
+        if (d.rev0 > 0) hipLaunchKernelGGL((k_ljm<L, NT, MODE, RED, true, UNIT>), grid, dim3(64), 0, s, A); \
+        else hipLaunchKernelGGL((k_ljm<L, NT, MODE, RED, false, UNIT>), grid, dim3(64), 0, s, A);           \
+    } while (0)
+        switch (lj_lanes(d)) {
+            case 2: hipLaunchKernelGGL((k_lj2<NT, MODE, RED, UNIT>), grid, dim3(64), 0, s, A); break;
+            case 4: LJM(4); break;
+            case 8: LJM(8); break;
+            case 16: LJM(16); break;
+            default: LJM(32); break;
+        }
+#undef LJM
     }
 }
 
@@ -2047,7 +2319,7 @@ __global__ __launch_bounds__(256) void k_pack_p_batch(const LJArgs *__restrict__
     const int n = A.counters[C_NLOCAL] + A.counters[C_NGHOST];
     double4 *P = (double4 *) A.P;  // the system's own packed buffer
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
-        P[i] = make_double4(A.X[i], A.Y[i], A.Z[i], 0.0);
+        P[i] = make_double4(A.X[i], A.Y[i], A.Z[i], type_w(A.type[i]));
 }
 
 void launch_pack_p_batch(hipStream_t s, const LJArgs *desc, int n, int max_cap) {
@@ -2058,7 +2330,7 @@ void launch_pack_p_batch(hipStream_t s, const LJArgs *desc, int n, int max_cap) 
 
 void launch_pack_p(hipStream_t s, const DevState &d, int cur) {
     hipLaunchKernelGGL(k_pack_p, dim3(std::max(1, std::min((d.cap + 255) / 256, 1024))), dim3(256), 0, s,
-                       d.counters, d.X[cur], d.Y[cur], d.Z[cur], d.P[cur]);
+                       d.counters, d.X[cur], d.Y[cur], d.Z[cur], d.type, d.P[cur]);
 }
 
 void launch_lj_full(hipStream_t s, const DevState &d, const Geom &g, const LJParams &prm, int cur, int next, int fuse,
@@ -2093,11 +2365,11 @@ void launch_vv_post(hipStream_t s, const DevState &d, const Geom &g, const LJPar
     if (reduce)
         hipLaunchKernelGGL(k_vv_post<true>, dim3(grid), dim3(256), 0, s, d.X[cur], d.Y[cur], d.Z[cur], d.X[next],
                            d.Y[next], d.Z[next], d.vx, d.vy, d.vz, d.fx, d.fy, d.fz, d.mass, d.flags, d.nlocal, prm.dt,
-                           prm.hdt, do_vv2, do_vv1, d.partials, images_of(d, do_vv1 && next != cur), g, Pn);
+                           prm.hdt, do_vv2, do_vv1, d.partials, images_of(d, do_vv1 && next != cur), g, d.type, Pn);
     else
         hipLaunchKernelGGL(k_vv_post<false>, dim3(grid), dim3(256), 0, s, d.X[cur], d.Y[cur], d.Z[cur], d.X[next],
                            d.Y[next], d.Z[next], d.vx, d.vy, d.vz, d.fx, d.fy, d.fz, d.mass, d.flags, d.nlocal, prm.dt,
-                           prm.hdt, do_vv2, do_vv1, d.partials, images_of(d, do_vv1 && next != cur), g, Pn);
+                           prm.hdt, do_vv2, do_vv1, d.partials, images_of(d, do_vv1 && next != cur), g, d.type, Pn);
 }
 
 void launch_ke_partial(hipStream_t s, const DevState &d) {

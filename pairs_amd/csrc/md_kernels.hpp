@@ -66,16 +66,26 @@ struct Geom {
 
 // Neighbour lists: entry k of physical local i.  Rows come in groups of four
 // so that one 16-byte load gives a lane four consecutive entries; a group
-// holds, for every particle, its four entries side by side.
+// holds, for every particle, its four entries side by side in the order 0, 2,
+// 1, 3 (list_pos): the halves of a group are then the entries that one lane
+// pair of the force kernel takes, so that its two pairs gather consecutive
+// entries -- often records of one cache line -- with one instruction.
+__host__ __device__ __forceinline__ int list_pos(int k) { return ((k & 1) << 1) | ((k >> 1) & 1); }
 __host__ __device__ __forceinline__ size_t nl_at(int k, int i, int nl_stride) {
-    return ((size_t) (k >> 2) * nl_stride + i) * 4 + (k & 3);
+    return ((size_t) (k >> 2) * nl_stride + i) * 4 + list_pos(k);
 }
+
+// list rows are allocated in multiples of this: the force kernel reads a
+// local's list up to 32 rows at a time, by whole rounds
+constexpr int LIST_ROWS = 32;
+__host__ __device__ __forceinline__ int list_rows(int ncap) { return (ncap + LIST_ROWS - 1) / LIST_ROWS * LIST_ROWS; }
 
 constexpr int IMG_MAX = 8;
 
 // what a position-advancing kernel needs to refresh the ghost images
 struct Images {
-    const int *cnt, *slot, *src, *mult;
+    const int *cnt;
+    const int4 *tab;
     int cap, on;
 };
 
@@ -122,7 +132,8 @@ struct DevState {
     // kernel that advances a local's position also writes its images' next
     // positions, so no separate ghost refresh runs between steps
     int *img_cnt;        // per physical local
-    int *img_slot;       // [k][cap]: ghost index (physical - nlocal) of image k
+    int4 *img_tab;       // [k][cap]: image k's ghost index (physical - nlocal), its source slot (-1: the
+                         // local itself), its shift (2 bits per dimension, + 1)
     int img_on;          // host: every local's images fit IMG_MAX
     int *tile_cnt;
     int *counters;
@@ -137,7 +148,7 @@ void launch_fill_i32(hipStream_t s, int *p, int v, int n);
 void launch_pack_p(hipStream_t s, const DevState &d, int cur);
 // waves of the force kernels: 64 locals each
 int force_waves(const DevState &d);
-// waves of the fused LJ force kernel (two lanes per local: 32 locals per wave)
+// waves of the timestep's LJ force kernel (two to 32 lanes per local)
 int lj_waves(const DevState &d);
 // the older API's modules (examples/lj_onetype.py): forces with its pair
 // expression (full lists), and its Euler update in the current buffer
@@ -220,6 +231,7 @@ void launch_thermo_reduce(hipStream_t s, const DevState &d, int nb_ke, int nb_f,
 // every argument of the full-list force kernel (one system)
 struct LJArgs {
     const int *counters;
+    int nlocal, rows;    // locals; allocated list rows of each part
     Geom g;
     const int *lstart, *gstart;
     const double *X, *Y, *Z;

@@ -7,10 +7,16 @@
 
 namespace pk {
 
-__device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    return v;
+// the largest v of the wave, as a uniform value: DPP row steps and row
+// broadcasts (a value >= 0)
+__device__ __forceinline__ int wave_max_uniform(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));  // row_shr 1, 2, 4, 8
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false));  // row_bcast 15
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false));  // row_bcast 31
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
 struct SegInfo {
@@ -129,8 +135,8 @@ __device__ __forceinline__ void list_walk32(const uint32_t *__restrict__ nl, int
 #pragma unroll
         for (int q = 0; q < G; q++) {
             j[4 * q + 0] = min(r.v[q].x, jmax);
-            j[4 * q + 1] = min(r.v[q].y, jmax);
-            j[4 * q + 2] = min(r.v[q].z, jmax);
+            j[4 * q + 2] = min(r.v[q].y, jmax);  // (a group holds its entries as 0, 2, 1, 3)
+            j[4 * q + 1] = min(r.v[q].z, jmax);
             j[4 * q + 3] = min(r.v[q].w, jmax);
         }
         body(k, j);
@@ -149,6 +155,9 @@ __device__ __forceinline__ void list_walk32(const uint32_t *__restrict__ nl, int
     }
 }
 
+// the fourth word of a packed position record: the particle's type (0.0 for type 0)
+__device__ __forceinline__ double type_w(int t) { return __longlong_as_double((long long) t); }
+
 // Next positions of local i's images (the stale multi-hop refresh of
 // src/pairs/sim/comm.py:45-54,369-442 one step early): an image of i itself
 // is i's new position + shift, an image of a ghost is that ghost's current
@@ -157,20 +166,20 @@ __device__ __forceinline__ void write_images(const Images &im, int i, int nlocal
                                              const double *__restrict__ X, const double *__restrict__ Y,
                                              const double *__restrict__ Z, double *__restrict__ Xn,
                                              double *__restrict__ Yn, double *__restrict__ Zn, const Geom &g,
-                                             double4 *__restrict__ Pn = nullptr) {
+                                             double4 *__restrict__ Pn, double tw) {
     const int n = min(im.cnt[i], IMG_MAX);
     for (int k = 0; k < n; k++) {
-        const int q = im.slot[(size_t) k * im.cap + i];
-        const int src = im.src[q];
-        const bool own = src == i;
+        const int4 t = im.tab[(size_t) k * im.cap + i];
+        const int q = t.x, src = t.y;
+        const bool own = src < 0;
         const double bx = own ? px : X[src], by = own ? py : Y[src], bz = own ? pz : Z[src];
-        const double x = bx + (double) im.mult[3 * q + 0] * g.len[0];
-        const double y = by + (double) im.mult[3 * q + 1] * g.len[1];
-        const double z = bz + (double) im.mult[3 * q + 2] * g.len[2];
+        const double x = bx + (double) ((t.z & 3) - 1) * g.len[0];
+        const double y = by + (double) (((t.z >> 2) & 3) - 1) * g.len[1];
+        const double z = bz + (double) (((t.z >> 4) & 3) - 1) * g.len[2];
         Xn[nlocal + q] = x;
         Yn[nlocal + q] = y;
         Zn[nlocal + q] = z;
-        if (Pn) Pn[nlocal + q] = make_double4(x, y, z, 0.0);
+        if (Pn) Pn[nlocal + q] = make_double4(x, y, z, tw);
     }
 }
 

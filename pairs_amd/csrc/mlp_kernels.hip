@@ -249,7 +249,7 @@ struct MLPSegArgs {
     // next positions and images if vv1)
     int vv, vv2, vv1;
     double dt, hdt;
-    const int *flags;
+    const int *flags, *type;
     const double *mass;
     double *vx, *vy, *vz;
     double *Xn, *Yn, *Zn;
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
         const bool live = i < nlocal;
         const int ii = live ? i : i0;
         const int n = live ? min(A.numneighs[ii], A.ncap) : 0;
-        const int nmax = __builtin_amdgcn_readfirstlane(wave_max(n));
+        const int nmax = wave_max_uniform(n);
         const double xi = A.X[ii], yi = A.Y[ii], zi = A.Z[ii];
         float acc[MLP_ND], di[MLP_ND];
 #pragma unroll
@@ -313,7 +313,8 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
 #pragma unroll
             for (int q = 0; q < U; q++) {
                 const int c = L * q + h;
-                const uint32_t e = (c & 2) ? ((c & 1) ? grp.w : grp.z) : ((c & 1) ? grp.y : grp.x);
+                // (a group holds its entries as 0, 2, 1, 3)
+                const uint32_t e = (c & 2) ? ((c & 1) ? grp.w : grp.y) : ((c & 1) ? grp.z : grp.x);
                 jq[q] = min(e, jmax);
             }
             double xj[U], yj[U], zj[U];
@@ -456,10 +457,11 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
                     }
                     if (A.vv1) {
                         A.Xn[i] = px; A.Yn[i] = py; A.Zn[i] = pz;
-                        if (A.Pn) A.Pn[i] = make_double4(px, py, pz, 0.0);
+                        const double tw = type_w(A.type[i]);
+                        if (A.Pn) A.Pn[i] = make_double4(px, py, pz, tw);
                         if (A.im.on)
                             write_images(A.im, i, A.counters[C_NLOCAL], px, py, pz, A.X, A.Y, A.Z, A.Xn, A.Yn, A.Zn,
-                                         A.g, A.Pn);
+                                         A.g, A.Pn, tw);
                     }
                 }
             }
@@ -1025,7 +1027,7 @@ void launch_mlp_forces(hipStream_t s, const DevState &d, const Geom &g, const ML
         A.vv = 1;
         A.vv2 = vv->vv2; A.vv1 = vv->vv1;
         A.dt = vv->prm->dt; A.hdt = vv->prm->hdt;
-        A.flags = d.flags; A.mass = d.mass;
+        A.flags = d.flags; A.type = d.type; A.mass = d.mass;
         A.vx = d.vx; A.vy = d.vy; A.vz = d.vz;
         A.Xn = d.X[vv->next]; A.Yn = d.Y[vv->next]; A.Zn = d.Z[vv->next];
         A.im = images_of(d, vv->vv1 && vv->next != cur);

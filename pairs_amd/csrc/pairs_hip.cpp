@@ -92,13 +92,11 @@ static void dfree(void *p) {
     if (p) hipFree(p);
 }
 
-// rows of the per-wave partials (force waves of 64 locals; blocks of 256 of
-// the stand-alone integrator)
-// one partial per wave of the reduction kernels: the fewest locals per wave
-// is 16 (the MLP list passes of a small system, four lanes per local)
+// row stride of the per-wave partials: the fewest locals per wave is 2 (the
+// force kernel of a small system, 32 lanes per local)
 static size_t pstride_of(const DevState &d, const Geom &g) {
     (void) g;
-    return (size_t) d.cap / 16 + 8;
+    return (size_t) d.cap / 2 + 8;
 }
 
 static void free_particle_arrays(DevState &d) {
@@ -109,8 +107,10 @@ static void free_particle_arrays(DevState &d) {
     for (auto p : dd) { dfree(*p); *p = nullptr; }
     int **ii[] = {&d.type, &d.flags, &d.uid, &d.shape, &d.ref, &d.phys, &d.alt_type, &d.alt_flags, &d.alt_uid,
                   &d.alt_shape, &d.alt_ref, &d.alt_cell, &d.numneighs, &d.particle_cell, &d.slot, &d.perm,
-                  &d.exchg_flag, &d.tile_cnt, &d.sync_src, &d.sync_mult, &d.img_cnt, &d.img_slot, &d.nrev};
+                  &d.exchg_flag, &d.tile_cnt, &d.sync_src, &d.sync_mult, &d.img_cnt, &d.nrev};
     for (auto p : ii) { dfree(*p); *p = nullptr; }
+    dfree(d.img_tab);
+    d.img_tab = nullptr;
 }
 
 static int alloc_particle_arrays(pairs_hip_ctx *ctx, DevState &d, int cap) {
@@ -126,7 +126,7 @@ static int alloc_particle_arrays(pairs_hip_ctx *ctx, DevState &d, int cap) {
     for (auto p : ii) r |= dalloc(ctx, p, cap);
     r |= dalloc(ctx, &d.sync_mult, 3 * (size_t) cap);
     r |= dalloc(ctx, &d.img_cnt, cap);
-    r |= dalloc(ctx, &d.img_slot, (size_t) IMG_MAX * cap);
+    r |= dalloc(ctx, &d.img_tab, (size_t) IMG_MAX * cap);
     r |= dalloc(ctx, &d.tile_cnt, 2 * ((size_t) cap / 256 + 2));
     d.cap = cap;
     d.pstride = (int) pstride_of(d, ctx->geom);
@@ -140,7 +140,7 @@ static int alloc_neighbor_arrays(pairs_hip_ctx *ctx, DevState &d, int ncap) {
     d.nl = nullptr;
     d.nl_stride = d.cap;
     // half lists: as many rows again for the mirror parts
-    const int rows = (ncap + 3) / 4 * 4;
+    const int rows = list_rows(ncap);
     d.rev0 = ctx->cfg.half ? rows : 0;
     if (dalloc(ctx, &d.nl, (size_t) rows * (ctx->cfg.half ? 2 : 1) * d.nl_stride)) return PAIRS_HIP_ERR_HIP;
     d.ncap = ncap;
