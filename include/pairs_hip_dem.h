@@ -165,7 +165,9 @@ int pairs_hip_dem_set_timing(pairs_hip_dem_ctx *ctx, int every_n);
 int pairs_hip_dem_contact_kernel_time(pairs_hip_dem_ctx *ctx, double *avg_ms, int *launches);
 /* The same timed steps split into phases, avg_ms[6]: prepare (exchange,
    borders, cell lists), contact search, history slots, spring-dashpot per
-   contact, per-particle sums + history clean-up, euler.
+   contact, per-particle sums + history clean-up, euler.  Slots to clean-up
+   are one kernel, timed as the spring-dashpot phase: the slot and sum phases
+   read about zero.
    No reference counterpart (the reference's timers are host-side). */
 int pairs_hip_dem_phase_times(pairs_hip_dem_ctx *ctx, double *avg_ms);
 

@@ -91,8 +91,8 @@ static void free_arrays(DemPtrs &p) {
     void *ptrs[] = {p.x, p.y, p.z, p.vx, p.vy, p.vz, p.wx, p.wy, p.wz, p.fx, p.fy, p.fz, p.tx, p.ty, p.tz, p.r, p.m,
                     p.nx, p.ny, p.nz, p.inv_i, p.rot_m, p.rot_q, p.uid, p.flags, p.type, p.shape, p.num_contacts,
                     p.c_uid, p.c_used, p.c_stick, p.c_tsd, p.c_ivm, p.cell_count, p.cell_start, p.cell_slot,
-                    p.cell_particles, p.particle_cell, p.nshapes, p.send_map, p.send_mult, p.exchg_flag, p.copy_to,
-                    p.blk, p.scan_tmp, p.buf, p.hbuf, p.cand_n, p.cand, p.cslot, p.cf};
+                    p.cell_particles, p.particle_cell, p.corder, p.cmixed, p.crec, p.rec, p.send_map, p.send_mult, p.exchg_flag, p.copy_to,
+                    p.blk, p.scan_tmp, p.buf, p.hbuf, p.cand_n, p.cand};
     for (void *q : ptrs)
         if (q) hipFree(q);
     const int cap = p.cap, ccap = p.ccap, send_cap = p.send_cap;
@@ -130,7 +130,6 @@ static int alloc_arrays(pairs_hip_dem_ctx *ctx, DemPtrs &p, size_t C, size_t K, 
     const size_t NC = (size_t) ctx->ncells_cap;
     r |= dalloc(ctx, &p.cell_count, NC + 1);
     r |= dalloc(ctx, &p.cell_start, NC + 1);
-    r |= dalloc(ctx, &p.nshapes, 2 * NC);
     r |= dalloc(ctx, &p.cell_particles, C);
     r |= dalloc(ctx, &p.scan_tmp, NC / 1024 + 8);
     r |= dalloc(ctx, &p.send_map, S);
@@ -141,8 +140,10 @@ static int alloc_arrays(pairs_hip_dem_ctx *ctx, DemPtrs &p, size_t C, size_t K, 
     r |= dalloc(ctx, &p.hbuf, (2 + 5 * K) * S);
     r |= dalloc(ctx, &p.cand_n, C);
     r |= dalloc(ctx, &p.cand, DCAND * C);
-    r |= dalloc(ctx, &p.cslot, DCAND * C);
-    r |= dalloc(ctx, &p.cf, 6 * DCAND * C);
+    r |= dalloc(ctx, &p.corder, C);
+    r |= dalloc(ctx, &p.cmixed, C);
+    r |= dalloc(ctx, &p.crec, C);
+    r |= dalloc(ctx, &p.rec, C);
     return r ? -1 : 0;
 }
 
@@ -517,7 +518,8 @@ static void enqueue_step(pairs_hip_dem_ctx *ctx, bool timed) {
     if (timed) hipEventRecord(ctx->ev[0], ctx->stream);
     launch_prepare(ctx->stream, ctx->p, ctx->counters, ctx->geom);
     if (timed) hipEventRecord(ctx->ev[1], ctx->stream);
-    launch_contacts(ctx->stream, ctx->p, ctx->counters, ctx->geom, ctx->prm, timed ? ctx->ev + 2 : nullptr);
+    launch_contacts(ctx->stream, ctx->p, ctx->counters, ctx->nlocal, ctx->geom, ctx->prm,
+                    timed ? ctx->ev + 2 : nullptr);
     if (timed) hipEventRecord(ctx->ev[5], ctx->stream);
     launch_euler(ctx->stream, ctx->p, ctx->counters, ctx->prm);
     if (timed) hipEventRecord(ctx->ev[6], ctx->stream);

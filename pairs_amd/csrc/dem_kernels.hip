@@ -408,13 +408,17 @@ __global__ __launch_bounds__(256) void k_cell_count(DemPtrs p, const int *__rest
     p.cell_slot[i] = atomicAdd(&p.cell_count[cell], 1);  // its place among the cell's entries
 }
 
-// exclusive scan of cell counts: block partials, then each block adds its offset
-__global__ __launch_bounds__(1024) void k_scan_partial(const int *__restrict__ in, int *__restrict__ out,
+// exclusive scan of cell counts: block partials, then each block adds its
+// offset; the counts are cleared behind the reads (nothing else uses them, so
+// the next binning starts from zeros)
+__global__ __launch_bounds__(1024) void k_scan_partial(int *__restrict__ in, int *__restrict__ out,
                                                        int *__restrict__ bsum, int n) {
     __shared__ int lds[20];
     const int i = blockIdx.x * 1024 + threadIdx.x;
     int t;
-    const int e = block_scan_excl<1024>(i < n ? in[i] : 0, lds, &t);
+    const int v = i < n ? in[i] : 0;
+    if (v) in[i] = 0;
+    const int e = block_scan_excl<1024>(v, lds, &t);
     if (i < n) out[i] = e;
     if (threadIdx.x == 0) bsum[blockIdx.x] = t;
 }
@@ -444,16 +448,11 @@ __global__ __launch_bounds__(256) void k_cell_fill(DemPtrs p, const int *__restr
     p.cell_particles[p.cell_start[cell] + p.cell_slot[i]] = i;
 }
 
-// per cell: index order (the CPU's insertion order), then PartitionCellLists
-// (cell_lists.py:137-171): in-place two-pointer partition by shape,
-// spheres then half-spaces
-__global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, int ncells) {
-    const int cell = blockIdx.x * 256 + threadIdx.x;
-    if (cell >= ncells) return;
-    const int s0 = p.cell_start[cell], cnt = p.cell_count[cell];
-    // the counts are not used after this pass: cleared for the next binning
-    p.cell_count[cell] = 0;
-    int *cp = p.cell_particles + s0;
+// PartitionCellLists (src/pairs/sim/cell_lists.py:137-171) of one cell, whose
+// entries cp[0, cnt) come in any order: index order (the CPU's insertion
+// order), then the in-place two-pointer partition by shape, spheres then
+// half-spaces
+__device__ __forceinline__ void partition_cell(const int *__restrict__ shape, int *cp, int cnt) {
     for (int a = 1; a < cnt; a++) {
         const int v = cp[a];
         int b = a - 1;
@@ -462,19 +461,79 @@ __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, int ncells) {
     }
     int lo = 0;
     for (int sh = 0; sh < 2; sh++) {
-        const int first = lo;
-        int hi = cnt - 1, ns = 0;
+        int hi = cnt - 1;
         while (lo <= hi) {
             const int q = cp[lo];
-            if (p.shape[q] != sh) {
+            if (shape[q] != sh) {
                 if (lo != hi) { cp[lo] = cp[hi]; cp[hi] = q; }
                 hi--;
             } else {
                 lo++;
-                ns = lo - first;
             }
         }
-        p.nshapes[2 * cell + sh] = ns;
+    }
+}
+
+// One thread per particle: its place in its cell's order, and the records the
+// contact kernels read -- by place: index, cell (bit 31: FIXED) and (x, y, z,
+// r); by index: everything a contact needs of its partner in one 128-byte line
+// (a gather of twelve arrays touches twelve lines).  In a cell of spheres the
+// order is the index order, so a particle's place is the number of smaller
+// indices in the cell; a cell that holds a half-space is ordered by the thread
+// of its first particle and written by it.  Bound by memory: 100 bytes in and
+// 136 out per particle, the records through LDS so that a wave writes whole
+// lines (13 us at 190000 particles; 42 with each thread storing its record).
+__global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__restrict__ c) {
+    constexpr int W = 13;  // LDS row of a record (doubles, one of padding)
+    __shared__ double s_rec[256 * W];
+    const int n = c[D_NLOCAL] + c[D_NGHOST];
+    const int b0 = blockIdx.x * 256;
+    const int i = b0 + threadIdx.x;
+    if (b0 >= n) return;
+    int sh = DSHAPE_SPHERE;
+    double x = 0.0, y = 0.0, z = 0.0, r = 0.0;
+    if (i < n) {
+        sh = p.shape[i];
+        x = p.x[i]; y = p.y[i]; z = p.z[i]; r = p.r[i];
+        double *R = s_rec + threadIdx.x * W;
+        R[0] = x; R[1] = y; R[2] = z; R[3] = r;
+        R[4] = p.vx[i]; R[5] = p.vy[i]; R[6] = p.vz[i]; R[7] = p.m[i];
+        R[8] = p.wx[i]; R[9] = p.wy[i]; R[10] = p.wz[i];
+        R[11] = __longlong_as_double((long long) p.uid[i] << 32 | (unsigned) p.type[i]);
+    }
+    __syncthreads();
+    // the block's records, 16 bytes per thread at consecutive addresses
+    const int nb = min(256, n - b0);
+    for (int u = threadIdx.x; u < 6 * nb; u += 256) {
+        const int k = u / 6, w = u - 6 * k;
+        const double *R = s_rec + k * W + 2 * w;
+        ((double2 *) (p.rec + b0 + k))[w] = make_double2(R[0], R[1]);
+    }
+    if (i >= n) return;
+    const int cell = p.particle_cell[i];
+    const int s0 = p.cell_start[cell], cnt = p.cell_start[cell + 1] - s0;
+    int rank = 0;
+    bool mixed = sh != DSHAPE_SPHERE;
+    if (cnt > 1)
+        for (int k = 0; k < cnt; k++) {
+            const int j = p.cell_particles[s0 + k];
+            rank += j < i ? 1 : 0;
+            mixed = mixed || p.shape[j] != DSHAPE_SPHERE;
+        }
+    auto put = [&](int q, int j, double jx, double jy, double jz, double jr, int jsh) {
+        p.corder[q] = make_int2(j, cell | ((p.flags[j] & DFLAG_FIXED) ? (int) 0x80000000 : 0));
+        p.crec[q] = make_double4(jx, jy, jz, jsh == DSHAPE_SPHERE ? jr : -1.0);
+    };
+    if (!mixed) {
+        put(s0 + rank, i, x, y, z, r, sh);
+    } else if (rank == 0) {
+        int *cp = p.cmixed + s0;
+        for (int k = 0; k < cnt; k++) cp[k] = p.cell_particles[s0 + k];
+        partition_cell(p.shape, cp, cnt);
+        for (int k = 0; k < cnt; k++) {
+            const int j = cp[k];
+            put(s0 + k, j, p.x[j], p.y[j], p.z[j], p.r[j], p.shape[j]);
+        }
     }
 }
 
@@ -483,16 +542,17 @@ __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, int ncells) {
 struct Acc3 { double x, y, z; };
 
 // linear_spring_dashpot (examples/dem.py:18-74) for one contact: normal n,
-// penetration delta, contact point cp, history slot k; updates the slot and
+// penetration delta, contact point cp, history slot k (fresh: a new slot, whose
+// history is zero and is not read); updates the slot and
 // returns the contact's force F and torque term T = (cp - x_i) x F
-__device__ __forceinline__ void spring_dashpot(const DemPtrs &p, const DemParams &prm, int i, int j, int k,
-                                               const double n[3], double delta, const double cp[3], double F[3],
-                                               double T[3]) {
+__device__ __forceinline__ void spring_dashpot(const DemPtrs &p, const DemParams &prm, const DemRec &ri,
+                                               const DemRec &rj, int i, int k, bool fresh, const double n[3],
+                                               double delta, const double cp[3], double F[3], double T[3]) {
     const size_t a = (size_t) k * p.cap + i;
-    const bool sticking = p.c_stick[a] == 1;
-    const double xi[3] = {p.x[i], p.y[i], p.z[i]}, xj[3] = {p.x[j], p.y[j], p.z[j]};
-    const double vi[3] = {p.vx[i], p.vy[i], p.vz[i]}, vj[3] = {p.vx[j], p.vy[j], p.vz[j]};
-    const double wi[3] = {p.wx[i], p.wy[i], p.wz[i]}, wj[3] = {p.wx[j], p.wy[j], p.wz[j]};
+    const bool sticking = !fresh && p.c_stick[a] == 1;
+    const double xi[3] = {ri.x, ri.y, ri.z}, xj[3] = {rj.x, rj.y, rj.z};
+    const double vi[3] = {ri.vx, ri.vy, ri.vz}, vj[3] = {rj.vx, rj.vy, rj.vz};
+    const double wi[3] = {ri.wx, ri.wy, ri.wz}, wj[3] = {rj.wx, rj.wy, rj.wz};
     double ai[3], aj[3], rel[3], reln[3], relt[3];
     for (int d = 0; d < 3; d++) { ai[d] = cp[d] - xi[d]; aj[d] = cp[d] - xj[d]; }
     double vwi[3], vwj[3];
@@ -507,13 +567,16 @@ __device__ __forceinline__ void spring_dashpot(const DemPtrs &p, const DemParams
     for (int d = 0; d < 3; d++) { reln[d] = rn * n[d]; relt[d] = rel[d] - reln[d]; }
     const double relt_len = sqrt((relt[0] * relt[0] + relt[1] * relt[1]) + relt[2] * relt[2]);
     const bool cond_a = sticking && relt_len < 1e-08;
-    const double meff = 1.0 / (1.0 / p.m[i] + 1.0 / p.m[j]);
+    const double meff = 1.0 / (1.0 / ri.m + 1.0 / rj.m);
     // stiffness from the collision time (examples/dem.py:34-35), or fixed
     const double kn = prm.kn_fixed > 0.0 ? prm.kn_fixed
                                          : (meff * (prm.pi * prm.pi + prm.ln_e * prm.ln_e)) / (prm.t_c * prm.t_c);
     const double kt = prm.kappa * kn;
-    const double h[3] = {p.c_tsd[3 * (size_t) k * p.cap + i], p.c_tsd[(3 * (size_t) k + 1) * p.cap + i],
-                         p.c_tsd[(3 * (size_t) k + 2) * p.cap + i]};
+    double h[3] = {0.0, 0.0, 0.0}, iv = 0.0;
+    if (!fresh) {
+        for (int d = 0; d < 3; d++) h[d] = p.c_tsd[(3 * (size_t) k + d) * p.cap + i];
+        iv = p.c_ivm[a];
+    }
     const double hn = (h[0] * n[0] + h[1] * n[1]) + h[2] * n[2];
     double rot[3], ntsd[3];
     for (int d = 0; d < 3; d++) rot[d] = h[d] - n[d] * hn;
@@ -529,7 +592,7 @@ __device__ __forceinline__ void spring_dashpot(const DemPtrs &p, const DemParams
     double ftls[3];
     for (int d = 0; d < 3; d++) ftls[d] = kt * ntsd[d] + dtan * relt[d];
     const double ftls_len = sqrt((ftls[0] * ftls[0] + ftls[1] * ftls[1]) + ftls[2] * ftls[2]);
-    const int tk = p.type[i] * prm.ntypes + p.type[j];
+    const int tk = ri.type * prm.ntypes + rj.type;
     double fn[3];
     for (int d = 0; d < 3; d++) fn[d] = (kn * delta) * n[d] + dn * reln[d];
     const double fn_len = sqrt((fn[0] * fn[0] + fn[1] * fn[1]) + fn[2] * fn[2]);
@@ -545,7 +608,6 @@ __device__ __forceinline__ void spring_dashpot(const DemPtrs &p, const DemParams
     for (int d = 0; d < 3; d++)
         p.c_tsd[(3 * (size_t) k + d) * p.cap + i] = slide ? (f_fric * tdir[d] - dtan * relt[d]) / kt : ntsd[d];
     const double rel_len = sqrt((rel[0] * rel[0] + rel[1] * rel[1]) + rel[2] * rel[2]);
-    const double iv = p.c_ivm[a];
     p.c_ivm[a] = (iv > 0.0) ? iv : rel_len;
     p.c_stick[a] = ((cond1 || cond2) || ftls_len < f_dynamic) ? 1 : 0;
     const double ft_abs = (f_fric < ftls_len) ? f_fric : ftls_len;
@@ -589,39 +651,45 @@ __device__ __forceinline__ int contact_slot(const DemPtrs &p, int *c, int i, int
     return slot;
 }
 
-// contact test of i (position xi, radius ri) against candidate j of the given
-// pass (0: sphere, 1: half-space), as linear_spring_dashpot's guard
-// (examples/dem.py:18-30 with the sphere/half-space geometry of
-// src/pairs/sim/interaction.py); on contact fills the normal, the contact
-// point and the penetration depth
-__device__ __forceinline__ bool contact_geom(const DemPtrs &p, const double xi[3], double ri, int j, int pass,
-                                             double nv[3], double cpt[3], double &delta) {
-    const double xj[3] = {p.x[j], p.y[j], p.z[j]};
-    if (pass == 0) {
-        const double d[3] = {xi[0] - xj[0], xi[1] - xj[1], xi[2] - xj[2]};
-        const double rsq = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
-        const double rj = p.r[j];
-        const double rs = ri + rj;
-        if (!(rsq < rs * (rs + 0.0))) return false;
-        const double dist = sqrt(rsq);
-        const double pen = (dist - ri) - rj;
-        delta = -(pen);
-        if (delta < 0.0) return false;
-        const double inv = 1.0 / dist;
-        for (int e = 0; e < 3; e++) nv[e] = d[e] * inv;
-        const double reach = rj + 0.5 * pen;
-        for (int e = 0; e < 3; e++) cpt[e] = xj[e] + nv[e] * reach;
-    } else {
-        const double nj[3] = {p.nx[j], p.ny[j], p.nz[j]};
-        const double pen = (((nj[0] * xi[0] + nj[1] * xi[1]) + nj[2] * xi[2]) - ri) -
-                           ((nj[0] * xj[0] + nj[1] * xj[1]) + nj[2] * xj[2]);
-        if (!(pen < 0.0)) return false;
-        delta = -(pen);
-        if (delta < 0.0) return false;
-        const double reach = ri + pen;
-        for (int e = 0; e < 3; e++) { nv[e] = nj[e]; cpt[e] = xi[e] - reach * nj[e]; }
-    }
+// contact test of i (position xi, radius ri) against a sphere (xj, rj), as
+// linear_spring_dashpot's guard (examples/dem.py:18-30 with the sphere
+// geometry of src/pairs/sim/interaction.py); on contact fills the normal, the
+// contact point and the penetration depth
+__device__ __forceinline__ bool sphere_contact(const double xi[3], double ri, const double xj[3], double rj,
+                                               double nv[3], double cpt[3], double &delta) {
+    const double d[3] = {xi[0] - xj[0], xi[1] - xj[1], xi[2] - xj[2]};
+    const double rsq = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
+    const double rs = ri + rj;
+    if (!(rsq < rs * (rs + 0.0))) return false;
+    const double dist = sqrt(rsq);
+    const double pen = (dist - ri) - rj;
+    delta = -(pen);
+    if (delta < 0.0) return false;
+    const double inv = 1.0 / dist;
+    for (int e = 0; e < 3; e++) nv[e] = d[e] * inv;
+    const double reach = rj + 0.5 * pen;
+    for (int e = 0; e < 3; e++) cpt[e] = xj[e] + nv[e] * reach;
     return true;
+}
+
+// the same against half-space j at xj
+__device__ __forceinline__ bool plane_contact(const DemPtrs &p, const double xi[3], double ri, int j,
+                                              const double xj[3], double nv[3], double cpt[3], double &delta) {
+    const double nj[3] = {p.nx[j], p.ny[j], p.nz[j]};
+    const double pen = (((nj[0] * xi[0] + nj[1] * xi[1]) + nj[2] * xi[2]) - ri) -
+                       ((nj[0] * xj[0] + nj[1] * xj[1]) + nj[2] * xj[2]);
+    if (!(pen < 0.0)) return false;
+    delta = -(pen);
+    if (delta < 0.0) return false;
+    const double reach = ri + pen;
+    for (int e = 0; e < 3; e++) { nv[e] = nj[e]; cpt[e] = xi[e] - reach * nj[e]; }
+    return true;
+}
+
+__device__ __forceinline__ bool contact_geom(const DemPtrs &p, const double xi[3], double ri, int j, const DemRec &rj,
+                                             int pass, double nv[3], double cpt[3], double &delta) {
+    const double xj[3] = {rj.x, rj.y, rj.z};
+    return pass == 0 ? sphere_contact(xi, ri, xj, rj.r, nv, cpt, delta) : plane_contact(p, xi, ri, j, xj, nv, cpt, delta);
 }
 
 // Candidates of i in the reference's visiting order: the spheres of cell 0
@@ -634,12 +702,9 @@ __device__ __forceinline__ void walk_candidates(const DemPtrs &p, const DemGeom 
         for (int s = -1; s < 27; s++) {
             const int cell = s < 0 ? 0 : ci + g.stencil[s];
             if (!(s < 0 || (cell > 0 && cell < g.ncells))) continue;
-            const int st = p.cell_start[cell], nsph = p.nshapes[2 * cell];
-            const int q0 = pass == 0 ? 0 : nsph;
-            const int q1 = pass == 0 ? nsph : nsph + p.nshapes[2 * cell + 1];
-            for (int q = q0; q < q1; q++) {
-                const int j = p.cell_particles[st + q];
-                if (j == i) continue;
+            for (int q = p.cell_start[cell]; q < p.cell_start[cell + 1]; q++) {
+                const int j = p.corder[q].x;
+                if (j == i || p.shape[j] != pass) continue;
                 if (!fn(j, pass)) return;
             }
         }
@@ -658,181 +723,242 @@ __device__ __forceinline__ int group_scan(int x) {
     return x;
 }
 
-// Contact search, LPS lanes per local particle.  The visiting order's 28
-// cells (cell 0, then the 27 stencil cells) are dealt to the lanes in
-// contiguous runs of CPL = ceil(28 / LPS).  Each lane counts the touching
-// spheres and half-spaces of its cells; prefix sums over the lanes give every
-// hit its place in the reference's visiting order (the spheres of cell 0 and
-// of the stencil cells, then the half-spaces of the same cells;
-// cell_lists.py partitions each cell spheres-first), and a second walk stores
-// them as cand[t][i] (half-spaces as ~j), from a bit mask of the lane's
-// first 32 candidates (beyond them the geometry test is repeated).
-// cand_n[i] = DCAND + 1 when more than DCAND touch (the force pass then walks
-// the cells itself).  Only geometry is read: no history is touched.
-template <int LPS>
+// Contact search, LPS lanes per local sphere, spheres in cell order (the
+// groups of a wave are neighbours and read the same records).  The visiting
+// order's 28 cells (cell 0, then the 27 stencil cells) are ten runs of the
+// cell order: cell 0, and the three cells of each of the nine z-columns, which
+// are consecutive.  Lane 0 takes cell 0 and column 0, lanes 1 to 6 a column
+// each, lane 7 columns 7 and 8.  Each lane counts the touching spheres and
+// half-spaces of its runs; prefix sums over the lanes give every hit its place
+// in the visiting order (all spheres, then all half-spaces), and the hits are
+// stored from a bit mask of the lane's first 32 candidates (beyond them the
+// test is repeated) as cand[i][t] (half-spaces as ~j).
+// cand_n[i] = DCAND + 1 when more than DCAND touch (the contact kernel then
+// walks the cells itself).  Only geometry is read: no history is touched.
+// Bound by the latency of its three dependent loads (place, run bounds,
+// candidates); the candidates of a run are consecutive 32-byte records.  By
+// particle index, cell by cell and from four arrays it took 105 us in a bed of
+// 187200 spheres and 59 us on the falling 200000; now 41 and 28.
+constexpr int LPS = 8;
 __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__restrict__ c, DemGeom g) {
-    constexpr int CPL = (28 + LPS - 1) / LPS;
     if (c[D_OVF]) return;
-    const int nl = c[D_NLOCAL];
-    const int i = (blockIdx.x * 256 + threadIdx.x) / LPS;
+    const int nl = c[D_NLOCAL], n = nl + c[D_NGHOST];
+    const int q0 = (blockIdx.x * 256 + threadIdx.x) / LPS;
     const int l = threadIdx.x & (LPS - 1);
-    const bool act = i < nl;
-    const int ii = act ? i : 0;
-    const bool fixed = !act || (p.flags[ii] & DFLAG_FIXED);
-    // this lane's cells: start, sphere count, candidate count, and the
-    // offset of each cell's candidates in the lane's sequence
-    int cst[CPL], csph[CPL], cn[CPL], cbase[CPL + 1];
-    const int ci = fixed ? 0 : p.particle_cell[ii];
-    cbase[0] = 0;
-#pragma unroll
-    for (int u = 0; u < CPL; u++) {
-        const int k = l * CPL + u;
-        cst[u] = 0; csph[u] = 0; cn[u] = 0;
-        if (!fixed && k < 28) {
-            const int cell = k == 0 ? 0 : ci + g.stencil[k - 1];
-            if (k == 0 || (cell > 0 && cell < g.ncells)) {
-                cst[u] = p.cell_start[cell];
-                const int2 ns = reinterpret_cast<const int2 *>(p.nshapes)[cell];
-                csph[u] = ns.x;
-                cn[u] = ns.x + ns.y;
-            }
+    const bool in = q0 < n;
+    const int qi = in ? q0 : 0;
+    const int2 own = p.corder[qi];
+    const int i = own.x, cc = own.y;
+    const double4 me = p.crec[qi];
+    const bool act = in && i < nl, look = act && cc >= 0;
+    const int ci = cc & 0x7fffffff;
+    // the lane's two runs [st, st + len)
+    int st[2] = {0, 0}, len[2] = {0, 0};
+    auto column = [&](int col, int &s0, int &ln) {
+        const int base = ci + g.stencil[3 * col + 1];
+        const int lo = max(base - 1, 1), hi = min(base + 1, g.ncells - 1);
+        if (lo <= hi) {
+            s0 = p.cell_start[lo];
+            ln = p.cell_start[hi + 1] - s0;
         }
-        cbase[u + 1] = cbase[u] + cn[u];
+    };
+    if (look) {
+        if (l == 0) { st[0] = p.cell_start[0]; len[0] = p.cell_start[1] - st[0]; }
+        column(l, st[1], len[1]);
+        if (l == LPS - 1) {
+            st[0] = st[1]; len[0] = len[1];
+            column(LPS, st[1], len[1]);
+        }
     }
-    const double ri = p.r[ii];
-    const double xi[3] = {p.x[ii], p.y[ii], p.z[ii]};
+    const double xi[3] = {me.x, me.y, me.z};
+    const double ri = me.w;
+    const int tot = len[0] + len[1];
+    auto place = [&](int b) { return b < len[0] ? st[0] + b : st[1] + (b - len[0]); };
+    // 0: no contact, 1: sphere, 2: half-space
+    auto touch = [&](int q, const double4 &r) {
+        double nv[3], cpt[3], delta;
+        const double xj[3] = {r.x, r.y, r.z};
+        if (r.w >= 0.0) return q != qi && sphere_contact(xi, ri, xj, r.w, nv, cpt, delta) ? 1 : 0;
+        const int j = p.corder[q].x;
+        return q != qi && plane_contact(p, xi, ri, j, xj, nv, cpt, delta) ? 2 : 0;
+    };
     int hs = 0, hh = 0;
     unsigned hit = 0u;
-#pragma unroll
-    for (int u = 0; u < CPL; u++)
-        for (int q = 0; q < cn[u]; q++) {
-            const int j = p.cell_particles[cst[u] + q];
-            const bool sph = q < csph[u];
-            double nv[3], cpt[3], delta;
-            if (j != ii && contact_geom(p, xi, ri, j, sph ? 0 : 1, nv, cpt, delta)) {
-                if (sph) hs++; else hh++;
-                const int b = cbase[u] + q;
-                if (b < 32) hit |= 1u << b;
-            }
-        }
+    for (int b = 0; b < tot; b += 2) {
+        const int qa = place(b), qb = place(min(b + 1, tot - 1));
+        const double4 ra = p.crec[qa], rb = p.crec[qb];
+        const int ta = touch(qa, ra), tb = b + 1 < tot ? touch(qb, rb) : 0;
+        hs += (ta == 1) + (tb == 1);
+        hh += (ta == 2) + (tb == 2);
+        if (b < 32) hit |= (unsigned) (ta != 0) << b | (unsigned) (tb != 0) << (b + 1);
+    }
     const int ps = group_scan<LPS>(hs), ph = group_scan<LPS>(hh);
     const int tot_s = __shfl(ps, LPS - 1, LPS), tot_h = __shfl(ph, LPS - 1, LPS);
-    const int n = tot_s + tot_h;
-    if (n <= DCAND) {
+    const int nt = tot_s + tot_h;
+    if (act && nt <= DCAND) {
         int os = ps - hs, oh = tot_s + ph - hh;
+        int *__restrict__ out = p.cand + (size_t) i * DCAND;
         while (hit) {
             const int b = __builtin_ctz(hit);
             hit &= hit - 1u;
-            int u = 0;
-#pragma unroll
-            for (int v = 1; v < CPL; v++) u += b >= cbase[v] ? 1 : 0;
-            int st = cst[0], q = b, sp = csph[0];
-#pragma unroll
-            for (int v = 1; v < CPL; v++)
-                if (u == v) { st = cst[v]; q = b - cbase[v]; sp = csph[v]; }
-            const int j = p.cell_particles[st + q];
-            const int t = q < sp ? os++ : oh++;
-            p.cand[(size_t) t * p.cap + ii] = q < sp ? j : ~j;
+            const int q = place(b), j = p.corder[q].x;
+            if (p.crec[q].w >= 0.0) out[os++] = j;
+            else out[oh++] = ~j;
         }
-        if (cbase[CPL] > 32) {
+        for (int b = 32; b < tot; b++) {
+            const int q = place(b);
+            const int t = touch(q, p.crec[q]);
+            if (t == 1) out[os++] = p.corder[q].x;
+            else if (t == 2) out[oh++] = ~p.corder[q].x;
+        }
+    }
+    if (act && l == 0) p.cand_n[i] = nt <= DCAND ? nt : DCAND + 1;
+}
+
+// The contacts of SPW consecutive local particles, one wave.  The wave's
+// contacts are numbered particle by particle in visiting order and dealt to
+// the lanes densely, 64 at a time, whichever particle they belong to:
+//  1. each contact looks its partner's uid up in its particle's history
+//     (reset_contact_history_usage_status and the slot rule of
+//     src/pairs/mapping/funcs.py:230-270: the last match, or a new slot); the
+//     particle's lane numbers the new slots in order;
+//  2. linear_spring_dashpot per contact, history updated, force and torque
+//     terms through LDS; the particle's lane adds them in contact order, with
+//     the reference's sphere / half-space grouping (force += sphere + plane
+//     sums, torque += plane + sphere sums) on top of gravity;
+//  3. clear_unused_contact_history from the particle's mask of used slots.
+// A particle with more than DCAND touching partners, more history than the
+// mask holds, or two contacts in one slot (a partner and its image) walks its
+// cells in its lane instead, one contact after the other, as the reference.
+// Bound by the gathers of the partners' records (0.9 M of 128 bytes in a bed of
+// 187200 spheres) and the FP64 divisions and roots of the contact law.  One
+// dense pass in place of a kernel per phase: the phases ran one thread per
+// possible contact (16 per particle) or per particle, and gathered a partner
+// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres.
+template <int SPW>
+__global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict__ c, DemGeom g, DemParams prm) {
+    __shared__ double s_term[64][7];
+    __shared__ int s_kind[64];
+    __shared__ int s_off[SPW], s_nc[SPW];
+    __shared__ int s_cand[SPW * DCAND], s_uid[SPW * DCAND], s_slot[SPW * DCAND];
+    __shared__ unsigned char s_own[SPW * DCAND];
+    if (c[D_OVF]) return;
+    const int nl = c[D_NLOCAL];
+    const int i0 = blockIdx.x * SPW, lane = threadIdx.x;
+    if (i0 >= nl) return;
+    const int i = i0 + lane;
+    const bool sph = lane < SPW && i < nl;
+    const size_t C = p.cap;
+    int nc = 0, nt = 0;
+    if (sph) { nc = p.num_contacts[i]; nt = p.cand_n[i]; }
+    const int nc0 = nc;
+    bool slow = nt > DCAND || nc + nt > 64;
+    const int n = slow ? 0 : nt;
+    int off = n;
 #pragma unroll
-            for (int u = 0; u < CPL; u++)
-                for (int q = max(0, 32 - cbase[u]); q < cn[u]; q++) {
-                    const int j = p.cell_particles[cst[u] + q];
-                    const bool sph = q < csph[u];
-                    double nv[3], cpt[3], delta;
-                    if (j != ii && contact_geom(p, xi, ri, j, sph ? 0 : 1, nv, cpt, delta)) {
-                        const int t = sph ? os++ : oh++;
-                        p.cand[(size_t) t * p.cap + ii] = sph ? j : ~j;
-                    }
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(off, o, 64);
+        if (lane >= o) off += y;
+    }
+    const int total = __shfl(off, 63, 64);
+    off -= n;
+    if (lane < SPW) { s_off[lane] = off; s_nc[lane] = nc0; }
+    for (int t = 0; t < n; t++) s_own[off + t] = (unsigned char) lane;
+    __syncthreads();
+    for (int k = lane; k < total; k += 64) {
+        const int s = s_own[k], ii = i0 + s;
+        const int e = p.cand[(size_t) ii * DCAND + (k - s_off[s])];
+        const int uid = p.rec[e < 0 ? ~e : e].uid;
+        const int m = s_nc[s];
+        int slot = -1;
+        for (int h = 0; h < m; h++)
+            if (p.c_uid[h * C + ii] == uid) slot = h;
+        s_cand[k] = e;
+        s_uid[k] = uid;
+        s_slot[k] = slot;
+    }
+    __syncthreads();
+    unsigned long long used = 0ull;
+    if (n > 0) {
+        // two contacts in one slot: not independent
+        bool fresh = false;
+        for (int t = 0; t < n; t++) {
+            const int slot = s_slot[off + t];
+            if (slot < 0) { fresh = true; continue; }
+            if (used >> slot & 1ull) slow = true;
+            used |= 1ull << slot;
+        }
+        if (fresh)
+            for (int t = 1; t < n; t++)
+                for (int u = 0; u < t; u++)
+                    if (s_slot[off + t] < 0 && s_slot[off + u] < 0 && s_uid[off + t] == s_uid[off + u]) slow = true;
+        if (slow) {
+            for (int t = 0; t < n; t++) s_slot[off + t] = -1;
+        } else if (fresh) {
+            for (int t = 0; t < n; t++) {
+                if (s_slot[off + t] >= 0) continue;
+                if (nc >= p.ccap) {
+                    atomicMax(&c[D_REQ_CONTACT], nc + 1);
+                    atomicMax(&c[D_OVF], DOVF_CONTACT);
+                    continue;
                 }
+                s_slot[off + t] = nc;
+                used |= 1ull << nc;
+                nc++;
+            }
         }
     }
-    if (act && l == 0) p.cand_n[i] = n <= DCAND ? n : DCAND + 1;
-}
-
-// One thread per local particle: reset_contact_history_usage_status, then the
-// history slot of each touching partner in order (the last match, or a new
-// slot; src/pairs/mapping/funcs.py:230-270), marked used.
-__global__ __launch_bounds__(256) void k_contact_slots(DemPtrs p, int *__restrict__ c) {
-    const int nl = c[D_NLOCAL];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= nl || c[D_OVF]) return;
-    const int nc0 = p.num_contacts[i];
-    for (int k = 0; k < nc0; k++) p.c_used[(size_t) k * p.cap + i] = 0;
-    const int nt = p.cand_n[i];
-    if (nt > DCAND) return;
-    for (int t = 0; t < nt; t++) {
-        const int e = p.cand[(size_t) t * p.cap + i];
-        p.cslot[(size_t) t * p.cap + i] = contact_slot(p, c, i, p.uid[e < 0 ? ~e : e]);
+    __syncthreads();
+    Acc3 fs = {0.0, 0.0, 0.0}, fp = {0.0, 0.0, 0.0}, ts = {0.0, 0.0, 0.0}, tp = {0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < total; k0 += 64) {
+        const int k = k0 + lane;
+        int kind = 2;
+        if (k < total && s_slot[k] >= 0) {
+            const int s = s_own[k], ii = i0 + s, slot = s_slot[k];
+            const int e = s_cand[k], j = e < 0 ? ~e : e;
+            const DemRec ri = p.rec[ii], rj = p.rec[j];
+            const double xi[3] = {ri.x, ri.y, ri.z};
+            const bool fresh = slot >= s_nc[s];
+            double nv[3], cpt[3], delta, F[3], T[3];
+            if (contact_geom(p, xi, ri.r, j, rj, e < 0 ? 1 : 0, nv, cpt, delta)) {
+                spring_dashpot(p, prm, ri, rj, ii, slot, fresh, nv, delta, cpt, F, T);
+                if (fresh) p.c_uid[slot * C + ii] = s_uid[k];
+                for (int d = 0; d < 3; d++) { s_term[lane][d] = F[d]; s_term[lane][3 + d] = T[d]; }
+                kind = e < 0 ? 1 : 0;
+            }
+        }
+        s_kind[lane] = kind;
+        __syncthreads();
+        for (int q = max(off, k0); q < min(off + n, k0 + 64); q++) {
+            const double *t = s_term[q - k0];
+            const int kd = s_kind[q - k0];
+            const double F[3] = {t[0], t[1], t[2]}, T[3] = {t[3], t[4], t[5]};
+            if (kd == 0) accumulate(fs, ts, F, T);
+            else if (kd == 1) accumulate(fp, tp, F, T);
+        }
+        __syncthreads();
     }
-}
-
-// One thread per (partner t, local particle i): linear_spring_dashpot of the
-// contact, its history slot updated, its force and torque term stored as
-// cf[6 t + 0..5][i] for the in-order sums of k_contacts.
-__global__ __launch_bounds__(256) void k_contact_pairs(DemPtrs p, const int *__restrict__ c, DemParams prm) {
-    const int nl = c[D_NLOCAL];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int t = blockIdx.y;
-    if (i >= nl || c[D_OVF]) return;
-    const int nt = p.cand_n[i];
-    if (t >= nt || nt > DCAND) return;
-    const size_t a = (size_t) t * p.cap + i;
-    const int slot = p.cslot[a];
-    if (slot < 0) return;
-    const int e = p.cand[a];
-    const int j = e < 0 ? ~e : e;
-    const double ri = p.r[i];
-    const double xi[3] = {p.x[i], p.y[i], p.z[i]};
-    double nv[3], cpt[3], delta, F[3], T[3];
-    if (!contact_geom(p, xi, ri, j, e < 0 ? 1 : 0, nv, cpt, delta)) return;
-    spring_dashpot(p, prm, i, j, slot, nv, delta, cpt, F, T);
-    for (int d = 0; d < 3; d++) {
-        p.cf[(6 * (size_t) t + d) * p.cap + i] = F[d];
-        p.cf[(6 * (size_t) t + 3 + d) * p.cap + i] = T[d];
-    }
-}
-
-// One thread per local particle: reset_volatile_properties, gravity, the
-// contacts' forces and torques summed in contact order (force += sphere +
-// plane sums, torque += plane + sphere sums) and
-// clear_unused_contact_history -- every one of them touches only the
-// thread's own particle and history rows.  A particle with more than DCAND
-// touching partners walks its cells here, slot search and spring-dashpot
-// inline.
-__global__ __launch_bounds__(128) void k_contacts(DemPtrs p, int *__restrict__ c, DemGeom g, DemParams prm) {
-    const int nl = c[D_NLOCAL];
-    const int i = blockIdx.x * 128 + threadIdx.x;
-    if (i >= nl || c[D_OVF]) return;
+    if (!sph) return;
     double f0 = 0.0, f1 = 0.0, f2 = 0.0, t0 = 0.0, t1 = 0.0, t2 = 0.0;
+    if (slow) {
+        for (int k = 0; k < nc0; k++) p.c_used[k * C + i] = 0;
+        p.num_contacts[i] = nc0;
+    }
     if (!(p.flags[i] & DFLAG_FIXED)) {
         // gravity (examples/dem.py:88-90)
         const double ri = p.r[i];
         const double vol = (((4.0 / 3.0) * prm.pi) * ri * ri) * ri;
         f2 = f2 - (prm.drho * vol) * prm.grav;
-        Acc3 fs = {0.0, 0.0, 0.0}, fp = {0.0, 0.0, 0.0}, ts = {0.0, 0.0, 0.0}, tp = {0.0, 0.0, 0.0};
-        const int nt = p.cand_n[i];
-        if (nt <= DCAND) {
-            for (int t = 0; t < nt; t++) {
-                const size_t a = (size_t) t * p.cap + i;
-                if (p.cslot[a] < 0) continue;
-                double F[3], T[3];
-                for (int d = 0; d < 3; d++) {
-                    F[d] = p.cf[(6 * (size_t) t + d) * p.cap + i];
-                    T[d] = p.cf[(6 * (size_t) t + 3 + d) * p.cap + i];
-                }
-                if (p.cand[a] >= 0) accumulate(fs, ts, F, T);
-                else accumulate(fp, tp, F, T);
-            }
-        } else {
-            const double xi[3] = {p.x[i], p.y[i], p.z[i]};
+        if (slow) {
+            const DemRec me = p.rec[i];
+            const double xi[3] = {me.x, me.y, me.z};
             walk_candidates(p, g, i, p.particle_cell[i], [&](int j, int pass) {
                 double nv[3], cpt[3], delta, F[3], T[3];
-                if (!contact_geom(p, xi, ri, j, pass, nv, cpt, delta)) return true;
-                const int slot = contact_slot(p, c, i, p.uid[j]);
+                const DemRec rj = p.rec[j];
+                if (!contact_geom(p, xi, ri, j, rj, pass, nv, cpt, delta)) return true;
+                const int slot = contact_slot(p, c, i, rj.uid);
                 if (slot < 0) return true;
-                spring_dashpot(p, prm, i, j, slot, nv, delta, cpt, F, T);
+                spring_dashpot(p, prm, me, rj, i, slot, false, nv, delta, cpt, F, T);
                 if (pass == 0) accumulate(fs, ts, F, T);
                 else accumulate(fp, tp, F, T);
                 return true;
@@ -844,20 +970,20 @@ __global__ __launch_bounds__(128) void k_contacts(DemPtrs p, int *__restrict__ c
     p.fx[i] = f0; p.fy[i] = f1; p.fz[i] = f2;
     p.tx[i] = t0; p.ty[i] = t1; p.tz[i] = t2;
     // clear_unused_contact_history (src/pairs/sim/contact_history.py:91-127)
+    if (slow) nc = p.num_contacts[i];
     int k = 0;
-    int nc = p.num_contacts[i];
     while (k < nc) {
-        const size_t a = (size_t) k * p.cap + i;
-        if (p.c_used[a] == 0) {
+        const size_t a = k * C + i;
+        if (slow ? p.c_used[a] == 0 : !(used >> k & 1ull)) {
             const int last = nc - 1;
             if (last > 0) {
-                const size_t b = (size_t) last * p.cap + i;
+                const size_t b = last * C + i;
                 p.c_stick[a] = p.c_stick[b];
-                for (int d = 0; d < 3; d++)
-                    p.c_tsd[(3 * (size_t) k + d) * p.cap + i] = p.c_tsd[(3 * (size_t) last + d) * p.cap + i];
+                for (int d = 0; d < 3; d++) p.c_tsd[(3 * (size_t) k + d) * C + i] = p.c_tsd[(3 * (size_t) last + d) * C + i];
                 p.c_ivm[a] = p.c_ivm[b];
                 p.c_uid[a] = p.c_uid[b];
-                p.c_used[a] = p.c_used[b];
+                if (slow) p.c_used[a] = p.c_used[b];
+                else used = (used & ~(1ull << k)) | (used >> last & 1ull) << k;
             }
             nc = nc - 1;
         } else {
@@ -975,7 +1101,7 @@ static void select_dim(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g
 }
 
 // exchange, borders, cells of one step (the cell counts are zero on entry:
-// allocated zeroed, cleared by every cell ordering pass)
+// allocated zeroed, cleared by every scan)
 void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
     // exchange, dimension by dimension (comm.py:100-151); one rank: only the
     // periodic dimensions send
@@ -995,23 +1121,28 @@ void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
     // cells
     const int pg = grid_of(p.cap, 256);
     hipLaunchKernelGGL(k_cell_count, dim3(pg), dim3(256), 0, s, p, c, g);
-    const int nb = grid_of(g.ncells, 1024);
-    hipLaunchKernelGGL(k_scan_partial, dim3(nb), dim3(1024), 0, s, p.cell_count, p.cell_start, p.scan_tmp, g.ncells);
-    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(1024), 0, s, p.cell_start, p.scan_tmp, g.ncells);
+    // (one entry past the cells, whose count stays zero: cell_start[ncells] is the total)
+    const int nb = grid_of(g.ncells + 1, 1024);
+    hipLaunchKernelGGL(k_scan_partial, dim3(nb), dim3(1024), 0, s, p.cell_count, p.cell_start, p.scan_tmp,
+                       g.ncells + 1);
+    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(1024), 0, s, p.cell_start, p.scan_tmp, g.ncells + 1);
     hipLaunchKernelGGL(k_cell_fill, dim3(pg), dim3(256), 0, s, p, c);
-    hipLaunchKernelGGL(k_cell_order, dim3(grid_of(g.ncells, 256)), dim3(256), 0, s, p, g.ncells);
+    hipLaunchKernelGGL(k_cell_order, dim3(pg), dim3(256), 0, s, p, c);
 }
 
 // forces + history bookkeeping, then integration
-void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, const DemParams &prm,
+void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
                      const hipEvent_t *between) {
-    hipLaunchKernelGGL(k_contact_find<DEM_LPS>, dim3(grid_of(p.cap, 256 / DEM_LPS)), dim3(256), 0, s, p, c, g);
-    if (between) hipEventRecord(between[0], s);
-    hipLaunchKernelGGL(k_contact_slots, dim3(grid_of(p.cap, 256)), dim3(256), 0, s, p, c);
-    if (between) hipEventRecord(between[1], s);
-    hipLaunchKernelGGL(k_contact_pairs, dim3(grid_of(p.cap, 256), DCAND), dim3(256), 0, s, p, c, prm);
+    hipLaunchKernelGGL(k_contact_find, dim3(grid_of(p.cap, 256 / LPS)), dim3(256), 0, s, p, c, g);
+    if (between) { hipEventRecord(between[0], s); hipEventRecord(between[1], s); }
+    // particles per wave: a wave's chain of look-ups is shorter with fewer (a
+    // small system is one wave of the chip long), its lanes fuller with more:
+    // beds of 2080 / 9600 / 39200 / 187200 spheres, ms a pass on 8, 16, 32:
+    // 16.1 16.8 17.8 / 4.58 4.76 4.99 / 6.41 6.24 6.45 / 28.8 27.3 26.4
+    if (nlocal < 16384) hipLaunchKernelGGL(k_contact_solve<8>, dim3(grid_of(nlocal, 8)), dim3(64), 0, s, p, c, g, prm);
+    else if (nlocal < 65536) hipLaunchKernelGGL(k_contact_solve<16>, dim3(grid_of(nlocal, 16)), dim3(64), 0, s, p, c, g, prm);
+    else hipLaunchKernelGGL(k_contact_solve<32>, dim3(grid_of(nlocal, 32)), dim3(64), 0, s, p, c, g, prm);
     if (between) hipEventRecord(between[2], s);
-    hipLaunchKernelGGL(k_contacts, dim3(grid_of(p.cap, 128)), dim3(128), 0, s, p, c, g, prm);
 }
 
 void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemParams &prm) {

@@ -28,10 +28,6 @@ enum {
 // touching partners recorded per particle by the contact search; a particle
 // with more walks its cells again in the force pass
 constexpr int DCAND = 16;
-// lanes per sphere of the contact search (each a run of the 28 cells)
-#ifndef DEM_LPS
-#define DEM_LPS 16
-#endif
 
 enum { DOVF_NONE = 0, DOVF_PART = 1, DOVF_CONTACT = 2, DOVF_SEND = 3, DOVF_CELLS = 4 };
 
@@ -52,6 +48,12 @@ struct DemParams {
     double mu_s[16], mu_d[16];
 };
 
+// everything a contact needs of a particle, one cache line
+struct alignas(128) DemRec {
+    double x, y, z, r, vx, vy, vz, m, wx, wy, wz;
+    int type, uid;
+};
+
 // every device array, passed by value to the kernels
 struct DemPtrs {
     int cap, ccap, send_cap;
@@ -61,13 +63,18 @@ struct DemPtrs {
     int *num_contacts, *c_uid, *c_used, *c_stick;  // [k][cap]
     double *c_tsd;                                 // [3k + d][cap]
     double *c_ivm;                                 // [k][cap]
-    int *cell_count, *cell_start, *cell_particles, *particle_cell, *nshapes;
+    int *cell_count, *cell_start, *cell_particles, *particle_cell;
     int *cell_slot;      // each particle's place in its cell, from the counting pass
     int *send_map, *send_mult, *exchg_flag, *copy_to, *blk, *scan_tmp;
     double *buf, *hbuf;
-    int *cand_n, *cand;  // touching partners found by the contact search: [t][cap], t < DCAND
-    int *cslot;          // their history slots [t][cap]
-    double *cf;          // their force and torque terms [6 t + d][cap]
+    // the particles in cell order (each cell in the reference's order): index
+    // and cell (bit 31: FIXED), (x, y, z, radius; -1 for a half-space); cmixed:
+    // scratch of cells that hold a half-space
+    int2 *corder;
+    int *cmixed;
+    double4 *crec;
+    DemRec *rec;         // by particle index, locals and ghosts
+    int *cand_n, *cand;  // touching partners found by the contact search: [i][t], t < DCAND
 };
 
 // one strided copy of 32-bit words: rows x words, row r from src + r * src_pitch
@@ -86,9 +93,9 @@ void launch_mass_inertia(hipStream_t s, const DemPtrs &p, int nl);
 // one step = prepare (exchange, borders, cells) + contacts (+ gravity and
 // history bookkeeping) + euler
 void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g);
-// between: three events recorded after the search, the slot and the pair
-// kernels (timed steps only)
-void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, const DemParams &prm,
+// nlocal: the host's count; between: three events recorded after the search
+// (two) and after the contact kernel (timed steps only)
+void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
                      const hipEvent_t *between = nullptr);
 void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemParams &prm);
 

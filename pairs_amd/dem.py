@@ -219,7 +219,9 @@ class DEMSystem:
 
     def phase_times(self):
         """Average ms of the timed steps' phases: prepare, contact search,
-        history slots, spring-dashpot, sums + history clean-up, euler."""
+        history slots, spring-dashpot, sums + history clean-up, euler.  Slots,
+        spring-dashpot, sums and clean-up are one kernel, timed as the
+        spring-dashpot phase; the slot and sum phases read about zero."""
         ms = (_D * 6)()
         self._check(self.L.pairs_hip_dem_phase_times(self.ctx, ms), "phase_times")
         return tuple(ms)

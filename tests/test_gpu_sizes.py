@@ -49,3 +49,71 @@ def test_lj_run_vs_oracle_at_size_edges(n, ntypes, half):
         for name, p, q in (("position", g.positions(True), o.positions(True)),
                            ("velocity", g.velocities(), o.velocities()), ("force", g.forces(), o.forces())):
             assert np.array_equal(p, q), f"{name} after step {b}: max |diff| {np.abs(p - q).max()}"
+
+
+def _spheres(case):
+    """uid, radius, position, velocity of a few spheres, domain, half-spaces"""
+    rng = np.random.default_rng(len(case))
+    d = 0.0029
+    planes = [(100000, (0.0, 0.0, 0.0), (0.0, 0.0, 1.0), 13)]
+    if case.startswith("pile"):  # a loose pile of n spheres
+        n = int(case[4:])
+        m = int(np.ceil(n ** (1.0 / 3.0)))
+        k = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+        x = (k + 0.5) * 0.97 * d + rng.uniform(-0.02, 0.02, (n, 3)) * d
+        r = 0.5 * d * rng.uniform(0.95, 1.05, n)
+        dom = (max(0.012, m * 0.97 * d + 0.001), max(0.012, m * 0.97 * d + 0.001), max(0.02, m * d + 0.01))
+    elif case == "crowd":  # one sphere with 30 small ones around it: more partners than the search keeps
+        u = rng.standard_normal((30, 3))
+        u /= np.linalg.norm(u, axis=1)[:, None]
+        x = np.concatenate([[[0.01, 0.01, 0.01]], 0.01 + u * 0.00198])
+        r = np.concatenate([[0.0016], np.full(30, 0.0004)])
+        dom = (0.02, 0.02, 0.02)
+    elif case == "dense":  # many small spheres per cell: more candidates than a lane's mask holds
+        k = np.stack(np.meshgrid(*[np.arange(9)] * 3, indexing="ij"), -1).reshape(-1, 3)
+        x = 0.002 + (k + 0.5) * 0.0008 + rng.uniform(-1e-5, 1e-5, (729, 3))
+        r = np.full(729, 0.00041)
+        dom = (0.02, 0.02, 0.02)
+    elif case == "image":  # a partner and its periodic image touch the same sphere
+        x = np.array([[0.0004, 0.006, 0.006], [0.0019, 0.0082, 0.006], [0.0011, 0.006, 0.0088]])
+        r = np.full(3, 0.00145)
+        dom = (0.0031, 0.012, 0.012)
+    else:  # half-spaces in cells of their own, among spheres
+        k = np.stack(np.meshgrid(*[np.arange(3)] * 3, indexing="ij"), -1).reshape(-1, 3)
+        x = 0.004 + (k + 0.5) * 0.98 * d
+        r = np.full(27, 0.5 * d)
+        planes += [(7, (0.0055, 0.0052, 0.0046), (0.0, 0.0, 1.0), 12), (900, (0.0055, 0.0052, 0.012), (0.0, 0.6, -0.8), 12)]
+        dom = (0.02, 0.02, 0.02)
+    return np.arange(1, len(r) + 1) + 10, r, x, rng.uniform(-0.05, 0.05, x.shape), dom, planes
+
+
+@pytest.mark.parametrize("case", ["pile1", "pile7", "pile9", "pile33", "pile257", "crowd", "dense", "image", "walls"])
+def test_dem_contacts_vs_oracle(case):
+    """contacts, history and trajectory of small arrangements that take every
+    form of the contact kernels, 30 steps against the oracle"""
+    from pairs_amd import dem
+    uid, r, x, v, dom, planes = _spheres(case)
+    g = dem.DEMSystem(dom, particle_capacity=16384, contact_capacity=48)
+    o = po.OracleDEM(dom, cap=16384, ccap=48, cellcap=256)
+    g.add_spheres(uid, r, x, v)
+    for k in range(len(r)):
+        o.add_sphere(int(uid[k]), r[k], x[k], v[k])
+    for s in (g, o):
+        for u, pos, nrm, fl in planes:
+            s.add_halfspace(u, pos, nrm, flags=fl)
+        s.setup()
+    for a, b in ((0, 1), (1, 4), (4, 30)):
+        g.run(a, b)
+        o.run(a, b)
+        assert g.nlocal == o.nlocal and g.nghost == o.nghost, b
+        assert np.array_equal(g.get("uid"), o.get("uid")), b
+        nc, cl, sk, tsd, iv = g.contacts()
+        onc, ocl, osk, otsd, oiv = o.contacts()
+        assert np.array_equal(nc, onc), b
+        for i in range(len(nc)):
+            m = nc[i]
+            assert np.array_equal(cl[i, :m], ocl[i, :m]) and np.array_equal(sk[i, :m], osk[i, :m]), (b, i)
+        # sin and cos of the rotation update differ in their last bits: 1e-10, as the DEM tests
+        for name, p, q in [(k, g.get(k), o.get(k)) for k in ("position", "linear_velocity", "angular_velocity",
+                                                              "force", "torque")]:
+            assert np.abs(p - q).max() <= 1e-10 * max(np.abs(q).max(), 1e-300), (b, name)
