@@ -929,14 +929,6 @@ __device__ __forceinline__ double odd_lane(double v) {
     return __longlong_as_double(((long long) hi << 32) | (unsigned int) lo);
 }
 
-// the 64-bit value of the other lane of each lane pair (DPP quad_perm 1,0,3,2)
-__device__ __forceinline__ double pair_swap(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int) b, 0xB1, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int) (b >> 32), 0xB1, 0xF, 0xF, true);
-    return __longlong_as_double(((long long) hi << 32) | (unsigned int) lo);
-}
-
 // the type word of a packed record's (z, type) half, from the other lane of the pair
 __device__ __forceinline__ int pair_swap_type(double w) {
     return __builtin_amdgcn_mov_dpp((int) __double_as_longlong(w), 0xB1, 0xF, 0xF, true);
@@ -1099,14 +1091,6 @@ __device__ __forceinline__ void lj_wave2(const LJArgs &A, int wv) {
 template <int NT, int MODE, bool RED, bool UNIT>
 __global__ __launch_bounds__(64) void k_lj2(LJArgs A) {
     lj_wave2<NT, MODE, RED, UNIT>(A, xcd_block(blockIdx.x, gridDim.x));
-}
-
-// LDS operations of one wave complete in order, so what a wave hands from
-// lane to lane needs no wait, only an order the compiler keeps
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // The force kernel of the timestep on L = 4 .. 32 lanes per local (M = 64 / L

@@ -19,6 +19,22 @@ __device__ __forceinline__ int wave_max_uniform(int v) {
     return __builtin_amdgcn_readlane(v, 63);
 }
 
+// the 64-bit value of the other lane of each lane pair (DPP quad_perm 1,0,3,2)
+__device__ __forceinline__ double pair_swap(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int) b, 0xB1, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int) (b >> 32), 0xB1, 0xF, 0xF, true);
+    return __longlong_as_double(((long long) hi << 32) | (unsigned int) lo);
+}
+
+// LDS operations of one wave complete in order, so what a wave hands from
+// lane to lane needs no wait, only an order the compiler keeps
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 struct SegInfo {
     int cx, cy, za, zb;  // column and z range [za, zb) of the home cells
     int ca, cb;          // flat cell ids of the first home cell and one past the last

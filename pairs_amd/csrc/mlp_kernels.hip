@@ -22,16 +22,17 @@ namespace pk {
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// FP32 -> BF16, round to nearest even (inputs are finite)
-__device__ __forceinline__ short f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (short) (u >> 16);
+// FP32 -> BF16, round to nearest even: the hardware's conversion of two values
+typedef __bf16 hwbf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    const f32x2 f = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, hwbf16x2));
 }
+__device__ __forceinline__ short f2bf(float f) { return (short) pack2(f, f); }
 __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
-    bf16x4 r;
-    r[0] = f2bf(a); r[1] = f2bf(b); r[2] = f2bf(c); r[3] = f2bf(d);
-    return r;
+    const uint2 u = make_uint2(pack2(a, b), pack2(c, d));
+    return __builtin_bit_cast(bf16x4, u);
 }
 __device__ __forceinline__ bf16x4 pack4(const f32x4 &x) { return pack4(x[0], x[1], x[2], x[3]); }
 __device__ __forceinline__ float bf2f(short b) { return __uint_as_float(((uint32_t) (uint16_t) b) << 16); }
@@ -185,11 +186,13 @@ __device__ __forceinline__ f32x4 mlp_input_grad(const MLPRegs &R, const f32x4 (&
     return d;
 }
 
-// E and dE/dG (raw descriptor units) of n rows; one wave per 16-row tile
-template <bool WANT_D>
+// E and dE/dG (raw descriptor units) of n rows; one wave per 16-row tile.
+// IMG: the rows are the locals of a force evaluation, and a local's dE/dG goes
+// to its ghost images too (im.on), in place of a copy pass over the ghosts.
+template <bool WANT_D, bool IMG>
 __global__ __launch_bounds__(256) void k_mlp_eval(const float *__restrict__ p, const float *__restrict__ sc,
                                                   const float *__restrict__ G, int n, float *__restrict__ E,
-                                                  float *__restrict__ D) {
+                                                  float *__restrict__ D, Images im) {
     const int lane = threadIdx.x & 63, q = lane >> 4, col = lane & 15;
     const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
     const int ntiles = (n + 15) >> 4;
@@ -216,6 +219,13 @@ __global__ __launch_bounds__(256) void k_mlp_eval(const float *__restrict__ p, c
                 o.z = R.es * d[2] * R.gi[2];
                 o.w = R.es * d[3] * R.gi[3];
                 *(float4 *) (D + (size_t) row * MLP_ND + 4 * q) = o;
+                if (IMG && im.on) {
+                    const int ni = min(im.cnt[row], IMG_MAX);
+                    for (int k = 0; k < ni; k++) {
+                        const int gq = im.tab[(size_t) k * im.cap + row].x;
+                        *(float4 *) (D + (size_t) (n + gq) * MLP_ND + 4 * q) = o;
+                    }
+                }
             }
         }
     }
@@ -270,11 +280,26 @@ struct MLPSegArgs {
 // the lanes at the end (FP32 / FP64 sums in any order: the potential is not
 // bit-matched to a reference), so L times as many waves hide the gathers'
 // latency.  Pairs at r >= 2.5 and entries past a lane's count are masked.
+//
+// Bound by vector work (210 operations per pair in MODE 1, 67 us' worth at
+// 131072 atoms) and, as each lane gathered its partners' rows by itself, by the
+// cache-line look-ups of those gathers (6 per pair in MODE 1, 107 us' worth at
+// one a cycle and CU).  So on two lanes per local MODE 1 loads each position
+// record with one instruction of the lane pair (x, y on one lane, z on the
+// other, swapped by DPP) and each 64-byte row of dE/dG with four lanes, handed
+// over through LDS (the chunks of a row are rotated by lane group: no bank
+// conflicts on either side): 2 look-ups per pair, the arithmetic unchanged.
+// 131072 atoms: MODE 1 89 -> 78 us, MODE 0 42 -> 39.  On four lanes (small
+// systems) the hand-over only lengthens a step's chain (16.6 -> 20 us at 2048
+// atoms), and in MODE 0 the swap costs more than the look-ups (39 -> 48): both
+// gather directly.
 template <int MODE, bool RED, int L>
 __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
     constexpr int U = 4 / L;  // entries per lane per step
+    constexpr bool ROWS = MODE == 1 && L == 2;  // dE/dG rows loaded by four lanes each
+    __shared__ __align__(16) float4 s_d[ROWS ? 256 : 1];
     const int wv = xcd_block(blockIdx.x, gridDim.x);
-    const int lane = threadIdx.x & 63, h = lane & (L - 1);
+    const int lane = threadIdx.x & 63, h = lane & (L - 1), odd = lane & 1;
     const int nlocal = A.counters[C_NLOCAL];
     const uint32_t jmax = (uint32_t) max(nlocal + A.counters[C_NGHOST] - 1, 0);
     const char *__restrict__ P = (const char *) A.P;
@@ -305,9 +330,13 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
         const uint4 *lp = (const uint4 *) A.nl + ii;
         const int gl = max((n + 3) / 4 - 1, 0);
         const int nst = (nmax + 3) / 4;
+        // the lane's chunk of the records the wave loads together: record
+        // 16 m + lane / 4, chunk rotated by the record's group of four
+        const int rsub = lane >> 2, rot = (lane >> 2) & 3;
+        const int chunk_in = (lane & 3) ^ ((rsub >> 2) & 3);
         for (int st = 0; st < nst; st++) {
-            // groups past the lane's list re-read its last group; entries are
-            // clamped to the last particle slot
+            // groups past the lane's list re-read its last group; entries past
+            // its count read the last particle slot, entries are clamped to it
             const uint4 grp = lp[(size_t) min(st, gl) * A.nl_stride];
             uint32_t jq[U];
 #pragma unroll
@@ -315,25 +344,33 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
                 const int c = L * q + h;
                 // (a group holds its entries as 0, 2, 1, 3)
                 const uint32_t e = (c & 2) ? ((c & 1) ? grp.w : grp.y) : ((c & 1) ? grp.z : grp.x);
-                jq[q] = min(e, jmax);
+                jq[q] = 4 * st + c < n ? min(e, jmax) : jmax;
             }
-            double xj[U], yj[U], zj[U];
-            float4 dj[U][4], rj[U];
-#pragma unroll
-            for (int q = 0; q < U; q++) {
-                const uint32_t off = jq[q] << 5;
-                const double2 pxy = *(const double2 *) (P + off);
-                xj[q] = pxy.x; yj[q] = pxy.y; zj[q] = *(const double *) (P + off + 16);
-                if (MODE == 1) {
-                    const float4 *dp = (const float4 *) (A.D + (size_t) jq[q] * MLP_ND);
-#pragma unroll
-                    for (int k4 = 0; k4 < 4; k4++) dj[q][k4] = dp[k4];
+            struct Ent { double2 a, b; float4 d0, d1, d2, d3, rho; };
+            auto gather = [&](uint32_t j, Ent &e) __attribute__((always_inline)) {
+                if (!ROWS) {
+                    e.a = *(const double2 *) (P + (j << 5));
+                    e.b.x = *(const double *) (P + (j << 5) + 16);
+                    if (MODE == 1) {
+                        const float4 *dp = (const float4 *) (A.D + (size_t) j * MLP_ND);
+                        e.d0 = dp[0]; e.d1 = dp[1]; e.d2 = dp[2]; e.d3 = dp[3];
+                    }
+                    if (MODE == 2) e.rho = A.rho[j];
+                    return;
                 }
-                if (MODE == 2) rj[q] = A.rho[jq[q]];
-            }
-#pragma unroll
-            for (int q = 0; q < U; q++) {
-                const double dx = xi - xj[q], dy = yi - yj[q], dz = zi - zj[q];
+                const uint32_t jp = (uint32_t) __builtin_amdgcn_mov_dpp((int) j, 0xB1, 0xF, 0xF, true);
+                const uint32_t je = odd ? jp : j, jo = odd ? j : jp;
+                e.a = *(const double2 *) (P + ((je << 5) + (odd ? 16u : 0u)));
+                e.b = *(const double2 *) (P + ((jo << 5) + (odd ? 0u : 16u)));
+                auto row = [&](int m) {
+                    return *((const float4 *) (A.D + (size_t) __shfl((int) j, 16 * m + rsub, 64) * MLP_ND) + chunk_in);
+                };
+                e.d0 = row(0); e.d1 = row(1); e.d2 = row(2); e.d3 = row(3);
+            };
+            auto pair = [&](int q, const Ent &e) __attribute__((always_inline)) {
+                const double2 xy = ROWS && odd ? e.b : e.a;
+                const double zj = ROWS ? pair_swap(odd ? e.a.x : e.b.x) : e.b.x;
+                const double dx = xi - xy.x, dy = yi - xy.y, dz = zi - zj;
                 double rsq = dx * dx + dy * dy;
                 rsq = rsq + dz * dz;
                 const bool in = (4 * st + L * q + h < n) && rsq < rc2;
@@ -348,10 +385,12 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
                 // computed anchors (k = 0 and k = 8): four exponentials per
                 // pair instead of sixteen, relative error below 1e-5
                 const float t0 = r - MLP_MU0;
+                // (arguments in the normal range of exp2, |t| < 1.8: the
+                // hardware's exponential as it is)
                 auto anchor = [&](int k0, float &g, float &a) {
                     const float t = t0 - (float) k0 * MLP_DMU;
-                    g = exp2f(-(t * t) * MLP_C);
-                    a = exp2f((2.0f * t - MLP_DMU) * MLP_DMU * MLP_C);
+                    g = __builtin_amdgcn_exp2f(-(t * t) * MLP_C);
+                    a = __builtin_amdgcn_exp2f((2.0f * t - MLP_DMU) * MLP_DMU * MLP_C);
                 };
                 float gk, ak;
                 if (MODE == 0) {
@@ -370,8 +409,8 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
                     const float sn = __builtin_amdgcn_sinf(ang), cs = __builtin_amdgcn_cosf(ang);
                     const float fc = 0.5f * (cs + 1.0f), dfc = -0.5f * MLP_PIRC * sn;
                     // (x_a - x_j) / r . (rho_a - rho_j), zero for a masked entry
-                    float proj = (float) dx * (rhoi.x - rj[q].x) + (float) dy * (rhoi.y - rj[q].y);
-                    proj = proj + (float) dz * (rhoi.z - rj[q].z);
+                    float proj = (float) dx * (rhoi.x - e.rho.x) + (float) dy * (rhoi.y - e.rho.y);
+                    proj = proj + (float) dz * (rhoi.z - e.rho.z);
                     proj = in ? -proj * rinv : 0.0f;
 #pragma unroll
                     for (int kk = 0; kk < MLP_ND; kk++) {
@@ -383,27 +422,43 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
                         ak *= gb;
                     }
                 } else {
+                    // this lane's row, from the lanes that loaded its chunks
+                    if (ROWS) {
+                        s_d[lane] = e.d0; s_d[64 + lane] = e.d1; s_d[128 + lane] = e.d2; s_d[192 + lane] = e.d3;
+                        wave_lds_sync();
+                    }
                     const float ang = r * (0.5f / (float) MLP_RC);
                     const float sn = __builtin_amdgcn_sinf(ang), cs = __builtin_amdgcn_cosf(ang);
                     const float fc = 0.5f * (cs + 1.0f), dfc = -0.5f * MLP_PIRC * sn;
                     float ci = 0.f, cj = 0.f;
-                    const float *djq = (const float *) dj[q];
 #pragma unroll
-                    for (int kk = 0; kk < MLP_ND; kk++) {
-                        if (kk % 8 == 0) anchor(kk, gk, ak);
-                        const float t = t0 - (float) kk * MLP_DMU;
-                        const float dphi = gk * fmaf(-t * MLP_IW2, fc, dfc);
-                        ci = fmaf(di[kk], dphi, ci);
-                        cj = fmaf(djq[kk], dphi, cj);
-                        gk *= ak;
-                        ak *= gb;
+                    for (int k4 = 0; k4 < 4; k4++) {
+                        const float4 d4 = ROWS ? s_d[4 * lane + (k4 ^ rot)] : k4 == 0 ? e.d0 : k4 == 1 ? e.d1 : k4 == 2 ? e.d2 : e.d3;
+                        const float dq[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const int kk = 4 * k4 + v;
+                            if (kk % 8 == 0) anchor(kk, gk, ak);
+                            const float t = t0 - (float) kk * MLP_DMU;
+                            const float dphi = gk * fmaf(-t * MLP_IW2, fc, dfc);
+                            ci = fmaf(di[kk], dphi, ci);
+                            cj = fmaf(dq[v], dphi, cj);
+                            gk *= ak;
+                            ak *= gb;
+                        }
                     }
+                    if (ROWS) wave_lds_sync();
                     const float cc = ci + cj;
                     const double coef = in ? (double) (-cc * rinv) : 0.0;
                     f0 += coef * dx; f1 += coef * dy; f2 += coef * dz;
                     if (RED) w += in ? (double) (-cc * r) : 0.0;
                 }
-            }
+            };
+            Ent e0, e1;
+            gather(jq[0], e0);
+            if (U == 2) gather(jq[U - 1], e1);
+            pair(0, e0);
+            if (U == 2) pair(U - 1, e1);
         }
         // the L lanes of a local: partial sums added
 #pragma unroll
@@ -1008,16 +1063,20 @@ static int eval_grid(int n) {
 
 void launch_mlp_eval(hipStream_t s, const float *p, const float *sc, const float *G, int n, float *E, float *D) {
     if (n <= 0) return;
-    if (D) hipLaunchKernelGGL(k_mlp_eval<true>, dim3(eval_grid(n)), dim3(256), 0, s, p, sc, G, n, E, D);
-    else hipLaunchKernelGGL(k_mlp_eval<false>, dim3(eval_grid(n)), dim3(256), 0, s, p, sc, G, n, E, D);
+    const Images none{};
+    if (D) hipLaunchKernelGGL((k_mlp_eval<true, false>), dim3(eval_grid(n)), dim3(256), 0, s, p, sc, G, n, E, D, none);
+    else hipLaunchKernelGGL((k_mlp_eval<false, false>), dim3(eval_grid(n)), dim3(256), 0, s, p, sc, G, n, E, D, none);
 }
 
 void launch_mlp_forces(hipStream_t s, const DevState &d, const Geom &g, const MLPBind &b, int cur, int reduce,
                        int ghost_grid, const MLPVV *vv, bool pack) {
     if (d.nlocal <= 0) return;
     launch_mlp_descriptors(s, d, g, cur, b.G, pack);
-    launch_mlp_eval(s, b.p, b.sc, b.G, d.nlocal, b.E, b.D);
-    hipLaunchKernelGGL(k_mlp_ghost_d, dim3(std::max(ghost_grid, 1)), dim3(256), 0, s, d.counters, d.sync_src, b.D);
+    const Images im = images_of(d, true);
+    hipLaunchKernelGGL((k_mlp_eval<true, true>), dim3(eval_grid(d.nlocal)), dim3(256), 0, s, b.p, b.sc, b.G, d.nlocal,
+                       b.E, b.D, im);
+    if (!im.on)
+        hipLaunchKernelGGL(k_mlp_ghost_d, dim3(std::max(ghost_grid, 1)), dim3(256), 0, s, d.counters, d.sync_src, b.D);
     MLPSegArgs A = seg_args(d, cur);
     A.D = b.D;
     A.E = b.E;
