@@ -56,82 +56,120 @@ __device__ __forceinline__ void silu(float z, float &h, float &dh) {
 
 // ---------------------------------------------------------------- network tile
 
-// A operands and per-lane constants of one wave (lane l: q = l / 16, col = l % 16)
-struct MLPRegs {
-    bf16x4 a1[4];      // W1 rows 16c + col, columns 4q..4q+3 (high BF16 part)
-    bf16x4 a1l[4];     // W1 - a1 (low part: the first layer runs at ~16-bit precision)
-    bf16x4 a2[4][4];   // W2 [c2][kc]: rows 16c2 + col, columns 16kc + 4q..
-    bf16x4 a2t[4][4];  // W2^T [c][kc]: W2[16kc + 4q + v][16c + col]
-    bf16x4 a1t[4];     // W1^T [kc]: W1[16kc + 4q + v][col] (high part)
-    bf16x4 a1tl[4];    // its low part
-    float b1[4][4], b2[4][4], w3[4][4];  // rows 16c + 4q + v
-    float b3, gm[4], gi[4], em, es;
+// The network of a workgroup in LDS: the A operands of every MFMA, converted
+// to BF16 once and laid out by fragment and lane (lane l: q = l / 16, col = l %
+// 16), and the FP32 constants.  In registers, one set per wave, they took 96 of
+// 243 registers and left two waves on a SIMD; a read from LDS is one
+// conflict-free 8-byte access per fragment and four waves fit (k_mlp_eval,
+// 131072 rows: 22.3 -> 18.1 us).
+enum {
+    NF_A1 = 0,     // W1 rows 16c + col, columns 4q..4q+3 (high BF16 part)
+    NF_A1L = 4,    // W1 - a1 (low part: the first layer runs at ~16-bit precision)
+    NF_A2 = 8,     // W2 [c][kc]: rows 16c + col, columns 16kc + 4q..
+    NF_A2T = 24,   // W2^T [c][kc]: W2[16kc + 4q + v][16c + col]
+    NF_A1T = 40,   // W1^T [kc]: W1[16kc + 4q + v][col] (high part)
+    NF_A1TL = 44,  // its low part
+    NF_COUNT = 48
+};
+struct MLPNet {
+    bf16x4 f[NF_COUNT][64];
+    f32x4 b1[4][4], b2[4][4], w3[4][4];  // [c][q]: rows 16c + 4q + v
+    f32x4 gm[4], gi[4];                  // [q]: features 4q + v
+    float b3, em, es;
 };
 
-template <bool BACK>
-__device__ __forceinline__ void mlp_load(MLPRegs &R, const float *__restrict__ p, const float *__restrict__ sc,
-                                         int lane) {
-    const int q = lane >> 4, col = lane & 15;
+// the waves of a workgroup of NT threads convert the fragments in turn, every
+// load in flight before the first conversion; ends with a barrier
+template <bool BACK, int NT>
+__device__ __forceinline__ void mlp_stage(MLPNet &N, const float *__restrict__ p, const float *__restrict__ sc) {
+    constexpr int NF = BACK ? NF_COUNT : NF_A2T, IT = (NF * 64 + NT - 1) / NT;
+    const int lane = threadIdx.x & 63, q = lane >> 4, col = lane & 15;
+    const int wl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float w[IT][4], c[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, y[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const float *w = p + MLP_W1 + (16 * c + col) * MLP_ND + 4 * q;
-        split4(w[0], w[1], w[2], w[3], R.a1[c], R.a1l[c]);
+    for (int it = 0; it < IT; it++) {
+        const int f = it * (NT / 64) + wl;
+        if (f >= NF) break;
+        const bool rows = f < NF_A2T;  // of W, else of W^T
+        const float *m;
+        if (f < NF_A2) m = p + MLP_W1 + (16 * (f & 3) + col) * MLP_ND + 4 * q;
+        else if (rows) m = p + MLP_W2 + (16 * ((f - NF_A2) >> 2) + col) * MLP_H + 16 * (f & 3) + 4 * q;
+        else if (f < NF_A1T) m = p + MLP_W2 + (16 * (f & 3) + 4 * q) * MLP_H + 16 * ((f - NF_A2T) >> 2) + col;
+        else m = p + MLP_W1 + (16 * (f & 3) + 4 * q) * MLP_ND + col;
+        const int step = rows ? 1 : f < NF_A1T ? MLP_H : MLP_ND;
 #pragma unroll
-        for (int kc = 0; kc < 4; kc++) {
-            const float *u = p + MLP_W2 + (16 * c + col) * MLP_H + 16 * kc + 4 * q;
-            R.a2[c][kc] = pack4(u[0], u[1], u[2], u[3]);
-            if (BACK) {
-                const float *t = p + MLP_W2 + (16 * kc + 4 * q) * MLP_H + 16 * c + col;
-                R.a2t[c][kc] = pack4(t[0], t[MLP_H], t[2 * MLP_H], t[3 * MLP_H]);
-            }
-        }
-        if (BACK) {
-            const float *t = p + MLP_W1 + (16 * c + 4 * q) * MLP_ND + col;
-            split4(t[0], t[MLP_ND], t[2 * MLP_ND], t[3 * MLP_ND], R.a1t[c], R.a1tl[c]);
-        }
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int h = 16 * c + 4 * q + v;
-            R.b1[c][v] = p[MLP_B1 + h];
-            R.b2[c][v] = p[MLP_B2 + h];
-            R.w3[c][v] = p[MLP_W3 + h];
-        }
+        for (int v = 0; v < 4; v++) w[it][v] = m[v * step];
     }
-    R.b3 = p[MLP_B3];
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        R.gm[v] = sc[MLP_GMEAN + 4 * q + v];
-        R.gi[v] = sc[MLP_GISTD + 4 * q + v];
+    if (wl == 0) {
+        c[0] = p[MLP_B1 + lane]; c[1] = p[MLP_B2 + lane]; c[2] = p[MLP_W3 + lane];
+        if (lane < 16) { c[3] = sc[MLP_GMEAN + lane]; c[4] = sc[MLP_GISTD + lane]; }
+        y[0] = p[MLP_B3]; y[1] = sc[MLP_EMEAN]; y[2] = sc[MLP_ESTD];
     }
-    R.em = sc[MLP_EMEAN];
-    R.es = sc[MLP_ESTD];
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        const int f = it * (NT / 64) + wl;
+        if (f >= NF) break;
+        bf16x4 hi, lo;
+        split4(w[it][0], w[it][1], w[it][2], w[it][3], hi, lo);
+        N.f[f][lane] = (f >= NF_A1L && f < NF_A2) || f >= NF_A1TL ? lo : hi;
+    }
+    if (wl == 0) {
+        ((float *) N.b1)[lane] = c[0]; ((float *) N.b2)[lane] = c[1]; ((float *) N.w3)[lane] = c[2];
+        if (lane < 16) { ((float *) N.gm)[lane] = c[3]; ((float *) N.gi)[lane] = c[4]; }
+        if (lane == 0) { N.b3 = y[0]; N.em = y[1]; N.es = y[2]; }
+    }
+    __syncthreads();
 }
 
+// keeps the compiler from hoisting a tile loop's LDS reads into registers
+__device__ __forceinline__ void mlp_keep_in_lds() { asm volatile("" ::: "memory"); }
+
+// one lane's view of the network
+struct MLPView {
+    const MLPNet &N;
+    int lane, q;
+    __device__ __forceinline__ bf16x4 f(int k) const { return N.f[k][lane]; }
+    __device__ __forceinline__ f32x4 b1(int c) const { return N.b1[c][q]; }
+    __device__ __forceinline__ f32x4 b2(int c) const { return N.b2[c][q]; }
+    __device__ __forceinline__ f32x4 w3(int c) const { return N.w3[c][q]; }
+    __device__ __forceinline__ float4 gi() const {
+        const f32x4 g = N.gi[q];
+        return make_float4(g[0], g[1], g[2], g[3]);
+    }
+};
+
 // standardised descriptors of the lane's particle, features 4q..4q+3
-__device__ __forceinline__ f32x4 mlp_input(const MLPRegs &R, float4 g) {
+__device__ __forceinline__ f32x4 mlp_input(const MLPView &R, float4 g) {
+    const f32x4 gm = R.N.gm[R.q], gi = R.N.gi[R.q];
     f32x4 s;
-    s[0] = (g.x - R.gm[0]) * R.gi[0];
-    s[1] = (g.y - R.gm[1]) * R.gi[1];
-    s[2] = (g.z - R.gm[2]) * R.gi[2];
-    s[3] = (g.w - R.gm[3]) * R.gi[3];
+    s[0] = (g.x - gm[0]) * gi[0];
+    s[1] = (g.y - gm[1]) * gi[1];
+    s[2] = (g.z - gm[2]) * gi[2];
+    s[3] = (g.w - gm[3]) * gi[3];
     return s;
+}
+
+// W1 x of output block c with both operands split: hi*hi + lo*hi + hi*lo
+__device__ __forceinline__ f32x4 mlp_layer1(const MLPView &R, int c, bf16x4 b0, bf16x4 b0l) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const bf16x4 a1 = R.f(NF_A1 + c);
+    f32x4 z = mfma16(R.f(NF_A1L + c), b0, zero);
+    z = mfma16(a1, b0l, z);
+    return mfma16(a1, b0, z);
 }
 
 // forward pass of one 16-particle tile: returns y of particle col (all four
 // lane groups hold it); keeps activations and SiLU derivatives
-__device__ __forceinline__ float mlp_forward(const MLPRegs &R, bf16x4 b0, bf16x4 b0l, f32x4 (&h1)[4],
+__device__ __forceinline__ float mlp_forward(const MLPView &R, bf16x4 b0, bf16x4 b0l, f32x4 (&h1)[4],
                                              f32x4 (&dh1)[4], bf16x4 (&bh1)[4], f32x4 (&h2)[4], f32x4 (&dh2)[4]) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        // W1 s with both operands split: hi*hi + lo*hi + hi*lo
-        f32x4 z = mfma16(R.a1l[c], b0, zero);
-        z = mfma16(R.a1[c], b0l, z);
-        z = mfma16(R.a1[c], b0, z);
+        const f32x4 z = mlp_layer1(R, c, b0, b0l), b1 = R.b1(c);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             float h, dh;
-            silu(z[v] + R.b1[c][v], h, dh);
+            silu(z[v] + b1[v], h, dh);
             h1[c][v] = h;
             dh1[c][v] = dh;
         }
@@ -140,48 +178,53 @@ __device__ __forceinline__ float mlp_forward(const MLPRegs &R, bf16x4 b0, bf16x4
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         f32x4 z = zero;
+        const f32x4 b2 = R.b2(c);
 #pragma unroll
-        for (int kc = 0; kc < 4; kc++) z = mfma16(R.a2[c][kc], bh1[kc], z);
+        for (int kc = 0; kc < 4; kc++) z = mfma16(R.f(NF_A2 + 4 * c + kc), bh1[kc], z);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             float h, dh;
-            silu(z[v] + R.b2[c][v], h, dh);
+            silu(z[v] + b2[v], h, dh);
             h2[c][v] = h;
             dh2[c][v] = dh;
         }
     }
     float y = 0.f;
 #pragma unroll
-    for (int c = 0; c < 4; c++)
+    for (int c = 0; c < 4; c++) {
+        const f32x4 w3 = R.w3(c);
 #pragma unroll
-        for (int v = 0; v < 4; v++) y = fmaf(R.w3[c][v], h2[c][v], y);
+        for (int v = 0; v < 4; v++) y = fmaf(w3[v], h2[c][v], y);
+    }
     y += __shfl_xor(y, 16, 64);
     y += __shfl_xor(y, 32, 64);
-    return y + R.b3;
+    return y + R.N.b3;
 }
 
 // dy/d(standardised descriptor) of particle col, features 4q..4q+3
-__device__ __forceinline__ f32x4 mlp_input_grad(const MLPRegs &R, const f32x4 (&dh1)[4], const f32x4 (&dh2)[4]) {
+__device__ __forceinline__ f32x4 mlp_input_grad(const MLPView &R, const f32x4 (&dh1)[4], const f32x4 (&dh2)[4]) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     bf16x4 bg2[4], bg1[4], bg1l[4];
 #pragma unroll
-    for (int c = 0; c < 4; c++)
-        bg2[c] = pack4(R.w3[c][0] * dh2[c][0], R.w3[c][1] * dh2[c][1], R.w3[c][2] * dh2[c][2],
-                       R.w3[c][3] * dh2[c][3]);
+    for (int c = 0; c < 4; c++) {
+        const f32x4 w3 = R.w3(c);
+        bg2[c] = pack4(w3[0] * dh2[c][0], w3[1] * dh2[c][1], w3[2] * dh2[c][2], w3[3] * dh2[c][3]);
+    }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         f32x4 a = zero;
 #pragma unroll
-        for (int kc = 0; kc < 4; kc++) a = mfma16(R.a2t[c][kc], bg2[kc], a);
+        for (int kc = 0; kc < 4; kc++) a = mfma16(R.f(NF_A2T + 4 * c + kc), bg2[kc], a);
         split4(a[0] * dh1[c][0], a[1] * dh1[c][1], a[2] * dh1[c][2], a[3] * dh1[c][3], bg1[c], bg1l[c]);
     }
     // W1^T g1, both split like the forward first layer
     f32x4 d = zero;
 #pragma unroll
     for (int kc = 0; kc < 4; kc++) {
-        d = mfma16(R.a1tl[kc], bg1[kc], d);
-        d = mfma16(R.a1t[kc], bg1l[kc], d);
-        d = mfma16(R.a1t[kc], bg1[kc], d);
+        const bf16x4 a1t = R.f(NF_A1T + kc);
+        d = mfma16(R.f(NF_A1TL + kc), bg1[kc], d);
+        d = mfma16(a1t, bg1l[kc], d);
+        d = mfma16(a1t, bg1[kc], d);
     }
     return d;
 }
@@ -189,39 +232,50 @@ __device__ __forceinline__ f32x4 mlp_input_grad(const MLPRegs &R, const f32x4 (&
 // E and dE/dG (raw descriptor units) of n rows; one wave per 16-row tile.
 // IMG: the rows are the locals of a force evaluation, and a local's dE/dG goes
 // to its ghost images too (im.on), in place of a copy pass over the ghosts.
-template <bool WANT_D, bool IMG>
-__global__ __launch_bounds__(256) void k_mlp_eval(const float *__restrict__ p, const float *__restrict__ sc,
+template <bool WANT_D, bool IMG, int NT>
+__global__ __launch_bounds__(NT) void k_mlp_eval(const float *__restrict__ p, const float *__restrict__ sc,
                                                   const float *__restrict__ G, int n, float *__restrict__ E,
                                                   float *__restrict__ D, Images im) {
     const int lane = threadIdx.x & 63, q = lane >> 4, col = lane & 15;
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
+    const int wave = blockIdx.x * (NT / 64) + (threadIdx.x >> 6), nw = gridDim.x * (NT / 64);
     const int ntiles = (n + 15) >> 4;
-    if (wave >= ntiles) return;  // wave-uniform
-    MLPRegs R;
-    mlp_load<WANT_D>(R, p, sc, lane);
+    __shared__ MLPNet N;
+    // a tile's rows are loaded a turn ahead, the first before the weights
+    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+    int ni = 0;
+    const auto load = [&](int t) __attribute__((always_inline)) {
+        const int row = t * 16 + col;
+        if (row >= n) return;
+        g = *(const float4 *) (G + (size_t) row * MLP_ND + 4 * q);
+        if (IMG && im.on) ni = min(im.cnt[row], IMG_MAX);
+    };
+    load(wave);
+    mlp_stage<WANT_D, NT>(N, p, sc);
     for (int t = wave; t < ntiles; t += nw) {
+        mlp_keep_in_lds();
+        const MLPView R{N, lane, q};
         const int row = t * 16 + col;
         const bool ok = row < n;
-        float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (ok) g = *(const float4 *) (G + (size_t) row * MLP_ND + 4 * q);
         bf16x4 b0, b0l;
         split4(mlp_input(R, g), b0, b0l);
+        const int images = ni;
+        load(t + nw);
         f32x4 h1[4], dh1[4], h2[4], dh2[4];
         bf16x4 bh1[4];
         const float y = mlp_forward(R, b0, b0l, h1, dh1, bh1, h2, dh2);
-        if (ok && q == 0 && E) E[row] = fmaf(R.es, y, R.em);
+        if (ok && q == 0 && E) E[row] = fmaf(R.N.es, y, R.N.em);
         if (WANT_D) {
             const f32x4 d = mlp_input_grad(R, dh1, dh2);
+            const float4 gi = R.gi();
             if (ok) {
                 float4 o;
-                o.x = R.es * d[0] * R.gi[0];
-                o.y = R.es * d[1] * R.gi[1];
-                o.z = R.es * d[2] * R.gi[2];
-                o.w = R.es * d[3] * R.gi[3];
+                o.x = R.N.es * d[0] * gi.x;
+                o.y = R.N.es * d[1] * gi.y;
+                o.z = R.N.es * d[2] * gi.z;
+                o.w = R.N.es * d[3] * gi.w;
                 *(float4 *) (D + (size_t) row * MLP_ND + 4 * q) = o;
                 if (IMG && im.on) {
-                    const int ni = min(im.cnt[row], IMG_MAX);
-                    for (int k = 0; k < ni; k++) {
+                    for (int k = 0; k < images; k++) {
                         const int gq = im.tab[(size_t) k * im.cap + row].x;
                         *(float4 *) (D + (size_t) (n + gq) * MLP_ND + 4 * q) = o;
                     }
@@ -569,122 +623,164 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
     return x ^ (x >> 31);
 }
 
+// What the gradient kernels accumulate over the tiles of one partial: bias
+// gradients and output-weight gradient per lane ([4 c + v][lane]; b1, b2, w3),
+// then db3 and the squared error.
+constexpr int GACC = 50;
+
+// the sums over the 16 particles of a lane group, written to the partial
+__device__ __forceinline__ void mlp_write_bias(const float (&acc)[GACC][64], float *__restrict__ out,
+                                               float *__restrict__ loss, int wl, int lane) {
+    const int q = lane >> 4, col = lane & 15;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int k = 4 * wl + v;
+        float a = acc[k][lane], b = acc[16 + k][lane], w = acc[32 + k][lane];
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            a += __shfl_xor(a, o, 64); b += __shfl_xor(b, o, 64); w += __shfl_xor(w, o, 64);
+        }
+        if (col == 0) {
+            const int hh = 16 * wl + 4 * q + v;
+            out[MLP_B1 + hh] = a; out[MLP_B2 + hh] = b; out[MLP_W3 + hh] = w;
+        }
+    }
+    if (wl == 0) {
+        float gb3 = acc[48][lane], lsum = acc[49][lane];
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) { gb3 += __shfl_xor(gb3, o, 64); lsum += __shfl_xor(lsum, o, 64); }
+        if (lane == 0) { out[MLP_B3] = gb3; *loss = lsum; }
+    }
+}
+
+// the partial's weight gradients: wave wl holds rows 16 wl .. 16 wl + 15
+__device__ __forceinline__ void mlp_write_weights(const f32x4 (&gW2)[4], const f32x4 &gW1, float *__restrict__ out,
+                                                  int wl, int lane) {
+    const int q = lane >> 4, col = lane & 15;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = 16 * wl + 4 * q + v;
+#pragma unroll
+        for (int c1 = 0; c1 < 4; c1++) out[MLP_W2 + row * MLP_H + 16 * c1 + col] = gW2[c1][v];
+        out[MLP_W1 + row * MLP_ND + col] = gW1[v];
+    }
+}
+
 // Gradient of L = (1/B) sum_b (y_b - (label_b - e_mean) / e_std)^2 over one
-// minibatch.  Every wave takes the same number of 16-row tiles (batch is a
-// multiple of 16 * waves); weight gradients are K = 16-particle MFMAs on
-// transposed tiles staged in LDS; bias gradients are lane sums.
+// minibatch into nwaves partials, one workgroup each: partial w sums the
+// 16-row tiles w, w + nwaves, ... in that order.  The four waves take four
+// consecutive tiles of the partial at once -- forward and backward pass of a
+// tile are one long chain of MFMAs and exponentials, which bounds the kernel --
+// and hand them over transposed in LDS; then each wave accumulates its quarter
+// of the weight gradients (K = 16-particle MFMAs) over the four tiles in order,
+// and the waves add their lanes' bias terms in turn, so every sum has the order
+// of one wave walking the tiles.  Batch 4096: 22.5 us with one wave per
+// partial, 12.9 so.
 __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ p, const float *__restrict__ sc,
                                                   MLPTrain t, uint64_t seed, int step) {
-    __shared__ short lds[4][3 * MLP_H * 16 + MLP_ND * 16];
+    __shared__ MLPNet N;
+    __shared__ short s_tile[4][3 * MLP_H * 16 + MLP_ND * 16];
+    __shared__ float s_acc[GACC][64];
     const int lane = threadIdx.x & 63, q = lane >> 4, col = lane & 15, wl = threadIdx.x >> 6;
-    const int wave = blockIdx.x * 4 + wl, nw = gridDim.x * 4;
-    short *sD2 = lds[wl], *sH1 = sD2 + MLP_H * 16, *sD1 = sH1 + MLP_H * 16, *sG = sD1 + MLP_H * 16;
-    MLPRegs R;
-    mlp_load<true>(R, p, sc, lane);
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 gW2[4][4], gW1[4];
-    float gb1[4][4], gb2[4][4], gw3[4][4], gb3 = 0.f, lsum = 0.f;
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        gW1[a] = zero;
-#pragma unroll
-        for (int b = 0; b < 4; b++) { gW2[a][b] = zero; gb1[a][b] = 0.f; gb2[a][b] = 0.f; gw3[a][b] = 0.f; }
-    }
-    const float inv_es = 1.0f / R.es, scale = 2.0f / (float) t.batch;
-    const int ntiles = t.batch >> 4;
-    for (int tile = wave; tile < ntiles; tile += nw) {
-        const uint64_t j = (uint64_t) (tile * 16 + col);
+    const int part = blockIdx.x, np = gridDim.x;
+    for (int k = threadIdx.x; k < GACC * 64; k += 256) (&s_acc[0][0])[k] = 0.f;
+    const int mine = ((t.batch >> 4) - part + np - 1) / np;  // tiles of this partial
+    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+    float lab = 0.f;
+    const auto load = [&](int k) __attribute__((always_inline)) {  // row col of the partial's tile k
+        if (k >= mine) return;
+        const uint64_t j = (uint64_t) ((part + k * np) * 16 + col);
         const uint64_t h = splitmix64(seed ^ ((uint64_t) step << 32) ^ j);
         const int idx = (int) (h % (uint64_t) t.rows);
-        const float4 g = *(const float4 *) (t.G + (size_t) idx * MLP_ND + 4 * q);
-        const float lab = t.label[idx];
-        bf16x4 b0, b0l;
-        split4(mlp_input(R, g), b0, b0l);
+        g = *(const float4 *) (t.G + (size_t) idx * MLP_ND + 4 * q);
+        lab = t.label[idx];
+    };
+    load(wl);
+    mlp_stage<true, 256>(N, p, sc);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 gW2[4] = {zero, zero, zero, zero}, gW1 = zero;
+    const float inv_es = 1.0f / N.es, scale = 2.0f / (float) t.batch;
+    for (int t0 = 0; t0 < mine; t0 += 4) {
+        mlp_keep_in_lds();
+        const MLPView R{N, lane, q};
+        const int nt = min(4, mine - t0);
+        float a1[4][4], a2[4][4], h3[4][4], e = 0.f, err = 0.f;
+        if (wl < nt) {
+            short *sD2 = s_tile[wl], *sH1 = sD2 + MLP_H * 16, *sD1 = sH1 + MLP_H * 16, *sG = sD1 + MLP_H * 16;
+            bf16x4 b0, b0l;
+            split4(mlp_input(R, g), b0, b0l);
 #pragma unroll
-        for (int v = 0; v < 4; v++) sG[(4 * q + v) * 16 + col] = b0[v];
-        f32x4 h1[4], dh1[4], h2[4], dh2[4];
-        bf16x4 bh1[4];
-        const float y = mlp_forward(R, b0, b0l, h1, dh1, bh1, h2, dh2);
+            for (int v = 0; v < 4; v++) sG[(4 * q + v) * 16 + col] = b0[v];
+            f32x4 h1[4], dh1[4], h2[4], dh2[4];
+            bf16x4 bh1[4];
+            const float y = mlp_forward(R, b0, b0l, h1, dh1, bh1, h2, dh2);
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+            for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) sH1[(16 * c + 4 * q + v) * 16 + col] = bh1[c][v];
-        const float err = y - (lab - R.em) * inv_es;
-        const float e = scale * err;
-        if (q == 0) { lsum = fmaf(err, err, lsum); gb3 += e; }
-        bf16x4 bd2[4];
+                for (int v = 0; v < 4; v++) sH1[(16 * c + 4 * q + v) * 16 + col] = bh1[c][v];
+            err = y - (lab - N.em) * inv_es;
+            load(t0 + 4 + wl);
+            e = scale * err;
+            bf16x4 bd2[4];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 d2;
+            for (int c = 0; c < 4; c++) {
+                const f32x4 w3 = R.w3(c);
+                f32x4 d2;
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                gw3[c][v] = fmaf(e, h2[c][v], gw3[c][v]);
-                d2[v] = e * R.w3[c][v] * dh2[c][v];
-                gb2[c][v] += d2[v];
+                for (int v = 0; v < 4; v++) {
+                    h3[c][v] = h2[c][v];
+                    d2[v] = e * w3[v] * dh2[c][v];
+                    a2[c][v] = d2[v];
+                }
+                bd2[c] = pack4(d2);
+#pragma unroll
+                for (int v = 0; v < 4; v++) sD2[(16 * c + 4 * q + v) * 16 + col] = bd2[c][v];
             }
-            bd2[c] = pack4(d2);
 #pragma unroll
-            for (int v = 0; v < 4; v++) sD2[(16 * c + 4 * q + v) * 16 + col] = bd2[c][v];
-        }
+            for (int c = 0; c < 4; c++) {
+                f32x4 a = zero;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 a = zero;
+                for (int kc = 0; kc < 4; kc++) a = mfma16(R.f(NF_A2T + 4 * c + kc), bd2[kc], a);
 #pragma unroll
-            for (int kc = 0; kc < 4; kc++) a = mfma16(R.a2t[c][kc], bd2[kc], a);
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float d1 = a[v] * dh1[c][v];
-                gb1[c][v] += d1;
-                sD1[(16 * c + 4 * q + v) * 16 + col] = f2bf(d1);
+                for (int v = 0; v < 4; v++) {
+                    const float d1 = a[v] * dh1[c][v];
+                    a1[c][v] = d1;
+                    sD1[(16 * c + 4 * q + v) * 16 + col] = f2bf(d1);
+                }
             }
         }
-        __syncthreads();
+        for (int u = 0; u < nt; u++) {
+            if (u == wl) {
 #pragma unroll
-        for (int c2 = 0; c2 < 4; c2++) {
-            const bf16x4 a = *(const bf16x4 *) (sD2 + (16 * c2 + col) * 16 + 4 * q);
+                for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int c1 = 0; c1 < 4; c1++) {
-                const bf16x4 b = *(const bf16x4 *) (sH1 + (16 * c1 + col) * 16 + 4 * q);
-                gW2[c2][c1] = mfma16(a, b, gW2[c2][c1]);
+                    for (int v = 0; v < 4; v++) {
+                        const int k = 4 * c + v;
+                        s_acc[k][lane] += a1[c][v];
+                        s_acc[16 + k][lane] += a2[c][v];
+                        s_acc[32 + k][lane] = fmaf(e, h3[c][v], s_acc[32 + k][lane]);
+                    }
+                if (q == 0) {
+                    s_acc[48][lane] += e;
+                    s_acc[49][lane] = fmaf(err, err, s_acc[49][lane]);
+                }
             }
+            __syncthreads();
         }
-        const bf16x4 bg = *(const bf16x4 *) (sG + col * 16 + 4 * q);
+        for (int u = 0; u < nt; u++) {
+            const short *sD2 = s_tile[u], *sH1 = sD2 + MLP_H * 16, *sD1 = sH1 + MLP_H * 16, *sG = sD1 + MLP_H * 16;
+            const bf16x4 a = *(const bf16x4 *) (sD2 + (16 * wl + col) * 16 + 4 * q);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const bf16x4 a = *(const bf16x4 *) (sD1 + (16 * c + col) * 16 + 4 * q);
-            gW1[c] = mfma16(a, bg, gW1[c]);
+            for (int c1 = 0; c1 < 4; c1++)
+                gW2[c1] = mfma16(a, *(const bf16x4 *) (sH1 + (16 * c1 + col) * 16 + 4 * q), gW2[c1]);
+            gW1 = mfma16(*(const bf16x4 *) (sD1 + (16 * wl + col) * 16 + 4 * q),
+                         *(const bf16x4 *) (sG + col * 16 + 4 * q), gW1);
         }
         __syncthreads();
     }
-    float *out = t.partial + (size_t) wave * MLP_NP;
-#pragma unroll
-    for (int c2 = 0; c2 < 4; c2++)
-#pragma unroll
-        for (int c1 = 0; c1 < 4; c1++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) out[MLP_W2 + (16 * c2 + 4 * q + v) * MLP_H + 16 * c1 + col] = gW2[c2][c1][v];
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) out[MLP_W1 + (16 * c + 4 * q + v) * MLP_ND + col] = gW1[c][v];
-    // bias sums over the 16 particles of a lane group
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            float a = gb1[c][v], b = gb2[c][v], w = gw3[c][v];
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                a += __shfl_xor(a, o, 64); b += __shfl_xor(b, o, 64); w += __shfl_xor(w, o, 64);
-            }
-            if (col == 0) {
-                const int hh = 16 * c + 4 * q + v;
-                out[MLP_B1 + hh] = a; out[MLP_B2 + hh] = b; out[MLP_W3 + hh] = w;
-            }
-        }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) { gb3 += __shfl_xor(gb3, o, 64); lsum += __shfl_xor(lsum, o, 64); }
-    if (lane == 0) { out[MLP_B3] = gb3; t.loss[wave] = lsum; }
+    float *out = t.partial + (size_t) part * MLP_NP;
+    mlp_write_weights(gW2, gW1, out, wl, lane);
+    mlp_write_bias(s_acc, out, t.loss + part, wl, lane);
 }
 
 // SiLU with its first and second derivatives:
@@ -708,191 +804,187 @@ __device__ __forceinline__ void silu3(float z, float &h, float &dh, float &ddh) 
 //   db1 = bar z1, db2 = bar z2, dw3 = eps h2 + h2' dz2, db3 = eps.
 // Layer products and weight gradients are MFMAs in the layout of k_mlp_grad
 // (BF16 operands, FP32 accumulation; s and u enter the first layer as hi + lo
-// pairs).  Every wave runs the same number of tile iterations (tiles past the
-// end have eps = u = 0 and add exact zeros), so the block barriers are uniform.
+// pairs), and the tiles of a partial are shared among the waves of its
+// workgroup as there (2048 rows: 18 -> 12.2 us).  Tiles past the end have eps =
+// u = 0 and add exact zeros.
 __global__ __launch_bounds__(256) void k_mlp_cgrad(const float *__restrict__ p, const float *__restrict__ sc,
                                                    MLPCfgGrad t) {
-    __shared__ short lds[4][6 * MLP_H * 16 + 2 * MLP_ND * 16];
+    __shared__ MLPNet N;
+    __shared__ short s_tile[4][6 * MLP_H * 16 + 2 * MLP_ND * 16];
+    __shared__ float s_acc[GACC][64];
     const int lane = threadIdx.x & 63, q = lane >> 4, col = lane & 15, wl = threadIdx.x >> 6;
-    const int wave = blockIdx.x * 4 + wl, nw = gridDim.x * 4;
-    short *sZ2 = lds[wl], *sH1 = sZ2 + MLP_H * 16, *sT2 = sH1 + MLP_H * 16, *sTH1 = sT2 + MLP_H * 16;
-    short *sZ1 = sTH1 + MLP_H * 16, *sT1 = sZ1 + MLP_H * 16, *sS = sT1 + MLP_H * 16, *sU = sS + MLP_ND * 16;
-    MLPRegs R;
-    mlp_load<true>(R, p, sc, lane);
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 gW2[4][4], gW1[4];
-    float gb1[4][4], gb2[4][4], gw3[4][4], gb3 = 0.f, lsum = 0.f;
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        gW1[a] = zero;
-#pragma unroll
-        for (int b = 0; b < 4; b++) { gW2[a][b] = zero; gb1[a][b] = 0.f; gb2[a][b] = 0.f; gw3[a][b] = 0.f; }
-    }
-    const float inv_es = 1.0f / R.es;
+    const int part = blockIdx.x, np = gridDim.x;
+    for (int k = threadIdx.x; k < GACC * 64; k += 256) (&s_acc[0][0])[k] = 0.f;
     const int ntiles = (t.n + 15) >> 4;
-    const int iters = (ntiles + nw - 1) / nw;
-    for (int it = 0; it < iters; it++) {
-        const int row = (wave + it * nw) * 16 + col;
-        const bool ok = row < t.n;
-        float4 g = make_float4(0.f, 0.f, 0.f, 0.f), uu = g;
-        double lab = 0.0;
-        if (ok) {
-            g = *(const float4 *) (t.G + (size_t) row * MLP_ND + 4 * q);
-            uu = *(const float4 *) (t.U + (size_t) row * MLP_ND + 4 * q);
-            lab = t.label[row];
-        }
-        bf16x4 b0, b0l, u0, u0l;
-        split4(mlp_input(R, g), b0, b0l);
-        split4(uu.x, uu.y, uu.z, uu.w, u0, u0l);
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            sS[(4 * q + v) * 16 + col] = b0[v];
-            sU[(4 * q + v) * 16 + col] = u0[v];
-        }
-        // forward, keeping h, h' and h'' of both layers
-        f32x4 h1[4], d1[4], e1[4], h2[4], d2[4], e2[4];
-        bf16x4 bh1[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 z = mfma16(R.a1l[c], b0, zero);
-            z = mfma16(R.a1[c], b0l, z);
-            z = mfma16(R.a1[c], b0, z);
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                float h, dh, ddh;
-                silu3(z[v] + R.b1[c][v], h, dh, ddh);
-                h1[c][v] = h; d1[c][v] = dh; e1[c][v] = ddh;
-            }
-            bh1[c] = pack4(h1[c]);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 z = zero;
-#pragma unroll
-            for (int kc = 0; kc < 4; kc++) z = mfma16(R.a2[c][kc], bh1[kc], z);
+    const int iters = (ntiles + np - 1) / np;
+    float4 g, uu;
+    double lab;
+    bool ok;
+    const auto load = [&](int k) __attribute__((always_inline)) {  // row col of the partial's tile k
+        const int row = (part + k * np) * 16 + col;
+        ok = k < iters && row < t.n;
+        g = uu = make_float4(0.f, 0.f, 0.f, 0.f);
+        lab = 0.0;
+        if (!ok) return;
+        g = *(const float4 *) (t.G + (size_t) row * MLP_ND + 4 * q);
+        uu = *(const float4 *) (t.U + (size_t) row * MLP_ND + 4 * q);
+        lab = t.label[row];
+    };
+    load(wl);
+    mlp_stage<true, 256>(N, p, sc);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 gW2[4] = {zero, zero, zero, zero}, gW1 = zero;
+    const float inv_es = 1.0f / N.es;
+    for (int t0 = 0; t0 < iters; t0 += 4) {
+        mlp_keep_in_lds();
+        const MLPView R{N, lane, q};
+        const int nt = min(4, iters - t0);
+        float a1[4][4], a2[4][4], h3[4][4], d3[4][4], x3[4][4], e = 0.f, err = 0.f;
+        if (wl < nt) {
+            short *sZ2 = s_tile[wl], *sH1 = sZ2 + MLP_H * 16, *sT2 = sH1 + MLP_H * 16, *sTH1 = sT2 + MLP_H * 16;
+            short *sZ1 = sTH1 + MLP_H * 16, *sT1 = sZ1 + MLP_H * 16, *sS = sT1 + MLP_H * 16, *sU = sS + MLP_ND * 16;
+            bf16x4 b0, b0l, u0, u0l;
+            split4(mlp_input(R, g), b0, b0l);
+            split4(uu.x, uu.y, uu.z, uu.w, u0, u0l);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                float h, dh, ddh;
-                silu3(z[v] + R.b2[c][v], h, dh, ddh);
-                h2[c][v] = h; d2[c][v] = dh; e2[c][v] = ddh;
+                sS[(4 * q + v) * 16 + col] = b0[v];
+                sU[(4 * q + v) * 16 + col] = u0[v];
+            }
+            // forward, keeping h, h' and h'' of both layers
+            f32x4 h1[4], d1[4], e1[4], h2[4], d2[4], e2[4];
+            bf16x4 bh1[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const f32x4 z = mlp_layer1(R, c, b0, b0l), b1 = R.b1(c);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    float h, dh, ddh;
+                    silu3(z[v] + b1[v], h, dh, ddh);
+                    h1[c][v] = h; d1[c][v] = dh; e1[c][v] = ddh;
+                }
+                bh1[c] = pack4(h1[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                f32x4 z = zero;
+                const f32x4 b2 = R.b2(c);
+#pragma unroll
+                for (int kc = 0; kc < 4; kc++) z = mfma16(R.f(NF_A2 + 4 * c + kc), bh1[kc], z);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    float h, dh, ddh;
+                    silu3(z[v] + b2[v], h, dh, ddh);
+                    h2[c][v] = h; d2[c][v] = dh; e2[c][v] = ddh;
+                }
+            }
+            float y = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const f32x4 w3 = R.w3(c);
+#pragma unroll
+                for (int v = 0; v < 4; v++) y = fmaf(w3[v], h2[c][v], y);
+            }
+            y += __shfl_xor(y, 16, 64);
+            y += __shfl_xor(y, 32, 64);
+            y += N.b3;
+            err = ok ? y - ((float) lab - N.em) * inv_es : 0.0f;
+            load(t0 + 4 + wl);
+            e = t.eps_scale * err;
+            // tangent along u
+            f32x4 t1[4];
+            bf16x4 bth1[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                t1[c] = mlp_layer1(R, c, u0, u0l);
+                bth1[c] = pack4(d1[c][0] * t1[c][0], d1[c][1] * t1[c][1], d1[c][2] * t1[c][2], d1[c][3] * t1[c][3]);
+            }
+            bf16x4 bz2[4], bt2[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                f32x4 t2 = zero;
+                const f32x4 w3 = R.w3(c);
+#pragma unroll
+                for (int kc = 0; kc < 4; kc++) t2 = mfma16(R.f(NF_A2 + 4 * c + kc), bth1[kc], t2);
+                f32x4 z2b, t2b;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float w = w3[v];
+                    h3[c][v] = h2[c][v];
+                    d3[c][v] = d2[c][v];
+                    x3[c][v] = t2[v];
+                    t2b[v] = w * d2[c][v];
+                    z2b[v] = w * fmaf(e, d2[c][v], e2[c][v] * t2[v]);
+                    a2[c][v] = z2b[v];
+                }
+                bz2[c] = pack4(z2b);
+                bt2[c] = pack4(t2b);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int f = (16 * c + 4 * q + v) * 16 + col;
+                    sZ2[f] = bz2[c][v];
+                    sT2[f] = bt2[c][v];
+                    sH1[f] = bh1[c][v];
+                    sTH1[f] = bth1[c][v];
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                f32x4 a = zero, at = zero;
+#pragma unroll
+                for (int kc = 0; kc < 4; kc++) {
+                    const bf16x4 w = R.f(NF_A2T + 4 * c + kc);
+                    a = mfma16(w, bz2[kc], a);
+                    at = mfma16(w, bt2[kc], at);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float z1b = fmaf(at[v] * e1[c][v], t1[c][v], a[v] * d1[c][v]);
+                    a1[c][v] = z1b;
+                    const int f = (16 * c + 4 * q + v) * 16 + col;
+                    sZ1[f] = f2bf(z1b);
+                    sT1[f] = f2bf(at[v] * d1[c][v]);
+                }
             }
         }
-        float y = 0.f;
+        // the waves in turn; dw3 = eps h2 + h2' dz2
+        for (int u = 0; u < nt; u++) {
+            if (u == wl) {
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+                for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) y = fmaf(R.w3[c][v], h2[c][v], y);
-        y += __shfl_xor(y, 16, 64);
-        y += __shfl_xor(y, 32, 64);
-        y += R.b3;
-        const float err = ok ? y - ((float) lab - R.em) * inv_es : 0.0f;
-        const float e = t.eps_scale * err;
-        if (q == 0) { lsum = fmaf(err, err, lsum); gb3 += e; }
-        // tangent along u
-        f32x4 t1[4];
-        bf16x4 bth1[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 z = mfma16(R.a1l[c], u0, zero);
-            z = mfma16(R.a1[c], u0l, z);
-            t1[c] = mfma16(R.a1[c], u0, z);
-            bth1[c] = pack4(d1[c][0] * t1[c][0], d1[c][1] * t1[c][1], d1[c][2] * t1[c][2], d1[c][3] * t1[c][3]);
+                    for (int v = 0; v < 4; v++) {
+                        const int k = 4 * c + v;
+                        s_acc[k][lane] += a1[c][v];
+                        s_acc[16 + k][lane] += a2[c][v];
+                        s_acc[32 + k][lane] = fmaf(e, h3[c][v], fmaf(d3[c][v], x3[c][v], s_acc[32 + k][lane]));
+                    }
+                if (q == 0) {
+                    s_acc[48][lane] += e;
+                    s_acc[49][lane] = fmaf(err, err, s_acc[49][lane]);
+                }
+            }
+            __syncthreads();
         }
-        bf16x4 bz2[4], bt2[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 t2 = zero;
-#pragma unroll
-            for (int kc = 0; kc < 4; kc++) t2 = mfma16(R.a2[c][kc], bth1[kc], t2);
-            f32x4 z2b, t2b;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float w = R.w3[c][v];
-                gw3[c][v] = fmaf(e, h2[c][v], fmaf(d2[c][v], t2[v], gw3[c][v]));
-                t2b[v] = w * d2[c][v];
-                z2b[v] = w * fmaf(e, d2[c][v], e2[c][v] * t2[v]);
-                gb2[c][v] += z2b[v];
-            }
-            bz2[c] = pack4(z2b);
-            bt2[c] = pack4(t2b);
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int f = (16 * c + 4 * q + v) * 16 + col;
-                sZ2[f] = bz2[c][v];
-                sT2[f] = bt2[c][v];
-                sH1[f] = bh1[c][v];
-                sTH1[f] = bth1[c][v];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 a = zero, at = zero;
-#pragma unroll
-            for (int kc = 0; kc < 4; kc++) {
-                a = mfma16(R.a2t[c][kc], bz2[kc], a);
-                at = mfma16(R.a2t[c][kc], bt2[kc], at);
-            }
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float z1b = fmaf(at[v] * e1[c][v], t1[c][v], a[v] * d1[c][v]);
-                gb1[c][v] += z1b;
-                const int f = (16 * c + 4 * q + v) * 16 + col;
-                sZ1[f] = f2bf(z1b);
-                sT1[f] = f2bf(at[v] * d1[c][v]);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int c2 = 0; c2 < 4; c2++) {
-            const bf16x4 az = *(const bf16x4 *) (sZ2 + (16 * c2 + col) * 16 + 4 * q);
-            const bf16x4 at = *(const bf16x4 *) (sT2 + (16 * c2 + col) * 16 + 4 * q);
+        for (int u = 0; u < nt; u++) {
+            const short *sZ2 = s_tile[u], *sH1 = sZ2 + MLP_H * 16, *sT2 = sH1 + MLP_H * 16, *sTH1 = sT2 + MLP_H * 16;
+            const short *sZ1 = sTH1 + MLP_H * 16, *sT1 = sZ1 + MLP_H * 16, *sS = sT1 + MLP_H * 16, *sU = sS + MLP_ND * 16;
+            const int at_row = (16 * wl + col) * 16 + 4 * q;
+            const bf16x4 az = *(const bf16x4 *) (sZ2 + at_row), at = *(const bf16x4 *) (sT2 + at_row);
 #pragma unroll
             for (int c1 = 0; c1 < 4; c1++) {
-                const bf16x4 bh = *(const bf16x4 *) (sH1 + (16 * c1 + col) * 16 + 4 * q);
-                const bf16x4 bt = *(const bf16x4 *) (sTH1 + (16 * c1 + col) * 16 + 4 * q);
-                gW2[c2][c1] = mfma16(az, bh, gW2[c2][c1]);
-                gW2[c2][c1] = mfma16(at, bt, gW2[c2][c1]);
+                const int b = (16 * c1 + col) * 16 + 4 * q;
+                gW2[c1] = mfma16(az, *(const bf16x4 *) (sH1 + b), gW2[c1]);
+                gW2[c1] = mfma16(at, *(const bf16x4 *) (sTH1 + b), gW2[c1]);
             }
-        }
-        const bf16x4 bs = *(const bf16x4 *) (sS + col * 16 + 4 * q);
-        const bf16x4 bu = *(const bf16x4 *) (sU + col * 16 + 4 * q);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const bf16x4 az = *(const bf16x4 *) (sZ1 + (16 * c + col) * 16 + 4 * q);
-            const bf16x4 at = *(const bf16x4 *) (sT1 + (16 * c + col) * 16 + 4 * q);
-            gW1[c] = mfma16(az, bs, gW1[c]);
-            gW1[c] = mfma16(at, bu, gW1[c]);
+            gW1 = mfma16(*(const bf16x4 *) (sZ1 + at_row), *(const bf16x4 *) (sS + col * 16 + 4 * q), gW1);
+            gW1 = mfma16(*(const bf16x4 *) (sT1 + at_row), *(const bf16x4 *) (sU + col * 16 + 4 * q), gW1);
         }
         __syncthreads();
     }
-    float *out = t.partial + (size_t) wave * MLP_NP;
-#pragma unroll
-    for (int c2 = 0; c2 < 4; c2++)
-#pragma unroll
-        for (int c1 = 0; c1 < 4; c1++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) out[MLP_W2 + (16 * c2 + 4 * q + v) * MLP_H + 16 * c1 + col] = gW2[c2][c1][v];
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) out[MLP_W1 + (16 * c + 4 * q + v) * MLP_ND + col] = gW1[c][v];
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            float a = gb1[c][v], b = gb2[c][v], w = gw3[c][v];
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                a += __shfl_xor(a, o, 64); b += __shfl_xor(b, o, 64); w += __shfl_xor(w, o, 64);
-            }
-            if (col == 0) {
-                const int hh = 16 * c + 4 * q + v;
-                out[MLP_B1 + hh] = a; out[MLP_B2 + hh] = b; out[MLP_W3 + hh] = w;
-            }
-        }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) { gb3 += __shfl_xor(gb3, o, 64); lsum += __shfl_xor(lsum, o, 64); }
-    if (lane == 0) { out[MLP_B3] = gb3; t.loss[wave] = lsum; }
+    float *out = t.partial + (size_t) part * MLP_NP;
+    mlp_write_weights(gW2, gW1, out, wl, lane);
+    mlp_write_bias(s_acc, out, t.loss + part, wl, lane);
 }
 
 // rho_i = 2 w_force (F_i - F*_i) / sum_j |F*_j|^2 for the locals; the sum is
@@ -927,27 +1019,42 @@ __global__ __launch_bounds__(256) void k_mlp_ghost_rho(const int *__restrict__ c
     }
 }
 
+// parameter k of the gradient: the partials added in order.  Thirty-two
+// loads are in flight before the first is added (64 partials: 16.6 us with one
+// load a turn, 4.3 so).
+__device__ __forceinline__ float sum_partials(const float *__restrict__ partial, int n, int k) {
+    float s = 0.f;
+    int w = 0;
+    for (; w + 32 <= n; w += 32) {
+        float v[32];
+#pragma unroll
+        for (int u = 0; u < 32; u++) v[u] = partial[(size_t) (w + u) * MLP_NP + k];
+#pragma unroll
+        for (int u = 0; u < 32; u++) s += v[u];
+    }
+    for (; w < n; w++) s += partial[(size_t) w * MLP_NP + k];
+    return s;
+}
+
 // acc += sum over waves of the gradient partials (in wave order); with out,
 // the sum itself is also written there
-__global__ __launch_bounds__(256) void k_mlp_accum(const float *__restrict__ partial, int nwaves,
+__global__ __launch_bounds__(64) void k_mlp_accum(const float *__restrict__ partial, int nwaves,
                                                    float *__restrict__ acc, float *__restrict__ out) {
-    const int k = blockIdx.x * 256 + threadIdx.x;
+    const int k = blockIdx.x * 64 + threadIdx.x;
     if (k >= MLP_NP) return;
-    float s = 0.f;
-    for (int w = 0; w < nwaves; w++) s += partial[(size_t) w * MLP_NP + k];
+    const float s = sum_partials(partial, nwaves, k);
     if (acc) acc[k] += s;
     if (out) out[k] = s;
 }
 
 // Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the summed wave partials
-__global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
+__global__ __launch_bounds__(64) void k_mlp_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
                                                   const float *__restrict__ partial, const float *__restrict__ loss,
                                                   int nwaves, int batch, float lr, float bc1, float bc2,
                                                   float gscale, float *__restrict__ loss_out) {
-    const int k = blockIdx.x * 256 + threadIdx.x;
+    const int k = blockIdx.x * 64 + threadIdx.x;
     if (k < MLP_NP) {
-        float gsum = 0.f;
-        for (int w = 0; w < nwaves; w++) gsum += partial[(size_t) w * MLP_NP + k];
+        float gsum = sum_partials(partial, nwaves, k);
         gsum *= gscale;
         const float mm = 0.9f * m[k] + 0.1f * gsum;
         const float vv = 0.999f * v[k] + 0.001f * gsum * gsum;
@@ -957,6 +1064,7 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ p, float *
     }
     if (k == 0 && loss_out) {
         float s = 0.f;
+#pragma unroll 16
         for (int w = 0; w < nwaves; w++) s += loss[w];
         *loss_out = s / (float) batch;
     }
@@ -1053,19 +1161,31 @@ void launch_mlp_descriptors(hipStream_t s, const DevState &d, const Geom &g, int
     launch_mlp_wave<0, false>(s, d, A);
 }
 
-// each wave converts the weights to BF16 registers once (about 21 KB read)
-// and then strides over 16-row tiles: 512 workgroups (two waves per SIMD)
-// amortise that over several tiles at 131072 rows
-static int eval_grid(int n) {
-    const int ntiles = (n + 15) / 16;
-    return std::max(1, std::min((ntiles + 3) / 4, 512));
+// k_mlp_eval by rows: workgroups of 16 waves convert the weights once per CU and
+// let four tiles share each SIMD, in at most 256 workgroups (one per CU); few
+// rows spread better over workgroups of 4.  Measured, 4 waves | 16: 2048 rows
+// 9.6 | 11.1 us; a step at 8400 rows 98.6 | 96.9, at 35152 100.2 | 97.8, at
+// 131072 167.5 | 164.1 (the pass itself 23 | 18 us).
+template <bool WANT_D, bool IMG, int NT>
+static void eval_launch(hipStream_t s, const float *p, const float *sc, const float *G, int n, float *E, float *D,
+                        const Images &im) {
+    const int ntiles = (n + 15) / 16, per = NT / 64;
+    const int grid = std::min((ntiles + per - 1) / per, 256);
+    hipLaunchKernelGGL((k_mlp_eval<WANT_D, IMG, NT>), dim3(grid), dim3(NT), 0, s, p, sc, G, n, E, D, im);
+}
+
+template <bool WANT_D, bool IMG>
+static void eval_any(hipStream_t s, const float *p, const float *sc, const float *G, int n, float *E, float *D,
+                     const Images &im) {
+    if (n < 8192) eval_launch<WANT_D, IMG, 256>(s, p, sc, G, n, E, D, im);
+    else eval_launch<WANT_D, IMG, 1024>(s, p, sc, G, n, E, D, im);
 }
 
 void launch_mlp_eval(hipStream_t s, const float *p, const float *sc, const float *G, int n, float *E, float *D) {
     if (n <= 0) return;
     const Images none{};
-    if (D) hipLaunchKernelGGL((k_mlp_eval<true, false>), dim3(eval_grid(n)), dim3(256), 0, s, p, sc, G, n, E, D, none);
-    else hipLaunchKernelGGL((k_mlp_eval<false, false>), dim3(eval_grid(n)), dim3(256), 0, s, p, sc, G, n, E, D, none);
+    if (D) eval_any<true, false>(s, p, sc, G, n, E, D, none);
+    else eval_any<false, false>(s, p, sc, G, n, E, D, none);
 }
 
 void launch_mlp_forces(hipStream_t s, const DevState &d, const Geom &g, const MLPBind &b, int cur, int reduce,
@@ -1073,8 +1193,7 @@ void launch_mlp_forces(hipStream_t s, const DevState &d, const Geom &g, const ML
     if (d.nlocal <= 0) return;
     launch_mlp_descriptors(s, d, g, cur, b.G, pack);
     const Images im = images_of(d, true);
-    hipLaunchKernelGGL((k_mlp_eval<true, true>), dim3(eval_grid(d.nlocal)), dim3(256), 0, s, b.p, b.sc, b.G, d.nlocal,
-                       b.E, b.D, im);
+    eval_any<true, true>(s, b.p, b.sc, b.G, d.nlocal, b.E, b.D, im);
     if (!im.on)
         hipLaunchKernelGGL(k_mlp_ghost_d, dim3(std::max(ghost_grid, 1)), dim3(256), 0, s, d.counters, d.sync_src, b.D);
     MLPSegArgs A = seg_args(d, cur);
@@ -1098,13 +1217,13 @@ void launch_mlp_forces(hipStream_t s, const DevState &d, const Geom &g, const ML
 }
 
 void launch_mlp_grad(hipStream_t s, const float *p, const float *sc, const MLPTrain &t, uint64_t seed, int step) {
-    hipLaunchKernelGGL(k_mlp_grad, dim3(t.nwaves / 4), dim3(256), 0, s, p, sc, t, seed, step);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(t.nwaves), dim3(256), 0, s, p, sc, t, seed, step);
 }
 
 void launch_mlp_adam(hipStream_t s, float *p, float *m, float *v, const MLPTrain &t, float lr, int step,
                      float *loss_out) {
     const float bc1 = 1.0f - powf(0.9f, (float) step), bc2 = 1.0f - powf(0.999f, (float) step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NP + 255) / 256), dim3(256), 0, s, p, m, v, t.partial, t.loss,
+    hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NP + 63) / 64), dim3(64), 0, s, p, m, v, t.partial, t.loss,
                        t.nwaves, t.batch, lr, bc1, bc2, t.gscale, loss_out);
 }
 
@@ -1132,11 +1251,11 @@ void launch_mlp_config_grad(hipStream_t s, const DevState &d, const Geom &g, con
     tt.U = U;
     tt.n = n;
     tt.eps_scale = (float) (2.0 * w_energy / n);
-    hipLaunchKernelGGL(k_mlp_cgrad, dim3(tt.nwaves / 4), dim3(256), 0, s, b.p, b.sc, tt);
+    hipLaunchKernelGGL(k_mlp_cgrad, dim3(tt.nwaves), dim3(256), 0, s, b.p, b.sc, tt);
 }
 
 void launch_mlp_accum(hipStream_t s, const float *partial, int nwaves, float *acc, float *out) {
-    hipLaunchKernelGGL(k_mlp_accum, dim3((MLP_NP + 255) / 256), dim3(256), 0, s, partial, nwaves, acc, out);
+    hipLaunchKernelGGL(k_mlp_accum, dim3((MLP_NP + 63) / 64), dim3(64), 0, s, partial, nwaves, acc, out);
 }
 
 void launch_mlp_moments(hipStream_t s, const float *G, const float *label, int n, double *partials, int nblocks) {

@@ -76,7 +76,7 @@ struct MLPTrain {
     const float *label;  // [rows] per-atom energies
     int rows;            // sample from [0, rows)
     int batch;           // rows per step (a multiple of 16)
-    int nwaves;          // waves of the gradient launch
+    int nwaves;          // partials (workgroups of the gradient launch)
     float *partial;      // [nwaves][MLP_NP]
     float *loss;         // [nwaves] partial squared errors
     float gscale = 1.0f; // Adam takes gscale * (sum of the partials)
@@ -90,14 +90,14 @@ struct MLPCfgGrad {
     const float *U;
     int n;
     float eps_scale;     // 2 w_energy / n
-    int nwaves;          // waves of the launch (a multiple of 4)
+    int nwaves;          // partials (workgroups of the launch)
     float *partial;      // [nwaves][MLP_NP]
     float *loss;         // [nwaves] partial sums of the squared standardised energy error
 };
 // gradient of the mean squared error of the standardised energy over one
 // minibatch (rows chosen by a counter hash of seed and step)
 void launch_mlp_grad(hipStream_t s, const float *p, const float *sc, const MLPTrain &t, uint64_t seed, int step);
-// sum the wave partials and take one Adam step (t = 1, 2, ...)
+// sum the partials and take one Adam step (t = 1, 2, ...)
 void launch_mlp_adam(hipStream_t s, float *p, float *m, float *v, const MLPTrain &t, float lr, int step,
                      float *loss_out);
 // Gradient of one configuration's loss on buffer `cur` (lists current):

@@ -117,3 +117,93 @@ def test_dem_contacts_vs_oracle(case):
         for name, p, q in [(k, g.get(k), o.get(k)) for k in ("position", "linear_velocity", "angular_velocity",
                                                               "force", "torque")]:
             assert np.abs(p - q).max() <= 1e-10 * max(np.abs(q).max(), 1e-300), (b, name)
+
+
+# k_mlp_eval takes workgroups of 4 waves below 8192 rows, of 16 from there; past
+# 65536 rows a wave walks several tiles
+@pytest.mark.parametrize("n", [1, 15, 17, 8191, 8192, 8193, 65537, 131089])
+def test_mlp_eval_vs_oracle_at_size_edges(n):
+    """energies and dE/dG against the BF16-emulating oracle at the tolerance of
+    the 1000-row test, on 300 rows drawn from all of them, and the first and
+    last 20; equal descriptors give equal results wherever their row lies"""
+    from oracle import mlp_oracle as mo
+    from pairs_amd import mlp
+    rng = np.random.default_rng(n)
+    p = mo.xavier(7).astype(np.float32)
+    sc = np.concatenate([rng.uniform(0.0, 3.0, 16), rng.uniform(0.3, 2.0, 16), [-5.5, 0.7]]).astype(np.float32)
+    m = mlp.MLPModel(seed=1)
+    m.set_params(p, sc)
+    base = rng.uniform(0.0, 4.0, (1000, 16)).astype(np.float32)
+    pick = rng.integers(0, 1000, n)
+    E, D = m.eval(base[pick])
+    Eb, Db = mo.forward_bf16(p, sc, base)
+    rows = np.unique(np.concatenate([np.arange(min(n, 20)), np.arange(max(n - 20, 0), n), rng.integers(0, n, 300)]))
+    err = np.sqrt(np.mean((E[rows] - Eb[pick[rows]]) ** 2))
+    assert err < 5e-3 * Eb.std(), err
+    ref = Db[pick[rows]]
+    assert np.sqrt(np.mean((D[rows] - ref) ** 2)) < 5e-3 * np.sqrt(np.mean(ref ** 2))
+    E0, D0 = m.eval(base)
+    assert np.array_equal(E, E0[pick]) and np.array_equal(D, D0[pick])
+
+
+# a partial's tiles are taken four at a time: 1, 3, 4, 5 and 9 of them
+@pytest.mark.parametrize("tiles", [1, 3, 4, 5, 9])
+def test_mlp_energy_grad_vs_oracle_by_tiles(tiles):
+    """k_mlp_grad on a minibatch of 64 partials of `tiles` 16-row tiles, at the
+    tolerance of the one-tile test"""
+    from oracle import mlp_oracle as mo
+    from pairs_amd import mlp
+    import test_gpu_mlp as tm
+    rng = np.random.default_rng(tiles)
+    rows, batch, seed, step = 3000, 1024 * tiles, 11, 5
+    G = rng.uniform(0.0, 4.0, (rows, 16)).astype(np.float32)
+    lab = rng.normal(-5.0, 0.8, rows).astype(np.float32)
+    p, sc = mo.xavier(5).astype(np.float32), tm._scale().astype(np.float32)
+    m = mlp.MLPModel(seed=1, dataset_capacity=rows)
+    m.set_params(p, sc)
+    assert m.add_rows(G, lab) == rows
+    g, loss = m.energy_grad(step, batch=batch, seed=seed)
+    idx = np.array([tm._splitmix64(seed ^ (step << 32) ^ j) % rows for j in range(batch)])
+    Lr, ref = mo.energy_loss_grad(p.astype(np.float64), sc.astype(np.float64), G[idx].astype(np.float64),
+                                  lab[idx].astype(np.float64))
+    assert abs(loss - Lr) <= 2e-2 * Lr, (loss, Lr)
+    tm._check_grad(g, ref, f"{tiles} tiles")
+
+
+# 864 to 5324 atoms: 1 to 6 tiles in a partial of k_mlp_cgrad, ragged ones among them
+@pytest.mark.parametrize("cells", [6, 9, 10, 11])
+def test_mlp_config_grad_vs_oracle_by_tiles(cells):
+    from oracle import mlp_oracle as mo
+    from pairs_amd import mlp
+    import test_gpu_mlp as tm
+    s, L = tm._state(cells, 40)
+    x = s.positions()
+    El, Fl = mo.lj_atom_energy(x, L), mo.lj_forces(x, L)
+    G = mo.descriptors(x, L)
+    sc = np.concatenate([G.mean(0), 1.0 / G.std(0), [El.mean(), El.std()]]).astype(np.float32)
+    p = mo.xavier(5).astype(np.float32)
+    m = mlp.MLPModel(seed=1, dataset_capacity=16)
+    m.set_params(p, sc)
+    g, (le, lf) = m.config_grad(s, 0.5, 1.0)
+    _, le_r, lf_r, ref = mo.config_loss_grad(p.astype(np.float64), sc.astype(np.float64), x, L, El, Fl, 0.5, 1.0)
+    assert abs(le - le_r) <= 3e-2 * le_r and abs(lf - lf_r) <= 3e-2 * lf_r
+    tm._check_grad(g, ref, f"{len(x)} atoms")
+
+
+# 6912 and 8788 atoms: either side of k_mlp_eval's rule, with its writes to ghost images
+@pytest.mark.parametrize("cells", [12, 13])
+def test_mlp_forces_vs_oracle_at_size_edges(cells):
+    from oracle import mlp_oracle as mo
+    from pairs_amd import mlp
+    import test_gpu_mlp as tm
+    s, L = tm._state(cells, 40)
+    x = s.positions()
+    G = mo.descriptors(x, L)
+    p = mo.xavier(5).astype(np.float32)
+    sc = np.concatenate([G.mean(0), 1.0 / G.std(0), [-5.5, 0.7]]).astype(np.float32)
+    m = mlp.MLPModel(seed=1)
+    m.set_params(p, sc)
+    e, _ = mlp.forces(s, m)
+    Fx, Ex = mo.forces(p, sc, x, L)
+    assert tm._rel_rms(s.forces(), Fx) < 3e-2
+    assert abs(e - Ex.sum()) < 1e-3 * abs(Ex.sum())
