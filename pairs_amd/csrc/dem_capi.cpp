@@ -91,7 +91,8 @@ static void free_arrays(DemPtrs &p) {
     void *ptrs[] = {p.x, p.y, p.z, p.vx, p.vy, p.vz, p.wx, p.wy, p.wz, p.fx, p.fy, p.fz, p.tx, p.ty, p.tz, p.r, p.m,
                     p.nx, p.ny, p.nz, p.inv_i, p.rot_m, p.rot_q, p.uid, p.flags, p.type, p.shape, p.num_contacts,
                     p.c_uid, p.c_used, p.c_stick, p.c_tsd, p.c_ivm, p.cell_count, p.cell_start, p.cell_slot,
-                    p.cell_particles, p.particle_cell, p.corder, p.cmixed, p.crec, p.rec, p.send_map, p.send_mult, p.exchg_flag, p.copy_to,
+                    p.cell_particles, p.particle_cell, p.corder, p.cmixed, p.crec, p.rec, p.cell_scan, p.leavers, p.send_map, p.send_side,
+                    p.exchg_flag, p.copy_to,
                     p.blk, p.scan_tmp, p.buf, p.hbuf, p.cand_n, p.cand};
     for (void *q : ptrs)
         if (q) hipFree(q);
@@ -130,12 +131,14 @@ static int alloc_arrays(pairs_hip_dem_ctx *ctx, DemPtrs &p, size_t C, size_t K, 
     const size_t NC = (size_t) ctx->ncells_cap;
     r |= dalloc(ctx, &p.cell_count, NC + 1);
     r |= dalloc(ctx, &p.cell_start, NC + 1);
+    r |= dalloc(ctx, &p.cell_scan, NC + 1);
     r |= dalloc(ctx, &p.cell_particles, C);
     r |= dalloc(ctx, &p.scan_tmp, NC / 1024 + 8);
     r |= dalloc(ctx, &p.send_map, S);
-    r |= dalloc(ctx, &p.send_mult, 3 * S);
+    r |= dalloc(ctx, &p.send_side, S);
     r |= dalloc(ctx, &p.copy_to, S);
-    r |= dalloc(ctx, &p.blk, 2 * (C / 256 + 2));
+    r |= dalloc(ctx, &p.blk, MAX_KIND * (C / 256 + 2));
+    r |= dalloc(ctx, &p.leavers, (size_t) LEAVE_CAP);
     r |= dalloc(ctx, &p.buf, 40 * S);
     r |= dalloc(ctx, &p.hbuf, (2 + 5 * K) * S);
     r |= dalloc(ctx, &p.cand_n, C);
@@ -521,7 +524,7 @@ static void enqueue_step(pairs_hip_dem_ctx *ctx, bool timed) {
     launch_contacts(ctx->stream, ctx->p, ctx->counters, ctx->nlocal, ctx->geom, ctx->prm,
                     timed ? ctx->ev + 2 : nullptr);
     if (timed) hipEventRecord(ctx->ev[5], ctx->stream);
-    launch_euler(ctx->stream, ctx->p, ctx->counters, ctx->prm);
+    launch_euler(ctx->stream, ctx->p, ctx->counters, ctx->geom, ctx->prm);
     if (timed) hipEventRecord(ctx->ev[6], ctx->stream);
 }
 
@@ -541,6 +544,8 @@ static int ensure_graph(pairs_hip_dem_ctx *ctx) {
 // (the timing cadence)
 static int enqueue_steps(pairs_hip_dem_ctx *ctx, int a, int b, int t0) {
     if (int e = ensure_graph(ctx)) return e;
+    launch_find_leavers(ctx->stream, ctx->p, ctx->counters, ctx->geom);
+    CHECK_LAUNCH();
     for (int ts = a; ts < b; ts++) {
         const bool timed = ctx->time_every > 0 && (ts - t0) % ctx->time_every == ctx->time_every - 1;
         if (timed) {

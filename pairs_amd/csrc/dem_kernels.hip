@@ -79,150 +79,35 @@ __device__ __forceinline__ void dsel(double xd, int fl, double lo, double hi, do
     s1 = ok && xd > hi - off;
 }
 
-// per-block counts of side 0 and side 1 over [0, nlocal + nghost); an
-// exchange, and the borders of the first periodic dimension, start from no
-// ghosts and an empty send map (comm.py:105-118: the counts are reset before
-// them), a later dimension selects among the locals and the ghosts so far and
-// appends behind them; workgroup 0 latches the range and the base for the
-// scatter (nothing writes them while this pass runs); an exchange clears
-// exchg_flag of locals
-__global__ __launch_bounds__(256) void k_sel_count(const double *__restrict__ Xd, const int *__restrict__ flags,
-                                                   int *__restrict__ c, double lo, double hi, double off, int exch,
-                                                   int first, int *__restrict__ blk, int *__restrict__ exchg_flag) {
-    __shared__ int s0c, s1c;
-    const bool fresh = exch || first;
-    const int nl = c[D_NLOCAL];
-    const int n = nl + (fresh ? 0 : c[D_NGHOST]);
-    if (threadIdx.x == 0) { s0c = 0; s1c = 0; }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        c[D_RANGE] = n;
-        c[D_BASE] = fresh ? 0 : c[D_NSEND_ALL];
-    }
-    __syncthreads();
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    bool a = false, b = false;
-    if (i < n) dsel(Xd[i], flags[i], lo, hi, off, a, b);
-    if (exch && i < nl) exchg_flag[i] = 0;
-    const unsigned long long ma = __ballot(a), mb = __ballot(b);
-    if ((threadIdx.x & 63) == 0) { atomicAdd(&s0c, __popcll(ma)); atomicAdd(&s1c, __popcll(mb)); }
-    __syncthreads();
-    if (threadIdx.x == 0) { blk[2 * blockIdx.x] = s0c; blk[2 * blockIdx.x + 1] = s1c; }
-}
-
-// sums of two per-thread values over a workgroup of 256 threads
-__device__ __forceinline__ void block_sum2_256(int a, int b, int *lds, int &sa, int &sb) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// a particle outside the box along a periodic dimension joins the list that the
+// next exchange reads.  An exchange shifts a particle only along its own
+// dimension, so whoever leaves along any of them is outside before the first.
+__device__ __forceinline__ void note_leaver(const DemPtrs &p, int *__restrict__ c, const DemGeom &g, int i, int fl,
+                                            double x, double y, double z) {
+    const double xs[3] = {x, y, z};
+    bool out = false;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        a += __shfl_xor(a, o, 64);
-        b += __shfl_xor(b, o, 64);
+    for (int d = 0; d < 3; d++) {
+        bool a, b;
+        dsel(xs[d], fl, g.lo[d], g.hi[d], 0.0, a, b);
+        out = out || (g.periodic[d] && (a || b));
     }
-    __syncthreads();
-    if (lane == 0) { lds[2 * wave] = a; lds[2 * wave + 1] = b; }
-    __syncthreads();
-    sa = lds[0] + lds[2] + lds[4] + lds[6];
-    sb = lds[1] + lds[3] + lds[5] + lds[7];
+    if (!out) return;
+    const int k = atomicAdd(&c[D_LEAVE], 1);
+    if (k < LEAVE_CAP) p.leavers[k] = i;
 }
 
-// ordered scatter into the send map (index order within each side, side 0
-// entries before side 1); borders also create the ghosts at nlocal + send
-// index (uid, type, mass, radius, position + shift, linear and angular
-// velocity, shape; flags are not sent, src/pairs/sim/comm.py:61-72).  Every
-// workgroup sums the per-block counts of the count pass itself (totals, and
-// the counts of the blocks before its own), so the offsets need no pass of
-// their own; all workgroups take the same capacity decision, and workgroup 0
-// updates the counts (a border dimension's ghosts join the ghost range), which
-// no other workgroup of this pass reads.
-__global__ __launch_bounds__(256) void k_sel_scatter(DemPtrs p, int *__restrict__ c, int dim, double lo, double hi,
-                                                     double off, double len, int exch, const int *__restrict__ blk,
-                                                     int pbc0, int pbc1, int send_cap, int cap) {
-    __shared__ int wbase[2][4];
-    __shared__ int red[8];
-    if (c[D_OVF]) return;
-    const int n = c[D_RANGE], nl = c[D_NLOCAL];
-    const int nblk = (n + 255) / 256;
-    if (blockIdx.x > 0 && (int) blockIdx.x >= nblk) return;  // workgroup 0 always writes the counts
-    const int base = c[D_BASE];
-    int t0 = 0, t1 = 0, q0 = 0, q1 = 0;
-    for (int u = threadIdx.x; u < nblk; u += 256) {
-        const int x = blk[2 * u], y = blk[2 * u + 1];
-        t0 += x; t1 += y;
-        if (u < (int) blockIdx.x) { q0 += x; q1 += y; }
-    }
-    int T0, T1, P0, P1;
-    block_sum2_256(t0, t1, red, T0, T1);
-    block_sum2_256(q0, q1, red, P0, P1);
-    const int need = base + T0 + T1;
-    if (need > send_cap || (!exch && nl + need > cap)) {
-        // the counts stay within the maps and arrays
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            if (need > send_cap) {
-                atomicMax(&c[D_REQ_SEND], need);
-                atomicMax(&c[D_OVF], DOVF_SEND);
-            } else {
-                atomicMax(&c[D_REQ_PART], nl + need);
-                atomicMax(&c[D_OVF], DOVF_PART);
-            }
-        }
-        return;
-    }
-    const double *Xd = dim == 0 ? p.x : (dim == 1 ? p.y : p.z);
+__global__ __launch_bounds__(256) void k_find_leavers(DemPtrs p, int *__restrict__ c, DemGeom g) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    bool a = false, b = false;
-    if (i < n) dsel(Xd[i], p.flags[i], lo, hi, off, a, b);
-    const unsigned long long ma = __ballot(a), mb = __ballot(b);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) { wbase[0][wave] = __popcll(ma); wbase[1][wave] = __popcll(mb); }
-    __syncthreads();
-    int pa = 0, pb = 0;
-    for (int w = 0; w < wave; w++) { pa += wbase[0][w]; pb += wbase[1][w]; }
-    for (int s = 0; s < 2; s++) {
-        const bool sel = s == 0 ? a : b;
-        if (!sel) continue;
-        const int idx = base + (s == 0 ? P0 + pa + lane_rank(ma) : T0 + P1 + pb + lane_rank(mb));
-        const int mult = s == 0 ? pbc0 : pbc1;
-        p.send_map[idx] = i;
-        p.send_mult[3 * idx + 0] = dim == 0 ? mult : 0;
-        p.send_mult[3 * idx + 1] = dim == 1 ? mult : 0;
-        p.send_mult[3 * idx + 2] = dim == 2 ? mult : 0;
-        if (exch) {
-            p.exchg_flag[i] = 1;
-        } else {
-            const int g = nl + idx;
-            // pack: src += send_mult * length (comm.py:312-318)
-            const double sh = (double) mult * len;
-            p.uid[g] = p.uid[i]; p.type[g] = p.type[i]; p.m[g] = p.m[i]; p.r[g] = p.r[i];
-            p.x[g] = dim == 0 ? p.x[i] + sh : p.x[i] + 0 * len;
-            p.y[g] = dim == 1 ? p.y[i] + sh : p.y[i] + 0 * len;
-            p.z[g] = dim == 2 ? p.z[i] + sh : p.z[i] + 0 * len;
-            p.vx[g] = p.vx[i]; p.vy[g] = p.vy[i]; p.vz[g] = p.vz[i];
-            p.wx[g] = p.wx[i]; p.wy[g] = p.wy[i]; p.wz[g] = p.wz[i];
-            p.shape[g] = p.shape[i];
-        }
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        c[D_NSEND + 2 * dim] = T0;
-        c[D_NSEND + 2 * dim + 1] = T1;
-        c[D_NSEND_ALL] = need;
-        if (!exch) c[D_NGHOST] = need;
-    }
-}
-
-__global__ void k_reset_comm(int *__restrict__ c) {
-    if (threadIdx.x == 0) {
-        c[D_NSEND_ALL] = 0;
-        c[D_NGHOST] = 0;
-        for (int k = 0; k < 6; k++) c[D_NSEND + k] = 0;
-    }
+    if (i < c[D_NLOCAL]) note_leaver(p, c, g, i, p.flags[i], p.x[i], p.y[i], p.z[i]);
 }
 
 // ---------------------------------------------------------------- exchange with contact history
 
 // remove_exchanged_particles_pt1 (src/pairs/sim/comm.py:445-470): holes of
 // leavers below nlocal - n are filled from the tail, skipping leavers
-__device__ __forceinline__ void exch_pt1(const int *__restrict__ c, const int *__restrict__ send_map,
+__device__ __forceinline__ void exch_pt1(int n, int nl, const int *__restrict__ send_map,
                                          const int *__restrict__ exchg_flag, int *__restrict__ copy_to) {
-    const int n = c[D_NSEND_ALL], nl = c[D_NLOCAL];
     int pos = nl - 1;
     for (int i = 0; i < n; i++) {
         if (send_map[i] < nl - n) {
@@ -235,155 +120,212 @@ __device__ __forceinline__ void exch_pt1(const int *__restrict__ c, const int *_
     }
 }
 
-constexpr int EXB = 40;  // doubles per packed particle (comm.py:61-72 property list of the exchange)
+// what travels with a particle (comm.py:61-72, the property list of the
+// exchange): arrays of doubles, then of words
+constexpr int EXD = 36, EXI = 4, EXB = EXD + EXI;
 
-__device__ __forceinline__ void copy_particle(DemPtrs &p, int dst, int src) {
-    p.uid[dst] = p.uid[src]; p.shape[dst] = p.shape[src]; p.flags[dst] = p.flags[src];
-    p.x[dst] = p.x[src]; p.y[dst] = p.y[src]; p.z[dst] = p.z[src];
-    p.m[dst] = p.m[src];
-    p.vx[dst] = p.vx[src]; p.vy[dst] = p.vy[src]; p.vz[dst] = p.vz[src];
-    p.wx[dst] = p.wx[src]; p.wy[dst] = p.wy[src]; p.wz[dst] = p.wz[src];
-    p.r[dst] = p.r[src];
-    p.nx[dst] = p.nx[src]; p.ny[dst] = p.ny[src]; p.nz[dst] = p.nz[src];
-    for (int k = 0; k < 9; k++) {
-        p.inv_i[(size_t) k * p.cap + dst] = p.inv_i[(size_t) k * p.cap + src];
-        p.rot_m[(size_t) k * p.cap + dst] = p.rot_m[(size_t) k * p.cap + src];
-    }
-    for (int k = 0; k < 4; k++) p.rot_q[(size_t) k * p.cap + dst] = p.rot_q[(size_t) k * p.cap + src];
-    p.type[dst] = p.type[src];
+__device__ __forceinline__ double *exch_array(const DemPtrs &p, int f) {
+    double *const a[14] = {p.x, p.y, p.z, p.m, p.vx, p.vy, p.vz, p.wx, p.wy, p.wz, p.r, p.nx, p.ny, p.nz};
+    double *r = a[0];
+#pragma unroll
+    for (int k = 1; k < 14; k++) r = f == k ? a[k] : r;
+    if (f >= 14) r = p.inv_i + (size_t) (f - 14) * p.cap;
+    if (f >= 23) r = p.rot_m + (size_t) (f - 23) * p.cap;
+    if (f >= 32) r = p.rot_q + (size_t) (f - 32) * p.cap;
+    return r;
 }
 
-// pack the leavers (all non-volatile properties, position shifted)
-__device__ __forceinline__ void exch_pack(DemPtrs &p, const int *__restrict__ c, double lx, double ly, double lz) {
-    const int n = c[D_NSEND_ALL];
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int m = p.send_map[i];
-        double *b = p.buf + (size_t) EXB * i;
-        const int *mu = p.send_mult + 3 * i;
-        b[0] = p.uid[m]; b[1] = p.shape[m]; b[2] = p.flags[m];
-        b[3] = p.x[m] + mu[0] * lx; b[4] = p.y[m] + mu[1] * ly; b[5] = p.z[m] + mu[2] * lz;
-        b[6] = p.m[m];
-        b[7] = p.vx[m]; b[8] = p.vy[m]; b[9] = p.vz[m];
-        b[10] = p.wx[m]; b[11] = p.wy[m]; b[12] = p.wz[m];
-        b[13] = p.r[m];
-        b[14] = p.nx[m]; b[15] = p.ny[m]; b[16] = p.nz[m];
-        for (int k = 0; k < 9; k++) { b[17 + k] = p.inv_i[(size_t) k * p.cap + m]; b[26 + k] = p.rot_m[(size_t) k * p.cap + m]; }
-        for (int k = 0; k < 4; k++) b[35 + k] = p.rot_q[(size_t) k * p.cap + m];
-        b[39] = p.type[m];
-    }
+__device__ __forceinline__ int *exch_words(const DemPtrs &p, int f) {
+    return f == 0 ? p.uid : f == 1 ? p.shape : f == 2 ? p.flags : p.type;
 }
 
-// remove_exchanged_particles_pt2 (comm.py:473-506): copy guard "src > 0",
-// properties and contact history move from the tail into the hole
-__device__ __forceinline__ void exch_pt2(DemPtrs &p, const int *__restrict__ c) {
-    const int n = c[D_NSEND_ALL];
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int src = p.copy_to[i];
+// slot k of the contact history of src written to dst
+__device__ __forceinline__ void copy_contact(const DemPtrs &p, int k, int dst, int src) {
+    const size_t a = (size_t) k * p.cap + dst, b = (size_t) k * p.cap + src;
+    const size_t ta = 3 * (size_t) k * p.cap + dst, tb = 3 * (size_t) k * p.cap + src, C = p.cap;
+    const int u = p.c_uid[b], w = p.c_used[b], s = p.c_stick[b];
+    const double t0 = p.c_tsd[tb], t1 = p.c_tsd[tb + C], t2 = p.c_tsd[tb + 2 * C], v = p.c_ivm[b];
+    p.c_uid[a] = u; p.c_used[a] = w; p.c_stick[a] = s;
+    p.c_tsd[ta] = t0; p.c_tsd[ta + C] = t1; p.c_tsd[ta + 2 * C] = t2;
+    p.c_ivm[a] = v;
+}
+
+// The leavers of one dimension moved: properties packed with the position
+// shifted (comm.py:312-318), the holes filled from the tail with their contact
+// history (remove_exchanged_particles_pt2, comm.py:473-506; copy guard "src >
+// 0"), the leavers unpacked at nlocal - n + i, and the history of the leaver's
+// slot as it is after the hole filling packed and unpacked (the reference packs
+// it then); every contact's uid lands in one buffer word, so the last contact's
+// uid is the one that travels.  Each phase is finished before the next begins.
+// A thread moves one word or one contact of one leaver.
+__device__ __forceinline__ void exch_move(const DemPtrs &p, double *const *s_arr, int n, int nl, int dim,
+                                          const DemGeom &g) {
+    const int nt = blockDim.x, base = nl - n, hb = 2 + 5 * p.ccap;
+    const size_t C = p.cap;
+    for (int e = threadIdx.x; e < n * EXB; e += nt) {
+        const int i = e / EXB, f = e - i * EXB, m = p.send_map[i];
+        double v;
+        if (f < EXD) {
+            v = s_arr[f][m];
+            if (f < 3) v = v + (f == dim ? (p.send_side[i] == 0 ? 1 : -1) : 0) * g.len[f];
+        } else {
+            v = exch_words(p, f - EXD)[m];
+        }
+        p.buf[e] = v;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * EXB; e += nt) {
+        const int i = e / EXB, f = e - i * EXB, src = p.copy_to[i];
         if (src <= 0) continue;
         const int dst = p.send_map[i];
-        copy_particle(p, dst, src);
-        const int nc = p.num_contacts[src];
-        for (int k = 0; k < nc; k++) {
-            const size_t a = (size_t) k * p.cap + dst, b = (size_t) k * p.cap + src;
-            p.c_uid[a] = p.c_uid[b];
-            p.c_used[a] = p.c_used[b];
-            p.c_stick[a] = p.c_stick[b];
-            p.c_tsd[3 * (size_t) k * p.cap + dst] = p.c_tsd[3 * (size_t) k * p.cap + src];
-            p.c_tsd[(3 * (size_t) k + 1) * p.cap + dst] = p.c_tsd[(3 * (size_t) k + 1) * p.cap + src];
-            p.c_tsd[(3 * (size_t) k + 2) * p.cap + dst] = p.c_tsd[(3 * (size_t) k + 2) * p.cap + src];
-            p.c_ivm[a] = p.c_ivm[b];
-        }
-        p.num_contacts[dst] = nc;
+        if (f < EXD) s_arr[f][dst] = s_arr[f][src];
+        else exch_words(p, f - EXD)[dst] = exch_words(p, f - EXD)[src];
     }
-}
-
-// unpack the leavers at nlocal - n + i; then pack their contact history from
-// the leaver's slot as it is after the hole filling (the reference packs the
-// history after pt2); every contact's uid lands in one buffer word, so the
-// last contact's uid is the one that travels
-__device__ __forceinline__ void exch_unpack(DemPtrs &p, const int *__restrict__ c) {
-    const int n = c[D_NSEND_ALL], base = c[D_NLOCAL] - n;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const double *b = p.buf + (size_t) EXB * i;
-        const int g = base + i;
-        p.uid[g] = (int) b[0]; p.shape[g] = (int) b[1]; p.flags[g] = (int) b[2];
-        p.x[g] = b[3]; p.y[g] = b[4]; p.z[g] = b[5];
-        p.m[g] = b[6];
-        p.vx[g] = b[7]; p.vy[g] = b[8]; p.vz[g] = b[9];
-        p.wx[g] = b[10]; p.wy[g] = b[11]; p.wz[g] = b[12];
-        p.r[g] = b[13];
-        p.nx[g] = b[14]; p.ny[g] = b[15]; p.nz[g] = b[16];
-        for (int k = 0; k < 9; k++) { p.inv_i[(size_t) k * p.cap + g] = b[17 + k]; p.rot_m[(size_t) k * p.cap + g] = b[26 + k]; }
-        for (int k = 0; k < 4; k++) p.rot_q[(size_t) k * p.cap + g] = b[35 + k];
-        p.type[g] = (int) b[39];
+    for (int e = threadIdx.x; e < n * p.ccap; e += nt) {
+        const int i = e / p.ccap, k = e - i * p.ccap, src = p.copy_to[i];
+        if (src <= 0) continue;
+        const int dst = p.send_map[i], nc = p.num_contacts[src];
+        if (k < nc) copy_contact(p, k, dst, src);
+        if (k == 0) p.num_contacts[dst] = nc;
     }
-}
-
-__device__ __forceinline__ void hist_pack(DemPtrs &p, const int *__restrict__ c) {
-    const int n = c[D_NSEND_ALL];
-    const int hb = 2 + 5 * p.ccap;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int m = p.send_map[i];
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * EXB; e += nt) {
+        const int i = e / EXB, f = e - i * EXB;
+        if (f < EXD) s_arr[f][base + i] = p.buf[e];
+        else exch_words(p, f - EXD)[base + i] = (int) p.buf[e];
+    }
+    for (int e = threadIdx.x; e < n * p.ccap; e += nt) {
+        const int i = e / p.ccap, k = e - i * p.ccap, m = p.send_map[i], nc = p.num_contacts[m];
         double *b = p.hbuf + (size_t) hb * i;
-        const int nc = p.num_contacts[m];
-        b[0] = nc;
-        double last = 0.0;
-        for (int k = 0; k < nc; k++) {
-            const size_t a = (size_t) k * p.cap + m;
-            last = p.c_uid[a];
-            b[2 + 5 * k] = p.c_stick[a];
-            b[3 + 5 * k] = p.c_tsd[3 * (size_t) k * p.cap + m];
-            b[4 + 5 * k] = p.c_tsd[(3 * (size_t) k + 1) * p.cap + m];
-            b[5 + 5 * k] = p.c_tsd[(3 * (size_t) k + 2) * p.cap + m];
-            b[6 + 5 * k] = p.c_ivm[a];
+        if (k == 0) {
+            b[0] = nc;
+            if (nc == 0) b[1] = 0.0;
         }
-        b[1] = last;
+        if (k >= nc) continue;
+        const size_t a = (size_t) k * C + m, t = 3 * (size_t) k * C + m;
+        if (k == nc - 1) b[1] = p.c_uid[a];
+        const int stick = p.c_stick[a];
+        const double t0 = p.c_tsd[t], t1 = p.c_tsd[t + C], t2 = p.c_tsd[t + 2 * C], v = p.c_ivm[a];
+        b += 2 + 5 * k;
+        b[0] = stick; b[1] = t0; b[2] = t1; b[3] = t2; b[4] = v;
     }
-}
-
-__device__ __forceinline__ void hist_unpack(DemPtrs &p, const int *__restrict__ c) {
-    const int n = c[D_NSEND_ALL], base = c[D_NLOCAL] - n;
-    const int hb = 2 + 5 * p.ccap;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * p.ccap; e += nt) {
+        const int i = e / p.ccap, k = e - i * p.ccap, to = base + i;
         const double *b = p.hbuf + (size_t) hb * i;
-        const int g = base + i;
-        const int nc = (int) b[0];
-        p.num_contacts[g] = nc;
-        for (int k = 0; k < nc; k++) {
-            const size_t a = (size_t) k * p.cap + g;
-            p.c_uid[a] = (int) b[1];
-            p.c_used[a] = 1;
-            p.c_stick[a] = (int) b[2 + 5 * k];
-            p.c_tsd[3 * (size_t) k * p.cap + g] = b[3 + 5 * k];
-            p.c_tsd[(3 * (size_t) k + 1) * p.cap + g] = b[4 + 5 * k];
-            p.c_tsd[(3 * (size_t) k + 2) * p.cap + g] = b[5 + 5 * k];
-            p.c_ivm[a] = b[6 + 5 * k];
+        const int nc = (int) b[0], uid = (int) b[1];
+        if (k == 0) p.num_contacts[to] = nc;
+        if (k >= nc) continue;
+        b += 2 + 5 * k;
+        const size_t a = (size_t) k * C + to, t = 3 * (size_t) k * C + to;
+        const double v0 = b[0], t0 = b[1], t1 = b[2], t2 = b[3], v = b[4];
+        p.c_uid[a] = uid; p.c_used[a] = 1; p.c_stick[a] = (int) v0;
+        p.c_tsd[t] = t0; p.c_tsd[t + C] = t1; p.c_tsd[t + 2 * C] = t2;
+        p.c_ivm[a] = v;
+    }
+    __syncthreads();
+}
+
+// The exchange, dimension by dimension (comm.py:100-151), in one workgroup: a
+// step moves few particles across a face, and they are on the list that the
+// integration before has left.  A thread holds one of them, follows it where an
+// exchange moves it, and ranks it among the leavers of a dimension (side 0
+// before side 1, each in index order: the reference's send order); the tail
+// that fills the holes is planned with two scans.  More leavers than the list
+// holds are found by a scan of the locals instead.  Bound by the latency of its
+// phases.  It replaces, per dimension, a count and a scatter pass over the
+// locals and a kernel whose thread 0 walked the tail through memory (bed of
+// 187200 spheres, two dimensions: 46 us -> 7.9).
+__global__ __launch_bounds__(1024) void k_exchange(DemPtrs p, int *__restrict__ c, DemGeom g) {
+    __shared__ int lds[20];
+    __shared__ double *s_arr[EXD];
+    __shared__ unsigned s_key[LEAVE_CAP];
+    __shared__ int s_map[LEAVE_CAP], s_fill[LEAVE_CAP], s_hole[LEAVE_CAP], s_tail[LEAVE_CAP];
+    const int tid = threadIdx.x, cnt = c[D_LEAVE], nl = c[D_NLOCAL], ovf = c[D_OVF];
+    __syncthreads();
+    if (tid == 0) c[D_LEAVE] = 0;
+    if (ovf || cnt == 0) return;
+    if (tid < EXD) s_arr[tid] = exch_array(p, tid);
+    const bool listed = cnt <= LEAVE_CAP;
+    int me = listed && tid < cnt ? p.leavers[tid] : -1;
+    for (int dim = 0; dim < 3; dim++) {
+        if (!g.periodic[dim]) continue;
+        const double *Xd = dim == 0 ? p.x : (dim == 1 ? p.y : p.z);
+        int n;
+        if (listed) {
+            bool a = false, b = false;
+            if (me >= 0) dsel(Xd[me], p.flags[me], g.lo[dim], g.hi[dim], 0.0, a, b);
+            const bool out = a || b;
+            const unsigned key = a ? (unsigned) me : b ? (unsigned) me | 0x80000000u : 0xffffffffu;
+            s_key[tid] = key;
+            s_tail[tid] = 0;
+            n = __syncthreads_count(out);
+            if (n == 0) continue;
+            if (n <= p.send_cap) {
+                int rank = 0;
+                for (int u = 0; u < cnt; u++) rank += s_key[u] < key ? 1 : 0;
+                if (out) {
+                    s_map[rank] = me;
+                    p.send_map[rank] = me;
+                    p.send_side[rank] = a ? 0 : 1;
+                    if (me >= nl - n) s_tail[nl - 1 - me] = 1;
+                }
+                __syncthreads();
+                int total;
+                const bool fills = tid < n && !s_tail[tid], hole = tid < n && s_map[tid] < nl - n;
+                const int ef = block_scan_excl<1024>(fills ? 1 : 0, lds, &total);
+                const int eh = block_scan_excl<1024>(hole ? 1 : 0, lds, &total);
+                if (fills) { s_fill[ef] = nl - 1 - tid; s_tail[tid] = 2 + ef; }
+                if (hole) s_hole[eh] = s_map[tid];
+                __syncthreads();
+                if (tid < n) p.copy_to[tid] = hole ? s_fill[eh] : -1;
+                if (out) me = nl - n + rank;
+                else if (me >= nl - n) me = s_hole[s_tail[nl - 1 - me] - 2];
+            }
+        } else {
+            // totals, then places in index order within each side
+            int t0 = 0, t1 = 0;
+            for (int i0 = 0; i0 < nl; i0 += 1024) {
+                const int i = i0 + tid;
+                bool a = false, b = false;
+                if (i < nl) dsel(Xd[i], p.flags[i], g.lo[dim], g.hi[dim], 0.0, a, b);
+                if (i < nl) p.exchg_flag[i] = a || b ? 1 : 0;
+                t0 += __syncthreads_count(a);
+                t1 += __syncthreads_count(b);
+            }
+            n = t0 + t1;
+            if (n == 0) continue;
+            if (n <= p.send_cap) {
+                int o0 = 0, o1 = t0;
+                for (int i0 = 0; i0 < nl; i0 += 1024) {
+                    const int i = i0 + tid;
+                    bool a = false, b = false;
+                    if (i < nl) dsel(Xd[i], p.flags[i], g.lo[dim], g.hi[dim], 0.0, a, b);
+                    int s0, s1;
+                    const int q0 = block_scan_excl<1024>(a ? 1 : 0, lds, &s0);
+                    const int q1 = block_scan_excl<1024>(b ? 1 : 0, lds, &s1);
+                    if (a) { p.send_map[o0 + q0] = i; p.send_side[o0 + q0] = 0; }
+                    if (b) { p.send_map[o1 + q1] = i; p.send_side[o1 + q1] = 1; }
+                    o0 += s0;
+                    o1 += s1;
+                }
+                __syncthreads();
+                if (tid == 0) exch_pt1(n, nl, p.send_map, p.exchg_flag, p.copy_to);
+            }
         }
+        if (n > p.send_cap) {
+            if (tid == 0) {
+                atomicMax(&c[D_REQ_SEND], n);
+                atomicMax(&c[D_OVF], DOVF_SEND);
+            }
+            return;
+        }
+        __syncthreads();
+        exch_move(p, s_arr, n, nl, dim, g);
     }
 }
 
-// The exchange of one dimension after its send map is built, in one
-// workgroup (a step moves few particles across a face): the tail fill plan
-// (pt1, sequential as the reference's), the leavers packed, the holes filled
-// from the tail with their contact history (pt2), the leavers unpacked at
-// nlocal - n + i, their history packed after the hole filling and unpacked --
-// the reference's order, each phase finished before the next begins.
-__global__ __launch_bounds__(1024) void k_exchange(DemPtrs p, const int *__restrict__ c, double lx, double ly,
-                                                   double lz) {
-    if (c[D_OVF] || c[D_NSEND_ALL] == 0) return;
-    if (threadIdx.x == 0) exch_pt1(c, p.send_map, p.exchg_flag, p.copy_to);
-    exch_pack(p, c, lx, ly, lz);
-    __syncthreads();
-    exch_pt2(p, c);
-    __syncthreads();
-    exch_unpack(p, c);
-    __syncthreads();
-    hist_pack(p, c);
-    __syncthreads();
-    hist_unpack(p, c);
-}
-
-// ---------------------------------------------------------------- cells
+// ---------------------------------------------------------------- borders and cell counts
 
 __device__ __forceinline__ int dcell_of(double x, double y, double z, const DemGeom &g) {
     const double xs[3] = {x, y, z};
@@ -398,19 +340,189 @@ __device__ __forceinline__ int dcell_of(double x, double y, double z, const DemG
     return idx + 1;
 }
 
-// BuildCellLists (src/pairs/sim/cell_lists.py:90-134): Infinite -> cell 0
-__global__ __launch_bounds__(256) void k_cell_count(DemPtrs p, const int *__restrict__ c, DemGeom g) {
-    const int n = c[D_NLOCAL] + c[D_NGHOST];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int cell = (p.flags[i] & DFLAG_INFINITE) ? 0 : dcell_of(p.x[i], p.y[i], p.z[i], g);
-    p.particle_cell[i] = cell;
-    p.cell_slot[i] = atomicAdd(&p.cell_count[cell], 1);  // its place among the cell's entries
+constexpr int pow3(int n) { return n == 0 ? 1 : 3 * pow3(n - 1); }
+
+// the k-th periodic dimension
+__device__ __forceinline__ int periodic_dim(const DemGeom &g, int k) {
+    int d = 0;
+    for (; d < 3; d++)
+        if (g.periodic[d] && k-- == 0) break;
+    return d;
 }
 
-// exclusive scan of cell counts: block partials, then each block adds its
-// offset; the counts are cleared behind the reads (nothing else uses them, so
-// the next binning starts from zeros)
+// Borders (comm.py:56-98): dimension by dimension, side 0 then side 1, every
+// local and every ghost of the dimensions before that lies within a cell width
+// of the face gets a ghost behind all others.  A ghost keeps its particle's
+// other coordinates, so whether it is selected along a later dimension depends
+// on the particle alone, and the ghosts of all dimensions fall into kinds: one
+// digit per periodic dimension (0 not shifted, 1 side 0, 2 side 1), the later
+// dimension the higher digit.  The order of the ghosts is that of their kind as
+// a number in base 3, and within a kind the index order of the particles.  So
+// one count per kind and block of particles (k_border_count) places them all.
+template <int ND>
+struct Kinds {
+    bool side[ND > 0 ? ND : 1][2];
+    __device__ __forceinline__ void set(const DemGeom &g, const double (&xs)[3], int fl, bool in) {
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            const int d = ND == 3 ? k : periodic_dim(g, k);
+            const double xd = d == 0 ? xs[0] : d == 1 ? xs[1] : xs[2];
+            bool a, b;
+            dsel(xd, fl, g.lo[d], g.hi[d], g.width, a, b);
+            side[k][0] = in && a;
+            side[k][1] = in && b;
+        }
+    }
+    __device__ __forceinline__ bool any() const {
+        bool r = false;
+#pragma unroll
+        for (int k = 0; k < ND; k++) r = r || side[k][0] || side[k][1];
+        return r;
+    }
+    __device__ __forceinline__ bool has(int kind) const {
+        bool r = true;
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            const int digit = kind % 3;
+            kind /= 3;
+            r = r && (digit == 0 || side[k][digit == 2 ? 1 : 0]);
+        }
+        return r;
+    }
+};
+
+template <int ND>
+__global__ __launch_bounds__(256) void k_border_count(DemPtrs p, const int *__restrict__ c, DemGeom g, int pitch) {
+    constexpr int NK = pow3(ND);
+    __shared__ int s_n[NK][4];
+    const int nl = c[D_NLOCAL];
+    if ((int) blockIdx.x * 256 >= nl) return;
+    const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Kinds<ND> K;
+    double xs[3] = {0.0, 0.0, 0.0};
+    int fl = 0;
+    if (i < nl) { xs[0] = p.x[i]; xs[1] = p.y[i]; xs[2] = p.z[i]; fl = p.flags[i]; }
+    K.set(g, xs, fl, i < nl);
+    const bool some = __ballot(K.any()) != 0;
+#pragma unroll
+    for (int k = 1; k < NK; k++) {
+        const int m = some ? __popcll(__ballot(K.has(k))) : 0;
+        if (lane == 0) s_n[k][wave] = m;
+    }
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k >= 1 && k < NK) p.blk[(size_t) k * pitch + blockIdx.x] = s_n[k][0] + s_n[k][1] + s_n[k][2] + s_n[k][3];
+}
+
+// The ghosts at nlocal + place (uid, type, mass, radius, position + shift,
+// linear and angular velocity, shape; flags are not sent, comm.py:61-72), and
+// the cells of locals and ghosts counted (BuildCellLists,
+// src/pairs/sim/cell_lists.py:90-134; Infinite -> cell 0).  Every workgroup sums
+// the counts of the blocks itself, so the places need no pass of their own, and
+// takes the same capacity decision, dimension by dimension; without room no
+// ghost is made and the cells hold the locals.  Bound by the returning atomics
+// of the cell counts (10 us at 190000 particles); with k_border_count 26 us
+// there, 33 for a count and a scatter pass per dimension and a pass of counts.
+template <int ND>
+__global__ __launch_bounds__(256) void k_border_cells(DemPtrs p, int *__restrict__ c, DemGeom g, int pitch) {
+    constexpr int NK = pow3(ND);
+    __shared__ int s_total[NK], s_before[NK], s_wave[NK][4];
+    const int nl = c[D_NLOCAL], ovf = c[D_OVF];
+    const int nblk = (nl + 255) / 256;
+    if (blockIdx.x > 0 && (int) blockIdx.x >= nblk) return;  // workgroup 0 always writes the count
+    const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Kinds<ND> K;
+    double xs[3] = {0.0, 0.0, 0.0};
+    int fl = 0;
+    if (i < nl) { xs[0] = p.x[i]; xs[1] = p.y[i]; xs[2] = p.z[i]; fl = p.flags[i]; }
+    K.set(g, xs, fl, i < nl);
+    if (i < nl) {
+        const int cell = (fl & DFLAG_INFINITE) ? 0 : dcell_of(xs[0], xs[1], xs[2], g);
+        p.particle_cell[i] = cell;
+        p.cell_slot[i] = atomicAdd(&p.cell_count[cell], 1);  // its place among the cell's entries
+    }
+    if (ND == 0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) c[D_NGHOST] = 0;
+        return;
+    }
+    const bool some = __ballot(K.any()) != 0;
+#pragma unroll
+    for (int k = 1; k < NK; k++) {
+        const int m = some ? __popcll(__ballot(K.has(k))) : 0;
+        if (lane == 0) s_wave[k][wave] = m;
+    }
+    for (int k = 1 + wave; k < NK; k += 4) {
+        int t = 0, q = 0;
+        for (int u = lane; u < nblk; u += 64) {
+            const int x = p.blk[(size_t) k * pitch + u];
+            t += x;
+            q += u < (int) blockIdx.x ? x : 0;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            t += __shfl_xor(t, o, 64);
+            q += __shfl_xor(q, o, 64);
+        }
+        if (lane == 0) { s_total[k] = t; s_before[k] = q; }
+    }
+    __syncthreads();
+    int need = 0, short_of = DOVF_NONE;
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+        if (short_of) break;
+        for (int k = pow3(d); k < pow3(d + 1); k++) need += s_total[k];
+        short_of = need > p.send_cap ? DOVF_SEND : nl + need > p.cap ? DOVF_PART : DOVF_NONE;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c[D_NGHOST] = ovf || short_of ? 0 : need;
+        if (!ovf && short_of) {
+            atomicMax(&c[short_of == DOVF_SEND ? D_REQ_SEND : D_REQ_PART], short_of == DOVF_SEND ? need : nl + need);
+            atomicMax(&c[D_OVF], short_of);
+        }
+    }
+    if (ovf || short_of || !some) return;
+    int uid = 0, type = 0, shape = 0;
+    double m = 0.0, r = 0.0, v[3] = {0.0, 0.0, 0.0}, w[3] = {0.0, 0.0, 0.0};
+    if (K.any()) {
+        uid = p.uid[i]; type = p.type[i]; shape = p.shape[i]; m = p.m[i]; r = p.r[i];
+        v[0] = p.vx[i]; v[1] = p.vy[i]; v[2] = p.vz[i]; w[0] = p.wx[i]; w[1] = p.wy[i]; w[2] = p.wz[i];
+    }
+    int at = nl;
+    for (int k = 1; k < NK; k++) {
+        const bool sel = K.has(k);
+        const unsigned long long mask = __ballot(sel);
+        int q = at + s_before[k];
+        for (int u = 0; u < wave; u++) q += s_wave[k][u];
+        at += s_total[k];
+        if (!sel) continue;
+        q += lane_rank(mask);
+        double y[3] = {xs[0], xs[1], xs[2]};
+        int digits = k;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            // src += send_mult * length (comm.py:312-318)
+            int mult = 0;
+            if (g.periodic[d]) {
+                mult = digits % 3 == 1 ? 1 : digits % 3 == 2 ? -1 : 0;
+                digits /= 3;
+            }
+            y[d] = xs[d] + (double) mult * g.len[d];
+        }
+        p.uid[q] = uid; p.type[q] = type; p.shape[q] = shape; p.m[q] = m; p.r[q] = r;
+        p.x[q] = y[0]; p.y[q] = y[1]; p.z[q] = y[2];
+        p.vx[q] = v[0]; p.vy[q] = v[1]; p.vz[q] = v[2];
+        p.wx[q] = w[0]; p.wy[q] = w[1]; p.wz[q] = w[2];
+        const int cell = dcell_of(y[0], y[1], y[2], g);
+        p.particle_cell[q] = cell;
+        p.cell_slot[q] = atomicAdd(&p.cell_count[cell], 1);
+    }
+}
+
+// ---------------------------------------------------------------- cells
+
+// exclusive scan of the cell counts: each block's own, and the block totals;
+// the counts are cleared behind the reads (nothing else uses them, so the next
+// binning starts from zeros)
 __global__ __launch_bounds__(1024) void k_scan_partial(int *__restrict__ in, int *__restrict__ out,
                                                        int *__restrict__ bsum, int n) {
     __shared__ int lds[20];
@@ -423,9 +535,9 @@ __global__ __launch_bounds__(1024) void k_scan_partial(int *__restrict__ in, int
     if (threadIdx.x == 0) bsum[blockIdx.x] = t;
 }
 
-// each block adds the totals of the blocks before it (it sums them itself:
-// a few hundred words, so the block offsets need no pass of their own)
-__global__ __launch_bounds__(1024) void k_scan_add(int *__restrict__ out, const int *__restrict__ bsum, int n) {
+// each block adds the totals of the blocks before it to the scan of its own
+__global__ __launch_bounds__(1024) void k_scan_add(const int *__restrict__ in, int *__restrict__ out,
+                                                   const int *__restrict__ bsum, int n) {
     __shared__ int red[16];
     int q = 0;
     for (int b = threadIdx.x; b < (int) blockIdx.x; b += 1024) q += bsum[b];
@@ -437,15 +549,40 @@ __global__ __launch_bounds__(1024) void k_scan_add(int *__restrict__ out, const 
 #pragma unroll
     for (int w = 0; w < 16; w++) off += red[w];
     const int i = blockIdx.x * 1024 + threadIdx.x;
-    if (i < n) out[i] += off;
+    if (i < n) out[i] = in[i] + off;
 }
 
-__global__ __launch_bounds__(256) void k_cell_fill(DemPtrs p, const int *__restrict__ c) {
+// The particles into their cells.  ADD: the blocks' offsets are not in
+// cell_start yet: every workgroup scans the block totals (at most SCAN_LDS of
+// them) in LDS and adds them where it needs them, and the workgroups share the
+// writing of cell_start for the passes behind.
+constexpr int SCAN_LDS = 2048;
+template <bool ADD>
+__global__ __launch_bounds__(256) void k_cell_fill(DemPtrs p, const int *__restrict__ c, int nstart, int nblk) {
+    __shared__ int s_off[ADD ? SCAN_LDS : 1];
+    __shared__ int lds[8];
     const int n = c[D_NLOCAL] + c[D_NGHOST];
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int cell = p.particle_cell[i];
-    p.cell_particles[p.cell_start[cell] + p.cell_slot[i]] = i;
+    int cell = 0, start = 0, slot = 0;
+    if (i < n) {
+        cell = p.particle_cell[i];
+        slot = p.cell_slot[i];
+        start = (ADD ? p.cell_scan : p.cell_start)[cell];
+    }
+    if (ADD) {
+        int at = 0;
+        for (int b0 = 0; b0 < nblk; b0 += 256) {
+            const int b = b0 + threadIdx.x;
+            int total;
+            const int e = block_scan_excl<256>(b < nblk ? p.scan_tmp[b] : 0, lds, &total);
+            if (b < nblk) s_off[b] = at + e;
+            at += total;
+        }
+        __syncthreads();
+        for (int k = i; k < nstart; k += gridDim.x * 256) p.cell_start[k] = p.cell_scan[k] + s_off[k >> 10];
+        start += s_off[cell >> 10];
+    }
+    if (i < n) p.cell_particles[start + slot] = i;
 }
 
 // PartitionCellLists (src/pairs/sim/cell_lists.py:137-171) of one cell, whose
@@ -996,11 +1133,17 @@ __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict
 // ---------------------------------------------------------------- integration
 
 // euler (examples/dem.py:77-85) with quaternion(phi, |phi|) and
-// quaternion_to_rotation_matrix (src/pairs/mapping/keywords.py:190-252)
-__global__ __launch_bounds__(256) void k_euler(DemPtrs p, const int *__restrict__ c, double dt) {
+// quaternion_to_rotation_matrix (src/pairs/mapping/keywords.py:190-252); the
+// particles it moves out of the box are noted for the next exchange
+__global__ __launch_bounds__(256) void k_euler(DemPtrs p, int *__restrict__ c, DemGeom g, double dt) {
     const int nl = c[D_NLOCAL];
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= nl || c[D_OVF] || (p.flags[i] & DFLAG_FIXED)) return;
+    if (i >= nl || c[D_OVF]) return;
+    const int fl = p.flags[i];
+    if (fl & DFLAG_FIXED) {
+        note_leaver(p, c, g, i, fl, p.x[i], p.y[i], p.z[i]);
+        return;
+    }
     const size_t C = p.cap;
     const double im = 1.0 / p.m[i];
     const double hm = 0.5 * im;
@@ -1043,6 +1186,7 @@ __global__ __launch_bounds__(256) void k_euler(DemPtrs p, const int *__restrict_
     R[7] = 2.0 * (q[2] * q[3] + q[0] * q[1]);
     R[8] = (1.0 - (2.0 * q[1]) * q[1]) - (2.0 * q[2]) * q[2];
     for (int d = 0; d < 3; d++) w[d] = w[d] + wd[d] * dt;
+    note_leaver(p, c, g, i, fl, x[0], x[1], x[2]);
     p.x[i] = x[0]; p.y[i] = x[1]; p.z[i] = x[2];
     p.vx[i] = v[0]; p.vy[i] = v[1]; p.vz[i] = v[2];
     p.wx[i] = w[0]; p.wy[i] = w[1]; p.wz[i] = w[2];
@@ -1090,43 +1234,38 @@ void launch_mass_inertia(hipStream_t s, const DemPtrs &p, int nl) {
     hipLaunchKernelGGL(k_mass_inertia, dim3(grid_of(nl, 256)), dim3(256), 0, s, p, nl);
 }
 
-static void select_dim(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, int dim, int exch, int first) {
-    const double *Xd = dim == 0 ? p.x : (dim == 1 ? p.y : p.z);
+template <int ND>
+static void launch_borders(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
     const int nb = grid_of(p.cap, 256);
-    const double off = exch ? 0.0 : g.width;
-    hipLaunchKernelGGL(k_sel_count, dim3(nb), dim3(256), 0, s, Xd, p.flags, c, g.lo[dim], g.hi[dim], off, exch, first,
-                       p.blk, p.exchg_flag);
-    hipLaunchKernelGGL(k_sel_scatter, dim3(nb), dim3(256), 0, s, p, c, dim, g.lo[dim], g.hi[dim], off,
-                       g.hi[dim] - g.lo[dim], exch, p.blk, 1, -1, p.send_cap, p.cap);
+    if constexpr (ND > 0) hipLaunchKernelGGL(k_border_count<ND>, dim3(nb), dim3(256), 0, s, p, c, g, nb);
+    hipLaunchKernelGGL(k_border_cells<ND>, dim3(nb), dim3(256), 0, s, p, c, g, nb);
+}
+
+void launch_find_leavers(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
+    if (!g.periodic[0] && !g.periodic[1] && !g.periodic[2]) return;
+    launch_fill(s, c + D_LEAVE, 0, 1);
+    hipLaunchKernelGGL(k_find_leavers, dim3(grid_of(p.cap, 256)), dim3(256), 0, s, p, c, g);
 }
 
 // exchange, borders, cells of one step (the cell counts are zero on entry:
-// allocated zeroed, cleared by every scan)
+// allocated zeroed, cleared by every scan); one rank: only the periodic
+// dimensions send
 void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
-    // exchange, dimension by dimension (comm.py:100-151); one rank: only the
-    // periodic dimensions send
-    for (int dim = 0; dim < 3; dim++) {
-        if (!g.periodic[dim]) continue;
-        select_dim(s, p, c, g, dim, 1, 0);
-        hipLaunchKernelGGL(k_exchange, dim3(1), dim3(1024), 0, s, p, c, g.len[0], g.len[1], g.len[2]);
-    }
-    // borders (comm.py:56-98)
-    bool first = true;
-    for (int dim = 0; dim < 3; dim++) {
-        if (!g.periodic[dim]) continue;
-        select_dim(s, p, c, g, dim, 0, first ? 1 : 0);
-        first = false;
-    }
-    if (first) hipLaunchKernelGGL(k_reset_comm, dim3(1), dim3(64), 0, s, c);  // no periodic dimension: no ghosts
-    // cells
-    const int pg = grid_of(p.cap, 256);
-    hipLaunchKernelGGL(k_cell_count, dim3(pg), dim3(256), 0, s, p, c, g);
+    const int nd = g.periodic[0] + g.periodic[1] + g.periodic[2];
+    if (nd > 0) hipLaunchKernelGGL(k_exchange, dim3(1), dim3(1024), 0, s, p, c, g);
+    if (nd == 0) launch_borders<0>(s, p, c, g);
+    else if (nd == 1) launch_borders<1>(s, p, c, g);
+    else if (nd == 2) launch_borders<2>(s, p, c, g);
+    else launch_borders<3>(s, p, c, g);
     // (one entry past the cells, whose count stays zero: cell_start[ncells] is the total)
-    const int nb = grid_of(g.ncells + 1, 1024);
-    hipLaunchKernelGGL(k_scan_partial, dim3(nb), dim3(1024), 0, s, p.cell_count, p.cell_start, p.scan_tmp,
-                       g.ncells + 1);
-    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(1024), 0, s, p.cell_start, p.scan_tmp, g.ncells + 1);
-    hipLaunchKernelGGL(k_cell_fill, dim3(pg), dim3(256), 0, s, p, c);
+    const int n = g.ncells + 1, nb = grid_of(n, 1024), pg = grid_of(p.cap, 256);
+    hipLaunchKernelGGL(k_scan_partial, dim3(nb), dim3(1024), 0, s, p.cell_count, p.cell_scan, p.scan_tmp, n);
+    if (nb <= SCAN_LDS) {
+        hipLaunchKernelGGL(k_cell_fill<true>, dim3(pg), dim3(256), 0, s, p, c, n, nb);
+    } else {
+        hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(1024), 0, s, p.cell_scan, p.cell_start, p.scan_tmp, n);
+        hipLaunchKernelGGL(k_cell_fill<false>, dim3(pg), dim3(256), 0, s, p, c, n, nb);
+    }
     hipLaunchKernelGGL(k_cell_order, dim3(pg), dim3(256), 0, s, p, c);
 }
 
@@ -1145,8 +1284,8 @@ void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const 
     if (between) hipEventRecord(between[2], s);
 }
 
-void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemParams &prm) {
-    hipLaunchKernelGGL(k_euler, dim3(grid_of(p.cap, 256)), dim3(256), 0, s, p, c, prm.dt);
+void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, const DemParams &prm) {
+    hipLaunchKernelGGL(k_euler, dim3(grid_of(p.cap, 256)), dim3(256), 0, s, p, c, g, prm.dt);
 }
 
 }  // namespace dk

@@ -14,11 +14,7 @@ enum { DSHAPE_SPHERE = 0, DSHAPE_HALFSPACE = 1 };
 enum {
     D_NLOCAL = 0,
     D_NGHOST = 1,
-    D_NSEND_ALL = 2,
-    D_NSEND = 3,   // 6 entries
-    D_RANGE = 9,   // nlocal + nghost latched by the selection of a dimension
-    D_BASE = 10,   // send entries before this dimension
-    D_UNUSED = 11,
+    D_LEAVE = 2,   // particles outside a periodic dimension, noted for the exchange
     D_OVF = 12,
     D_REQ_SEND = 13,
     D_REQ_CONTACT = 14,
@@ -28,6 +24,10 @@ enum {
 // touching partners recorded per particle by the contact search; a particle
 // with more walks its cells again in the force pass
 constexpr int DCAND = 16;
+// leavers noted by index; with more the exchange scans the locals itself
+constexpr int LEAVE_CAP = 1024;
+// ghost kinds: per periodic dimension none, side 0 or side 1
+constexpr int MAX_KIND = 27;
 
 enum { DOVF_NONE = 0, DOVF_PART = 1, DOVF_CONTACT = 2, DOVF_SEND = 3, DOVF_CELLS = 4 };
 
@@ -65,7 +65,9 @@ struct DemPtrs {
     double *c_ivm;                                 // [k][cap]
     int *cell_count, *cell_start, *cell_particles, *particle_cell;
     int *cell_slot;      // each particle's place in its cell, from the counting pass
-    int *send_map, *send_mult, *exchg_flag, *copy_to, *blk, *scan_tmp;
+    int *cell_scan;      // cell starts within a block of the scan
+    int *leavers;        // [LEAVE_CAP] particles that the next exchange looks at
+    int *send_map, *send_side, *exchg_flag, *copy_to, *blk, *scan_tmp;
     double *buf, *hbuf;
     // the particles in cell order (each cell in the reference's order): index
     // and cell (bit 31: FIXED), (x, y, z, radius; -1 for a half-space); cmixed:
@@ -93,10 +95,12 @@ void launch_mass_inertia(hipStream_t s, const DemPtrs &p, int nl);
 // one step = prepare (exchange, borders, cells) + contacts (+ gravity and
 // history bookkeeping) + euler
 void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g);
+// the leavers of the first of several steps (each step notes those of the next)
+void launch_find_leavers(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g);
 // nlocal: the host's count; between: three events recorded after the search
 // (two) and after the contact kernel (timed steps only)
 void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
                      const hipEvent_t *between = nullptr);
-void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemParams &prm);
+void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, const DemParams &prm);
 
 }  // namespace dk

@@ -207,3 +207,62 @@ def test_mlp_forces_vs_oracle_at_size_edges(cells):
     Fx, Ex = mo.forces(p, sc, x, L)
     assert tm._rel_rms(s.forces(), Fx) < 3e-2
     assert abs(e - Ex.sum()) < 1e-3 * abs(Ex.sum())
+
+
+# exchange and borders: 0 to 3 periodic dimensions; the leavers of a step fit the
+# list that the integration keeps (1024) or do not; a box narrower than two
+# cell widths, whose particles have images on both sides; a cell grid whose
+# block totals do not fit the fill kernel's scan (2048 * 1024 cells)
+@pytest.mark.parametrize("pairs,periodic,dom,speed", [
+    (300, (True, True, False), (0.03, 0.02, 0.03), 20.0),
+    (300, (False, True, False), (0.03, 0.02, 0.03), 20.0),
+    (300, (True, True, True), (0.03, 0.02, 0.03), 20.0),
+    (300, (False, False, False), (0.03, 0.02, 0.03), 20.0),
+    (2500, (True, True, False), (0.06, 0.06, 0.06), 300.0),
+    (2500, (True, False, True), (0.06, 0.06, 0.06), 300.0),
+    (2500, (True, True, True), (0.06, 0.06, 0.06), 300.0),
+    (40, (True, True, True), (0.0045, 0.03, 0.0041), 20.0),
+    (200, (True, True, False), (0.41, 0.41, 0.41), 400.0),
+])
+def test_dem_exchange_and_borders_vs_oracle(pairs, periodic, dom, speed):
+    """touching pairs that fly through the faces together, their order, ghosts
+    and contact history against the oracle, with a run cut into chunks"""
+    from pairs_amd import dem
+    rng = np.random.default_rng(pairs)
+    dom = np.asarray(dom)
+    r = 0.0001
+    x = rng.uniform(0.0006, 1.0, (pairs, 3)) * (dom - 0.0012) + 0.0003
+    u = rng.standard_normal((pairs, 3))
+    u *= 1.94 * r / np.linalg.norm(u, axis=1)[:, None]
+    v = rng.uniform(-speed, speed, (pairs, 3)) * np.asarray(periodic)
+    pos, vel = np.concatenate([x, x + u]), np.concatenate([v, v + rng.uniform(-0.05, 0.05, v.shape)])
+    order = rng.permutation(2 * pairs)
+    pos, vel = pos[order], vel[order]
+    uid = np.arange(1, 2 * pairs + 1)
+    cells = int(np.prod(np.ceil(dom / 0.0025) + 4)) + 2
+    g = dem.DEMSystem(tuple(dom), periodic=periodic, particle_capacity=40000, contact_capacity=6, send_capacity=30000,
+                      ncells_capacity=cells)
+    o = po.OracleDEM(tuple(dom), periodic=periodic, cap=40000, ccap=6, cellcap=16 if cells > 1000000 else 256,
+                     send_cap=30000, ncells_cap=cells)
+    g.add_spheres(uid, np.full(2 * pairs, r), pos, vel)
+    for k in range(2 * pairs):
+        o.add_sphere(int(uid[k]), r, pos[k], vel[k])
+    for s in (g, o):
+        s.setup()
+    for a, b in ((0, 1), (1, 3), (3, 8)):
+        g.run(a, b)
+        o.run(a, b)
+        assert g.nlocal == o.nlocal and g.nghost == o.nghost, b
+        assert np.array_equal(g.get("uid", ghosts=True), o.get("uid", ghosts=True)), b
+        nc, cl, sk, tsd, iv = g.contacts()
+        onc, ocl, osk, otsd, oiv = o.contacts()
+        assert np.array_equal(nc, onc), b
+        for i in range(len(nc)):
+            m = nc[i]
+            assert np.array_equal(cl[i, :m], ocl[i, :m]) and np.array_equal(sk[i, :m], osk[i, :m]), (b, i)
+            if m:
+                assert np.abs(tsd[i, :m] - otsd[i, :m]).max() <= 1e-9 * np.abs(otsd).max(), (b, i)
+        for name in ("position", "linear_velocity"):
+            p, q = g.get(name, ghosts=True), o.get(name, ghosts=True)
+            assert np.abs(p - q).max() <= 1e-10 * np.abs(q).max(), (b, name)
+    assert nc.max() > 0
