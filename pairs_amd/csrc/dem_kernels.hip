@@ -56,14 +56,17 @@ __device__ __forceinline__ int block_scan_excl(int v, int *lds, int *total) {
     }
     if (lane == 63) lds[wave] = x;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int w = 0; w < BS / 64; w++) { const int t = lds[w]; lds[w] = acc; acc += t; }
-        lds[BS / 64] = acc;
+    // every wave sums the wave totals itself
+    constexpr int NW = BS / 64;
+    const int w = lane < NW ? lds[lane] : 0;
+    int t = w;
+#pragma unroll
+    for (int off = 1; off < NW; off <<= 1) {
+        const int y = __shfl_up(t, off, 64);
+        if (lane >= off) t += y;
     }
-    __syncthreads();
-    const int r = lds[wave] + x - v;
-    *total = lds[BS / 64];
+    *total = __shfl(t, NW - 1, 64);
+    const int r = __shfl(t - w, wave, 64) + x - v;
     __syncthreads();
     return r;
 }
@@ -327,17 +330,18 @@ __global__ __launch_bounds__(1024) void k_exchange(DemPtrs p, int *__restrict__ 
 
 // ---------------------------------------------------------------- borders and cell counts
 
+__device__ __forceinline__ int dcell_dim(double x, int d, const DemGeom &g) {
+    const double q = (x - (g.lo[d] - g.width)) / g.width;
+    const int cc = (int) q >= 0 ? (int) q : 0;
+    return cc < g.dim_cells[d] ? cc : g.dim_cells[d] - 1;
+}
+
+__device__ __forceinline__ int dcell_index(int cx, int cy, int cz, const DemGeom &g) {
+    return (cx * g.dim_cells[1] + cy) * g.dim_cells[2] + cz + 1;
+}
+
 __device__ __forceinline__ int dcell_of(double x, double y, double z, const DemGeom &g) {
-    const double xs[3] = {x, y, z};
-    int idx = 0;
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        const double q = (xs[d] - (g.lo[d] - g.width)) / g.width;
-        int cc = (int) q >= 0 ? (int) q : 0;
-        cc = cc < g.dim_cells[d] ? cc : g.dim_cells[d] - 1;
-        idx = d == 0 ? cc : idx * g.dim_cells[d] + cc;
-    }
-    return idx + 1;
+    return dcell_index(dcell_dim(x, 0, g), dcell_dim(y, 1, g), dcell_dim(z, 2, g), g);
 }
 
 constexpr int pow3(int n) { return n == 0 ? 1 : 3 * pow3(n - 1); }
@@ -391,40 +395,55 @@ struct Kinds {
     }
 };
 
+// Locals into their cells (BuildCellLists, src/pairs/sim/cell_lists.py:90-134;
+// Infinite -> cell 0) and the ghosts of each kind counted by block.  Bound by
+// the returning atomics of the cell counts.
 template <int ND>
-__global__ __launch_bounds__(256) void k_border_count(DemPtrs p, const int *__restrict__ c, DemGeom g, int pitch) {
+__global__ __launch_bounds__(256) void k_cell_count(DemPtrs p, int *__restrict__ c, DemGeom g, int pitch) {
     constexpr int NK = pow3(ND);
     __shared__ int s_n[NK][4];
     const int nl = c[D_NLOCAL];
+    if (ND == 0 && blockIdx.x == 0 && threadIdx.x == 0) c[D_NGHOST] = 0;
     if ((int) blockIdx.x * 256 >= nl) return;
     const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     Kinds<ND> K;
     double xs[3] = {0.0, 0.0, 0.0};
-    int fl = 0;
-    if (i < nl) { xs[0] = p.x[i]; xs[1] = p.y[i]; xs[2] = p.z[i]; fl = p.flags[i]; }
-    K.set(g, xs, fl, i < nl);
-    const bool some = __ballot(K.any()) != 0;
-#pragma unroll
-    for (int k = 1; k < NK; k++) {
-        const int m = some ? __popcll(__ballot(K.has(k))) : 0;
-        if (lane == 0) s_n[k][wave] = m;
+    int fl = 0, cell = 0, slot = 0;
+    if (i < nl) {
+        xs[0] = p.x[i]; xs[1] = p.y[i]; xs[2] = p.z[i]; fl = p.flags[i];
+        cell = (fl & DFLAG_INFINITE) ? 0 : dcell_of(xs[0], xs[1], xs[2], g);
+        slot = atomicAdd(&p.cell_count[cell], 1);  // its place among the cell's entries
     }
-    __syncthreads();
-    const int k = threadIdx.x;
-    if (k >= 1 && k < NK) p.blk[(size_t) k * pitch + blockIdx.x] = s_n[k][0] + s_n[k][1] + s_n[k][2] + s_n[k][3];
+    if (ND > 0) {
+        K.set(g, xs, fl, i < nl);
+        const bool some = __ballot(K.any()) != 0;
+#pragma unroll
+        for (int k = 1; k < NK; k++) {
+            const int m = some ? __popcll(__ballot(K.has(k))) : 0;
+            if (lane == 0) s_n[k][wave] = m;
+        }
+        __syncthreads();
+        const int k = threadIdx.x;
+        if (k >= 1 && k < NK) p.blk[(size_t) k * pitch + blockIdx.x] = s_n[k][0] + s_n[k][1] + s_n[k][2] + s_n[k][3];
+    }
+    if (i < nl) {
+        p.particle_cell[i] = cell;
+        p.cell_slot[i] = slot;
+    }
 }
 
 // The ghosts at nlocal + place (uid, type, mass, radius, position + shift,
 // linear and angular velocity, shape; flags are not sent, comm.py:61-72), and
-// the cells of locals and ghosts counted (BuildCellLists,
-// src/pairs/sim/cell_lists.py:90-134; Infinite -> cell 0).  Every workgroup sums
-// the counts of the blocks itself, so the places need no pass of their own, and
-// takes the same capacity decision, dimension by dimension; without room no
-// ghost is made and the cells hold the locals.  Bound by the returning atomics
-// of the cell counts (10 us at 190000 particles); with k_border_count 26 us
-// there, 33 for a count and a scatter pass per dimension and a pass of counts.
+// their cells counted.  Every workgroup sums the counts of the blocks itself,
+// so the places need no pass of their own, and takes the same capacity
+// decision, dimension by dimension; without room no ghost is made and the cells
+// hold the locals.  Bound by latency: the particle's fields are loaded before
+// the sums and the atomics of all kinds are in flight before the first place
+// is stored.  2080 | 187200 spheres, us: with the locals' atomics here, a kind
+// and its cell at a time 12 | 22 on top of 2.6 | 4.7 for the counts; so 7.7 |
+// 9.4 on top of 3.1 | 9.6 for k_cell_count.
 template <int ND>
-__global__ __launch_bounds__(256) void k_border_cells(DemPtrs p, int *__restrict__ c, DemGeom g, int pitch) {
+__global__ __launch_bounds__(256) void k_border_ghosts(DemPtrs p, int *__restrict__ c, DemGeom g, int pitch) {
     constexpr int NK = pow3(ND);
     __shared__ int s_total[NK], s_before[NK], s_wave[NK][4];
     const int nl = c[D_NLOCAL], ovf = c[D_OVF];
@@ -436,34 +455,41 @@ __global__ __launch_bounds__(256) void k_border_cells(DemPtrs p, int *__restrict
     int fl = 0;
     if (i < nl) { xs[0] = p.x[i]; xs[1] = p.y[i]; xs[2] = p.z[i]; fl = p.flags[i]; }
     K.set(g, xs, fl, i < nl);
-    if (i < nl) {
-        const int cell = (fl & DFLAG_INFINITE) ? 0 : dcell_of(xs[0], xs[1], xs[2], g);
-        p.particle_cell[i] = cell;
-        p.cell_slot[i] = atomicAdd(&p.cell_count[cell], 1);  // its place among the cell's entries
+    int uid = 0, type = 0, shape = 0;
+    double m = 0.0, r = 0.0, v[3] = {0.0, 0.0, 0.0}, w[3] = {0.0, 0.0, 0.0};
+    const bool mine = K.any();
+    if (mine) {
+        uid = p.uid[i]; type = p.type[i]; shape = p.shape[i]; m = p.m[i]; r = p.r[i];
+        v[0] = p.vx[i]; v[1] = p.vy[i]; v[2] = p.vz[i]; w[0] = p.wx[i]; w[1] = p.wy[i]; w[2] = p.wz[i];
     }
-    if (ND == 0) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) c[D_NGHOST] = 0;
-        return;
-    }
-    const bool some = __ballot(K.any()) != 0;
+    const bool some = __ballot(mine) != 0;
 #pragma unroll
     for (int k = 1; k < NK; k++) {
-        const int m = some ? __popcll(__ballot(K.has(k))) : 0;
-        if (lane == 0) s_wave[k][wave] = m;
+        const int n = some ? __popcll(__ballot(K.has(k))) : 0;
+        if (lane == 0) s_wave[k][wave] = n;
     }
-    for (int k = 1 + wave; k < NK; k += 4) {
-        int t = 0, q = 0;
-        for (int u = lane; u < nblk; u += 64) {
-            const int x = p.blk[(size_t) k * pitch + u];
-            t += x;
-            q += u < (int) blockIdx.x ? x : 0;
+    constexpr int PER = (NK + 2) / 4;  // kinds of a wave: 1 + wave, 5 + wave, ..
+    constexpr int AHEAD = ND == 3 ? 1 : 8;
+    int t[PER] = {}, q[PER] = {};
+#pragma unroll AHEAD
+    for (int u = lane; u < nblk; u += 64) {
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int k = 1 + wave + 4 * e;
+            const int x = k < NK ? p.blk[(size_t) k * pitch + u] : 0;
+            t[e] += x;
+            q[e] += u < (int) blockIdx.x ? x : 0;
         }
+    }
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
-            t += __shfl_xor(t, o, 64);
-            q += __shfl_xor(q, o, 64);
+            t[e] += __shfl_xor(t[e], o, 64);
+            q[e] += __shfl_xor(q[e], o, 64);
         }
-        if (lane == 0) { s_total[k] = t; s_before[k] = q; }
+        const int k = 1 + wave + 4 * e;
+        if (lane == 0 && k < NK) { s_total[k] = t[e]; s_before[k] = q[e]; }
     }
     __syncthreads();
     int need = 0, short_of = DOVF_NONE;
@@ -481,44 +507,51 @@ __global__ __launch_bounds__(256) void k_border_cells(DemPtrs p, int *__restrict
         }
     }
     if (ovf || short_of || !some) return;
-    int uid = 0, type = 0, shape = 0;
-    double m = 0.0, r = 0.0, v[3] = {0.0, 0.0, 0.0}, w[3] = {0.0, 0.0, 0.0};
-    if (K.any()) {
-        uid = p.uid[i]; type = p.type[i]; shape = p.shape[i]; m = p.m[i]; r = p.r[i];
-        v[0] = p.vx[i]; v[1] = p.vy[i]; v[2] = p.vz[i]; w[0] = p.wx[i]; w[1] = p.wy[i]; w[2] = p.wz[i];
-    }
-    int at = nl;
+    // places by kind, cells by dimension and shift
+    int to[NK], slot[NK], at = nl;
+#pragma unroll
     for (int k = 1; k < NK; k++) {
-        const bool sel = K.has(k);
-        const unsigned long long mask = __ballot(sel);
-        int q = at + s_before[k];
-        for (int u = 0; u < wave; u++) q += s_wave[k][u];
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < 3; u++) n += u < wave ? s_wave[k][u] : 0;
+        to[k] = at + s_before[k] + n + lane_rank(__ballot(K.has(k)));
         at += s_total[k];
-        if (!sel) continue;
-        q += lane_rank(mask);
-        double y[3] = {xs[0], xs[1], xs[2]};
-        int digits = k;
+    }
+    if (!mine) return;
+    double y[3][3];
+    int cc[3][3];
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            // src += send_mult * length (comm.py:312-318)
+            y[d][e] = xs[d] + (double) (e == 1 ? 1 : e == 2 ? -1 : 0) * g.len[d];
+            cc[d][e] = e == 0 || g.periodic[d] ? dcell_dim(y[d][e], d, g) : 0;
+        }
+#pragma unroll
+    for (int k = 1; k < NK; k++) {
+        if (!K.has(k)) continue;
+        int digits = k, cell[3];
+        double z[3];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-            // src += send_mult * length (comm.py:312-318)
-            int mult = 0;
-            if (g.periodic[d]) {
-                mult = digits % 3 == 1 ? 1 : digits % 3 == 2 ? -1 : 0;
-                digits /= 3;
-            }
-            y[d] = xs[d] + (double) mult * g.len[d];
+            int e = 0;
+            if (g.periodic[d]) { e = digits % 3; digits /= 3; }
+            z[d] = e == 0 ? y[d][0] : e == 1 ? y[d][1] : y[d][2];
+            cell[d] = e == 0 ? cc[d][0] : e == 1 ? cc[d][1] : cc[d][2];
         }
-        p.uid[q] = uid; p.type[q] = type; p.shape[q] = shape; p.m[q] = m; p.r[q] = r;
-        p.x[q] = y[0]; p.y[q] = y[1]; p.z[q] = y[2];
-        p.vx[q] = v[0]; p.vy[q] = v[1]; p.vz[q] = v[2];
-        p.wx[q] = w[0]; p.wy[q] = w[1]; p.wz[q] = w[2];
-        const int cell = dcell_of(y[0], y[1], y[2], g);
-        p.particle_cell[q] = cell;
-        p.cell_slot[q] = atomicAdd(&p.cell_count[cell], 1);
+        const int to_k = to[k], ck = dcell_index(cell[0], cell[1], cell[2], g);
+        slot[k] = atomicAdd(&p.cell_count[ck], 1);
+        p.particle_cell[to_k] = ck;
+        p.uid[to_k] = uid; p.type[to_k] = type; p.shape[to_k] = shape; p.m[to_k] = m; p.r[to_k] = r;
+        p.x[to_k] = z[0]; p.y[to_k] = z[1]; p.z[to_k] = z[2];
+        p.vx[to_k] = v[0]; p.vy[to_k] = v[1]; p.vz[to_k] = v[2];
+        p.wx[to_k] = w[0]; p.wy[to_k] = w[1]; p.wz[to_k] = w[2];
     }
+#pragma unroll
+    for (int k = 1; k < NK; k++)
+        if (K.has(k)) p.cell_slot[to[k]] = slot[k];
 }
-
-// ---------------------------------------------------------------- cells
 
 // exclusive scan of the cell counts: each block's own, and the block totals;
 // the counts are cleared behind the reads (nothing else uses them, so the next
@@ -552,19 +585,21 @@ __global__ __launch_bounds__(1024) void k_scan_add(const int *__restrict__ in, i
     if (i < n) out[i] = in[i] + off;
 }
 
-// The particles into their cells.  ADD: the blocks' offsets are not in
+// The particles into their cells (a half-space's entry carries a mark).  ADD: the blocks' offsets are not in
 // cell_start yet: every workgroup scans the block totals (at most SCAN_LDS of
 // them) in LDS and adds them where it needs them, and the workgroups share the
 // writing of cell_start for the passes behind.
 constexpr int SCAN_LDS = 2048;
+constexpr int CELL_PLANE = (int) 0x80000000;
 template <bool ADD>
 __global__ __launch_bounds__(256) void k_cell_fill(DemPtrs p, const int *__restrict__ c, int nstart, int nblk) {
     __shared__ int s_off[ADD ? SCAN_LDS : 1];
     __shared__ int lds[8];
     const int n = c[D_NLOCAL] + c[D_NGHOST];
     const int i = blockIdx.x * 256 + threadIdx.x;
-    int cell = 0, start = 0, slot = 0;
+    int cell = 0, start = 0, slot = 0, sh = 0;
     if (i < n) {
+        sh = p.shape[i];
         cell = p.particle_cell[i];
         slot = p.cell_slot[i];
         start = (ADD ? p.cell_scan : p.cell_start)[cell];
@@ -582,7 +617,7 @@ __global__ __launch_bounds__(256) void k_cell_fill(DemPtrs p, const int *__restr
         for (int k = i; k < nstart; k += gridDim.x * 256) p.cell_start[k] = p.cell_scan[k] + s_off[k >> 10];
         start += s_off[cell >> 10];
     }
-    if (i < n) p.cell_particles[start + slot] = i;
+    if (i < n) p.cell_particles[start + slot] = i | (sh != DSHAPE_SPHERE ? CELL_PLANE : 0);
 }
 
 // PartitionCellLists (src/pairs/sim/cell_lists.py:137-171) of one cell, whose
@@ -620,6 +655,8 @@ __device__ __forceinline__ void partition_cell(const int *__restrict__ shape, in
 // of its first particle and written by it.  Bound by memory: 100 bytes in and
 // 136 out per particle, the records through LDS so that a wave writes whole
 // lines (13 us at 190000 particles; 42 with each thread storing its record).
+// A cell's entries are read four at a time and say themselves which of them is
+// a half-space (15 us with an entry and its shape at a time).
 __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__restrict__ c) {
     constexpr int W = 13;  // LDS row of a record (doubles, one of padding)
     __shared__ double s_rec[256 * W];
@@ -627,16 +664,20 @@ __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__rest
     const int b0 = blockIdx.x * 256;
     const int i = b0 + threadIdx.x;
     if (b0 >= n) return;
-    int sh = DSHAPE_SPHERE;
+    int sh = DSHAPE_SPHERE, fl = 0, cell = 0, s0 = 0, cnt = 0;
     double x = 0.0, y = 0.0, z = 0.0, r = 0.0;
     if (i < n) {
+        cell = p.particle_cell[i];
         sh = p.shape[i];
+        fl = p.flags[i];
         x = p.x[i]; y = p.y[i]; z = p.z[i]; r = p.r[i];
         double *R = s_rec + threadIdx.x * W;
         R[0] = x; R[1] = y; R[2] = z; R[3] = r;
         R[4] = p.vx[i]; R[5] = p.vy[i]; R[6] = p.vz[i]; R[7] = p.m[i];
         R[8] = p.wx[i]; R[9] = p.wy[i]; R[10] = p.wz[i];
         R[11] = __longlong_as_double((long long) p.uid[i] << 32 | (unsigned) p.type[i]);
+        s0 = p.cell_start[cell];
+        cnt = p.cell_start[cell + 1] - s0;
     }
     __syncthreads();
     // the block's records, 16 bytes per thread at consecutive addresses
@@ -647,29 +688,32 @@ __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__rest
         ((double2 *) (p.rec + b0 + k))[w] = make_double2(R[0], R[1]);
     }
     if (i >= n) return;
-    const int cell = p.particle_cell[i];
-    const int s0 = p.cell_start[cell], cnt = p.cell_start[cell + 1] - s0;
     int rank = 0;
     bool mixed = sh != DSHAPE_SPHERE;
     if (cnt > 1)
-        for (int k = 0; k < cnt; k++) {
-            const int j = p.cell_particles[s0 + k];
-            rank += j < i ? 1 : 0;
-            mixed = mixed || p.shape[j] != DSHAPE_SPHERE;
+        for (int k0 = 0; k0 < cnt; k0 += 4) {
+            int e[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) e[u] = p.cell_particles[s0 + min(k0 + u, cnt - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                rank += k0 + u < cnt && (e[u] & ~CELL_PLANE) < i ? 1 : 0;
+                mixed = mixed || e[u] < 0;
+            }
         }
-    auto put = [&](int q, int j, double jx, double jy, double jz, double jr, int jsh) {
-        p.corder[q] = make_int2(j, cell | ((p.flags[j] & DFLAG_FIXED) ? (int) 0x80000000 : 0));
+    auto put = [&](int q, int j, int jf, double jx, double jy, double jz, double jr, int jsh) {
+        p.corder[q] = make_int2(j, cell | ((jf & DFLAG_FIXED) ? (int) 0x80000000 : 0));
         p.crec[q] = make_double4(jx, jy, jz, jsh == DSHAPE_SPHERE ? jr : -1.0);
     };
     if (!mixed) {
-        put(s0 + rank, i, x, y, z, r, sh);
+        put(s0 + rank, i, fl, x, y, z, r, sh);
     } else if (rank == 0) {
         int *cp = p.cmixed + s0;
-        for (int k = 0; k < cnt; k++) cp[k] = p.cell_particles[s0 + k];
+        for (int k = 0; k < cnt; k++) cp[k] = p.cell_particles[s0 + k] & ~CELL_PLANE;
         partition_cell(p.shape, cp, cnt);
         for (int k = 0; k < cnt; k++) {
             const int j = cp[k];
-            put(s0 + k, j, p.x[j], p.y[j], p.z[j], p.r[j], p.shape[j]);
+            put(s0 + k, j, p.flags[j], p.x[j], p.y[j], p.z[j], p.r[j], p.shape[j]);
         }
     }
 }
@@ -971,7 +1015,8 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
 // 187200 spheres) and the FP64 divisions and roots of the contact law.  One
 // dense pass in place of a kernel per phase: the phases ran one thread per
 // possible contact (16 per particle) or per particle, and gathered a partner
-// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres.
+// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres;
+// eight history slots compared at a time 53 -> 48.
 template <int SPW>
 __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict__ c, DemGeom g, DemParams prm) {
     __shared__ double s_term[64][7];
@@ -1008,8 +1053,14 @@ __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict
         const int uid = p.rec[e < 0 ? ~e : e].uid;
         const int m = s_nc[s];
         int slot = -1;
-        for (int h = 0; h < m; h++)
-            if (p.c_uid[h * C + ii] == uid) slot = h;
+        for (int h0 = 0; h0 < m; h0 += 8) {
+            int u[8];
+#pragma unroll
+            for (int v = 0; v < 8; v++) u[v] = p.c_uid[min(h0 + v, m - 1) * C + ii];
+#pragma unroll
+            for (int v = 0; v < 8; v++)
+                if (h0 + v < m && u[v] == uid) slot = h0 + v;
+        }
         s_cand[k] = e;
         s_uid[k] = uid;
         s_slot[k] = slot;
@@ -1237,8 +1288,8 @@ void launch_mass_inertia(hipStream_t s, const DemPtrs &p, int nl) {
 template <int ND>
 static void launch_borders(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
     const int nb = grid_of(p.cap, 256);
-    if constexpr (ND > 0) hipLaunchKernelGGL(k_border_count<ND>, dim3(nb), dim3(256), 0, s, p, c, g, nb);
-    hipLaunchKernelGGL(k_border_cells<ND>, dim3(nb), dim3(256), 0, s, p, c, g, nb);
+    hipLaunchKernelGGL(k_cell_count<ND>, dim3(nb), dim3(256), 0, s, p, c, g, nb);
+    if constexpr (ND > 0) hipLaunchKernelGGL(k_border_ghosts<ND>, dim3(nb), dim3(256), 0, s, p, c, g, nb);
 }
 
 void launch_find_leavers(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
