@@ -439,9 +439,8 @@ __global__ __launch_bounds__(256) void k_cell_count(DemPtrs p, int *__restrict__
 // decision, dimension by dimension; without room no ghost is made and the cells
 // hold the locals.  Bound by latency: the particle's fields are loaded before
 // the sums and the atomics of all kinds are in flight before the first place
-// is stored.  2080 | 187200 spheres, us: with the locals' atomics here, a kind
-// and its cell at a time 12 | 22 on top of 2.6 | 4.7 for the counts; so 7.7 |
-// 9.4 on top of 3.1 | 9.6 for k_cell_count.
+// is stored (with the locals' atomics here and a kind at a time 12 us at 2080
+// spheres and 22 at 187200, TIMEB so with k_cell_count).
 template <int ND>
 __global__ __launch_bounds__(256) void k_border_ghosts(DemPtrs p, int *__restrict__ c, DemGeom g, int pitch) {
     constexpr int NK = pow3(ND);
@@ -655,8 +654,6 @@ __device__ __forceinline__ void partition_cell(const int *__restrict__ shape, in
 // of its first particle and written by it.  Bound by memory: 100 bytes in and
 // 136 out per particle, the records through LDS so that a wave writes whole
 // lines (13 us at 190000 particles; 42 with each thread storing its record).
-// A cell's entries are read four at a time and say themselves which of them is
-// a half-space (15 us with an entry and its shape at a time).
 __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__restrict__ c) {
     constexpr int W = 13;  // LDS row of a record (doubles, one of padding)
     __shared__ double s_rec[256 * W];
@@ -908,25 +905,30 @@ __device__ __forceinline__ int group_scan(int x) {
 // groups of a wave are neighbours and read the same records).  The visiting
 // order's 28 cells (cell 0, then the 27 stencil cells) are ten runs of the
 // cell order: cell 0, and the three cells of each of the nine z-columns, which
-// are consecutive.  Lane 0 takes cell 0 and column 0, lanes 1 to 6 a column
-// each, lane 7 columns 7 and 8.  Each lane counts the touching spheres and
-// half-spaces of its runs; prefix sums over the lanes give every hit its place
-// in the visiting order (all spheres, then all half-spaces), and the hits are
-// stored from a bit mask of the lane's first 32 candidates (beyond them the
-// test is repeated) as cand[i][t] (half-spaces as ~j).
+// are consecutive.  Lane l finds the bounds of column l, lane 0 those of cell 0
+// and lane 7 those of the last column too; the runs are laid end to end in LDS
+// (a window of FIND_WIN candidates at a time) and the lanes take the candidates
+// in turn, so that all have the same number whatever the runs' lengths.  A
+// group's part of the wave's ballot gives every hit its place in the visiting
+// order (all spheres, then all half-spaces); they are stored to cand[i][t]
+// (half-spaces as ~j).
 // cand_n[i] = DCAND + 1 when more than DCAND touch (the contact kernel then
 // walks the cells itself).  Only geometry is read: no history is touched.
-// Bound by the latency of its three dependent loads (place, run bounds,
-// candidates); the candidates of a run are consecutive 32-byte records.  By
-// particle index, cell by cell and from four arrays it took 105 us in a bed of
-// 187200 spheres and 59 us on the falling 200000; now 41 and 28.
-constexpr int LPS = 8;
+// Bound by vector work, then by the latency of its dependent loads (place, run
+// bounds, candidates).  Bed of 187200 spheres | 200000 falling, us: by particle
+// index, cell by cell, from four arrays 105 | 59; a lane per column of the
+// ordered records, as slow as its longest column, 41 | 28; TIMEF so.
+constexpr int LPS = 8, FIND_WIN = 64;
 __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__restrict__ c, DemGeom g) {
+    constexpr int GROUPS = 256 / LPS;
+    __shared__ int s_place[GROUPS][FIND_WIN + 1];
+    __shared__ int s_hit[GROUPS][DCAND + 1], s_wall[GROUPS][DCAND + 1];
     if (c[D_OVF]) return;
     const int nl = c[D_NLOCAL], n = nl + c[D_NGHOST];
     const int q0 = (blockIdx.x * 256 + threadIdx.x) / LPS;
-    const int l = threadIdx.x & (LPS - 1);
+    const int l = threadIdx.x & (LPS - 1), grp = threadIdx.x / LPS;
     const bool in = q0 < n;
+    if (!__ballot(in)) return;
     const int qi = in ? q0 : 0;
     const int2 own = p.corder[qi];
     const int i = own.x, cc = own.y;
@@ -953,47 +955,70 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
     }
     const double xi[3] = {me.x, me.y, me.z};
     const double ri = me.w;
-    const int tot = len[0] + len[1];
-    auto place = [&](int b) { return b < len[0] ? st[0] + b : st[1] + (b - len[0]); };
+    const int upto = group_scan<LPS>(len[0] + len[1]);
+    const int total = __shfl(upto, LPS - 1, LPS);
+    const int at[2] = {upto - len[0] - len[1], upto - len[1]};  // the runs' first candidates
     // 0: no contact, 1: sphere, 2: half-space
     auto touch = [&](int q, const double4 &r) {
         double nv[3], cpt[3], delta;
         const double xj[3] = {r.x, r.y, r.z};
-        if (r.w >= 0.0) return q != qi && sphere_contact(xi, ri, xj, r.w, nv, cpt, delta) ? 1 : 0;
-        const int j = p.corder[q].x;
-        return q != qi && plane_contact(p, xi, ri, j, xj, nv, cpt, delta) ? 2 : 0;
+        if (q == qi) return 0;
+        if (r.w >= 0.0) {
+            // sqrt(d2) - ri - rj <= 0 without the root where d2 is below (ri +
+            // rj)^2 by more than 1e-12 of it (the rounding errors are 1e-15)
+            const double d0 = xi[0] - xj[0], d1 = xi[1] - xj[1], d2 = xi[2] - xj[2], rs = ri + r.w;
+            const double dd = (d0 * d0 + d1 * d1) + d2 * d2, rr = rs * rs;
+            if (ri >= 0.0 && rr > 1e-280 && dd < rr * (1.0 - 1e-12)) return 1;
+            return sphere_contact(xi, ri, xj, r.w, nv, cpt, delta) ? 1 : 0;
+        }
+        return plane_contact(p, xi, ri, p.corder[q].x, xj, nv, cpt, delta) ? 2 : 0;
     };
-    int hs = 0, hh = 0;
-    unsigned hit = 0u;
-    for (int b = 0; b < tot; b += 2) {
-        const int qa = place(b), qb = place(min(b + 1, tot - 1));
-        const double4 ra = p.crec[qa], rb = p.crec[qb];
-        const int ta = touch(qa, ra), tb = b + 1 < tot ? touch(qb, rb) : 0;
-        hs += (ta == 1) + (tb == 1);
-        hh += (ta == 2) + (tb == 2);
-        if (b < 32) hit |= (unsigned) (ta != 0) << b | (unsigned) (tb != 0) << (b + 1);
-    }
-    const int ps = group_scan<LPS>(hs), ph = group_scan<LPS>(hh);
-    const int tot_s = __shfl(ps, LPS - 1, LPS), tot_h = __shfl(ph, LPS - 1, LPS);
-    const int nt = tot_s + tot_h;
-    if (act && nt <= DCAND) {
-        int os = ps - hs, oh = tot_s + ph - hh;
-        int *__restrict__ out = p.cand + (size_t) i * DCAND;
-        while (hit) {
-            const int b = __builtin_ctz(hit);
-            hit &= hit - 1u;
-            const int q = place(b), j = p.corder[q].x;
-            if (p.crec[q].w >= 0.0) out[os++] = j;
-            else out[oh++] = ~j;
+    const int shift = (threadIdx.x & 63) & ~(LPS - 1);
+    const unsigned below = (1u << l) - 1u;
+    int ns = 0, nh = 0;  // hits of the group
+    for (int w0 = 0; __ballot(w0 < total); w0 += FIND_WIN) {
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+            for (int k = max(0, w0 - at[e]); k < min(len[e], w0 + FIND_WIN - at[e]); k++)
+                s_place[grp][at[e] + k - w0] = st[e] + k;
+        wave_lds_sync();
+        const int m = min(total - w0, FIND_WIN);
+        for (int b = 0; __ballot(b < m); b += 2 * LPS) {
+            const int ba = b + l, bb = b + LPS + l;
+            const bool ina = ba < m, inb = bb < m;
+            const int qa = ina ? s_place[grp][ba] : qi, qb = inb ? s_place[grp][bb] : qi;
+            const double4 ra = p.crec[qa], rb = p.crec[qb];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int q = e == 0 ? qa : qb;
+                const int t = touch(q, e == 0 ? ra : rb);  // none for its own record
+                const unsigned sph = (unsigned) (__ballot(t == 1) >> shift) & 0xffu;
+                if (t == 1) {
+                    const int r = ns + __popc(sph & below);
+                    if (r < DCAND) s_hit[grp][r] = q;
+                }
+                ns += __popc(sph);
+                const unsigned long long walls = __ballot(t == 2);
+                if (walls) {
+                    const unsigned pl = (unsigned) (walls >> shift) & 0xffu;
+                    if (t == 2) {
+                        const int r = nh + __popc(pl & below);
+                        if (r < DCAND) s_wall[grp][r] = q;
+                    }
+                    nh += __popc(pl);
+                }
+            }
         }
-        for (int b = 32; b < tot; b++) {
-            const int q = place(b);
-            const int t = touch(q, p.crec[q]);
-            if (t == 1) out[os++] = p.corder[q].x;
-            else if (t == 2) out[oh++] = ~p.corder[q].x;
-        }
+        wave_lds_sync();
     }
-    if (act && l == 0) p.cand_n[i] = nt <= DCAND ? nt : DCAND + 1;
+    const int nt = ns + nh;
+    if (!act) return;
+    if (nt <= DCAND)
+        for (int t = l; t < nt; t += LPS) {
+            const int j = p.corder[t < ns ? s_hit[grp][t] : s_wall[grp][t - ns]].x;
+            p.cand[(size_t) i * DCAND + t] = t < ns ? j : ~j;
+        }
+    if (l == 0) p.cand_n[i] = nt <= DCAND ? nt : DCAND + 1;
 }
 
 // The contacts of SPW consecutive local particles, one wave.  The wave's
@@ -1015,8 +1040,7 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
 // 187200 spheres) and the FP64 divisions and roots of the contact law.  One
 // dense pass in place of a kernel per phase: the phases ran one thread per
 // possible contact (16 per particle) or per particle, and gathered a partner
-// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres;
-// eight history slots compared at a time 53 -> 48.
+// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres.
 template <int SPW>
 __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict__ c, DemGeom g, DemParams prm) {
     __shared__ double s_term[64][7];

@@ -27,14 +27,6 @@ __device__ __forceinline__ double pair_swap(double v) {
     return __longlong_as_double(((long long) hi << 32) | (unsigned int) lo);
 }
 
-// LDS operations of one wave complete in order, so what a wave hands from
-// lane to lane needs no wait, only an order the compiler keeps
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct SegInfo {
     int cx, cy, za, zb;  // column and z range [za, zb) of the home cells
     int ca, cb;          // flat cell ids of the first home cell and one past the last
