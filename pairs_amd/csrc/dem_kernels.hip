@@ -439,8 +439,9 @@ __global__ __launch_bounds__(256) void k_cell_count(DemPtrs p, int *__restrict__
 // decision, dimension by dimension; without room no ghost is made and the cells
 // hold the locals.  Bound by latency: the particle's fields are loaded before
 // the sums and the atomics of all kinds are in flight before the first place
-// is stored (with the locals' atomics here and a kind at a time 12 us at 2080
-// spheres and 22 at 187200, TIMEB so with k_cell_count).
+// is stored.  2080 | 187200 spheres, us: with the locals' atomics here, a kind
+// and its cell at a time 12 | 22 on top of 2.6 | 4.7 for the counts; so 7.7 |
+// 9.4 on top of 3.1 | 9.6 for k_cell_count.
 template <int ND>
 __global__ __launch_bounds__(256) void k_border_ghosts(DemPtrs p, int *__restrict__ c, DemGeom g, int pitch) {
     constexpr int NK = pow3(ND);
@@ -654,6 +655,8 @@ __device__ __forceinline__ void partition_cell(const int *__restrict__ shape, in
 // of its first particle and written by it.  Bound by memory: 100 bytes in and
 // 136 out per particle, the records through LDS so that a wave writes whole
 // lines (13 us at 190000 particles; 42 with each thread storing its record).
+// A cell's entries are read four at a time and say themselves which of them is
+// a half-space (15 us with an entry and its shape at a time).
 __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__restrict__ c) {
     constexpr int W = 13;  // LDS row of a record (doubles, one of padding)
     __shared__ double s_rec[256 * W];
@@ -917,7 +920,7 @@ __device__ __forceinline__ int group_scan(int x) {
 // Bound by vector work, then by the latency of its dependent loads (place, run
 // bounds, candidates).  Bed of 187200 spheres | 200000 falling, us: by particle
 // index, cell by cell, from four arrays 105 | 59; a lane per column of the
-// ordered records, as slow as its longest column, 41 | 28; TIMEF so.
+// the ordered records, as slow as its longest column, 41 | 28; so 31 | 25.
 constexpr int LPS = 8, FIND_WIN = 64;
 __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__restrict__ c, DemGeom g) {
     constexpr int GROUPS = 256 / LPS;
@@ -1040,7 +1043,8 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
 // 187200 spheres) and the FP64 divisions and roots of the contact law.  One
 // dense pass in place of a kernel per phase: the phases ran one thread per
 // possible contact (16 per particle) or per particle, and gathered a partner
-// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres.
+// from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres;
+// eight history slots compared at a time 53 -> 48.
 template <int SPW>
 __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict__ c, DemGeom g, DemParams prm) {
     __shared__ double s_term[64][7];
