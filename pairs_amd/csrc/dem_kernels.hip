@@ -242,7 +242,7 @@ __device__ __forceinline__ void exch_move(const DemPtrs &p, double *const *s_arr
 __global__ __launch_bounds__(1024) void k_exchange(DemPtrs p, int *__restrict__ c, DemGeom g) {
     __shared__ int lds[20];
     __shared__ double *s_arr[EXD];
-    __shared__ unsigned s_key[LEAVE_CAP];
+    __shared__ __align__(16) unsigned s_key[LEAVE_CAP];
     __shared__ int s_map[LEAVE_CAP], s_fill[LEAVE_CAP], s_hole[LEAVE_CAP], s_tail[LEAVE_CAP];
     const int tid = threadIdx.x, cnt = c[D_LEAVE], nl = c[D_NLOCAL], ovf = c[D_OVF];
     __syncthreads();
@@ -266,7 +266,14 @@ __global__ __launch_bounds__(1024) void k_exchange(DemPtrs p, int *__restrict__ 
             if (n == 0) continue;
             if (n <= p.send_cap) {
                 int rank = 0;
-                for (int u = 0; u < cnt; u++) rank += s_key[u] < key ? 1 : 0;
+                if (__ballot(out)) {  // (the entries past cnt are the largest key)
+                    const uint4 *k4 = (const uint4 *) s_key;
+#pragma unroll 4
+                    for (int u = 0; u < (cnt + 3) / 4; u++) {
+                        const uint4 k = k4[u];
+                        rank += (k.x < key ? 1 : 0) + (k.y < key ? 1 : 0) + (k.z < key ? 1 : 0) + (k.w < key ? 1 : 0);
+                    }
+                }
                 if (out) {
                     s_map[rank] = me;
                     p.send_map[rank] = me;

@@ -1567,9 +1567,9 @@ __device__ __forceinline__ void k_sel_count_body(const double *__restrict__ Xd, 
 
 __global__ __launch_bounds__(256) void k_sel_count(const double *__restrict__ Xd, const int *__restrict__ flags,
                                                    const int *__restrict__ phys, int *__restrict__ counters, Geom g,
-                                                   int dim, int exch, int first, int *__restrict__ tile_cnt,
+                                                   int dim, int *__restrict__ tile_cnt,
                                                    int *__restrict__ exchg_flag) {
-    k_sel_count_body(Xd, flags, phys, counters, g, dim, exch, first, tile_cnt, exchg_flag);
+    k_sel_count_body(Xd, flags, phys, counters, g, dim, 1, 0, tile_cnt, exchg_flag);
 }
 
 // sums of two per-thread values over a workgroup of 256 threads
@@ -1697,10 +1697,10 @@ __global__ __launch_bounds__(256) void k_sel_scatter(double *__restrict__ X, dou
                                                      int *__restrict__ uid, int *__restrict__ shape,
                                                      int *__restrict__ flags, int *__restrict__ ref,
                                                      int *__restrict__ phys, int *__restrict__ counters, Geom g,
-                                                     int dim, int exch, const int *__restrict__ tile_cnt,
+                                                     int dim, const int *__restrict__ tile_cnt,
                                                      int *__restrict__ send_map, int *__restrict__ send_mult,
                                                      int send_cap, int cap) {
-    k_sel_scatter_body(X, Y, Z, vx, vy, vz, mass, type, uid, shape, flags, ref, phys, counters, g, dim, exch,
+    k_sel_scatter_body(X, Y, Z, vx, vy, vz, mass, type, uid, shape, flags, ref, phys, counters, g, dim, 1,
                        tile_cnt, send_map, send_mult, send_cap, cap);
 }
 
@@ -1715,7 +1715,7 @@ __global__ __launch_bounds__(256) void k_sel_scatter(double *__restrict__ X, dou
 // index below nlocal (descending).  One workgroup: a rebuild moves few particles.
 __device__ __forceinline__ void k_exchange_relabel_body(double *__restrict__ X, double *__restrict__ Y,
                                                            double *__restrict__ Z, int *__restrict__ ref,
-                                                           int *__restrict__ phys, const int *__restrict__ counters,
+                                                           int *__restrict__ phys, int n, int nlocal,
                                                            Geom g, const int *__restrict__ send_map,
                                                            const int *__restrict__ send_mult,
                                                            const int *__restrict__ exchg_flag, int *__restrict__ tail,
@@ -1723,10 +1723,7 @@ __device__ __forceinline__ void k_exchange_relabel_body(double *__restrict__ X, 
                                                            int *__restrict__ p_src) {
     __shared__ int lds[20];
     __shared__ int s_tail[1024];
-    if (counters[C_OVF]) return;
-    const int n = counters[C_NSEND_ALL];
     if (n == 0) return;
-    const int nlocal = counters[C_NLOCAL];
     if (n <= 1024) {
         // one leaver per thread (the usual case): the tail list in LDS and
         // each leaver's entries in registers, the same steps as below
@@ -1807,7 +1804,399 @@ __global__ __launch_bounds__(1024) void k_exchange_relabel(double *__restrict__ 
                                                            const int *__restrict__ exchg_flag, int *__restrict__ tail,
                                                            int *__restrict__ copy_to, int *__restrict__ p_leaver,
                                                            int *__restrict__ p_src) {
-    k_exchange_relabel_body(X, Y, Z, ref, phys, counters, g, send_map, send_mult, exchg_flag, tail, copy_to, p_leaver, p_src);
+    if (counters[C_OVF]) return;
+    k_exchange_relabel_body(X, Y, Z, ref, phys, counters[C_NSEND_ALL], counters[C_NLOCAL], g, send_map, send_mult,
+                            exchg_flag, tail, copy_to, p_leaver, p_src);
+}
+
+// ---------------------------------------------------------------- exchange from a list of leavers
+
+// a local outside the box along a periodic dimension joins the list that the
+// exchange reads.  An exchange shifts a particle only along its own dimension,
+// so whoever leaves along any of them is outside before the first.
+__global__ __launch_bounds__(256) void k_find_leavers(const double *__restrict__ X, const double *__restrict__ Y,
+                                                      const double *__restrict__ Z, const int *__restrict__ flags,
+                                                      int *__restrict__ counters, Geom g, int px, int py, int pz,
+                                                      int *__restrict__ leavers) {
+    if (counters[C_OVF]) return;
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= counters[C_NLOCAL]) return;
+    const int fl = flags[p];
+    bool out = false, a, b;
+    if (px) { ghost_sel(X[p], fl, 0, g, true, a, b); out = out || a || b; }
+    if (py) { ghost_sel(Y[p], fl, 1, g, true, a, b); out = out || a || b; }
+    if (pz) { ghost_sel(Z[p], fl, 2, g, true, a, b); out = out || a || b; }
+    if (!out) return;
+    const int k = atomicAdd(&counters[C_LEAVE], 1);
+    if (k < LEAVE_CAP) leavers[k] = p;
+}
+
+// The exchange of all periodic dimensions in one workgroup, a leaver per
+// thread.  A particle keeps its physical slot; what moves is its reference
+// index.  Per dimension the leavers are ranked by side and reference index (the
+// reference's send order), the tail walk is planned with two scans, and the
+// relabeling is that of k_exchange_relabel_body.  More leavers than the list
+// holds are found by a scan of the locals in reference order instead.  Bound by
+// the latency of its phases; with k_find_leavers it takes the place of three
+// kernels per dimension (us per rebuild: 256 atoms 27 -> LJX1, 131072 45 ->
+// LJX2).  Beyond some 200000 locals the leavers of a rebuild no longer fit
+// and the three kernels remain (exch_listed).
+__global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, double *__restrict__ Y,
+                                                   double *__restrict__ Z, const int *__restrict__ flags,
+                                                   int *__restrict__ ref, int *__restrict__ phys,
+                                                   int *__restrict__ counters, Geom g, int px, int py, int pz,
+                                                   const int *__restrict__ leavers, int *__restrict__ send_map,
+                                                   int *__restrict__ send_mult, int *__restrict__ exchg_flag,
+                                                   int *__restrict__ scratch, int send_cap) {
+    __shared__ int lds[20];
+    __shared__ __align__(16) unsigned s_key[LEAVE_CAP];
+    __shared__ int s_map[LEAVE_CAP], s_fill[LEAVE_CAP], s_hole[LEAVE_CAP], s_tail[LEAVE_CAP];
+    const int tid = threadIdx.x, cnt = counters[C_LEAVE], nl = counters[C_NLOCAL], ovf = counters[C_OVF];
+    __syncthreads();
+    if (tid == 0) { counters[C_LEAVE] = 0; counters[C_LEAVE_MAX] = cnt; }
+    if (ovf) return;
+    const bool listed = cnt <= LEAVE_CAP;
+    const int me = listed && tid < cnt ? leavers[tid] : -1;
+    const int periodic[3] = {px, py, pz};
+#pragma unroll
+    for (int dim = 0; dim < 3; dim++) {
+        if (!periodic[dim]) continue;
+        const double *Xd = dim == 0 ? X : (dim == 1 ? Y : Z);
+        int n0 = 0, n1 = 0, r = -1;
+        bool a = false, b = false;
+        if (listed) {
+            if (me >= 0) {
+                r = ref[me];
+                ghost_sel(Xd[me], flags[me], dim, g, true, a, b);
+            }
+            s_key[tid] = a ? (unsigned) r : b ? (unsigned) r | 0x80000000u : 0xffffffffu;
+            s_tail[tid] = 0;
+            n0 = __syncthreads_count(a);
+            n1 = __syncthreads_count(b);
+        } else {
+            for (int i0 = 0; i0 < nl; i0 += 1024) {
+                const int i = i0 + tid;
+                bool c0 = false, c1 = false;
+                if (i < nl) {
+                    const int p = phys[i];
+                    ghost_sel(Xd[p], flags[p], dim, g, true, c0, c1);
+                    exchg_flag[i] = c0 || c1 ? 1 : 0;
+                }
+                n0 += __syncthreads_count(c0);
+                n1 += __syncthreads_count(c1);
+            }
+        }
+        const int n = n0 + n1;
+        if (n > send_cap) {
+            if (tid == 0) {
+                counters[C_OVF] = OVF_SEND;
+                counters[C_REQ_SEND] = max(counters[C_REQ_SEND], n);
+            }
+            return;
+        }
+        if (tid == 0) {
+            counters[C_NSEND + 2 * dim] = n0;
+            counters[C_NSEND + 2 * dim + 1] = n1;
+            counters[C_NSEND_ALL] = n;
+        }
+        if (n == 0) continue;
+        auto send = [&](int pos, int idx, int side) {
+            const int mult = side == 0 ? 1 : -1;  // pbc_prev = +1, pbc_next = -1 on one rank
+            send_map[pos] = idx;
+            send_mult[3 * pos + 0] = dim == 0 ? mult : 0;
+            send_mult[3 * pos + 1] = dim == 1 ? mult : 0;
+            send_mult[3 * pos + 2] = dim == 2 ? mult : 0;
+        };
+        if (listed) {
+            const unsigned key = s_key[tid];
+            int rank = 0;
+            if (__ballot(a || b)) {  // (the entries past cnt are the largest key)
+                const uint4 *k4 = (const uint4 *) s_key;
+#pragma unroll 4
+                for (int u = 0; u < (cnt + 3) / 4; u++) {
+                    const uint4 k = k4[u];
+                    rank += (k.x < key ? 1 : 0) + (k.y < key ? 1 : 0) + (k.z < key ? 1 : 0) + (k.w < key ? 1 : 0);
+                }
+            }
+            if (a || b) {
+                s_map[rank] = r;
+                send(rank, r, a ? 0 : 1);
+                if (r >= nl - n) s_tail[nl - 1 - r] = 1;
+            }
+            __syncthreads();
+            int fills_all, holes;
+            const bool fills = tid < n && !s_tail[tid], hole = tid < n && s_map[tid] < nl - n;
+            const int ef = block_exclusive_scan<1024>(fills ? 1 : 0, lds, &fills_all);
+            const int eh = block_exclusive_scan<1024>(hole ? 1 : 0, lds, &holes);
+            if (fills) s_fill[ef] = nl - 1 - tid;
+            if (hole) s_hole[eh] = s_map[tid];
+            __syncthreads();
+            const int src = tid < holes ? s_fill[tid] : -1;
+            const int ps = src > 0 ? phys[src] : -1;
+            __syncthreads();
+            if (ps >= 0) { const int dst = s_hole[tid]; ref[ps] = dst; phys[dst] = ps; }
+            if (a || b) {
+                const double mult = a ? 1.0 : -1.0;
+                X[me] = X[me] + (dim == 0 ? mult : 0.0) * g.len[0];
+                Y[me] = Y[me] + (dim == 1 ? mult : 0.0) * g.len[1];
+                Z[me] = Z[me] + (dim == 2 ? mult : 0.0) * g.len[2];
+                ref[me] = nl - n + rank;
+                phys[nl - n + rank] = me;
+            }
+        } else {
+            int o0 = 0, o1 = n0;
+            for (int i0 = 0; i0 < nl; i0 += 1024) {
+                const int i = i0 + tid;
+                bool c0 = false, c1 = false;
+                if (i < nl) {
+                    const int p = phys[i];
+                    ghost_sel(Xd[p], flags[p], dim, g, true, c0, c1);
+                }
+                int t0, t1;
+                const int q0 = block_exclusive_scan<1024>(c0 ? 1 : 0, lds, &t0);
+                const int q1 = block_exclusive_scan<1024>(c1 ? 1 : 0, lds, &t1);
+                if (c0) send(o0 + q0, i, 0);
+                if (c1) send(o1 + q1, i, 1);
+                o0 += t0;
+                o1 += t1;
+            }
+            __syncthreads();
+            k_exchange_relabel_body(X, Y, Z, ref, phys, n, nl, g, send_map, send_mult, exchg_flag, scratch,
+                                    scratch + send_cap, scratch + 2 * send_cap, scratch + 3 * send_cap);
+        }
+        __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------- borders in two passes
+
+constexpr int pow3(int n) { return n == 0 ? 1 : 3 * pow3(n - 1); }
+
+// Borders (comm.py:56-98): dimension by dimension, side 0 then side 1, every
+// local and every ghost of the dimensions before that lies within a cell
+// spacing of the face gets a ghost behind all others.  A ghost keeps its
+// particle's other coordinates (and its flags read 0), so whether it is selected
+// along a later dimension depends on the particle alone, and the ghosts fall
+// into kinds: one digit per periodic dimension (0 not shifted, 1 side 0, 2 side
+// 1), the later dimension the higher digit.  The order of the ghosts is that of
+// their kind as a number in base 3, and within a kind the reference order of the
+// particles; the source of a ghost is the ghost, or the particle, of the kind
+// without the top digit.  So one count per kind and tile of BORDER_T reference
+// indices places them all.
+constexpr int BORDER_T = 1024;
+
+template <int ND>
+struct Kinds {
+    bool side[ND][2];
+    int dim[ND];
+    __device__ __forceinline__ void set(const Geom &g, int px, int py, int pz, const double (&xs)[3], int fl, bool in) {
+#pragma unroll
+        for (int k = 0; k < ND; k++) dim[k] = k;
+        if (ND == 2) { dim[0] = px ? 0 : 1; dim[ND - 1] = pz ? 2 : 1; }
+        if (ND == 1) dim[0] = px ? 0 : py ? 1 : 2;
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            const int d = dim[k];
+            bool a, b;
+            ghost_sel(d == 0 ? xs[0] : d == 1 ? xs[1] : xs[2], fl, d, g, false, a, b);
+            side[k][0] = in && a;
+            side[k][1] = in && b;
+        }
+    }
+    __device__ __forceinline__ bool any() const {
+        bool r = false;
+#pragma unroll
+        for (int k = 0; k < ND; k++) r = r || side[k][0] || side[k][1];
+        return r;
+    }
+    __device__ __forceinline__ bool has(int kind) const {
+        bool r = true;
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            const int digit = kind % 3;
+            kind /= 3;
+            r = r && (digit == 0 || side[k][digit == 2 ? 1 : 0]);
+        }
+        return r;
+    }
+};
+
+struct BorderArgs {
+    double *X, *Y, *Z, *vx, *vy, *vz, *mass;
+    int *type, *uid, *shape, *flags, *ref, *phys, *counters;
+    Geom g;
+    int px, py, pz, pitch, send_cap, cap;
+    int *cnt;  // [kind][tile], kinds pitch apart
+    int *send_map, *send_mult;
+};
+
+template <int ND>
+__global__ __launch_bounds__(BORDER_T) void k_border_count(BorderArgs A) {
+    constexpr int NK = pow3(ND), NW = BORDER_T / 64;
+    __shared__ int s_n[NK][NW];
+    if (A.counters[C_OVF]) return;
+    const int nl = A.counters[C_NLOCAL], r = blockIdx.x * BORDER_T + threadIdx.x;
+    if ((int) blockIdx.x * BORDER_T >= nl) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double xs[3] = {0.0, 0.0, 0.0};
+    int fl = 0;
+    if (r < nl) {
+        const int p = A.phys[r];
+        xs[0] = A.X[p]; xs[1] = A.Y[p]; xs[2] = A.Z[p]; fl = A.flags[p];
+    }
+    Kinds<ND> K;
+    K.set(A.g, A.px, A.py, A.pz, xs, fl, r < nl);
+    const bool some = __ballot(K.any()) != 0;
+#pragma unroll
+    for (int k = 1; k < NK; k++) {
+        const int m = some ? __popcll(__ballot(K.has(k))) : 0;
+        if (lane == 0) s_n[k][wave] = m;
+    }
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k >= 1 && k < NK) {
+        int n = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) n += s_n[k][w];
+        A.cnt[(size_t) k * A.pitch + blockIdx.x] = n;
+    }
+}
+
+// The ghosts (pack, communicateData's self-copy and unpack of comm.py:291-366:
+// uid, type, mass, position + shift, velocity, shape) at physical slot =
+// reference index nlocal + place, and their send map entries.  Every workgroup
+// sums the tiles' counts itself and takes the same capacity decision, dimension
+// by dimension; on overflow the counts stay as they were.  Bound by latency in
+// small systems and by the ghosts' writes in large ones; with k_border_count it
+// takes the place of a count and a scatter pass per dimension (us per rebuild:
+// 256 atoms 20 -> LJB1, 131072 31 -> LJB2, 1048576 111 -> LJB3).
+template <int ND>
+__global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
+    constexpr int NK = pow3(ND), NW = BORDER_T / 64;
+    __shared__ int s_total[NK], s_before[NK], s_n[NK][NW], s_pre[NK][NW];
+    int *c = A.counters;
+    if (c[C_OVF]) return;
+    const int nl = c[C_NLOCAL], ntiles = (nl + BORDER_T - 1) / BORDER_T;
+    if (blockIdx.x > 0 && (int) blockIdx.x >= ntiles) return;  // workgroup 0 always writes the counts
+    const int r = blockIdx.x * BORDER_T + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int p = 0, fl = 0, uid = 0, type = 0, shape = 0;
+    double xs[3] = {0.0, 0.0, 0.0}, m = 0.0, v[3] = {0.0, 0.0, 0.0};
+    if (r < nl) {
+        p = A.phys[r];
+        xs[0] = A.X[p]; xs[1] = A.Y[p]; xs[2] = A.Z[p]; fl = A.flags[p];
+    }
+    Kinds<ND> K;
+    K.set(A.g, A.px, A.py, A.pz, xs, fl, r < nl);
+    const bool mine = K.any();
+    if (mine) {
+        uid = A.uid[p]; type = A.type[p]; shape = A.shape[p]; m = A.mass[p];
+        v[0] = A.vx[p]; v[1] = A.vy[p]; v[2] = A.vz[p];
+    }
+    const bool some = __ballot(mine) != 0;
+#pragma unroll
+    for (int k = 1; k < NK; k++) {
+        const int n = some ? __popcll(__ballot(K.has(k))) : 0;
+        if (lane == 0) s_n[k][wave] = n;
+    }
+    constexpr int PER = (NK - 1 + NW - 1) / NW;  // kinds of a wave
+    int t[PER] = {}, q[PER] = {};
+#pragma unroll 4
+    for (int u = lane; u < ntiles; u += 64) {
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int k = 1 + wave + NW * e;
+            const int x = k < NK ? A.cnt[(size_t) k * A.pitch + u] : 0;
+            t[e] += x;
+            q[e] += u < (int) blockIdx.x ? x : 0;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            t[e] += __shfl_xor(t[e], o, 64);
+            q[e] += __shfl_xor(q[e], o, 64);
+        }
+        const int k = 1 + wave + NW * e;
+        if (lane == 0 && k < NK) { s_total[k] = t[e]; s_before[k] = q[e]; }
+    }
+    __syncthreads();
+    if ((int) threadIdx.x < (NK - 1) * NW) {
+        const int k = 1 + threadIdx.x / NW, w = threadIdx.x % NW;
+        int n = s_before[k];
+#pragma unroll
+        for (int u = 0; u < NW - 1; u++) n += u < w ? s_n[k][u] : 0;
+        s_pre[k][w] = n;
+    }
+    __syncthreads();
+    int need = 0;
+    bool ovf_send = false, ovf_part = false;
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+        if (ovf_send || ovf_part) break;
+#pragma unroll
+        for (int k = pow3(d); k < pow3(d + 1); k++) need += s_total[k];
+        ovf_send = need > A.send_cap;
+        ovf_part = nl + need > A.cap;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (ovf_send) {
+            c[C_OVF] = OVF_SEND;
+            c[C_REQ_SEND] = max(c[C_REQ_SEND], need);
+        }
+        if (ovf_part) {
+            c[C_OVF] = OVF_PART;
+            c[C_REQ_PART] = max(c[C_REQ_PART], nl + need);
+        }
+        if (!ovf_send && !ovf_part) {
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+#pragma unroll
+                for (int side = 0; side < 2; side++) {
+                    int n = 0;
+#pragma unroll
+                    for (int k = (side + 1) * pow3(d); k < (side + 2) * pow3(d); k++) n += s_total[k];
+                    c[C_NSEND + 2 * K.dim[d] + side] = n;
+                }
+            c[C_NSEND_ALL] = need;
+            c[C_NGHOST] = need;
+        }
+    }
+    if (ovf_send || ovf_part || !some) return;
+    int to[pow3(ND - 1)];  // places of the kinds without the last dimension
+    int at = 0;
+#pragma unroll
+    for (int k = 1; k < NK; k++) {
+        const unsigned long long mask = __ballot(K.has(k));
+        const int pos = at + s_pre[k][wave] + lane_rank(mask);
+        at += s_total[k];
+        if (k < pow3(ND - 1)) to[k] = pos;
+        if (!K.has(k)) continue;
+        int top = 0, digits = k, mult[3] = {0, 0, 0};
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            const int e = digits % 3;
+            digits /= 3;
+            if (e) top = d;
+            const int s = e == 1 ? 1 : e == 2 ? -1 : 0;
+#pragma unroll
+            for (int x = 0; x < 3; x++) mult[x] += K.dim[d] == x ? s : 0;
+        }
+        const int from = k % pow3(top), tk = k / pow3(top) == 1 ? 1 : -1;
+        A.send_map[pos] = from == 0 ? r : nl + to[from];
+        A.send_mult[3 * pos + 0] = K.dim[top] == 0 ? tk : 0;
+        A.send_mult[3 * pos + 1] = K.dim[top] == 1 ? tk : 0;
+        A.send_mult[3 * pos + 2] = K.dim[top] == 2 ? tk : 0;
+        const int gp = nl + pos;
+        A.X[gp] = xs[0] + (double) mult[0] * A.g.len[0];
+        A.Y[gp] = xs[1] + (double) mult[1] * A.g.len[1];
+        A.Z[gp] = xs[2] + (double) mult[2] * A.g.len[2];
+        A.vx[gp] = v[0]; A.vy[gp] = v[1]; A.vz[gp] = v[2];
+        A.mass[gp] = m; A.type[gp] = type; A.uid[gp] = uid; A.shape[gp] = shape;
+        A.flags[gp] = 0;
+        A.ref[gp] = gp;
+        A.phys[gp] = gp;
+    }
 }
 
 // Comm.synchronize with the stale multi-hop semantics of the reference (all
@@ -1975,9 +2364,10 @@ __global__ __launch_bounds__(256) void k_sel_scatter_batch(const RepDesc *__rest
 __global__ __launch_bounds__(1024) void k_exchange_relabel_batch(const RepDesc *__restrict__ D, int dim) {
     REP_ARGS;
     if (!R.periodic[dim]) return;
+    if (d.counters[C_OVF]) return;
     int *sc = d.scratch_i;
-    k_exchange_relabel_body(d.X[c], d.Y[c], d.Z[c], d.ref, d.phys, d.counters, g, d.send_map, d.send_mult,
-                            d.exchg_flag, sc, sc + d.send_cap, sc + 2 * d.send_cap, sc + 3 * d.send_cap);
+    k_exchange_relabel_body(d.X[c], d.Y[c], d.Z[c], d.ref, d.phys, d.counters[C_NSEND_ALL], d.counters[C_NLOCAL], g,
+                            d.send_map, d.send_mult, d.exchg_flag, sc, sc + d.send_cap, sc + 2 * d.send_cap, sc + 3 * d.send_cap);
 }
 
 // which: 0 lcount, 1 gcount (ncells + 1 entries), 2 img_cnt (cap entries)
@@ -2117,40 +2507,53 @@ void launch_expand_neighbors(hipStream_t s, const DevState &d, const Geom &g, in
                        s, d.counters, d.ref, d.nl, d.nl_stride, d.numneighs, out_ref, ncap_out);
 }
 
-static void launch_select_dim(hipStream_t s, const DevState &d, const Geom &g, int dim, int exch, int first) {
-    const int grid = tile_grid(d.cap);
-    const int c = d.cur;
-    const double *Xd = dim == 0 ? d.X[c] : (dim == 1 ? d.Y[c] : d.Z[c]);
-    hipLaunchKernelGGL(k_sel_count, dim3(grid), dim3(256), 0, s, Xd, d.flags, d.phys, d.counters, g, dim, exch, first,
-                       d.tile_cnt, d.exchg_flag);
-    hipLaunchKernelGGL(k_sel_scatter, dim3(grid), dim3(256), 0, s, d.X[c], d.Y[c], d.Z[c], d.vx, d.vy, d.vz, d.mass,
-                       d.type, d.uid, d.shape, d.flags, d.ref, d.phys, d.counters, g, dim, exch, d.tile_cnt,
-                       d.send_map, d.send_mult, d.send_cap, d.cap);
-}
-
 void launch_exchange(hipStream_t s, const DevState &d, const Geom &g, const int *periodic) {
     const int c = d.cur;
+    int *sc = d.scratch_i;
+    if (!periodic[0] && !periodic[1] && !periodic[2]) return;
+    if (d.exch_listed) {
+        hipLaunchKernelGGL(k_find_leavers, dim3((d.cap + 255) / 256), dim3(256), 0, s, d.X[c], d.Y[c], d.Z[c], d.flags,
+                           d.counters, g, periodic[0], periodic[1], periodic[2], d.leavers);
+        hipLaunchKernelGGL(k_exchange, dim3(1), dim3(1024), 0, s, d.X[c], d.Y[c], d.Z[c], d.flags, d.ref, d.phys,
+                           d.counters, g, periodic[0], periodic[1], periodic[2], d.leavers, d.send_map, d.send_mult,
+                           d.exchg_flag, sc, d.send_cap);
+        return;
+    }
+    const int grid = tile_grid(d.cap);
     for (int dim = 0; dim < 3; dim++) {
         if (!periodic[dim]) continue;
-        launch_select_dim(s, d, g, dim, 1, 0);
-        int *sc = d.scratch_i;
+        const double *Xd = dim == 0 ? d.X[c] : (dim == 1 ? d.Y[c] : d.Z[c]);
+        hipLaunchKernelGGL(k_sel_count, dim3(grid), dim3(256), 0, s, Xd, d.flags, d.phys, d.counters, g, dim,
+                           d.tile_cnt, d.exchg_flag);
+        hipLaunchKernelGGL(k_sel_scatter, dim3(grid), dim3(256), 0, s, d.X[c], d.Y[c], d.Z[c], d.vx, d.vy, d.vz,
+                           d.mass, d.type, d.uid, d.shape, d.flags, d.ref, d.phys, d.counters, g, dim, d.tile_cnt,
+                           d.send_map, d.send_mult, d.send_cap, d.cap);
         hipLaunchKernelGGL(k_exchange_relabel, dim3(1), dim3(1024), 0, s, d.X[c], d.Y[c], d.Z[c], d.ref, d.phys,
                            d.counters, g, d.send_map, d.send_mult, d.exchg_flag, sc, sc + d.send_cap,
                            sc + 2 * d.send_cap, sc + 3 * d.send_cap);
     }
 }
 
+template <int ND>
+static void borders_nd(hipStream_t s, const BorderArgs &A) {
+    hipLaunchKernelGGL(k_border_count<ND>, dim3(A.pitch), dim3(BORDER_T), 0, s, A);
+    hipLaunchKernelGGL(k_border_ghosts<ND>, dim3(A.pitch), dim3(BORDER_T), 0, s, A);
+}
+
 void launch_borders(hipStream_t s, const DevState &d, const Geom &g, const int *periodic) {
-    // the first periodic dimension starts from no ghosts and an empty send map
-    bool first = true;
-    for (int dim = 0; dim < 3; dim++) {
-        if (!periodic[dim]) continue;
-        launch_select_dim(s, d, g, dim, 0, first ? 1 : 0);
-        first = false;
-    }
+    const int c = d.cur, nd = (periodic[0] != 0) + (periodic[1] != 0) + (periodic[2] != 0);
     // no periodic dimension: no ghosts, nothing sent (adjacent counters)
     static_assert(C_NSEND_ALL == C_NGHOST + 1 && C_NSEND == C_NSEND_ALL + 1, "counter layout");
-    if (first) launch_set_counters(s, d.counters, C_NGHOST, 8, 0);
+    if (nd == 0) {
+        launch_set_counters(s, d.counters, C_NGHOST, 8, 0);
+        return;
+    }
+    const BorderArgs A = {d.X[c], d.Y[c], d.Z[c], d.vx, d.vy, d.vz, d.mass, d.type, d.uid, d.shape, d.flags, d.ref,
+                          d.phys, d.counters, g, periodic[0], periodic[1], periodic[2],
+                          (d.cap + BORDER_T - 1) / BORDER_T, d.send_cap, d.cap, d.tile_cnt, d.send_map, d.send_mult};
+    if (nd == 1) borders_nd<1>(s, A);
+    else if (nd == 2) borders_nd<2>(s, A);
+    else borders_nd<3>(s, A);
 }
 
 void launch_sync_pp(hipStream_t s, const DevState &d, const Geom &g, int cur, int prev, int grid) {

@@ -47,7 +47,9 @@ enum {
     C_TILE_MAX = 16,  // largest segment tile of the current lists
     C_UNSUPPORTED = 17,
     C_IMG_OVF = 18,   // a local has more periodic images than IMG_MAX
-    C_COUNT = 19
+    C_LEAVE = 19,     // locals outside a periodic dimension, listed for the exchange
+    C_LEAVE_MAX = 20, // their number at the last exchange
+    C_COUNT = 21
 };
 enum { OVF_NONE = 0, OVF_PART = 1, OVF_NEIGH = 2, OVF_SEND = 3, OVF_TILE = 4 };
 
@@ -81,6 +83,10 @@ constexpr int LIST_ROWS = 32;
 __host__ __device__ __forceinline__ int list_rows(int ncap) { return (ncap + LIST_ROWS - 1) / LIST_ROWS * LIST_ROWS; }
 
 constexpr int IMG_MAX = 8;
+// leavers that the one-workgroup exchange takes from its list
+constexpr int LEAVE_CAP = 1024;
+// ghost kinds: per periodic dimension none, side 0 or side 1
+constexpr int MAX_KIND = 27;
 
 // what a position-advancing kernel needs to refresh the ghost images
 struct Images {
@@ -136,6 +142,8 @@ struct DevState {
                          // local itself), its shift (2 bits per dimension, + 1)
     int img_on;          // host: every local's images fit IMG_MAX
     int *tile_cnt;
+    int *leavers;        // [LEAVE_CAP] physical slots
+    int exch_listed;     // host: the exchange works from the list of leavers
     int *counters;
     int *scratch_i;      // 4 * send_cap
     double *stage;       // 10 * send_cap doubles

@@ -107,7 +107,7 @@ static void free_particle_arrays(DevState &d) {
     for (auto p : dd) { dfree(*p); *p = nullptr; }
     int **ii[] = {&d.type, &d.flags, &d.uid, &d.shape, &d.ref, &d.phys, &d.alt_type, &d.alt_flags, &d.alt_uid,
                   &d.alt_shape, &d.alt_ref, &d.alt_cell, &d.numneighs, &d.particle_cell, &d.slot, &d.perm,
-                  &d.exchg_flag, &d.tile_cnt, &d.sync_src, &d.sync_mult, &d.img_cnt, &d.nrev};
+                  &d.exchg_flag, &d.tile_cnt, &d.leavers, &d.sync_src, &d.sync_mult, &d.img_cnt, &d.nrev};
     for (auto p : ii) { dfree(*p); *p = nullptr; }
     dfree(d.img_tab);
     d.img_tab = nullptr;
@@ -127,7 +127,8 @@ static int alloc_particle_arrays(pairs_hip_ctx *ctx, DevState &d, int cap) {
     r |= dalloc(ctx, &d.sync_mult, 3 * (size_t) cap);
     r |= dalloc(ctx, &d.img_cnt, cap);
     r |= dalloc(ctx, &d.img_tab, (size_t) IMG_MAX * cap);
-    r |= dalloc(ctx, &d.tile_cnt, 2 * ((size_t) cap / 256 + 2));
+    r |= dalloc(ctx, &d.tile_cnt, std::max(2 * ((size_t) cap / 256 + 2), MAX_KIND * ((size_t) cap / 1024 + 2)));
+    r |= dalloc(ctx, &d.leavers, (size_t) LEAVE_CAP);
     d.cap = cap;
     d.pstride = (int) pstride_of(d, ctx->geom);
     r |= dalloc(ctx, &d.partials, 3 * (size_t) d.pstride);
@@ -223,6 +224,12 @@ static void take_counters(pairs_hip_ctx *ctx) {
     ctx->nghost = ctx->h_counters[C_NGHOST];
     ctx->nsend_all = ctx->h_counters[C_NSEND_ALL];
     ctx->ghost_grid = std::max(1, std::min((ctx->nsend_all + 255) / 256 + 1, 4096));
+    if (ctx->d.exch_listed && ctx->h_counters[C_LEAVE_MAX] > LEAVE_CAP) {
+        // the list does not hold the leavers of a rebuild (and the exchange
+        // scanned the locals in one workgroup): the wide kernels from now on
+        ctx->d.exch_listed = 0;
+        drop_reb_graphs(ctx);
+    }
 }
 
 static int read_counters(pairs_hip_ctx *ctx) {
@@ -471,6 +478,9 @@ int pairs_hip_upload(pairs_hip_ctx *ctx, int n, const double *x, const double *v
     CHECK_LAUNCH();
     HIP_OK(hipStreamSynchronize(ctx->stream));
     d.nlocal = n;
+    // the leavers of a rebuild (some 600 at 131072 locals of the LJ fluid) fit the
+    // list of the one-workgroup exchange; EXCHMEAS
+    d.exch_listed = getenv("EXL") ? atoi(getenv("EXL")) : n < 200000;
     ctx->nghost = 0;
     ctx->nsend_all = 0;
     setup_segments(ctx, ctx->zc_override);

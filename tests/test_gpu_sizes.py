@@ -266,3 +266,44 @@ def test_dem_exchange_and_borders_vs_oracle(pairs, periodic, dom, speed):
             p, q = g.get(name, ghosts=True), o.get(name, ghosts=True)
             assert np.abs(p - q).max() <= 1e-10 * np.abs(q).max(), (b, name)
     assert nc.max() > 0
+
+
+# exchange and borders of a rebuild: 0 to 3 periodic dimensions; leavers that fit
+# the list of the one-workgroup exchange (1024) or do not (then, from the next
+# rebuild on, the wide kernels run); a box narrower than two cell spacings; more
+# than one border tile (1024 reference indices)
+@pytest.mark.parametrize("n,periodic,edge,speed", [
+    (1, (1, 1, 1), 39.0, 300.0), (1023, (1, 1, 1), 21.0, 200.0), (1025, (1, 1, 1), 22.0, 200.0),
+    (6000, (1, 1, 1), 39.0, 200.0), (6000, (1, 1, 1), 39.0, 2500.0), (6000, (0, 1, 1), 39.0, 3500.0),
+    (6000, (1, 1, 0), 39.0, 200.0), (6000, (1, 0, 1), 39.0, 200.0), (3000, (0, 1, 0), 31.0, 200.0),
+    (3000, (0, 0, 1), 31.0, 200.0), (3000, (1, 0, 0), 31.0, 200.0), (3000, (0, 0, 0), 31.0, 200.0),
+    (100, (1, 1, 1), 5.04, 100.0)])
+def test_lj_exchange_and_borders_vs_oracle(n, periodic, edge, speed):
+    """free flight through the faces with a rebuild after every step: order,
+    ghosts, maps and lists against the oracle"""
+    from pairs_amd import md
+    import test_gpu_md as tm
+    rng = np.random.default_rng(n + int(speed))
+    box = [(0.0, edge)] * 3
+    x = rng.uniform(0.0, edge, (n, 3))
+    v = rng.uniform(-speed, speed, (n, 3)) * np.asarray(periodic)
+    flags = np.where(rng.random(n) < 0.02, 4, 0).astype(np.int32)
+    flags[rng.random(n) < 0.01] = 8
+    g = md.LJSystem(box, particle_capacity=40000, neighbor_capacity=200, send_capacity=30000, periodic=periodic)
+    o = po.OracleMD(box, 40000, ncap=200, ccap=256, send_cap=30000, periodic=periodic)
+    g.upload(x, v, flags=flags)
+    o.set_particles(x, v, flags=flags)
+    o.setup_cells()
+    for step in range(4):
+        g.euler()
+        o.euler()
+        g.exchange()
+        g.borders()
+        g.build_cell_lists()
+        g.build_neighbor_lists()
+        o.rebuild()
+        assert o.overflow == 0
+        assert np.array_equal(g.nsend(), o.nsend()), step
+        assert np.array_equal(g.positions(True), o.positions(True)), step
+        assert np.array_equal(g.velocities(), o.velocities()), step
+        tm._compare_lists(g, o, step)
