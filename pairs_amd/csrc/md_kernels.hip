@@ -1838,8 +1838,8 @@ __global__ __launch_bounds__(256) void k_find_leavers(const double *__restrict__
 // relabeling is that of k_exchange_relabel_body.  More leavers than the list
 // holds are found by a scan of the locals in reference order instead.  Bound by
 // the latency of its phases; with k_find_leavers it takes the place of three
-// kernels per dimension (us per rebuild: 256 atoms 27 -> LJX1, 131072 45 ->
-// LJX2).  Beyond some 200000 locals the leavers of a rebuild no longer fit
+// kernels per dimension (us per rebuild: 256 atoms 27 -> 12, 131072 45 ->
+// 35).  Beyond some 200000 locals the leavers of a rebuild no longer fit
 // and the three kernels remain (exch_listed).
 __global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, double *__restrict__ Y,
                                                    double *__restrict__ Z, const int *__restrict__ flags,
@@ -2069,7 +2069,7 @@ __global__ __launch_bounds__(BORDER_T) void k_border_count(BorderArgs A) {
 // by dimension; on overflow the counts stay as they were.  Bound by latency in
 // small systems and by the ghosts' writes in large ones; with k_border_count it
 // takes the place of a count and a scatter pass per dimension (us per rebuild:
-// 256 atoms 20 -> LJB1, 131072 31 -> LJB2, 1048576 111 -> LJB3).
+// 256 atoms 20 -> 15, 131072 31 -> 25, 1048576 111 -> 61).
 template <int ND>
 __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
     constexpr int NK = pow3(ND), NW = BORDER_T / 64;
