@@ -154,71 +154,79 @@ __global__ __launch_bounds__(256) void k_bin_count(const double *__restrict__ X,
 }
 
 // exclusive scans of the local and ghost cell counts -> lstart, gstart
-// [0..ncells], one workgroup of 16 waves: each wave takes a contiguous run
-// of rows of 64 cells (coalesced loads), the wave totals give each run's
-// base, and each row is scanned across the lanes.  The counts are cleared
-// behind the reads (nothing else uses them, so the next binning starts from
-// zeros).  The flags the rest of the rebuild raises by atomics (images,
-// largest tile) are cleared here too.
+// [0..ncells], one workgroup of 16 waves: a lane takes four consecutive cells
+// (16-byte loads), a wave a contiguous run of rows of 256, all of a round's
+// loads in flight; the rows are scanned across the lanes with DPP, the wave
+// totals give each run's base.  The counts are cleared behind the reads (nothing
+// else uses them, so the next binning starts from zeros).  The flags the rest of
+// the rebuild raises by atomics (images, largest tile) are cleared here too.
+// Bound by latency (a cell per lane and 16 shuffled rows per wave whatever the
+// number of cells: 14 us at 217 cells, 15 at 12168, 74 at 74089; 4, 6
+// and 26 so).
 __device__ __forceinline__ void k_scan_cells_body(int *__restrict__ counters, int *__restrict__ lcount,
                                                      int *__restrict__ gcount, int *__restrict__ lstart,
                                                      int *__restrict__ gstart, int ncells) {
     __shared__ int tot[2][16];
     if (threadIdx.x == 0) { counters[C_IMG_OVF] = 0; counters[C_TILE_MAX] = 0; }
     if (counters[C_OVF]) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int RW = 16;
-    constexpr int ROUND = 16 * RW * 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int RW = 4;
+    constexpr int ROUND = 16 * RW * 256;
+    // (the arrays hold a multiple of four entries)
+    auto load = [&](const int *p, int c) {
+        int4 v = make_int4(0, 0, 0, 0);
+        if (c < ncells) {
+            v = *(const int4 *) (p + c);
+            if (c + 1 >= ncells) v.y = 0;
+            if (c + 2 >= ncells) v.z = 0;
+            if (c + 3 >= ncells) v.w = 0;
+        }
+        return v;
+    };
+    auto store = [&](int *p, int c, int b, const int4 &v) {
+        if (c < ncells) *(int4 *) (p + c) = make_int4(b, b + v.x, b + v.x + v.y, b + v.x + v.y + v.z);
+    };
     int carry_l = 0, carry_g = 0;
     for (int r0 = 0; r0 < ncells; r0 += ROUND) {
-        const int rn = min(ncells - r0, ROUND);
-        const int rows = (rn + 63) / 64;
-        const int per = (rows + 15) / 16;
-        const int row0 = wave * per;
-        int vl[RW], vg[RW];
-        int sl = 0, sg = 0;
+        const int w0 = r0 + wave * RW * 256;
+        int4 vl[RW], vg[RW];
+        int xl[RW], xg[RW], sl = 0, sg = 0;
 #pragma unroll
         for (int k = 0; k < RW; k++) {
-            const int cr = (row0 + k) * 64 + lane;
-            const bool in = k < per && cr < rn;
-            vl[k] = in ? lcount[r0 + cr] : 0;
-            vg[k] = in ? gcount[r0 + cr] : 0;
-            sl += vl[k];
-            sg += vg[k];
+            vl[k] = load(lcount, w0 + k * 256 + lane * 4);
+            vg[k] = load(gcount, w0 + k * 256 + lane * 4);
         }
 #pragma unroll
         for (int k = 0; k < RW; k++) {
-            const int cr = (row0 + k) * 64 + lane;
-            if (k < per && cr < rn) { lcount[r0 + cr] = 0; gcount[r0 + cr] = 0; }
+            const int c = w0 + k * 256 + lane * 4;
+            if (c < ncells) {
+                *(int4 *) (lcount + c) = make_int4(0, 0, 0, 0);
+                *(int4 *) (gcount + c) = make_int4(0, 0, 0, 0);
+            }
         }
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            sl += __shfl_xor(sl, off, 64);
-            sg += __shfl_xor(sg, off, 64);
+        for (int k = 0; k < RW; k++) {
+            if (w0 + k * 256 >= ncells) { xl[k] = xg[k] = 0; continue; }
+            const int tl = vl[k].x + vl[k].y + vl[k].z + vl[k].w, tg = vg[k].x + vg[k].y + vg[k].z + vg[k].w;
+            const int il = wave_scan(tl), ig = wave_scan(tg);
+            xl[k] = sl + il - tl;
+            xg[k] = sg + ig - tg;
+            sl += __builtin_amdgcn_readlane(il, 63);
+            sg += __builtin_amdgcn_readlane(ig, 63);
         }
         if (lane == 0) { tot[0][wave] = sl; tot[1][wave] = sg; }
         __syncthreads();
-        int bl = carry_l, bg = carry_g, al = carry_l, ag = carry_g;
-        for (int w = 0; w < 16; w++) {
-            const int a = tot[0][w], b = tot[1][w];
-            if (w < wave) { bl += a; bg += b; }
-            al += a; ag += b;
-        }
+        const int al = lane < 16 ? tot[0][lane] : 0, ag = lane < 16 ? tot[1][lane] : 0;
+        const int pl = wave_scan(al), pg = wave_scan(ag);
+        const int bl = carry_l + __builtin_amdgcn_readlane(pl - al, wave);
+        const int bg = carry_g + __builtin_amdgcn_readlane(pg - ag, wave);
+        carry_l += __builtin_amdgcn_readlane(pl, 15);
+        carry_g += __builtin_amdgcn_readlane(pg, 15);
 #pragma unroll
         for (int k = 0; k < RW; k++) {
-            int xl = vl[k], xg = vg[k];
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int yl = __shfl_up(xl, off, 64), yg = __shfl_up(xg, off, 64);
-                if (lane >= off) { xl += yl; xg += yg; }
-            }
-            const int cr = (row0 + k) * 64 + lane;
-            if (k < per && cr < rn) { lstart[r0 + cr] = bl + xl - vl[k]; gstart[r0 + cr] = bg + xg - vg[k]; }
-            bl += __shfl(xl, 63, 64);
-            bg += __shfl(xg, 63, 64);
+            store(lstart, w0 + k * 256 + lane * 4, bl + xl[k], vl[k]);
+            store(gstart, w0 + k * 256 + lane * 4, bg + xg[k], vg[k]);
         }
-        carry_l = al;
-        carry_g = ag;
         __syncthreads();
     }
     if (threadIdx.x == 0) { lstart[ncells] = carry_l; gstart[ncells] = carry_g; }
@@ -426,8 +434,8 @@ __global__ __launch_bounds__(256) void k_img_build(int *__restrict__ counters, c
 // reference-index order; accepted when j != i (full) or i < j (half, point
 // masses) and rsq < (rc + skin)^2.
 //
-// One workgroup of BB threads (BW waves) per segment; each wave takes home
-// cells of the segment in turn.  The tile (positions, + reference indices
+// One workgroup of NT threads per segment; each wave takes home cells of the
+// segment in turn, or a part of a cell's home particles.  The tile (positions, + reference indices
 // for half lists) is staged in LDS and a table gives, per column of the tile,
 // each flat cell's local and ghost sub-range (tile offset, length).  For a
 // home cell the wave lays out its candidates in the reference's order (cell
@@ -438,9 +446,14 @@ __global__ __launch_bounds__(256) void k_img_build(int *__restrict__ counters, c
 // count append the accepted candidates in candidate order, written to the
 // list directly (the four entries of a group share 16 bytes, so the L2
 // merges the appends of a cell's home particles before they reach HBM; an
-// LDS row buffer that wrote whole groups cost more in occupancy than it saved).
+// LDS row buffer that wrote whole groups lengthened the chain: 113 -> 135 us at
+// 131072 atoms).  Bound half by vector work (500 distances per particle), half
+// by latency.  Lanes without a candidate hold NaN and full lists hold physical
+// slots, which spares the inner loop a test and a look-up, the runs are summed
+// with DPP and the table's cell starts are loaded ahead: 119 -> 113 us at
+// 131072 atoms, 603 -> 556 at 1048576.
 constexpr int BB = 128;        // threads per build workgroup
-constexpr int BW = BB / 64;    // waves per build workgroup
+constexpr int BB_SMALL = 512;  // in small systems
 constexpr int NB_CAND = 2048;  // candidates of one home cell
 // half lists: mirror entries of one home particle collected in the top
 // RMAX slots of the wave's candidate buffer before they are sorted
@@ -454,8 +467,9 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
     return __longlong_as_double(((long long) hi << 32) | lo);
 }
 
-template <bool HALF>
+template <bool HALF, int NT>
 __device__ __forceinline__ void build_segment(const BuildArgs &A, int seg) {
+    constexpr int BW = NT / 64;  // waves
     const int *__restrict__ counters = A.counters;
     const Geom &g = A.g;
     const int *__restrict__ lstart = A.lstart, *__restrict__ gstart = A.gstart;
@@ -470,73 +484,85 @@ __device__ __forceinline__ void build_segment(const BuildArgs &A, int seg) {
     int *ctab = tslot + tcap;                                   // [9][zt][4]: local st, len, ghost st, len
     int *tref = ctab + 9 * zt * 4;                              // [tcap] half lists only
     uint16_t *cand_all = (uint16_t *) (tref + (HALF ? tcap : 0));  // [BW][NB_CAND]
-    __shared__ int r_start[NRUNS], r_len[NRUNS], r_off[NRUNS + 1], col_lo[9];
+    __shared__ int r_start[NRUNS], r_off[NRUNS + 1], col_lo[9];
     if (counters[C_OVF]) return;
     const int nlocal = counters[C_NLOCAL];
     if (seg >= g.nsegs) return;
     const SegInfo si = seg_info(seg, g);
+    const int nz = si.zb - si.za + 2;  // flat cells B+za-1 .. B+zb of each column
+    // what a table entry needs of the cell starts (loaded before the runs are known)
+    struct Sub { int l0 = 0, l1 = 0, g0 = 0, g1 = 0, lb = 0, gb = 0; bool on = false; };
+    auto sub = [&](int e) {
+        Sub r;
+        const int col = e / nz, zz = e - col * nz;
+        const int B = ((si.cx + col / 3 - 1) * g.dim_cells[1] + (si.cy + col % 3 - 1)) * g.dim_cells[2] + 1;
+        const int cc = B + si.za - 1 + zz, lo = max(B + si.za - 1, 1);
+        // a flat cell is a stencil cell of the reference iff 0 < cc < ncells
+        // (interaction.py:92-98)
+        r.on = cc > 0 && cc < g.ncells;
+        if (r.on) {
+            r.l0 = lstart[cc]; r.l1 = lstart[cc + 1]; r.g0 = gstart[cc]; r.g1 = gstart[cc + 1];
+            r.lb = lstart[lo]; r.gb = gstart[lo];
+        }
+        return r;
+    };
+    Sub first;
+    if ((int) threadIdx.x < 9 * nz) first = sub(threadIdx.x);
     const int h0 = lstart[si.ca], h1 = lstart[si.cb];
     if (h1 <= h0) return;
-    seg_runs(si, g, lstart, gstart, nlocal, r_start, r_len, r_off, col_lo);
+    seg_runs(si, g, lstart, gstart, nlocal, r_start, r_off, col_lo);
     const int T = r_off[NRUNS];
-    const int nz = si.zb - si.za + 2;  // flat cells B+za-1 .. B+zb of each column
     if (T > tcap || nz > zt) {
         if (threadIdx.x == 0) { atomicMax(&ctr[C_TILE_MAX], T); atomicMax(&ctr[C_OVF], OVF_TILE); }
         return;
     }
     if (threadIdx.x == 0) atomicMax(&ctr[C_TILE_MAX], T);
     stage_slots(r_start, r_off, T, tslot);
-    __syncthreads();
-    if (HALF)
-        for (int p = threadIdx.x; p < T; p += BB)
-            tref[p] = ref[tslot[p]] | ((flags[tslot[p]] & FLAG_FIXED) ? (1 << 30) : 0);
-    // sub-range table: a flat cell cc of column col is a stencil cell of the
-    // reference iff 0 < cc < ncells (interaction.py:92-98)
-    for (int e = threadIdx.x; e < 9 * nz; e += BB) {
+    // sub-range table
+    for (int e = threadIdx.x; e < 9 * nz; e += NT) {
+        const Sub r = e == (int) threadIdx.x ? first : sub(e);
         const int col = e / nz, zz = e - col * nz;
-        const int dx = col / 3 - 1, dy = col % 3 - 1;
-        const int cc = ((si.cx + dx) * g.dim_cells[1] + (si.cy + dy)) * g.dim_cells[2] + 1 + si.za - 1 + zz;
-        int v0 = 0, v1 = 0, v2 = 0, v3 = 0;
-        if (cc > 0 && cc < g.ncells) {
-            const int lo = col_lo[col];
-            v0 = r_off[2 + 2 * col] + (lstart[cc] - lstart[lo]);
-            v1 = lstart[cc + 1] - lstart[cc];
-            v2 = r_off[3 + 2 * col] + (gstart[cc] - gstart[lo]);
-            v3 = gstart[cc + 1] - gstart[cc];
-        }
         int *t = ctab + (col * zt + zz) * 4;
-        t[0] = v0; t[1] = v1; t[2] = v2; t[3] = v3;
+        t[0] = r.on ? r_off[2 + 2 * col] + (r.l0 - r.lb) : 0;
+        t[1] = r.l1 - r.l0;
+        t[2] = r.on ? r_off[3 + 2 * col] + (r.g0 - r.gb) : 0;
+        t[3] = r.g1 - r.g0;
     }
     __syncthreads();
+    if (HALF) {
+        for (int p = threadIdx.x; p < T; p += NT)
+            tref[p] = ref[tslot[p]] | ((flags[tslot[p]] & FLAG_FIXED) ? (1 << 30) : 0);
+        __syncthreads();
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint16_t *cand = cand_all + wave * NB_CAND;
     // home particles are the locals of the centre column (col 4), table rows
     // 1 .. nz-2; a home particle's index in the segment is its tile offset
     // minus own_base (= its physical slot minus h0)
     const int own_base = r_off[2 + 2 * 4] + (h0 - lstart[col_lo[4]]);
-    for (int zz = 1 + wave; zz <= nz - 2; zz += BW) {
+    // a cell's home particles are shared by SP waves where the workgroup has
+    // more waves than the segment cells
+    const int ncells = nz - 2, SP = max(1, BW / ncells);
+    for (int item = wave; item < ncells * SP; item += BW) {
+        const int zz = 1 + item / SP, part = item % SP;
         const int *tc = ctab + (4 * zt + zz) * 4;
-        const int hst = tc[0], hlen = tc[1];
+        const int hall = tc[1], hfrom = part * hall / SP;
+        const int hst = tc[0] + hfrom, hlen = (part + 1) * hall / SP - hfrom;
         if (hlen == 0) continue;
         // candidate sub-ranges, one per lane: cell 0 locals, ghosts; then per
         // column (dx outer, dy inner) and dz = -1, 0, 1: locals, ghosts
         int st = 0, ln = 0;
         if (lane < 2) {
             st = r_off[lane];
-            ln = r_len[lane];
+            ln = r_off[lane + 1] - st;
         } else if (lane < 56) {
             const int u = lane - 2, col = u / 6, dz = (u % 6) / 2 - 1, gh = u & 1;
             const int *t = ctab + (col * zt + zz + dz) * 4;
             st = t[2 * gh];
             ln = t[2 * gh + 1];
         }
-        int incl = ln;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int v = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += v;
-        }
-        const int ncand = __shfl(incl, 63, 64);
+        const int incl = wave_scan(ln);
+        const int ncand = __builtin_amdgcn_readlane(incl, 63);
         if (ncand > (HALF ? NB_CAND - RMAX : NB_CAND)) {
             if (lane == 0) { atomicMax(&ctr[C_TILE_MAX], tcap + 1); atomicMax(&ctr[C_OVF], OVF_TILE); }
             continue;
@@ -556,13 +582,13 @@ __device__ __forceinline__ void build_segment(const BuildArgs &A, int seg) {
 #pragma unroll
         for (int c = 0; c < CREG; c++) {
             rco[c] = 0; rcr[c] = 0;
-            rcx[c] = 0.0; rcy[c] = 0.0; rcz[c] = 0.0;
+            rcx[c] = NAN; rcy[c] = 0.0; rcz[c] = 0.0;  // no candidate: fails every test
             if (c < nchunk) {
                 const int q = c * 64 + lane;
                 const int o = q < ncand ? cand[q] : 0;
                 const int pc = tslot[o];
-                rco[c] = o;
-                rcx[c] = X[pc]; rcy[c] = Y[pc]; rcz[c] = Z[pc];
+                rco[c] = HALF ? o : pc;
+                rcx[c] = q < ncand ? X[pc] : NAN; rcy[c] = Y[pc]; rcz[c] = Z[pc];
                 if (HALF) rcr[c] = tref[o];
             }
         }
@@ -584,21 +610,20 @@ __device__ __forceinline__ void build_segment(const BuildArgs &A, int seg) {
                     const double xi = readlane_f64(hx, h), yi = readlane_f64(hy, h), zi = readlane_f64(hz, h);
                     const int hr = HALF ? __builtin_amdgcn_readlane(href, h) : 0;
                     // one chunk: accepted candidates append in lane (= candidate) order
-                    auto test = [&](int c0, int o, double cx, double cy, double cz, int cr) {
-                        const bool qv = c0 + lane < ncand;
+                    auto test = [&](int o, double cx, double cy, double cz, int cr) {
                         const double dx = xi - cx, dy = yi - cy, dz = zi - cz;
                         double rsq = dx * dx + dy * dy;
                         rsq = rsq + dz * dz;
                         const int crf = cr & REF_MASK;
-                        const bool keep = HALF ? (hr < crf) : (o != ownh);
-                        const bool acc = qv && keep && rsq < rc2;
+                        const bool keep = HALF ? (hr < crf) : (o != h0 + idx);
+                        const bool acc = keep && rsq < rc2;
                         const unsigned long long m = __ballot(acc);
                         const int k = cnt + lane_rank(m);
-                        if (acc && k < ncap) nl[nl_at(k, h0 + idx, nl_stride)] = (uint32_t) tslot[o];
+                        if (acc && k < ncap) nl[nl_at(k, h0 + idx, nl_stride)] = HALF ? (uint32_t) tslot[o] : (uint32_t) o;
                         cnt += __popcll(m);
                         if (HALF) {
                             // a mirror entry: an earlier-index local, not fixed
-                            const bool mir = qv && crf < hr && !(cr >> 30) && rsq < rc2;
+                            const bool mir = crf < hr && !(cr >> 30) && rsq < rc2;
                             const unsigned long long mr = __ballot(mir);
                             const int kr = cntr + lane_rank(mr);
                             if (mir && kr < RMAX) rbuf[kr] = (uint16_t) o;
@@ -607,12 +632,12 @@ __device__ __forceinline__ void build_segment(const BuildArgs &A, int seg) {
                     };
 #pragma unroll
                     for (int c = 0; c < CREG; c++)
-                        if (c < nchunk) test(c * 64, rco[c], rcx[c], rcy[c], rcz[c], rcr[c]);
+                        if (c < nchunk) test(rco[c], rcx[c], rcy[c], rcz[c], rcr[c]);
                     for (int c = CREG; c < nchunk; c++) {  // more candidates than the registers hold
                         const int q = c * 64 + lane;
                         const int o = q < ncand ? cand[q] : 0;
                         const int pc = tslot[o];
-                        test(c * 64, o, X[pc], Y[pc], Z[pc], HALF ? tref[o] : 0);
+                        test(HALF ? o : pc, q < ncand ? X[pc] : NAN, Y[pc], Z[pc], HALF ? tref[o] : 0);
                     }
                 }
                 if (HALF) {
@@ -667,9 +692,9 @@ __device__ __forceinline__ void build_segment(const BuildArgs &A, int seg) {
     }
 }
 
-template <bool HALF>
-__global__ __launch_bounds__(BB) void k_build_neighbors(BuildArgs A) {
-    build_segment<HALF>(A, xcd_block(blockIdx.x, gridDim.x));
+template <bool HALF, int NT>
+__global__ __launch_bounds__(NT) void k_build_neighbors(BuildArgs A) {
+    build_segment<HALF, NT>(A, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // the segments of many independent systems in one launch: block b belongs to
@@ -680,7 +705,7 @@ __global__ __launch_bounds__(BB) void k_build_neighbors_batch(const BuildArgs *_
                                                               const int *__restrict__ seg_base) {
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r = rep[b];
-    build_segment<HALF>(desc[r], b - seg_base[r]);
+    build_segment<HALF, BB>(desc[r], b - seg_base[r]);
 }
 
 // Expand the lists into reference indices (for download):
@@ -2454,9 +2479,9 @@ void launch_cells_batch(hipStream_t s, const RepDesc *D, int n, int max_cap, int
 
 int build_zt(const Geom &g) { return g.nchunks == 1 ? g.dim_cells[2] + 2 : g.zc + 3; }
 
-static size_t build_lds(const DevState &d, const Geom &g, int half, int tcap) {
+static size_t build_lds(const DevState &d, const Geom &g, int half, int tcap, int nt = BB) {
     (void) d;
-    return (size_t) tcap * (sizeof(int) + (half ? sizeof(int) : 0)) + (size_t) BW * NB_CAND * sizeof(uint16_t) +
+    return (size_t) tcap * (sizeof(int) + (half ? sizeof(int) : 0)) + (size_t) (nt / 64) * NB_CAND * sizeof(uint16_t) +
            (size_t) 9 * build_zt(g) * 4 * sizeof(int);
 }
 
@@ -2487,11 +2512,22 @@ size_t build_lds_bytes(const DevState &d, const Geom &g, int half) {
     return build_lds(d, g, half, min(d.tile_cap, build_tile_limit(d, g, half)));
 }
 
+template <int NT>
+static void build_launch(hipStream_t s, const DevState &d, const Geom &g, int half, const BuildArgs &A) {
+    const size_t lds = build_lds(d, g, half, A.tcap, NT);
+    if (half) hipLaunchKernelGGL((k_build_neighbors<true, NT>), dim3(g.nsegs), dim3(NT), lds, s, A);
+    else hipLaunchKernelGGL((k_build_neighbors<false, NT>), dim3(g.nsegs), dim3(NT), lds, s, A);
+}
+
 void launch_build_neighbors(hipStream_t s, const DevState &d, const Geom &g, int half, double rc2) {
     const BuildArgs A = build_args(d, g, half, rc2);
-    const size_t lds = build_lds(d, g, half, A.tcap);
-    if (half) hipLaunchKernelGGL(k_build_neighbors<true>, dim3(g.nsegs), dim3(BB), lds, s, A);
-    else hipLaunchKernelGGL(k_build_neighbors<false>, dim3(g.nsegs), dim3(BB), lds, s, A);
+    // eight waves per segment share its cells' home particles where the segments
+    // are too few to fill the chip.  Build, us, on 2 | 8 waves: 256 atoms 30 | 18,
+    // 19200 40 | 35; 200 steps of 70304 atoms 6.89 | 6.84 ms; 131072 atoms 113 |
+    // 122 (half lists 263 | 305).  (A larger tile leaves no room for eight
+    // candidate buffers at the occupancy measured.)
+    if (d.nlocal < 80000 && A.tcap <= 8192) build_launch<BB_SMALL>(s, d, g, half, A);
+    else build_launch<BB>(s, d, g, half, A);
 }
 
 void launch_build_batch(hipStream_t s, const BuildArgs *desc, const int *rep, const int *seg_base, int nblocks,

@@ -52,18 +52,18 @@ constexpr int NRUNS = 20;
 // stencil (dx outer, dy inner; src/pairs/sim/cell_lists.py:70-87), each over
 // flat cells [B + za - 1, B + zb] clipped to the grid (a stencil cell of the
 // reference is valid iff 0 < nc < ncells, interaction.py:92-98), locals then
-// ghosts.  Written by threads 0..19; r_off is the exclusive prefix (r_off[20]
+// ghosts.  Written by the first wave; r_off is the exclusive prefix (r_off[20]
 // = tile size).  lo of each column is kept for candidate enumeration.
 __device__ __forceinline__ void seg_runs(const SegInfo &si, const Geom &g, const int *__restrict__ lstart,
-                                         const int *__restrict__ gstart, int nlocal, int *r_start, int *r_len,
-                                         int *r_off, int *col_lo) {
+                                         const int *__restrict__ gstart, int nlocal, int *r_start, int *r_off,
+                                         int *col_lo) {
     const int t = threadIdx.x;
-    if (t < NRUNS) {
+    if (t < 64) {
         int start = 0, len = 0;
         if (t < 2) {
             if (t == 0) { start = lstart[0]; len = lstart[1] - lstart[0]; }
             else { start = nlocal + gstart[0]; len = gstart[1] - gstart[0]; }
-        } else {
+        } else if (t < NRUNS) {
             const int col = (t - 2) >> 1, loc = ((t - 2) & 1) == 0;
             const int dx = col / 3 - 1, dy = col % 3 - 1;
             const int B = ((si.cx + dx) * g.dim_cells[1] + (si.cy + dy)) * g.dim_cells[2] + 1;
@@ -76,14 +76,12 @@ __device__ __forceinline__ void seg_runs(const SegInfo &si, const Geom &g, const
             }
             if (loc) col_lo[col] = lo;
         }
-        r_start[t] = start;
-        r_len[t] = len;
-    }
-    __syncthreads();
-    if (t == 0) {
-        int off = 0;
-        for (int r = 0; r < NRUNS; r++) { r_off[r] = off; off += r_len[r]; }
-        r_off[NRUNS] = off;
+        const int upto = wave_scan(len);
+        if (t < NRUNS) {
+            r_start[t] = start;
+            r_off[t + 1] = upto;
+        }
+        if (t == 0) r_off[0] = 0;
     }
     __syncthreads();
 }

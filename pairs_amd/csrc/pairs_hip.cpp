@@ -332,8 +332,10 @@ int pairs_hip_create(pairs_hip_ctx **out, const pairs_hip_md_config *cfg) {
     if (alloc_particle_arrays(ctx, d, cfg->particle_capacity)) return fail(PAIRS_HIP_ERR_HIP);
     if (alloc_neighbor_arrays(ctx, d, cfg->neighbor_capacity)) return fail(PAIRS_HIP_ERR_HIP);
     if (alloc_send_arrays(ctx, d, cfg->send_capacity)) return fail(PAIRS_HIP_ERR_HIP);
-    if (dalloc(ctx, &d.lcount, (size_t) d.ncells_cap + 1) || dalloc(ctx, &d.gcount, (size_t) d.ncells_cap + 1) ||
-        dalloc(ctx, &d.lstart, (size_t) d.ncells_cap + 1) || dalloc(ctx, &d.gstart, (size_t) d.ncells_cap + 1) ||
+    // (a multiple of four entries: the scan moves them by 16 bytes)
+    const size_t cells = ((size_t) d.ncells_cap + 4) / 4 * 4;
+    if (dalloc(ctx, &d.lcount, cells) || dalloc(ctx, &d.gcount, cells) || dalloc(ctx, &d.lstart, cells) ||
+        dalloc(ctx, &d.gstart, cells) ||
         dalloc(ctx, &d.counters, C_COUNT) || dalloc(ctx, &d.thermo, 5 * 4096))
         return fail(PAIRS_HIP_ERR_HIP);
     launch_fill_i32(ctx->stream, d.counters, 0, C_COUNT);

@@ -277,7 +277,7 @@ def test_dem_exchange_and_borders_vs_oracle(pairs, periodic, dom, speed):
     (6000, (1, 1, 1), 39.0, 200.0), (6000, (1, 1, 1), 39.0, 2500.0), (6000, (0, 1, 1), 39.0, 3500.0),
     (6000, (1, 1, 0), 39.0, 200.0), (6000, (1, 0, 1), 39.0, 200.0), (3000, (0, 1, 0), 31.0, 200.0),
     (3000, (0, 0, 1), 31.0, 200.0), (3000, (1, 0, 0), 31.0, 200.0), (3000, (0, 0, 0), 31.0, 200.0),
-    (100, (1, 1, 1), 5.04, 100.0)])
+    (100, (1, 1, 1), 5.04, 100.0), (3000, (1, 1, 1), 100.0, 300.0)])  # (54873 cells: several rounds of the scan)
 def test_lj_exchange_and_borders_vs_oracle(n, periodic, edge, speed):
     """free flight through the faces with a rebuild after every step: order,
     ghosts, maps and lists against the oracle"""
