@@ -1340,6 +1340,364 @@ __global__ __launch_bounds__(64) void k_ljm(LJArgs A) {
     lj_multi<L, NT, MODE, RED, HALF, UNIT>(A, xcd_block(blockIdx.x, gridDim.x));
 }
 
+// ---------------------------------------------------------------- Lennard-Jones over LDS tiles
+
+// Large systems of one type take their timestep forces from LDS.  The locals
+// are cut into groups of whole cells of one z-column, at most TILE_G of them
+// (k_tile_groups); a group's tile is the particles its lists name, in the order
+// of the runs of its candidate cells, and a second copy of the lists names them
+// by 16-bit byte offsets into the tile, eight to a 16-byte load, padded with
+// the offset of a particle out of reach (k_tile_build).  k_ljt then gathers each
+// neighbour once per group from memory and once per entry from LDS.
+
+// One wave per z-column of cells (and one for cell 0): its locals packed into
+// groups (first local, count, first and last cell).  A group's id is the order
+// of arrival; results do not depend on it.
+__global__ __launch_bounds__(256) void k_tile_groups(TileArgs A) {
+    __shared__ int4 s_out[4][64];
+    int *__restrict__ c = A.counters;
+    if (c[C_OVF]) return;
+    const Geom &g = A.g;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = blockIdx.x * 4 + wave - 1, ncol = g.dim_cells[0] * g.dim_cells[1];
+    if (col >= ncol) return;
+    const int c0 = col < 0 ? 0 : 1 + col * g.dim_cells[2], c1 = col < 0 ? 1 : c0 + g.dim_cells[2];
+    int n = 0;  // groups in s_out
+    auto flush = [&]() {
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&c[C_NGROUPS], n);
+        base = __builtin_amdgcn_readfirstlane(base);
+        wave_lds_sync();
+        if (lane < n && base + lane < A.gmax) A.grp[base + lane] = s_out[wave][lane];
+        wave_lds_sync();
+        n = 0;
+    };
+    auto emit = [&](int first, int cnt, int ca, int cb) {
+        if (lane == 0) s_out[wave][n] = make_int4(first, cnt, ca, cb);
+        if (++n == 64) flush();
+    };
+    int first = __builtin_amdgcn_readfirstlane(A.lstart[c0]), cnt = 0, ca = c0;
+    for (int z0 = c0; z0 < c1; z0 += 64) {
+        const int z = z0 + lane;
+        const int len = z < c1 ? A.lstart[z + 1] - A.lstart[z] : 0;
+        for (int k = 0; k < min(64, c1 - z0); k++) {
+            int m = __builtin_amdgcn_readlane(len, k);
+            if (m == 0) continue;
+            if (cnt > 0 && (cnt + m > TILE_G || z0 + k - ca >= TILE_SPAN)) {
+                emit(first, cnt, ca, min(z0 + k - 1, ca + TILE_SPAN - 1));
+                first += cnt;
+                cnt = 0;
+            }
+            if (cnt == 0) ca = z0 + k;
+            for (; m > TILE_G; m -= TILE_G) {
+                emit(first, TILE_G, ca, ca);
+                first += TILE_G;
+            }
+            cnt += m;
+        }
+    }
+    if (cnt > 0) emit(first, cnt, ca, min(c1, ca + TILE_SPAN) - 1);
+    if (n > 0) flush();
+}
+
+// The tile of a group and its locals' lists over it, one local per thread.  A
+// group whose tile or candidates do not fit (or in cell 0) gets size 0: its
+// forces come from the 32-bit lists.  Twice over the lists: the entries'
+// places among the candidates (binary search of the slot among the sorted
+// runs) mark the used ones, whose ranks are the tile's order; then places
+// become byte offsets.  1048576 atoms: 200 us per rebuild, and 24 for the groups.
+template <bool HALF>
+__global__ __launch_bounds__(TILE_G) void k_tile_build(TileArgs A) {
+    constexpr int CMAX = 4096 / TILE_G * TILE_G, W = TILE_G / 64;
+    __shared__ int r_start[NRUNS], r_off[NRUNS + 1], col_lo[9];
+    __shared__ int s_from[32], s_delta[32], s_cnt[W * ((CMAX + TILE_G - 1) / TILE_G)], s_total;
+    __shared__ unsigned char s_mark[CMAX];
+    __shared__ uint16_t s_rank[CMAX];
+    if (A.counters[C_OVF]) return;
+    const int ng = min(A.counters[C_NGROUPS], A.gmax), t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // tile b is made by workgroup b and used by workgroup b of the force kernel
+    // (consecutive groups on one XCD); the rest of the table is empty
+    const int tile = blockIdx.x;
+    if (tile >= ng) {
+        if (t == 0) A.tile[tile] = make_int4(0, 0, 0, 0);
+        return;
+    }
+    const int4 G = A.grp[xcd_block(tile, ng)];
+    const Geom &g = A.g;
+    auto done = [&](int size) {
+        if (t == 0) A.tile[tile] = make_int4(G.x, G.y, size, 0);
+    };
+    if (G.z == 0) {
+        done(0);
+        return;
+    }
+    SegInfo si;
+    const int col = (G.z - 1) / g.dim_cells[2];
+    si.cx = col / g.dim_cells[1];
+    si.cy = col % g.dim_cells[1];
+    si.za = G.z - 1 - col * g.dim_cells[2];
+    si.zb = si.za + G.w - G.z + 1;
+    si.ca = G.z;
+    si.cb = G.z + (si.zb - si.za);
+    seg_runs(si, g, A.lstart, A.gstart, A.nlocal, r_start, r_off, col_lo);
+    const int T = r_off[NRUNS];
+    auto give_up = [&]() {
+        done(0);
+        if (t == 0) atomicAdd(&A.counters[C_BIG], 1);
+    };
+    if (T > CMAX) {
+        give_up();
+        return;
+    }
+    if (t < 32) { s_from[t] = 0x7fffffff; s_delta[t] = 0; }
+    for (int k = t; k < CMAX / 4; k += TILE_G) ((int *) s_mark)[k] = 0;
+    __syncthreads();
+    // the runs by start, empty ones left out
+    if (t < NRUNS && r_off[t + 1] > r_off[t]) {
+        int rank = 0;
+        for (int k = 0; k < NRUNS; k++) rank += r_off[k + 1] > r_off[k] && r_start[k] < r_start[t] ? 1 : 0;
+        s_from[rank] = r_start[t];
+        s_delta[rank] = r_off[t] - r_start[t];
+    }
+    __syncthreads();
+    const int i = G.x + t;
+    const bool live = t < G.y;
+    const size_t stride = A.nl_stride;
+    auto place = [&](uint32_t j) {
+        int p = 0;
+#pragma unroll
+        for (int s = 16; s > 0; s >>= 1) p += s_from[p + s] <= (int) j ? s : 0;
+        return min((unsigned) ((int) j + s_delta[p]), (unsigned) CMAX - 1);
+    };
+    // pass over one part of the list: rows of eight, to the wave's depth
+    auto mark = [&](int n, int row0, int out0) {
+        const int rows = (wave_max_uniform(n) + 7) / 8;
+        const uint4 *from = (const uint4 *) A.nl + (size_t) (row0 >> 2) * stride + i;
+        for (int r = 0; r < rows; r++) {
+            if (!live) continue;
+            uint32_t c[8];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint4 e = from[(size_t) min(2 * r + h, A.rows / 4 - 1) * stride];
+                c[4 * h + 0] = e.x; c[4 * h + 2] = e.y; c[4 * h + 1] = e.z; c[4 * h + 3] = e.w;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const bool in = 8 * r + q < n;
+                c[q] = in ? place(c[q]) : 0xffffu;
+                if (in) s_mark[c[q]] = 1;
+            }
+            A.nl16[(size_t) (out0 + r) * stride + i] =
+                make_uint4(c[0] | c[1] << 16, c[2] | c[3] << 16, c[4] | c[5] << 16, c[6] | c[7] << 16);
+        }
+    };
+    auto rename = [&](int n, int out0) {
+        const int rows = (wave_max_uniform(n) + 7) / 8;
+        for (int r = 0; r < rows; r++) {
+            if (!live) continue;
+            uint4 *at = A.nl16 + (size_t) (out0 + r) * stride + i;
+            const uint4 v = *at;
+            auto two = [&](uint32_t w) {
+                const uint32_t a = w & 0xffffu, b = w >> 16;
+                const uint32_t x = a == 0xffffu ? 0u : (uint32_t) s_rank[a] * 8u;
+                const uint32_t y = b == 0xffffu ? 0u : (uint32_t) s_rank[b] * 8u;
+                return x | y << 16;
+            };
+            *at = make_uint4(two(v.x), two(v.y), two(v.z), two(v.w));
+        }
+    };
+    const int n = live ? min(A.numneighs[i], A.ncap) : 0, nr = HALF && live ? min(A.nrev[i], A.rev0) : 0;
+    mark(n, 0, 0);
+    if (HALF) mark(nr, A.rev0, A.rows / 8);
+    __syncthreads();
+    // ranks of the marked places (1..; 0 is the particle out of reach)
+    const int its = (T + TILE_G - 1) / TILE_G;
+    for (int k = 0; k < its; k++) {
+        const unsigned long long m = __ballot(s_mark[k * TILE_G + t] != 0);
+        if (lane == 0) s_cnt[W * k + wave] = __popcll(m);
+    }
+    __syncthreads();
+    if (t < 64) {
+        const int v = t < W * its ? s_cnt[t] : 0, u = wave_scan(v);
+        if (t < W * its) s_cnt[t] = u - v;
+        if (t == 63) s_total = u;
+    }
+    __syncthreads();
+    const int size = 1 + s_total;
+    if (size > TILE_CAP) {
+        give_up();
+        return;
+    }
+    for (int k = 0; k < its; k++) {
+        const int c = k * TILE_G + t;
+        const unsigned long long m = __ballot(s_mark[c] != 0);
+        if (!s_mark[c]) continue;
+        const int rank = 1 + s_cnt[W * k + wave] + lane_rank(m), run = run_of(r_off, c);
+        s_rank[c] = (uint16_t) rank;
+        A.slots[(size_t) tile * TILE_CAP + rank] = r_start[run] + (c - r_off[run]);
+    }
+    done(size);
+    __syncthreads();
+    rename(n, 0);
+    if (HALF) rename(nr, A.rows / 8);
+}
+
+// The force kernel of the timestep over a group's tile (MODE 0 and 1, HALF,
+// UNIT as lj_wave; one type, no reduction), one lane per local: positions of
+// the tile staged in LDS by component, the lists' byte offsets used as they are
+// (padding names a particle at 1e100, which fails the cutoff test and adds a
+// signed zero), the pairs of a row of eight computed together and added in list
+// order.  Bound by vector work (32 operations per entry, 26 of them FP64: 95 of
+// 163 us at 1048576 atoms) and by memory (11 records staged per local, 2 bytes
+// per entry: 690 MB), with 12 waves on a CU.  Against two lanes per local that
+// gather from memory (k_lj2): 283 -> 163 us there, half lists 42.6 -> 38.8 us at
+// 131072 atoms, full lists there 31 either way (a tile's latency is not hidden
+// by other tiles).  Groups of 192 or 256 locals keep fewer waves resident: 182
+// and 209 us at 1048576.
+template <int MODE, bool HALF, bool UNIT>
+__global__ __launch_bounds__(TILE_G) void k_ljt(LJArgs A, TileArgs B) {
+    __shared__ double s_pos[3 * TILE_CAP];
+    const int t = threadIdx.x;
+    // the tile: slots (loaded whatever its size), then records, then LDS
+    constexpr int PER = (TILE_CAP + TILE_G - 1) / TILE_G;
+    int sl[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+        sl[k] = B.slots[(size_t) blockIdx.x * TILE_CAP + min(k * TILE_G + t, TILE_CAP - 1)];
+    const int4 G = B.tile[blockIdx.x];
+    if (G.y == 0) return;
+    const int size = G.z;
+    const int nlocal = A.nlocal;
+    const int i = G.x + t;
+    const bool live = t < G.y && i < nlocal;
+    const int ii = live ? i : G.x;
+    const char *__restrict__ P = (const char *) A.P;
+    const size_t stride = A.nl_stride;
+    // the first rows of the list, and what the integration needs
+    const uint4 *lp = B.nl16 + ii;
+    uint4 L = lp[0], M = lp[stride];
+    const int fl = live ? A.flags[ii] : FLAG_FIXED;
+    const int nn = A.numneighs[ii], nm = HALF ? A.nrev[ii] : 0;
+    const double xi = A.X[ii], yi = A.Y[ii], zi = A.Z[ii];
+    double m = 0.0, v0 = 0.0, v1 = 0.0, v2 = 0.0;
+    if (MODE == 1) { m = A.mass[ii]; v0 = A.vx[ii]; v1 = A.vy[ii]; v2 = A.vz[ii]; }
+    {
+        double2 xy[PER];
+        double z[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int e = k * TILE_G + t;
+            xy[k] = make_double2(1e100, 0.0);
+            z[k] = 0.0;
+            if (e > 0 && e < size) {
+                xy[k] = *(const double2 *) (P + ((size_t) sl[k] << 5));
+                z[k] = *(const double *) (P + ((size_t) sl[k] << 5) + 16);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int e = k * TILE_G + t;
+            if (e < size) {
+                s_pos[e] = xy[k].x;
+                s_pos[TILE_CAP + e] = xy[k].y;
+                s_pos[2 * TILE_CAP + e] = z[k];
+            }
+        }
+    }
+    const bool moves = !(fl & FLAG_FIXED);
+    const int n = moves ? min(nn, A.ncap) : 0, nr = HALF && moves ? min(nm, A.rev0) : 0;
+    const double rc2 = A.rc2, dt = A.dt, hdt = A.hdt, eps0 = A.tab.eps[0], sig0 = A.tab.sig6[0];
+    __syncthreads();
+    auto walk = [&](int cnt, int row0, int out0, double &a0, double &a1, double &a2) {
+        const int nmax = wave_max_uniform(cnt);
+        double uu, ww;
+        if (size > 0) {
+            const int rows = (nmax + 7) / 8;
+            const uint4 *lq = lp + (size_t) out0 * stride;
+            const char *S = (const char *) s_pos;
+            if (out0 > 0) { L = lq[0]; M = lq[stride]; }
+            for (int r = 0; r < rows; r++) {
+                const uint4 N = lq[(size_t) min(r + 2, rows - 1) * stride];
+                const uint32_t o[8] = {L.x & 0xffffu, L.x >> 16, L.y & 0xffffu, L.y >> 16,
+                                       L.z & 0xffffu, L.z >> 16, L.w & 0xffffu, L.w >> 16};
+                double x[8], y[8], z[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    x[q] = *(const double *) (S + o[q]);
+                    y[q] = *(const double *) (S + o[q] + 8 * TILE_CAP);
+                    z[q] = *(const double *) (S + o[q] + 16 * TILE_CAP);
+                }
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    double g0, g1, g2;
+                    lj_pair<false, false, UNIT>(xi, yi, zi, x[q], y[q], z[q], true, rc2, sig0, eps0, g0, g1, g2, uu,
+                                                ww);
+                    a0 = a0 + g0; a1 = a1 + g1; a2 = a2 + g2;
+                }
+                L = M;
+                M = N;
+            }
+        } else {
+            // eight entries at a time from memory (a local's own record past its end)
+            const uint4 *from = (const uint4 *) A.nl + (size_t) (row0 >> 2) * stride + ii;
+            for (int k = 0; k < nmax; k += 8) {
+                uint32_t c[8];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const uint4 e = from[(size_t) min(k / 4 + h, A.rows / 4 - 1) * stride];
+                    c[4 * h + 0] = e.x; c[4 * h + 2] = e.y; c[4 * h + 1] = e.z; c[4 * h + 3] = e.w;
+                }
+                double2 xy[8];
+                double z[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const size_t at = (size_t) (k + q < cnt ? c[q] : (uint32_t) ii) << 5;
+                    xy[q] = *(const double2 *) (P + at);
+                    z[q] = *(const double *) (P + at + 16);
+                }
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    double g0, g1, g2;
+                    lj_pair<false, false, UNIT>(xi, yi, zi, xy[q].x, xy[q].y, z[q], k + q < cnt, rc2, sig0, eps0, g0,
+                                                g1, g2, uu, ww);
+                    a0 = a0 + g0; a1 = a1 + g1; a2 = a2 + g2;
+                }
+            }
+        }
+    };
+    double t0 = 0.0, t1 = 0.0, t2 = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0;
+    walk(n, 0, 0, t0, t1, t2);
+    if (HALF) walk(nr, A.rev0, A.rows / 8, r0, r1, r2);
+    if (!live) return;
+    // reset_volatile_properties, the mirror contributions (half lists), then
+    // force[i] = force[i] + reduction
+    const double f0 = r0 + t0, f1 = r1 + t1, f2 = r2 + t2;
+    A.fx[i] = f0; A.fy[i] = f1; A.fz[i] = f2;
+    if (MODE == 1) {
+        double px = xi, py = yi, pz = zi;
+        if (moves && A.do_vv2) {  // final_integrate(ts)
+            double b0 = hdt * f0, b1 = hdt * f1, b2 = hdt * f2;
+            b0 = b0 / m; b1 = b1 / m; b2 = b2 / m;
+            v0 = v0 + b0; v1 = v1 + b1; v2 = v2 + b2;
+        }
+        if (moves) {
+            if (A.do_vv1) {  // initial_integrate(ts+1)
+                double b0 = hdt * f0, b1 = hdt * f1, b2 = hdt * f2;
+                b0 = b0 / m; b1 = b1 / m; b2 = b2 / m;
+                v0 = v0 + b0; v1 = v1 + b1; v2 = v2 + b2;
+                px = xi + dt * v0; py = yi + dt * v1; pz = zi + dt * v2;
+            }
+            A.vx[i] = v0; A.vy[i] = v1; A.vz[i] = v2;
+        }
+        if (A.do_vv1) {
+            A.Xn[i] = px; A.Yn[i] = py; A.Zn[i] = pz;
+            if (A.Pn) A.Pn[i] = make_double4(px, py, pz, 0.0);
+            if (A.im.on)
+                write_images(A.im, i, nlocal, px, py, pz, A.X, A.Y, A.Z, A.Xn, A.Yn, A.Zn, A.g, A.Pn, 0.0);
+        }
+    }
+}
+
 // the waves of many independent systems in one persistent launch: the grid
 // is what the device holds resident at once, and workgroup w takes the
 // consecutive table entries [w * per, (w + 1) * per); entry b belongs to
@@ -2512,6 +2870,23 @@ size_t build_lds_bytes(const DevState &d, const Geom &g, int half) {
     return build_lds(d, g, half, min(d.tile_cap, build_tile_limit(d, g, half)));
 }
 
+static TileArgs tile_args(const DevState &d, const Geom &g) {
+    TileArgs T;
+    T.counters = d.counters;
+    T.g = g;
+    T.lstart = d.lstart; T.gstart = d.gstart; T.numneighs = d.numneighs; T.nrev = d.nrev;
+    T.nl = d.nl; T.nl16 = d.nl16;
+    T.nlocal = d.nlocal; T.nl_stride = d.nl_stride; T.ncap = d.ncap; T.rows = list_rows(d.ncap); T.rev0 = d.rev0;
+    T.grp = d.tile_grp; T.tile = d.tile_tab; T.slots = d.tile_slots; T.gmax = d.tile_gmax;
+    return T;
+}
+
+// (a group and the next of its column hold more than TILE_G locals together, or
+// start TILE_SPAN cells apart)
+int tile_groups_max(int nlocal, const Geom &g) {
+    return 2 * (nlocal / TILE_G) + g.dim_cells[0] * g.dim_cells[1] * (g.dim_cells[2] / TILE_SPAN + 1) + 2;
+}
+
 template <int NT>
 static void build_launch(hipStream_t s, const DevState &d, const Geom &g, int half, const BuildArgs &A) {
     const size_t lds = build_lds(d, g, half, A.tcap, NT);
@@ -2528,6 +2903,12 @@ void launch_build_neighbors(hipStream_t s, const DevState &d, const Geom &g, int
     // candidate buffers at the occupancy measured.)
     if (d.nlocal < 80000 && A.tcap <= 8192) build_launch<BB_SMALL>(s, d, g, half, A);
     else build_launch<BB>(s, d, g, half, A);
+    if (!d.tiles) return;
+    const TileArgs T = tile_args(d, g);
+    launch_set_counters(s, d.counters, C_NGROUPS, 2, 0);
+    hipLaunchKernelGGL(k_tile_groups, dim3((g.dim_cells[0] * g.dim_cells[1] + 1 + 3) / 4), dim3(256), 0, s, T);
+    if (half) hipLaunchKernelGGL(k_tile_build<true>, dim3(T.gmax), dim3(TILE_G), 0, s, T);
+    else hipLaunchKernelGGL(k_tile_build<false>, dim3(T.gmax), dim3(TILE_G), 0, s, T);
 }
 
 void launch_build_batch(hipStream_t s, const BuildArgs *desc, const int *rep, const int *seg_base, int nblocks,
@@ -2680,6 +3061,13 @@ static void lj_launch(hipStream_t s, const DevState &d, const Geom &g, const LJP
         if (d.rev0 > 0) hipLaunchKernelGGL((k_lj<NT, MODE, RED, true, false, UNIT>), grid, dim3(64), 0, s, A);
         else hipLaunchKernelGGL((k_lj<NT, MODE, RED, false, false, UNIT>), grid, dim3(64), 0, s, A);
     } else if constexpr (MODE != 2) {
+        if constexpr (NT == 1 && !RED)
+            if (d.tiles) {
+                const TileArgs T = tile_args(d, g);
+                if (d.rev0 > 0) hipLaunchKernelGGL((k_ljt<MODE, true, UNIT>), dim3(T.gmax), dim3(TILE_G), 0, s, A, T);
+                else hipLaunchKernelGGL((k_ljt<MODE, false, UNIT>), dim3(T.gmax), dim3(TILE_G), 0, s, A, T);
+                return;
+            }
         const dim3 grid(lj_waves(d));
 #define LJM(L)                                                                                            \
     do {                                                                                                  \

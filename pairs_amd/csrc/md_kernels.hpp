@@ -49,7 +49,9 @@ enum {
     C_IMG_OVF = 18,   // a local has more periodic images than IMG_MAX
     C_LEAVE = 19,     // locals outside a periodic dimension, listed for the exchange
     C_LEAVE_MAX = 20, // their number at the last exchange
-    C_COUNT = 21
+    C_NGROUPS = 21,   // groups of the force tiles
+    C_BIG = 22,       // those whose tile does not fit
+    C_COUNT = 23
 };
 enum { OVF_NONE = 0, OVF_PART = 1, OVF_NEIGH = 2, OVF_SEND = 3, OVF_TILE = 4 };
 
@@ -81,6 +83,12 @@ __host__ __device__ __forceinline__ size_t nl_at(int k, int i, int nl_stride) {
 // local's list up to 32 rows at a time, by whole rounds
 constexpr int LIST_ROWS = 32;
 __host__ __device__ __forceinline__ int list_rows(int ncap) { return (ncap + LIST_ROWS - 1) / LIST_ROWS * LIST_ROWS; }
+
+// force tiles: locals of a group, cells it spans, particles of a tile (six
+// tiles in a CU's LDS)
+constexpr int TILE_G = 128;
+constexpr int TILE_SPAN = 8;
+constexpr int TILE_CAP = 1088;
 
 constexpr int IMG_MAX = 8;
 // leavers that the one-workgroup exchange takes from its list
@@ -141,6 +149,13 @@ struct DevState {
     int4 *img_tab;       // [k][cap]: image k's ghost index (physical - nlocal), its source slot (-1: the
                          // local itself), its shift (2 bits per dimension, + 1)
     int img_on;          // host: every local's images fit IMG_MAX
+    // force tiles of a large system (k_ljt): a group's locals and its tile's
+    // size (0: does not fit), the tile's slots, the lists as offsets into it
+    int tiles;           // host: the neighbour build makes them
+    int tile_gmax;
+    int4 *tile_grp, *tile_tab;
+    int *tile_slots;
+    uint4 *nl16;
     int *tile_cnt;
     int *leavers;        // [LEAVE_CAP] physical slots
     int exch_listed;     // host: the exchange works from the list of leavers
@@ -210,6 +225,21 @@ struct BuildArgs {
     int *numneighs, *nrev;
 };
 BuildArgs build_args(const DevState &d, const Geom &g, int half, double rc2);
+// the force tiles of one system
+struct TileArgs {
+    int *counters;
+    Geom g;
+    const int *lstart, *gstart, *numneighs, *nrev;
+    const uint32_t *nl;
+    uint4 *nl16;         // row r of local i: entries 8 r .. 8 r + 7; half lists: mirror rows from rows / 8 on
+    int nlocal, nl_stride, ncap, rows, rev0;
+    int4 *grp;           // first local, locals, first cell, last cell
+    int4 *tile;          // by workgroup: first local, locals (0: none), the tile's size (0: does not fit)
+    int *slots;
+    int gmax;
+};
+// the most groups of a system's tiles
+int tile_groups_max(int nlocal, const Geom &g);
 // dynamic LDS of one system's build workgroup
 size_t build_lds_bytes(const DevState &d, const Geom &g, int half);
 // the builds of many systems in one launch (block b: system rep[b], its

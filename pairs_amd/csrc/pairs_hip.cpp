@@ -148,6 +148,45 @@ static int alloc_neighbor_arrays(pairs_hip_ctx *ctx, DevState &d, int ncap) {
     return 0;
 }
 
+static void free_tiles(DevState &d) {
+    dfree(d.tile_grp); dfree(d.tile_tab); dfree(d.tile_slots); dfree(d.nl16);
+    d.tile_grp = d.tile_tab = nullptr; d.tile_slots = nullptr; d.nl16 = nullptr;
+    d.tiles = 0;
+}
+
+// Force tiles (k_ljt) or not, and their arrays: called where the number of
+// locals or the lists' capacity changes, when no lists are valid.  The tiles
+// cost a rebuild some 40 us per 100000 locals and save each step's force pass
+// half its memory traffic.  A rebuild every 20 steps, ms without | with:
+// 157216 locals (100 steps) 7.29 | 7.43, 186624 8.18 | 8.08 (half lists 11.2 |
+// 11.4), 198400 (200) 14.8 | 13.7, 389344 (100) 15.8 | 14.7 (half 24.1 | 19.9),
+// 1048576 (200) 86.0 | 65.2 (half, 60: 46.0 | 38.7); at 200000 they pay from 8
+// steps between rebuilds on.  A group takes up to 128 locals of one z-column of
+// cells, so short columns would leave its lanes idle.
+static int setup_tiles(pairs_hip_ctx *ctx) {
+    DevState &d = ctx->d;
+    const Geom &g = ctx->geom;
+    free_tiles(d);
+    const double per_column = d.nlocal * (g.spacing / g.len[0]) * (g.spacing / g.len[1]);
+    if (ctx->tiles_off || ctx->cfg.ntypes != 1 || d.nlocal < 200000 || ctx->cfg.reneighbor_every < 10 ||
+        per_column < 96.0)
+        return 0;
+    d.tile_gmax = tile_groups_max(d.nlocal, g);
+    const size_t gm = (size_t) d.tile_gmax;
+    if (dalloc(ctx, &d.tile_grp, gm) || dalloc(ctx, &d.tile_tab, gm) || dalloc(ctx, &d.tile_slots, gm * TILE_CAP) ||
+        dalloc(ctx, &d.nl16, (size_t) list_rows(d.ncap) / 8 * (d.rev0 > 0 ? 2 : 1) * d.nl_stride))
+        return PAIRS_HIP_ERR_HIP;
+    launch_set_counters(ctx->stream, d.counters, C_NGROUPS, 2, 0);
+    // until a build has made tiles: every local, over the 32-bit lists
+    std::vector<int4> tab((d.nlocal + TILE_G - 1) / TILE_G);
+    for (size_t k = 0; k < tab.size(); k++)
+        tab[k] = make_int4((int) k * TILE_G, std::min(TILE_G, d.nlocal - (int) k * TILE_G), 0, 0);
+    HIP_OK(hipMemcpyAsync(d.tile_tab, tab.data(), tab.size() * sizeof(int4), hipMemcpyHostToDevice, ctx->stream));
+    HIP_OK(hipStreamSynchronize(ctx->stream));
+    d.tiles = 1;
+    return 0;
+}
+
 static int alloc_send_arrays(pairs_hip_ctx *ctx, DevState &d, int send_cap) {
     dfree(d.send_map); dfree(d.send_mult); dfree(d.scratch_i); dfree(d.stage);
     d.send_map = d.send_mult = d.scratch_i = nullptr;
@@ -229,6 +268,12 @@ static void take_counters(pairs_hip_ctx *ctx) {
         // scanned the locals in one workgroup): the wide kernels from now on
         ctx->d.exch_listed = 0;
         drop_reb_graphs(ctx);
+    }
+    if (ctx->d.tiles && ctx->h_counters[C_BIG] > ctx->h_counters[C_NGROUPS] / 16) {
+        // too many groups whose tile does not fit (they walk the 32-bit lists)
+        ctx->tiles_off = true;
+        ctx->d.tiles = 0;
+        drop_graphs(ctx);
     }
 }
 
@@ -356,6 +401,7 @@ int pairs_hip_destroy(pairs_hip_ctx *ctx) {
     for (auto e : ctx->ev_end) hipEventDestroy(e);
     DevState &d = ctx->d;
     free_particle_arrays(d);
+    free_tiles(d);
     dfree(d.nl); dfree(d.send_map); dfree(d.send_mult); dfree(d.scratch_i); dfree(d.stage);
     dfree(d.lcount); dfree(d.gcount); dfree(d.lstart); dfree(d.gstart); dfree(d.counters); dfree(d.thermo);
     dfree(ctx->d_eatom); dfree(ctx->d_expand);
@@ -419,6 +465,7 @@ int pairs_hip_reserve(pairs_hip_ctx *ctx, int particle_capacity, int neighbor_ca
     } else if (neighbor_capacity > d.ncap) {
         if (alloc_neighbor_arrays(ctx, d, neighbor_capacity)) return PAIRS_HIP_ERR_HIP;
         launch_fill_i32(ctx->stream, d.numneighs, 0, d.cap);
+        if (setup_tiles(ctx)) return PAIRS_HIP_ERR_HIP;
     }
     if (send_capacity > d.send_cap) {
         if (alloc_send_arrays(ctx, d, send_capacity)) return PAIRS_HIP_ERR_HIP;
@@ -487,7 +534,7 @@ int pairs_hip_upload(pairs_hip_ctx *ctx, int n, const double *x, const double *v
     ctx->nghost = 0;
     ctx->nsend_all = 0;
     setup_segments(ctx, ctx->zc_override);
-    return 0;
+    return setup_tiles(ctx);
 }
 
 // Park-Miller minimal standard generator without masking (runtime/copper_fcc_lattice.hpp:11-26)
@@ -1683,6 +1730,8 @@ int pairs_hip_mlp_attach(pairs_hip_ctx *ctx, pairs_hip_mlp *m, double max_rel_rm
     }
     ctx->mlp = mlp_bind(ctx, m);
     ctx->mlp_on = true;
+    ctx->tiles_off = true;
+    ctx->d.tiles = 0;
     DevState &d = ctx->d;
     launch_mlp_forces(ctx->stream, d, ctx->geom, ctx->mlp, d.cur, 0, ctx->ghost_grid);
     CHECK_LAUNCH();
@@ -1952,6 +2001,7 @@ int pairs_hip_batch_create(pairs_hip_batch **out, int nreplicas, const pairs_hip
         pairs_hip_ctx *ctx = nullptr;
         const int e = pairs_hip_create(&ctx, &c);
         if (e) { pairs_hip_batch_destroy(b); return e; }
+        ctx->tiles_off = true;  // the batched kernels neither make nor use force tiles
         b->rep.push_back(ctx);
         b->unit = b->unit && b->ntypes1 && ctx->prm.eps[0] == 1.0 && ctx->prm.sig6[0] == 1.0;
     }

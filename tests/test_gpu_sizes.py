@@ -307,3 +307,36 @@ def test_lj_exchange_and_borders_vs_oracle(n, periodic, edge, speed):
         assert np.array_equal(g.positions(True), o.positions(True)), step
         assert np.array_equal(g.velocities(), o.velocities()), step
         tm._compare_lists(g, o, step)
+
+
+# large systems of one type take the timestep's forces from LDS tiles; two types
+# with the same parameters do not, and give the same bits
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("sites,spacing,every", [
+    ((59, 59, 59), 1.06, 10),     # the LJ fluid; a last column of cells nearly empty
+    ((26, 29, 271), 1.06, 12),    # long columns
+    ((61, 61, 55), 0.93, 10),     # dense: tiles that do not fit, the 32-bit lists instead
+    ((130, 130, 12), 1.06, 10)])  # short columns: no tiles
+def test_lj_tiles_vs_gathers(half, sites, spacing, every):
+    from pairs_amd import md
+    rng = np.random.default_rng(sum(sites))
+    k = np.stack(np.meshgrid(*[np.arange(m) for m in sites], indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    k = k[rng.permutation(n)]
+    box = [(0.0, m * spacing) for m in sites]
+    x = (k + 0.5 + rng.uniform(-0.08, 0.08, k.shape)) * spacing
+    v = rng.standard_normal(k.shape)
+    flags = np.where(rng.random(n) < 0.02, 4, 0).astype(np.int32)
+    v[flags == 4] = 0.0
+    out = []
+    for nt in (1, 2):
+        g = md.LJSystem(box, particle_capacity=2 * n, send_capacity=n, neighbor_capacity=140, half=half, ntypes=nt,
+                        reneighbor_every=every, thermo_every=16, ncells_capacity=200000)
+        g.upload(x, v, flags=flags, types=np.arange(n, dtype=np.int32) % nt)
+        got = []
+        for a, b in ((0, 1), (1, 6), (6, 27)):
+            g.run(a, b, 100)
+            got += [g.positions(True), g.velocities(), g.forces()]
+        out.append(got)
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
