@@ -16,6 +16,7 @@
 
 #include "../../include/pairs_hip_dem.h"
 #include "dem_kernels.hpp"
+#include "host_rows.hpp"
 
 using namespace dk;
 
@@ -51,6 +52,7 @@ struct pairs_hip_dem_ctx {
     CopyDesc *h_copy = nullptr; // pinned copy tables (checkpoint, restore)
     CopyDesc *d_copy = nullptr;
     int resizes = 0;            // capacity growths so far
+    HostRows rows;
 };
 
 #define HIP_OK(expr)                                                                                   \
@@ -672,20 +674,12 @@ int pairs_hip_dem_download(pairs_hip_dem_ctx *ctx, int what, void *host, int cou
     const size_t C = p.cap;
     // at most what exists: locals and ghosts, or the locals of local-only arrays
     const int n_all = std::min(count, nall), n_loc = std::min(count, nl);
-    auto get_d = [&](const double *d, double *h, int n) { return hipMemcpy(h, d, n * sizeof(double), hipMemcpyDeviceToHost); };
     auto get_i = [&](const int *d, int *h, int n) -> int {
-        HIP_OK(hipMemcpy(h, d, n * sizeof(int), hipMemcpyDeviceToHost));
+        HIP_OK(ctx->rows.fetch<int>(ctx->stream, {d}, nullptr, n, h));
         return n;
     };
     auto interleave = [&](std::initializer_list<const double *> cols, double *out, int n) -> int {
-        const int nc = (int) cols.size();
-        std::vector<double> tmp(std::max(n, 1));
-        int c = 0;
-        for (const double *col : cols) {
-            HIP_OK(get_d(col, tmp.data(), n));
-            for (int i = 0; i < n; i++) out[(size_t) i * nc + c] = tmp[i];
-            c++;
-        }
+        HIP_OK(ctx->rows.fetch<double>(ctx->stream, cols, nullptr, n, out));
         return n;
     };
     double *hd = (double *) host;
@@ -696,8 +690,8 @@ int pairs_hip_dem_download(pairs_hip_dem_ctx *ctx, int what, void *host, int cou
     case PAIRS_HIP_DEM_ANGULAR_VELOCITY: return interleave({p.wx, p.wy, p.wz}, hd, n_all);
     case PAIRS_HIP_DEM_FORCE: return interleave({p.fx, p.fy, p.fz}, hd, n_loc);
     case PAIRS_HIP_DEM_TORQUE: return interleave({p.tx, p.ty, p.tz}, hd, n_loc);
-    case PAIRS_HIP_DEM_RADIUS: HIP_OK(get_d(p.r, hd, n_all)); return n_all;
-    case PAIRS_HIP_DEM_MASS: HIP_OK(get_d(p.m, hd, n_all)); return n_all;
+    case PAIRS_HIP_DEM_RADIUS: return interleave({p.r}, hd, n_all);
+    case PAIRS_HIP_DEM_MASS: return interleave({p.m}, hd, n_all);
     case PAIRS_HIP_DEM_ROTATION_QUAT:
         return interleave({p.rot_q, p.rot_q + C, p.rot_q + 2 * C, p.rot_q + 3 * C}, hd, n_loc);
     case PAIRS_HIP_DEM_ROTATION_MATRIX:

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/pairs_hip.h"
+#include "host_rows.hpp"
 #include "md_kernels.hpp"
 #include "mlp_kernels.hpp"
 
@@ -23,6 +24,8 @@ struct pairs_hip_ctx {
     std::string err;
     int req[5] = {0, 0, 0, 0, 0};
     int h_counters[C_COUNT];
+    int *h_pin = nullptr;      // pinned, C_COUNT
+    HostRows rows;
     int nghost = 0, nsend_all = 0;
     int ghost_grid = 1;
     int max_lds = 65536;       // shared memory a workgroup may allocate

@@ -278,8 +278,9 @@ static void take_counters(pairs_hip_ctx *ctx) {
 }
 
 static int read_counters(pairs_hip_ctx *ctx) {
-    HIP_OK(hipMemcpyAsync(ctx->h_counters, ctx->d.counters, sizeof(int) * C_COUNT, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_OK(hipMemcpyAsync(ctx->h_pin, ctx->d.counters, sizeof(int) * C_COUNT, hipMemcpyDeviceToHost, ctx->stream));
     HIP_OK(hipStreamSynchronize(ctx->stream));
+    std::memcpy(ctx->h_counters, ctx->h_pin, sizeof(int) * C_COUNT);
     take_counters(ctx);
     return 0;
 }
@@ -312,15 +313,11 @@ static int host_phys(pairs_hip_ctx *ctx, int n, std::vector<int> &phys) {
     return download_raw(ctx, phys.data(), ctx->d.phys, n * sizeof(int));
 }
 
+// rows of arrays in reference order, entry r from the slot of reference index r
 template <typename T>
-static int ref_order(pairs_hip_ctx *ctx, const T *dev, int n, const std::vector<int> &phys, T *out, int stride,
-                     int comp) {
+static int ref_rows(pairs_hip_ctx *ctx, std::initializer_list<const T *> cols, int n, T *out) {
     if (n <= 0) return 0;
-    int maxp = 0;
-    for (int r = 0; r < n; r++) maxp = std::max(maxp, phys[r]);
-    std::vector<T> tmp(maxp + 1);
-    if (download_raw(ctx, tmp.data(), dev, (maxp + 1) * sizeof(T))) return PAIRS_HIP_ERR_HIP;
-    for (int r = 0; r < n; r++) out[(size_t) r * stride + comp] = tmp[phys[r]];
+    HIP_OK(ctx->rows.fetch(ctx->stream, cols, ctx->d.phys, n, out));
     return 0;
 }
 
@@ -369,6 +366,7 @@ int pairs_hip_create(pairs_hip_ctx **out, const pairs_hip_md_config *cfg) {
     if (noalloc_resolve(dev, ctx->err)) return fail(PAIRS_HIP_ERR_HIP);
     DevState &d = ctx->d;
     d.max_lds = ctx->max_lds;
+    if (hipHostMalloc((void **) &ctx->h_pin, sizeof(int) * C_COUNT) != hipSuccess) return fail(PAIRS_HIP_ERR_HIP);
     if (const char *e = getenv("PAIRS_HIP_HOME")) ctx->home_target = std::max(8, atoi(e));
     setup_geometry(ctx);
     // the cell grid is fixed by the box; its arrays are sized to fit it
@@ -409,6 +407,7 @@ int pairs_hip_destroy(pairs_hip_ctx *ctx) {
     dfree(ctx->mlp_rho); dfree(ctx->mlp_U);
     dfree(ctx->ckpt);
     if (ctx->h_spec) hipHostFree(ctx->h_spec);
+    if (ctx->h_pin) hipHostFree(ctx->h_pin);
     if (ctx->spec_ev) hipEventDestroy(ctx->spec_ev);
     if (ctx->reb_ev) hipEventDestroy(ctx->reb_ev);
     if (ctx->side) { hipStreamSynchronize(ctx->side); hipStreamDestroy(ctx->side); }
@@ -429,19 +428,12 @@ static int fetch_locals(pairs_hip_ctx *ctx, HostLocals &h) {
     if (read_counters(ctx)) return PAIRS_HIP_ERR_HIP;
     const int n = ctx->h_counters[C_NLOCAL];
     h.n = n;
-    std::vector<int> phys;
-    if (host_phys(ctx, n, phys)) return PAIRS_HIP_ERR_HIP;
     h.x.resize(3 * (size_t) n); h.v.resize(3 * (size_t) n); h.m.resize(n); h.t.resize(n); h.f.resize(n); h.u.resize(n);
     const int c = d.cur;
-    const double *pos[3] = {d.X[c], d.Y[c], d.Z[c]}, *vel[3] = {d.vx, d.vy, d.vz};
-    for (int k = 0; k < 3; k++) {
-        if (ref_order(ctx, pos[k], n, phys, h.x.data(), 3, k)) return PAIRS_HIP_ERR_HIP;
-        if (ref_order(ctx, vel[k], n, phys, h.v.data(), 3, k)) return PAIRS_HIP_ERR_HIP;
-    }
-    if (ref_order(ctx, (const double *) d.mass, n, phys, h.m.data(), 1, 0) ||
-        ref_order(ctx, (const int *) d.type, n, phys, h.t.data(), 1, 0) ||
-        ref_order(ctx, (const int *) d.flags, n, phys, h.f.data(), 1, 0) ||
-        ref_order(ctx, (const int *) d.uid, n, phys, h.u.data(), 1, 0))
+    if (ref_rows<double>(ctx, {d.X[c], d.Y[c], d.Z[c]}, n, h.x.data()) ||
+        ref_rows<double>(ctx, {d.vx, d.vy, d.vz}, n, h.v.data()) || ref_rows<double>(ctx, {d.mass}, n, h.m.data()) ||
+        ref_rows<int>(ctx, {d.type}, n, h.t.data()) || ref_rows<int>(ctx, {d.flags}, n, h.f.data()) ||
+        ref_rows<int>(ctx, {d.uid}, n, h.u.data()))
         return PAIRS_HIP_ERR_HIP;
     return 0;
 }
@@ -670,35 +662,29 @@ int pairs_hip_download(pairs_hip_ctx *ctx, int what, void *host, int count) {
         case PAIRS_HIP_VELOCITY:
         case PAIRS_HIP_FORCE: {
             const int n = lim(what == PAIRS_HIP_FORCE ? nlocal : nall);
-            if (host_phys(ctx, n, phys)) return PAIRS_HIP_ERR_HIP;
-            const double *src[3];
-            if (what == PAIRS_HIP_POSITION) { src[0] = d.X[c]; src[1] = d.Y[c]; src[2] = d.Z[c]; }
-            else if (what == PAIRS_HIP_VELOCITY) { src[0] = d.vx; src[1] = d.vy; src[2] = d.vz; }
-            else { src[0] = d.fx; src[1] = d.fy; src[2] = d.fz; }
-            for (int k = 0; k < 3; k++)
-                if (ref_order(ctx, src[k], n, phys, (double *) host, 3, k)) return PAIRS_HIP_ERR_HIP;
-            return n;
+            double *h = (double *) host;
+            const int e = what == PAIRS_HIP_POSITION   ? ref_rows<double>(ctx, {d.X[c], d.Y[c], d.Z[c]}, n, h)
+                          : what == PAIRS_HIP_VELOCITY ? ref_rows<double>(ctx, {d.vx, d.vy, d.vz}, n, h)
+                                                       : ref_rows<double>(ctx, {d.fx, d.fy, d.fz}, n, h);
+            return e ? PAIRS_HIP_ERR_HIP : n;
         }
         case PAIRS_HIP_MASS: {
             const int n = lim(nall);
-            if (host_phys(ctx, n, phys)) return PAIRS_HIP_ERR_HIP;
-            return ref_order(ctx, (const double *) d.mass, n, phys, (double *) host, 1, 0) ? PAIRS_HIP_ERR_HIP : n;
+            return ref_rows<double>(ctx, {d.mass}, n, (double *) host) ? PAIRS_HIP_ERR_HIP : n;
         }
         case PAIRS_HIP_TYPE:
         case PAIRS_HIP_FLAGS:
         case PAIRS_HIP_UID:
         case PAIRS_HIP_PARTICLE_CELL: {
             const int n = lim(nall);
-            if (host_phys(ctx, n, phys)) return PAIRS_HIP_ERR_HIP;
             const int *src = what == PAIRS_HIP_TYPE ? d.type
                              : what == PAIRS_HIP_FLAGS ? d.flags
                              : what == PAIRS_HIP_UID ? d.uid : d.particle_cell;
-            return ref_order(ctx, src, n, phys, (int *) host, 1, 0) ? PAIRS_HIP_ERR_HIP : n;
+            return ref_rows<int>(ctx, {src}, n, (int *) host) ? PAIRS_HIP_ERR_HIP : n;
         }
         case PAIRS_HIP_NUMNEIGHS: {
             const int n = lim(nlocal);
-            if (host_phys(ctx, n, phys)) return PAIRS_HIP_ERR_HIP;
-            return ref_order(ctx, (const int *) d.numneighs, n, phys, (int *) host, 1, 0) ? PAIRS_HIP_ERR_HIP : n;
+            return ref_rows<int>(ctx, {d.numneighs}, n, (int *) host) ? PAIRS_HIP_ERR_HIP : n;
         }
         case PAIRS_HIP_NEIGHBORLISTS: {
             const int n = lim(nlocal);
@@ -758,8 +744,7 @@ int pairs_hip_download(pairs_hip_ctx *ctx, int what, void *host, int count) {
         case PAIRS_HIP_ATOM_ENERGY: {
             const int n = lim(std::min(nlocal, ctx->eatom_cap));
             if (!ctx->d_eatom || n == 0) return 0;
-            if (host_phys(ctx, n, phys)) return PAIRS_HIP_ERR_HIP;
-            return ref_order(ctx, (const double *) ctx->d_eatom, n, phys, (double *) host, 1, 0) ? PAIRS_HIP_ERR_HIP : n;
+            return ref_rows<double>(ctx, {ctx->d_eatom}, n, (double *) host) ? PAIRS_HIP_ERR_HIP : n;
         }
     }
     return PAIRS_HIP_ERR_ARG;

@@ -261,7 +261,8 @@ class DEMSystem:
                 "num_contacts": (NUM_CONTACTS, np.int32, None)}
         which, dt, cols = spec[name]
         n = self.nlocal + (self.nghost if ghosts else 0)
-        out = np.zeros((n, cols) if cols else n, dt)
+        # (an array of locals only leaves the ghosts' rows at zero)
+        out = (np.zeros if ghosts else np.empty)((n, cols) if cols else n, dt)
         self._check(self.L.pairs_hip_dem_download(self.ctx, which, out.ctypes.data_as(_P), n), "download")
         return out
 

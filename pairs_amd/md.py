@@ -247,7 +247,7 @@ class LJSystem:
         return self.count(nat.NCELLS)
 
     def _dl(self, what, shape, dtype, n):
-        a = np.zeros(shape, dtype)
+        a = np.empty(shape, dtype)  # (what the call does not fill is cut off)
         if n == 0:
             return a
         got = self._call("pairs_hip_download", what, a.ctypes.data_as(ctypes.c_void_p), n)

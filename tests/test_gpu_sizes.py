@@ -340,3 +340,22 @@ def test_lj_tiles_vs_gathers(half, sites, spacing, every):
         out.append(got)
     for p, q in zip(*out):
         assert np.array_equal(p, q)
+
+
+# downloads come in blocks of 1 MiB: 43690 rows of three doubles, 131072 doubles, 262144 words
+@pytest.mark.parametrize("n", [1, 43690, 43691, 87381, 131073, 262145])
+def test_downloads_at_block_edges(n):
+    from pairs_amd import dem, md
+    rng = np.random.default_rng(n)
+    L = 2.0 * n ** (1.0 / 3.0)
+    x, v = rng.uniform(0.0, L, (n, 3)), rng.standard_normal((n, 3))
+    t, fl = rng.integers(0, 3, n).astype(np.int32), rng.integers(0, 2, n).astype(np.int32) * 4
+    g = md.LJSystem([(0.0, L)] * 3, particle_capacity=n, send_capacity=16, neighbor_capacity=16, ntypes=3)
+    g.upload(x, v, types=t, flags=fl)
+    assert np.array_equal(g.positions(), x) and np.array_equal(g.velocities(), v) and np.array_equal(g.types(), t)
+    s = dem.DEMSystem((L, L, L), particle_capacity=n + 1, contact_capacity=4, send_capacity=16, cell_width=L / 4,
+                      ncells_capacity=1000)
+    r = rng.uniform(0.1, 0.2, n)
+    s.add_spheres(np.arange(n) + 5, r, x, v)
+    assert np.array_equal(s.get("position"), x) and np.array_equal(s.get("linear_velocity"), v)
+    assert np.array_equal(s.get("uid"), np.arange(n) + 5) and np.array_equal(s.get("radius"), r)
