@@ -258,173 +258,140 @@ __global__ __launch_bounds__(256) void k_bin_scatter(const int *__restrict__ cou
 }
 
 // Order the locals and the ghosts of every cell by reference index -- the
-// order in which the CPU program's sequential insertion fills cell_particles.
-// One wave per (cell, locals|ghosts) run: a rank sort of up to 64 keys in
-// registers, a serial insertion sort beyond that.
-// one wave per item (cell c = item / 2; its locals, or its ghosts)
-__device__ __forceinline__ void k_sort_cells_body(const int *__restrict__ counters, const int *__restrict__ lstart,
-                                                    const int *__restrict__ gstart, const int *__restrict__ ref,
-                                                    int *__restrict__ perm, int ncells, int item) {
-    if (counters[C_OVF]) return;
-    const int nlocal = counters[C_NLOCAL];
+// order in which the CPU program's sequential insertion fills cell_particles --
+// move every particle array into that order (into the spare arrays), update
+// phys[reference index] and clear the locals' image counts.  One wave per (cell,
+// locals|ghosts) run: a rank sort of up to 64 keys in registers, each lane
+// moving its particle to its place; a serial insertion sort beyond that.  Sort
+// and move in kernels of their own took 6.8 us at 256 atoms, 18 at 131072 and 88
+// at 1048576; so 6.1, 17 and 102, with a launch less.
+struct OrderArgs {
+    const int *counters, *lstart, *gstart;
+    int *perm;
+    const double *X, *Y, *Z, *vx, *vy, *vz, *mass;
+    const int *type, *flags, *uid, *shape, *ref;
+    double *Xn, *Yn, *Zn, *avx, *avy, *avz, *amass;
+    int *atype, *aflags, *auid, *ashape, *aref, *acell, *phys, *img_cnt;
+    int ncells;
+};
+
+// item: cell item / 2, its locals or (odd) its ghosts
+__device__ __forceinline__ void k_order_body(const OrderArgs &A, int item) {
+    if (A.counters[C_OVF]) return;
+    const int nlocal = A.counters[C_NLOCAL];
     const int lane = threadIdx.x & 63;
-    if (item >= 2 * ncells) return;
+    if (item >= 2 * A.ncells) return;
     const int c = item >> 1, ghosts = item & 1;
-    const int b = ghosts ? nlocal + gstart[c] : lstart[c];
-    const int e = ghosts ? nlocal + gstart[c + 1] : lstart[c + 1];
+    const int b = ghosts ? nlocal + A.gstart[c] : A.lstart[c];
+    const int e = ghosts ? nlocal + A.gstart[c + 1] : A.lstart[c + 1];
     const int len = e - b;
-    if (len <= 1) return;
+    auto move = [&](int p, int r, int np) {
+        A.Xn[np] = A.X[p]; A.Yn[np] = A.Y[p]; A.Zn[np] = A.Z[p];
+        A.avx[np] = A.vx[p]; A.avy[np] = A.vy[p]; A.avz[np] = A.vz[p]; A.amass[np] = A.mass[p];
+        A.atype[np] = A.type[p]; A.aflags[np] = A.flags[p]; A.auid[np] = A.uid[p]; A.ashape[np] = A.shape[p];
+        A.aref[np] = r;
+        A.acell[np] = c;
+        A.phys[r] = np;
+        if (!ghosts) A.img_cnt[np] = 0;
+    };
     if (len <= 64) {
-        const int p = lane < len ? perm[b + lane] : 0;
-        const int key = lane < len ? ref[p] : 0x7fffffff;
+        const int p = lane < len ? A.perm[b + lane] : 0;
+        const int key = lane < len ? A.ref[p] : 0x7fffffff;
         int rank = 0;
-        for (int q = 0; q < len; q++) {
-            const int kq = __shfl(key, q, 64);
-            rank += (kq < key) ? 1 : 0;
-        }
-        if (lane < len) perm[b + rank] = p;
-    } else if (lane == 0) {
+        for (int q = 0; q < len; q++) rank += __builtin_amdgcn_readlane(key, q) < key ? 1 : 0;
+        if (lane < len) move(p, key, b + rank);
+        return;
+    }
+    if (lane == 0) {
         for (int k = b + 1; k < e; k++) {
-            const int v = perm[k], kv = ref[v];
+            const int v = A.perm[k], kv = A.ref[v];
             int q = k - 1;
-            while (q >= b && ref[perm[q]] > kv) { perm[q + 1] = perm[q]; q--; }
-            perm[q + 1] = v;
+            while (q >= b && A.ref[A.perm[q]] > kv) { A.perm[q + 1] = A.perm[q]; q--; }
+            A.perm[q + 1] = v;
         }
     }
-}
-
-__global__ __launch_bounds__(256) void k_sort_cells(const int *__restrict__ counters, const int *__restrict__ lstart,
-                                                    const int *__restrict__ gstart, const int *__restrict__ ref,
-                                                    int *__restrict__ perm, int ncells) {
-    k_sort_cells_body(counters, lstart, gstart, ref, perm, ncells, blockIdx.x * 4 + (threadIdx.x >> 6));
-}
-
-// Move every particle array into cell order (into the spare arrays) and
-// update phys[reference index].
-__device__ __forceinline__ void k_permute_body(const int *__restrict__ counters, const int *__restrict__ perm,
-                                                 const double *__restrict__ X, const double *__restrict__ Y,
-                                                 const double *__restrict__ Z, double *__restrict__ Xn,
-                                                 double *__restrict__ Yn, double *__restrict__ Zn,
-                                                 const double *__restrict__ vx, const double *__restrict__ vy,
-                                                 const double *__restrict__ vz, const double *__restrict__ mass,
-                                                 const int *__restrict__ type, const int *__restrict__ flags,
-                                                 const int *__restrict__ uid, const int *__restrict__ shape,
-                                                 const int *__restrict__ ref, const int *__restrict__ cell,
-                                                 double *__restrict__ avx, double *__restrict__ avy,
-                                                 double *__restrict__ avz, double *__restrict__ amass,
-                                                 int *__restrict__ atype, int *__restrict__ aflags,
-                                                 int *__restrict__ auid, int *__restrict__ ashape,
-                                                 int *__restrict__ aref, int *__restrict__ acell,
-                                                 int *__restrict__ phys) {
-    if (counters[C_OVF]) return;
-    const int n = counters[C_NLOCAL] + counters[C_NGHOST];
-    for (int np = blockIdx.x * 256 + threadIdx.x; np < n; np += gridDim.x * 256) {
-        const int p = perm[np];
-        Xn[np] = X[p]; Yn[np] = Y[p]; Zn[np] = Z[p];
-        avx[np] = vx[p]; avy[np] = vy[p]; avz[np] = vz[p]; amass[np] = mass[p];
-        atype[np] = type[p]; aflags[np] = flags[p]; auid[np] = uid[p]; ashape[np] = shape[p];
-        const int r = ref[p];
-        aref[np] = r;
-        acell[np] = cell[p];
-        phys[r] = np;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (int k = b + lane; k < e; k += 64) {
+        const int p = A.perm[k];
+        move(p, A.ref[p], k);
     }
 }
 
-__global__ __launch_bounds__(256) void k_permute(const int *__restrict__ counters, const int *__restrict__ perm,
-                                                 const double *__restrict__ X, const double *__restrict__ Y,
-                                                 const double *__restrict__ Z, double *__restrict__ Xn,
-                                                 double *__restrict__ Yn, double *__restrict__ Zn,
-                                                 const double *__restrict__ vx, const double *__restrict__ vy,
-                                                 const double *__restrict__ vz, const double *__restrict__ mass,
-                                                 const int *__restrict__ type, const int *__restrict__ flags,
-                                                 const int *__restrict__ uid, const int *__restrict__ shape,
-                                                 const int *__restrict__ ref, const int *__restrict__ cell,
-                                                 double *__restrict__ avx, double *__restrict__ avy,
-                                                 double *__restrict__ avz, double *__restrict__ amass,
-                                                 int *__restrict__ atype, int *__restrict__ aflags,
-                                                 int *__restrict__ auid, int *__restrict__ ashape,
-                                                 int *__restrict__ aref, int *__restrict__ acell,
-                                                 int *__restrict__ phys) {
-    k_permute_body(counters, perm, X, Y, Z, Xn, Yn, Zn, vx, vy, vz, mass, type, flags, uid, shape, ref, cell, avx, avy, avz, amass, atype, aflags, auid, ashape, aref, acell, phys);
+__global__ __launch_bounds__(256) void k_order(OrderArgs A) {
+    k_order_body(A, blockIdx.x * 4 + (threadIdx.x >> 6));
+}
+
+// from position buffer c into the other
+__host__ __device__ __forceinline__ OrderArgs order_args(const DevState &d, const Geom &g, int c) {
+    const int o = 1 - c;
+    return {d.counters, d.lstart, d.gstart, d.perm, d.X[c], d.Y[c], d.Z[c], d.vx, d.vy, d.vz, d.mass, d.type, d.flags,
+            d.uid, d.shape, d.ref, d.X[o], d.Y[o], d.Z[o], d.alt_vx, d.alt_vy, d.alt_vz, d.alt_mass, d.alt_type,
+            d.alt_flags, d.alt_uid, d.alt_shape, d.alt_ref, d.alt_cell, d.phys, d.img_cnt, g.ncells};
 }
 
 // Copy the permuted arrays back (array addresses stay fixed, so captured
-// graphs remain valid across rebuilds), clear the locals' image counts, and
-// build the ghost refresh maps in physical order: the physical slot of each
-// ghost's source and its image multipliers (send_map / send_mult are in
-// reference ghost order: ghost g = reference index nlocal + g, read from the
-// permuted copy of ref).
-__device__ __forceinline__ void k_copy_back_maps_body(
-    const int *__restrict__ counters, const double *__restrict__ avx, const double *__restrict__ avy,
-    const double *__restrict__ avz, const double *__restrict__ amass, const int *__restrict__ atype,
-    const int *__restrict__ aflags, const int *__restrict__ auid, const int *__restrict__ ashape,
-    const int *__restrict__ aref, const int *__restrict__ acell, double *__restrict__ vx, double *__restrict__ vy,
-    double *__restrict__ vz, double *__restrict__ mass, int *__restrict__ type, int *__restrict__ flags,
-    int *__restrict__ uid, int *__restrict__ shape, int *__restrict__ ref, int *__restrict__ cell,
-    const int *__restrict__ phys, const int *__restrict__ send_map, const int *__restrict__ send_mult,
-    int *__restrict__ sync_src, int *__restrict__ sync_mult, int *__restrict__ img_cnt) {
-    if (counters[C_OVF]) return;
-    const int nlocal = counters[C_NLOCAL], ng = counters[C_NGHOST];
+// graphs remain valid across rebuilds), and build the ghost refresh maps in
+// physical order: the physical slot of each ghost's source and its image
+// multipliers (send_map / send_mult are in reference ghost order: ghost g =
+// reference index nlocal + g, read from the permuted copy of ref).  A ghost's
+// chain of sources ends at its root local, whose image table it joins (order
+// irrelevant: positions are written to the next buffer from values of the
+// current one).  P, if given, gets the packed copy of the new positions, which
+// the force step behind a rebuild gathers from.
+struct CopyBackArgs {
+    int *counters;
+    const double *avx, *avy, *avz, *amass;
+    const int *atype, *aflags, *auid, *ashape, *aref, *acell;
+    double *vx, *vy, *vz, *mass;
+    int *type, *flags, *uid, *shape, *ref, *cell;
+    const int *phys, *send_map, *send_mult;
+    int *sync_src, *sync_mult, *img_cnt;
+    int4 *img_tab;
+    int cap;
+    const double *X, *Y, *Z;
+    double4 *P;
+};
+
+__device__ __forceinline__ void k_copy_back_body(const CopyBackArgs &A) {
+    if (A.counters[C_OVF]) return;
+    const int nlocal = A.counters[C_NLOCAL], ng = A.counters[C_NGHOST];
     const int n = nlocal + ng;
     for (int p = blockIdx.x * 256 + threadIdx.x; p < n; p += gridDim.x * 256) {
-        vx[p] = avx[p]; vy[p] = avy[p]; vz[p] = avz[p]; mass[p] = amass[p];
-        type[p] = atype[p]; flags[p] = aflags[p]; uid[p] = auid[p]; shape[p] = ashape[p];
-        ref[p] = aref[p]; cell[p] = acell[p];
-        if (p < nlocal) img_cnt[p] = 0;
-    }
-    for (int q = blockIdx.x * 256 + threadIdx.x; q < ng; q += gridDim.x * 256) {
-        const int g = aref[nlocal + q] - nlocal;
-        sync_src[q] = phys[send_map[g]];
-        sync_mult[3 * q + 0] = send_mult[3 * g + 0];
-        sync_mult[3 * q + 1] = send_mult[3 * g + 1];
-        sync_mult[3 * q + 2] = send_mult[3 * g + 2];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_copy_back_maps(
-    const int *__restrict__ counters, const double *__restrict__ avx, const double *__restrict__ avy,
-    const double *__restrict__ avz, const double *__restrict__ amass, const int *__restrict__ atype,
-    const int *__restrict__ aflags, const int *__restrict__ auid, const int *__restrict__ ashape,
-    const int *__restrict__ aref, const int *__restrict__ acell, double *__restrict__ vx, double *__restrict__ vy,
-    double *__restrict__ vz, double *__restrict__ mass, int *__restrict__ type, int *__restrict__ flags,
-    int *__restrict__ uid, int *__restrict__ shape, int *__restrict__ ref, int *__restrict__ cell,
-    const int *__restrict__ phys, const int *__restrict__ send_map, const int *__restrict__ send_mult,
-    int *__restrict__ sync_src, int *__restrict__ sync_mult, int *__restrict__ img_cnt) {
-    k_copy_back_maps_body(counters, avx, avy, avz, amass, atype, aflags, auid, ashape, aref, acell, vx, vy, vz, mass,
-                          type, flags, uid, shape, ref, cell, phys, send_map, send_mult, sync_src, sync_mult, img_cnt);
-}
-
-// A segment's tile as physical slots: entry p of the tile is particle
-// tslot[p] (the force kernels gather positions from HBM through it, so the
-// tile costs 4 B of LDS per entry and many workgroups share a CU).
-// Images of each local: every ghost's chain of sources ends at its root
-// local; a root gets a slot per image (order irrelevant: positions are
-// written to the next buffer from values of the current one).
-__device__ __forceinline__ void k_img_build_body(int *__restrict__ counters, const int *__restrict__ sync_src,
-                                                   const int *__restrict__ sync_mult, int *__restrict__ img_cnt,
-                                                   int4 *__restrict__ img_tab, int cap) {
-    if (counters[C_OVF]) return;
-    const int nlocal = counters[C_NLOCAL], ng = counters[C_NGHOST];
-    for (int q = blockIdx.x * 256 + threadIdx.x; q < ng; q += gridDim.x * 256) {
-        int root = sync_src[q];
-        for (int hop = 0; root >= nlocal && hop < 64; hop++) root = sync_src[root - nlocal];
-        if (root >= nlocal) { atomicMax(&counters[C_IMG_OVF], 1); continue; }
-        const int k = atomicAdd(&img_cnt[root], 1);
-        if (k < IMG_MAX) {
-            const int src = sync_src[q];
-            const int m = (sync_mult[3 * q] + 1) | (sync_mult[3 * q + 1] + 1) << 2 | (sync_mult[3 * q + 2] + 1) << 4;
-            img_tab[(size_t) k * cap + root] = make_int4(q, src == root ? -1 : src, m, 0);
-        }
-        else atomicMax(&counters[C_IMG_OVF], 1);
+        A.vx[p] = A.avx[p]; A.vy[p] = A.avy[p]; A.vz[p] = A.avz[p]; A.mass[p] = A.amass[p];
+        const int t = A.atype[p];
+        A.type[p] = t; A.flags[p] = A.aflags[p]; A.uid[p] = A.auid[p]; A.shape[p] = A.ashape[p];
+        const int r = A.aref[p];
+        A.ref[p] = r; A.cell[p] = A.acell[p];
+        if (A.P) A.P[p] = make_double4(A.X[p], A.Y[p], A.Z[p], type_w(t));
+        if (p < nlocal) continue;
+        const int q = p - nlocal, g = r - nlocal;
+        int from = A.send_map[g];
+        const int src = A.phys[from];
+        const int m0 = A.send_mult[3 * g + 0], m1 = A.send_mult[3 * g + 1], m2 = A.send_mult[3 * g + 2];
+        A.sync_src[q] = src;
+        A.sync_mult[3 * q + 0] = m0; A.sync_mult[3 * q + 1] = m1; A.sync_mult[3 * q + 2] = m2;
+        for (int hop = 0; from >= nlocal && hop < 64; hop++) from = A.send_map[from - nlocal];
+        if (from >= nlocal) { atomicMax(&A.counters[C_IMG_OVF], 1); continue; }
+        const int root = A.phys[from];
+        const int k = atomicAdd(&A.img_cnt[root], 1);
+        if (k < IMG_MAX)
+            A.img_tab[(size_t) k * A.cap + root] =
+                make_int4(q, src == root ? -1 : src, (m0 + 1) | (m1 + 1) << 2 | (m2 + 1) << 4, 0);
+        else atomicMax(&A.counters[C_IMG_OVF], 1);
     }
 }
 
-__global__ __launch_bounds__(256) void k_img_build(int *__restrict__ counters, const int *__restrict__ sync_src,
-                                                   const int *__restrict__ sync_mult, int *__restrict__ img_cnt,
-                                                   int4 *__restrict__ img_tab, int cap) {
-    k_img_build_body(counters, sync_src, sync_mult, img_cnt, img_tab, cap);
-}
+__global__ __launch_bounds__(256) void k_copy_back(CopyBackArgs A) { k_copy_back_body(A); }
 
+// o: the position buffer that holds the permuted particles
+__host__ __device__ __forceinline__ CopyBackArgs copy_back_args(const DevState &d, int o, double4 *P) {
+    return {d.counters, d.alt_vx, d.alt_vy, d.alt_vz, d.alt_mass, d.alt_type, d.alt_flags, d.alt_uid, d.alt_shape,
+            d.alt_ref, d.alt_cell, d.vx, d.vy, d.vz, d.mass, d.type, d.flags, d.uid, d.shape, d.ref,
+            d.particle_cell, d.phys, d.send_map, d.send_mult, d.sync_src, d.sync_mult, d.img_cnt, d.img_tab, d.cap,
+            d.X[o], d.Y[o], d.Z[o], P};
+}
 
 // ---------------------------------------------------------------- neighbour lists
 
@@ -2676,7 +2643,7 @@ void launch_gather_counters(hipStream_t s, const int *const *src, int n, int *ds
 static int tile_grid(int cap) { return max(1, min((cap + 255) / 256, 2048)); }
 
 // (the cell counts are zero on entry: allocated zeroed, cleared by every scan)
-void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g) {
+void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g, bool pack) {
     const int grid = tile_grid(d.cap);
     const int c = d.cur, o = 1 - d.cur;
     hipLaunchKernelGGL(k_bin_count, dim3(grid), dim3(256), 0, s, d.X[c], d.Y[c], d.Z[c], d.flags, d.counters, g,
@@ -2685,19 +2652,9 @@ void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g) {
                        g.ncells);
     hipLaunchKernelGGL(k_bin_scatter, dim3(grid), dim3(256), 0, s, d.counters, d.particle_cell, d.slot, d.lstart,
                        d.gstart, d.perm);
-    hipLaunchKernelGGL(k_sort_cells, dim3((2 * g.ncells + 3) / 4), dim3(256), 0, s, d.counters, d.lstart, d.gstart,
-                       d.ref, d.perm, g.ncells);
-    hipLaunchKernelGGL(k_permute, dim3(grid), dim3(256), 0, s, d.counters, d.perm, d.X[c], d.Y[c], d.Z[c], d.X[o],
-                       d.Y[o], d.Z[o], d.vx, d.vy, d.vz, d.mass, d.type, d.flags, d.uid, d.shape, d.ref,
-                       d.particle_cell, d.alt_vx, d.alt_vy, d.alt_vz, d.alt_mass, d.alt_type, d.alt_flags,
-                       d.alt_uid, d.alt_shape, d.alt_ref, d.alt_cell, d.phys);
+    hipLaunchKernelGGL(k_order, dim3((2 * g.ncells + 3) / 4), dim3(256), 0, s, order_args(d, g, c));
     d.cur = o;
-    hipLaunchKernelGGL(k_copy_back_maps, dim3(grid), dim3(256), 0, s, d.counters, d.alt_vx, d.alt_vy, d.alt_vz,
-                       d.alt_mass, d.alt_type, d.alt_flags, d.alt_uid, d.alt_shape, d.alt_ref, d.alt_cell, d.vx,
-                       d.vy, d.vz, d.mass, d.type, d.flags, d.uid, d.shape, d.ref, d.particle_cell, d.phys,
-                       d.send_map, d.send_mult, d.sync_src, d.sync_mult, d.img_cnt);
-    hipLaunchKernelGGL(k_img_build, dim3(grid), dim3(256), 0, s, d.counters, d.sync_src, d.sync_mult, d.img_cnt, d.img_tab,
-                       d.cap);
+    hipLaunchKernelGGL(k_copy_back, dim3(grid), dim3(256), 0, s, copy_back_args(d, o, pack ? d.P[o] : nullptr));
 }
 
 // ---------------------------------------------------------------- batched cell phase
@@ -2776,31 +2733,15 @@ __global__ __launch_bounds__(256) void k_bin_scatter_batch(const RepDesc *__rest
     k_bin_scatter_body(d.counters, d.particle_cell, d.slot, d.lstart, d.gstart, d.perm);
 }
 
-__global__ __launch_bounds__(256) void k_sort_cells_batch(const RepDesc *__restrict__ D) {
+__global__ __launch_bounds__(256) void k_order_batch(const RepDesc *__restrict__ D) {
     REP_ARGS;
-    for (int item = blockIdx.x * 4 + (threadIdx.x >> 6); item < 2 * g.ncells; item += gridDim.x * 4)
-        k_sort_cells_body(d.counters, d.lstart, d.gstart, d.ref, d.perm, g.ncells, item);
+    const OrderArgs A = order_args(d, g, c);
+    for (int item = blockIdx.x * 4 + (threadIdx.x >> 6); item < 2 * g.ncells; item += gridDim.x * 4) k_order_body(A, item);
 }
 
-__global__ __launch_bounds__(256) void k_permute_batch(const RepDesc *__restrict__ D) {
+__global__ __launch_bounds__(256) void k_copy_back_batch(const RepDesc *__restrict__ D) {
     REP_ARGS;
-    const int o = 1 - c;
-    k_permute_body(d.counters, d.perm, d.X[c], d.Y[c], d.Z[c], d.X[o], d.Y[o], d.Z[o], d.vx, d.vy, d.vz, d.mass,
-                   d.type, d.flags, d.uid, d.shape, d.ref, d.particle_cell, d.alt_vx, d.alt_vy, d.alt_vz, d.alt_mass,
-                   d.alt_type, d.alt_flags, d.alt_uid, d.alt_shape, d.alt_ref, d.alt_cell, d.phys);
-}
-
-__global__ __launch_bounds__(256) void k_copy_back_maps_batch(const RepDesc *__restrict__ D) {
-    REP_ARGS;
-    k_copy_back_maps_body(d.counters, d.alt_vx, d.alt_vy, d.alt_vz, d.alt_mass, d.alt_type, d.alt_flags, d.alt_uid,
-                          d.alt_shape, d.alt_ref, d.alt_cell, d.vx, d.vy, d.vz, d.mass, d.type, d.flags, d.uid,
-                          d.shape, d.ref, d.particle_cell, d.phys, d.send_map, d.send_mult, d.sync_src, d.sync_mult,
-                          d.img_cnt);
-}
-
-__global__ __launch_bounds__(256) void k_img_build_batch(const RepDesc *__restrict__ D) {
-    REP_ARGS;
-    k_img_build_body(d.counters, d.sync_src, d.sync_mult, d.img_cnt, d.img_tab, d.cap);
+    k_copy_back_body(copy_back_args(d, 1 - c, nullptr));
 }
 
 #undef REP_ARGS
@@ -2829,10 +2770,8 @@ void launch_cells_batch(hipStream_t s, const RepDesc *D, int n, int max_cap, int
     hipLaunchKernelGGL(k_bin_count_batch, tiles, dim3(256), 0, s, D);
     hipLaunchKernelGGL(k_scan_cells_batch, one, dim3(1024), 0, s, D);
     hipLaunchKernelGGL(k_bin_scatter_batch, tiles, dim3(256), 0, s, D);
-    hipLaunchKernelGGL(k_sort_cells_batch, cells, dim3(256), 0, s, D);
-    hipLaunchKernelGGL(k_permute_batch, tiles, dim3(256), 0, s, D);
-    hipLaunchKernelGGL(k_copy_back_maps_batch, tiles, dim3(256), 0, s, D);
-    hipLaunchKernelGGL(k_img_build_batch, tiles, dim3(256), 0, s, D);
+    hipLaunchKernelGGL(k_order_batch, cells, dim3(256), 0, s, D);
+    hipLaunchKernelGGL(k_copy_back_batch, tiles, dim3(256), 0, s, D);
 }
 
 int build_zt(const Geom &g) { return g.nchunks == 1 ? g.dim_cells[2] + 2 : g.zc + 3; }

@@ -193,7 +193,8 @@ void launch_exchange(hipStream_t s, const DevState &d, const Geom &g, const int 
 void launch_borders(hipStream_t s, const DevState &d, const Geom &g, const int *periodic);
 // bins locals and ghosts into cells and permutes every particle array into
 // cell order (swapping d's spare arrays in), then builds the ghost sync maps
-void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g);
+// (pack: and the packed copy of the new positions)
+void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g, bool pack = false);
 void launch_build_neighbors(hipStream_t s, const DevState &d, const Geom &g, int half, double rc2);
 // largest tile (entries) the build and force kernels can stage in LDS
 int build_tile_limit(const DevState &d, const Geom &g, int half);

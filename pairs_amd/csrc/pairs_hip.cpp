@@ -1008,12 +1008,12 @@ static inline bool every(int ts, int n) { return n > 0 && (((ts + 1) % n) == 0 |
 static void enqueue_rebuild(pairs_hip_ctx *ctx, hipStream_t s) {
     launch_exchange(s, ctx->d, ctx->geom, ctx->cfg.periodic);
     launch_borders(s, ctx->d, ctx->geom, ctx->cfg.periodic);
-    launch_bin_sort(s, ctx->d, ctx->geom);  // flips d.cur; clears the image and tile flags
+    // flips d.cur; clears the image and tile flags; the packed copy is for the
+    // force step behind the rebuild
+    launch_bin_sort(s, ctx->d, ctx->geom, true);
     // the neighbour build runs right behind the cell phase; every rebuild kernel
     // returns at once when an earlier one has set an overflow
     enqueue_build(ctx, s, false);
-    // the packed (x, y, z) copy of the new buffer, for the force step after it
-    launch_pack_p(s, ctx->d, ctx->d.cur);
 }
 
 // The rebuild's ~37 small kernels have grids that depend only on
