@@ -525,9 +525,10 @@ static void enqueue_step(pairs_hip_dem_ctx *ctx, bool timed) {
     if (timed) hipEventRecord(ctx->ev[1], ctx->stream);
     launch_contacts(ctx->stream, ctx->p, ctx->counters, ctx->nlocal, ctx->geom, ctx->prm,
                     timed ? ctx->ev + 2 : nullptr);
-    if (timed) hipEventRecord(ctx->ev[5], ctx->stream);
+    if (!timed) return;  // integrated by the contact kernel
+    hipEventRecord(ctx->ev[5], ctx->stream);
     launch_euler(ctx->stream, ctx->p, ctx->counters, ctx->geom, ctx->prm);
-    if (timed) hipEventRecord(ctx->ev[6], ctx->stream);
+    hipEventRecord(ctx->ev[6], ctx->stream);
 }
 
 static int ensure_graph(pairs_hip_dem_ctx *ctx) {

@@ -725,6 +725,75 @@ __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__rest
     }
 }
 
+// ---------------------------------------------------------------- integration
+
+// euler (examples/dem.py:77-85) of particle i under force f and torque tq, with
+// quaternion(phi, |phi|) and quaternion_to_rotation_matrix
+// (src/pairs/mapping/keywords.py:190-252); a particle it moves out of the box is
+// noted for the next exchange
+__device__ __forceinline__ void euler_particle(const DemPtrs &p, int *__restrict__ c, const DemGeom &g, double dt,
+                                               int i, int fl, const double (&f)[3], const double (&tq)[3]) {
+    if (fl & DFLAG_FIXED) {
+        note_leaver(p, c, g, i, fl, p.x[i], p.y[i], p.z[i]);
+        return;
+    }
+    const size_t C = p.cap;
+    const double im = 1.0 / p.m[i];
+    const double hm = 0.5 * im;
+    double x[3] = {p.x[i], p.y[i], p.z[i]}, v[3] = {p.vx[i], p.vy[i], p.vz[i]}, w[3] = {p.wx[i], p.wy[i], p.wz[i]};
+    for (int d = 0; d < 3; d++) x[d] = x[d] + (((hm * f[d]) * dt) * dt + v[d] * dt);
+    for (int d = 0; d < 3; d++) v[d] = v[d] + (im * f[d]) * dt;
+    double I[9], R[9], q[4];
+    for (int k = 0; k < 9; k++) { I[k] = p.inv_i[k * C + i]; R[k] = p.rot_m[k * C + i]; }
+    for (int k = 0; k < 4; k++) q[k] = p.rot_q[k * C + i];
+    double a[3], b[3], wd[3];
+    for (int r = 0; r < 3; r++) a[r] = (I[3 * r] * tq[0] + I[3 * r + 1] * tq[1]) + I[3 * r + 2] * tq[2];
+    for (int r = 0; r < 3; r++) b[r] = (R[3 * r] * a[0] + R[3 * r + 1] * a[1]) + R[3 * r + 2] * a[2];
+    for (int cc = 0; cc < 3; cc++) wd[cc] = (b[0] * R[cc] + b[1] * R[3 + cc]) + b[2] * R[6 + cc];
+    double phi[3];
+    for (int d = 0; d < 3; d++) phi[d] = w[d] * dt + ((0.5 * wd[d]) * dt) * dt;
+    const double plen = sqrt((phi[0] * phi[0] + phi[1] * phi[1]) + phi[2] * phi[2]);
+    double dq[4];
+    if (fabs(plen) < 1e-06) {
+        dq[0] = 1.0; dq[1] = 0.0; dq[2] = 0.0; dq[3] = 0.0;
+    } else {
+        const double cs = cos(plen * 0.5), sn = sin(plen * 0.5), inv = 1.0 / plen;
+        dq[0] = cs;
+        for (int d = 0; d < 3; d++) dq[1 + d] = sn * (phi[d] * inv);
+    }
+    const double p0 = ((dq[0] * q[0] - dq[1] * q[1]) - dq[2] * q[2]) - dq[3] * q[3];
+    const double p1 = ((dq[0] * q[1] + dq[1] * q[0]) + dq[2] * q[3]) - dq[3] * q[2];
+    const double p2 = ((dq[0] * q[2] + dq[2] * q[0]) + dq[3] * q[1]) - dq[1] * q[3];
+    const double p3 = ((dq[0] * q[3] + dq[3] * q[0]) + dq[1] * q[2]) - dq[2] * q[1];
+    const double n2 = ((p0 * p0 + p1 * p1) + p2 * p2) + p3 * p3;
+    const double sc = (fabs(n2 - 1.0) < 1e-08) ? 1.0 : 1.0 / sqrt(n2);
+    q[0] = p0 * sc; q[1] = p1 * sc; q[2] = p2 * sc; q[3] = p3 * sc;
+    R[0] = (1.0 - (2.0 * q[2]) * q[2]) - (2.0 * q[3]) * q[3];
+    R[1] = 2.0 * (q[1] * q[2] - q[0] * q[3]);
+    R[2] = 2.0 * (q[1] * q[3] + q[0] * q[2]);
+    R[3] = 2.0 * (q[1] * q[2] + q[0] * q[3]);
+    R[4] = (1.0 - (2.0 * q[1]) * q[1]) - (2.0 * q[3]) * q[3];
+    R[5] = 2.0 * (q[2] * q[3] - q[0] * q[1]);
+    R[6] = 2.0 * (q[1] * q[3] - q[0] * q[2]);
+    R[7] = 2.0 * (q[2] * q[3] + q[0] * q[1]);
+    R[8] = (1.0 - (2.0 * q[1]) * q[1]) - (2.0 * q[2]) * q[2];
+    for (int d = 0; d < 3; d++) w[d] = w[d] + wd[d] * dt;
+    note_leaver(p, c, g, i, fl, x[0], x[1], x[2]);
+    p.x[i] = x[0]; p.y[i] = x[1]; p.z[i] = x[2];
+    p.vx[i] = v[0]; p.vy[i] = v[1]; p.vz[i] = v[2];
+    p.wx[i] = w[0]; p.wy[i] = w[1]; p.wz[i] = w[2];
+    for (int k = 0; k < 9; k++) p.rot_m[k * C + i] = R[k];
+    for (int k = 0; k < 4; k++) p.rot_q[k * C + i] = q[k];
+}
+
+__global__ __launch_bounds__(256) void k_euler(DemPtrs p, int *__restrict__ c, DemGeom g, double dt) {
+    const int nl = c[D_NLOCAL];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= nl || c[D_OVF]) return;
+    const double f[3] = {p.fx[i], p.fy[i], p.fz[i]}, tq[3] = {p.tx[i], p.ty[i], p.tz[i]};
+    euler_particle(p, c, g, dt, i, p.flags[i], f, tq);
+}
+
 // ---------------------------------------------------------------- contacts
 
 struct Acc3 { double x, y, z; };
@@ -1042,7 +1111,9 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
 //     terms through LDS; the particle's lane adds them in contact order, with
 //     the reference's sphere / half-space grouping (force += sphere + plane
 //     sums, torque += plane + sphere sums) on top of gravity;
-//  3. clear_unused_contact_history from the particle's mask of used slots.
+//  3. clear_unused_contact_history from the particle's mask of used slots;
+//  4. EULER: the particle integrated (nothing here reads another particle's
+//     position but from the records made before).
 // A particle with more than DCAND touching partners, more history than the
 // mask holds, or two contacts in one slot (a partner and its image) walks its
 // cells in its lane instead, one contact after the other, as the reference.
@@ -1051,8 +1122,9 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
 // dense pass in place of a kernel per phase: the phases ran one thread per
 // possible contact (16 per particle) or per particle, and gathered a partner
 // from twelve arrays: 134 -> 53 us in that bed, 29 -> 11 us at 2080 spheres;
-// eight history slots compared at a time 53 -> 48.
-template <int SPW>
+// eight history slots compared at a time 53 -> 48.  With the integration 60,
+// for 48 and 18 us apart; 12.0 for 10.8 and 4.3 at 2080 spheres.
+template <int SPW, bool EULER>
 __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict__ c, DemGeom g, DemParams prm) {
     __shared__ double s_term[64][7];
     __shared__ int s_kind[64];
@@ -1167,7 +1239,8 @@ __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict
         for (int k = 0; k < nc0; k++) p.c_used[k * C + i] = 0;
         p.num_contacts[i] = nc0;
     }
-    if (!(p.flags[i] & DFLAG_FIXED)) {
+    const int fl = p.flags[i];
+    if (!(fl & DFLAG_FIXED)) {
         // gravity (examples/dem.py:88-90)
         const double ri = p.r[i];
         const double vol = (((4.0 / 3.0) * prm.pi) * ri * ri) * ri;
@@ -1214,70 +1287,10 @@ __global__ __launch_bounds__(64) void k_contact_solve(DemPtrs p, int *__restrict
         }
     }
     p.num_contacts[i] = nc;
-}
-
-// ---------------------------------------------------------------- integration
-
-// euler (examples/dem.py:77-85) with quaternion(phi, |phi|) and
-// quaternion_to_rotation_matrix (src/pairs/mapping/keywords.py:190-252); the
-// particles it moves out of the box are noted for the next exchange
-__global__ __launch_bounds__(256) void k_euler(DemPtrs p, int *__restrict__ c, DemGeom g, double dt) {
-    const int nl = c[D_NLOCAL];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= nl || c[D_OVF]) return;
-    const int fl = p.flags[i];
-    if (fl & DFLAG_FIXED) {
-        note_leaver(p, c, g, i, fl, p.x[i], p.y[i], p.z[i]);
-        return;
+    if (EULER) {
+        const double f[3] = {f0, f1, f2}, tq[3] = {t0, t1, t2};
+        euler_particle(p, c, g, prm.dt, i, fl, f, tq);
     }
-    const size_t C = p.cap;
-    const double im = 1.0 / p.m[i];
-    const double hm = 0.5 * im;
-    const double f[3] = {p.fx[i], p.fy[i], p.fz[i]}, tq[3] = {p.tx[i], p.ty[i], p.tz[i]};
-    double x[3] = {p.x[i], p.y[i], p.z[i]}, v[3] = {p.vx[i], p.vy[i], p.vz[i]}, w[3] = {p.wx[i], p.wy[i], p.wz[i]};
-    for (int d = 0; d < 3; d++) x[d] = x[d] + (((hm * f[d]) * dt) * dt + v[d] * dt);
-    for (int d = 0; d < 3; d++) v[d] = v[d] + (im * f[d]) * dt;
-    double I[9], R[9], q[4];
-    for (int k = 0; k < 9; k++) { I[k] = p.inv_i[k * C + i]; R[k] = p.rot_m[k * C + i]; }
-    for (int k = 0; k < 4; k++) q[k] = p.rot_q[k * C + i];
-    double a[3], b[3], wd[3];
-    for (int r = 0; r < 3; r++) a[r] = (I[3 * r] * tq[0] + I[3 * r + 1] * tq[1]) + I[3 * r + 2] * tq[2];
-    for (int r = 0; r < 3; r++) b[r] = (R[3 * r] * a[0] + R[3 * r + 1] * a[1]) + R[3 * r + 2] * a[2];
-    for (int cc = 0; cc < 3; cc++) wd[cc] = (b[0] * R[cc] + b[1] * R[3 + cc]) + b[2] * R[6 + cc];
-    double phi[3];
-    for (int d = 0; d < 3; d++) phi[d] = w[d] * dt + ((0.5 * wd[d]) * dt) * dt;
-    const double plen = sqrt((phi[0] * phi[0] + phi[1] * phi[1]) + phi[2] * phi[2]);
-    double dq[4];
-    if (fabs(plen) < 1e-06) {
-        dq[0] = 1.0; dq[1] = 0.0; dq[2] = 0.0; dq[3] = 0.0;
-    } else {
-        const double cs = cos(plen * 0.5), sn = sin(plen * 0.5), inv = 1.0 / plen;
-        dq[0] = cs;
-        for (int d = 0; d < 3; d++) dq[1 + d] = sn * (phi[d] * inv);
-    }
-    const double p0 = ((dq[0] * q[0] - dq[1] * q[1]) - dq[2] * q[2]) - dq[3] * q[3];
-    const double p1 = ((dq[0] * q[1] + dq[1] * q[0]) + dq[2] * q[3]) - dq[3] * q[2];
-    const double p2 = ((dq[0] * q[2] + dq[2] * q[0]) + dq[3] * q[1]) - dq[1] * q[3];
-    const double p3 = ((dq[0] * q[3] + dq[3] * q[0]) + dq[1] * q[2]) - dq[2] * q[1];
-    const double n2 = ((p0 * p0 + p1 * p1) + p2 * p2) + p3 * p3;
-    const double sc = (fabs(n2 - 1.0) < 1e-08) ? 1.0 : 1.0 / sqrt(n2);
-    q[0] = p0 * sc; q[1] = p1 * sc; q[2] = p2 * sc; q[3] = p3 * sc;
-    R[0] = (1.0 - (2.0 * q[2]) * q[2]) - (2.0 * q[3]) * q[3];
-    R[1] = 2.0 * (q[1] * q[2] - q[0] * q[3]);
-    R[2] = 2.0 * (q[1] * q[3] + q[0] * q[2]);
-    R[3] = 2.0 * (q[1] * q[2] + q[0] * q[3]);
-    R[4] = (1.0 - (2.0 * q[1]) * q[1]) - (2.0 * q[3]) * q[3];
-    R[5] = 2.0 * (q[2] * q[3] - q[0] * q[1]);
-    R[6] = 2.0 * (q[1] * q[3] - q[0] * q[2]);
-    R[7] = 2.0 * (q[2] * q[3] + q[0] * q[1]);
-    R[8] = (1.0 - (2.0 * q[1]) * q[1]) - (2.0 * q[2]) * q[2];
-    for (int d = 0; d < 3; d++) w[d] = w[d] + wd[d] * dt;
-    note_leaver(p, c, g, i, fl, x[0], x[1], x[2]);
-    p.x[i] = x[0]; p.y[i] = x[1]; p.z[i] = x[2];
-    p.vx[i] = v[0]; p.vy[i] = v[1]; p.vz[i] = v[2];
-    p.wx[i] = w[0]; p.wy[i] = w[1]; p.wz[i] = w[2];
-    for (int k = 0; k < 9; k++) p.rot_m[k * C + i] = R[k];
-    for (int k = 0; k < 4; k++) p.rot_q[k * C + i] = q[k];
 }
 
 // update_mass_and_inertia (examples/dem.py:6-15)
@@ -1355,18 +1368,26 @@ void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g) {
     hipLaunchKernelGGL(k_cell_order, dim3(pg), dim3(256), 0, s, p, c);
 }
 
-// forces + history bookkeeping, then integration
-void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
-                     const hipEvent_t *between) {
-    hipLaunchKernelGGL(k_contact_find, dim3(grid_of(p.cap, 256 / LPS)), dim3(256), 0, s, p, c, g);
-    if (between) { hipEventRecord(between[0], s); hipEventRecord(between[1], s); }
+template <bool EULER>
+static void launch_solve(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm) {
     // particles per wave: a wave's chain of look-ups is shorter with fewer (a
     // small system is one wave of the chip long), its lanes fuller with more:
     // beds of 2080 / 9600 / 39200 / 187200 spheres, ms a pass on 8, 16, 32:
     // 16.1 16.8 17.8 / 4.58 4.76 4.99 / 6.41 6.24 6.45 / 28.8 27.3 26.4
-    if (nlocal < 16384) hipLaunchKernelGGL(k_contact_solve<8>, dim3(grid_of(nlocal, 8)), dim3(64), 0, s, p, c, g, prm);
-    else if (nlocal < 65536) hipLaunchKernelGGL(k_contact_solve<16>, dim3(grid_of(nlocal, 16)), dim3(64), 0, s, p, c, g, prm);
-    else hipLaunchKernelGGL(k_contact_solve<32>, dim3(grid_of(nlocal, 32)), dim3(64), 0, s, p, c, g, prm);
+    const int spw = nlocal < 16384 ? 8 : nlocal < 65536 ? 16 : 32;
+    const dim3 grid(grid_of(nlocal, spw));
+    if (spw == 8) hipLaunchKernelGGL((k_contact_solve<8, EULER>), grid, dim3(64), 0, s, p, c, g, prm);
+    else if (spw == 16) hipLaunchKernelGGL((k_contact_solve<16, EULER>), grid, dim3(64), 0, s, p, c, g, prm);
+    else hipLaunchKernelGGL((k_contact_solve<32, EULER>), grid, dim3(64), 0, s, p, c, g, prm);
+}
+
+// forces, history bookkeeping and integration
+void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
+                     const hipEvent_t *between) {
+    hipLaunchKernelGGL(k_contact_find, dim3(grid_of(p.cap, 256 / LPS)), dim3(256), 0, s, p, c, g);
+    if (between) { hipEventRecord(between[0], s); hipEventRecord(between[1], s); }
+    if (between) launch_solve<false>(s, p, c, nlocal, g, prm);
+    else launch_solve<true>(s, p, c, nlocal, g, prm);
     if (between) hipEventRecord(between[2], s);
 }
 
