@@ -2181,15 +2181,15 @@ __global__ __launch_bounds__(256) void k_find_leavers(const double *__restrict__
     if (k < LEAVE_CAP) leavers[k] = p;
 }
 
-// The exchange of all periodic dimensions in one workgroup, a leaver per
-// thread.  A particle keeps its physical slot; what moves is its reference
-// index.  Per dimension the leavers are ranked by side and reference index (the
-// reference's send order), the tail walk is planned with two scans, and the
-// relabeling is that of k_exchange_relabel_body.  More leavers than the list
+// The exchange of all periodic dimensions in one workgroup.  A particle keeps
+// its physical slot; what moves is its reference index.  Per dimension the
+// leavers among those listed are collected and ranked by side and reference
+// index (the reference's send order), the tail walk is planned with two scans,
+// and the relabeling is that of k_exchange_relabel_body.  More leavers than the list
 // holds are found by a scan of the locals in reference order instead.  Bound by
 // the latency of its phases; with k_find_leavers it takes the place of three
 // kernels per dimension (us per rebuild: 256 atoms 27 -> 12, 131072 45 ->
-// 35).  Beyond some 200000 locals the leavers of a rebuild no longer fit
+// 25; a lattice start, where 3072 leave at once, 1.82 -> 1.70 ms for 25 steps).  Beyond some 200000 locals the leavers of a rebuild no longer fit
 // and the three kernels remain (exch_listed).
 __global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, double *__restrict__ Y,
                                                    double *__restrict__ Z, const int *__restrict__ flags,
@@ -2198,31 +2198,39 @@ __global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, doubl
                                                    const int *__restrict__ leavers, int *__restrict__ send_map,
                                                    int *__restrict__ send_mult, int *__restrict__ exchg_flag,
                                                    int *__restrict__ scratch, int send_cap) {
-    __shared__ int lds[20];
+    constexpr int PER = LEAVE_CAP / 1024;
+    constexpr unsigned SIDE1 = 0x80000000u;
+    __shared__ int lds[20], s_n[2];
     __shared__ __align__(16) unsigned s_key[LEAVE_CAP];
-    __shared__ int s_map[LEAVE_CAP], s_fill[LEAVE_CAP], s_hole[LEAVE_CAP], s_tail[LEAVE_CAP];
+    __shared__ unsigned s_map[LEAVE_CAP];
+    __shared__ int s_fill[LEAVE_CAP], s_hole[LEAVE_CAP];
+    __shared__ unsigned char s_tail[LEAVE_CAP];
     const int tid = threadIdx.x, cnt = counters[C_LEAVE], nl = counters[C_NLOCAL], ovf = counters[C_OVF];
     __syncthreads();
     if (tid == 0) { counters[C_LEAVE] = 0; counters[C_LEAVE_MAX] = cnt; }
     if (ovf) return;
     const bool listed = cnt <= LEAVE_CAP;
-    const int me = listed && tid < cnt ? leavers[tid] : -1;
     const int periodic[3] = {px, py, pz};
 #pragma unroll
     for (int dim = 0; dim < 3; dim++) {
         if (!periodic[dim]) continue;
         const double *Xd = dim == 0 ? X : (dim == 1 ? Y : Z);
-        int n0 = 0, n1 = 0, r = -1;
-        bool a = false, b = false;
+        int n0 = 0, n1 = 0;
         if (listed) {
-            if (me >= 0) {
-                r = ref[me];
-                ghost_sel(Xd[me], flags[me], dim, g, true, a, b);
+            // the dimension's leavers among those listed, in any order
+            if (tid < 2) s_n[tid] = 0;
+            __syncthreads();
+            for (int c = tid; c < cnt; c += 1024) {
+                const int p = leavers[c];
+                bool a, b;
+                ghost_sel(Xd[p], flags[p], dim, g, true, a, b);
+                if (!(a || b)) continue;
+                s_key[atomicAdd(&s_n[0], 1)] = (unsigned) ref[p] | (a ? 0u : SIDE1);
+                if (!a) atomicAdd(&s_n[1], 1);
             }
-            s_key[tid] = a ? (unsigned) r : b ? (unsigned) r | 0x80000000u : 0xffffffffu;
-            s_tail[tid] = 0;
-            n0 = __syncthreads_count(a);
-            n1 = __syncthreads_count(b);
+            __syncthreads();
+            n1 = s_n[1];
+            n0 = s_n[0] - n1;
         } else {
             for (int i0 = 0; i0 < nl; i0 += 1024) {
                 const int i = i0 + tid;
@@ -2249,7 +2257,10 @@ __global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, doubl
             counters[C_NSEND + 2 * dim + 1] = n1;
             counters[C_NSEND_ALL] = n;
         }
-        if (n == 0) continue;
+        if (n == 0) {
+            __syncthreads();
+            continue;
+        }
         auto send = [&](int pos, int idx, int side) {
             const int mult = side == 0 ? 1 : -1;  // pbc_prev = +1, pbc_next = -1 on one rank
             send_map[pos] = idx;
@@ -2258,40 +2269,62 @@ __global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, doubl
             send_mult[3 * pos + 2] = dim == 2 ? mult : 0;
         };
         if (listed) {
-            const unsigned key = s_key[tid];
-            int rank = 0;
-            if (__ballot(a || b)) {  // (the entries past cnt are the largest key)
+            if (tid < 3 && n + tid < LEAVE_CAP) s_key[n + tid] = 0xffffffffu;  // to whole reads of four
+            for (int t = tid; t < n; t += 1024) s_tail[t] = 0;
+            __syncthreads();
+            for (int t = tid; t < n; t += 1024) {
+                const unsigned key = s_key[t];
                 const uint4 *k4 = (const uint4 *) s_key;
+                int rank = 0;
 #pragma unroll 4
-                for (int u = 0; u < (cnt + 3) / 4; u++) {
+                for (int u = 0; u < (n + 3) / 4; u++) {
                     const uint4 k = k4[u];
                     rank += (k.x < key ? 1 : 0) + (k.y < key ? 1 : 0) + (k.z < key ? 1 : 0) + (k.w < key ? 1 : 0);
                 }
-            }
-            if (a || b) {
-                s_map[rank] = r;
-                send(rank, r, a ? 0 : 1);
+                const int r = (int) (key & ~SIDE1);
+                s_map[rank] = key;
+                send(rank, r, key & SIDE1 ? 1 : 0);
                 if (r >= nl - n) s_tail[nl - 1 - r] = 1;
             }
             __syncthreads();
-            int fills_all, holes;
-            const bool fills = tid < n && !s_tail[tid], hole = tid < n && s_map[tid] < nl - n;
-            const int ef = block_exclusive_scan<1024>(fills ? 1 : 0, lds, &fills_all);
-            const int eh = block_exclusive_scan<1024>(hole ? 1 : 0, lds, &holes);
-            if (fills) s_fill[ef] = nl - 1 - tid;
-            if (hole) s_hole[eh] = s_map[tid];
+            // the tail that fills, and the holes, in order
+            int nfill = 0, nhole = 0;
+            for (int t0 = 0; t0 < n; t0 += 1024) {
+                const int t = t0 + tid;
+                const int r = t < n ? (int) (s_map[t] & ~SIDE1) : 0;
+                const bool fills = t < n && !s_tail[t], hole = t < n && r < nl - n;
+                int tf, th;
+                const int ef = block_exclusive_scan<1024>(fills ? 1 : 0, lds, &tf);
+                const int eh = block_exclusive_scan<1024>(hole ? 1 : 0, lds, &th);
+                if (fills) s_fill[nfill + ef] = nl - 1 - t;
+                if (hole) s_hole[nhole + eh] = r;
+                nfill += tf;
+                nhole += th;
+            }
             __syncthreads();
-            const int src = tid < holes ? s_fill[tid] : -1;
-            const int ps = src > 0 ? phys[src] : -1;
+            // every slot read before the first is relabeled
+            int ps[PER], pl[PER];
+#pragma unroll
+            for (int k = 0; k < PER; k++) {
+                const int t = k * 1024 + tid;
+                const int src = t < nhole ? s_fill[t] : -1;
+                ps[k] = src > 0 ? phys[src] : -1;
+                pl[k] = t < n ? phys[s_map[t] & ~SIDE1] : -1;
+            }
             __syncthreads();
-            if (ps >= 0) { const int dst = s_hole[tid]; ref[ps] = dst; phys[dst] = ps; }
-            if (a || b) {
-                const double mult = a ? 1.0 : -1.0;
-                X[me] = X[me] + (dim == 0 ? mult : 0.0) * g.len[0];
-                Y[me] = Y[me] + (dim == 1 ? mult : 0.0) * g.len[1];
-                Z[me] = Z[me] + (dim == 2 ? mult : 0.0) * g.len[2];
-                ref[me] = nl - n + rank;
-                phys[nl - n + rank] = me;
+#pragma unroll
+            for (int k = 0; k < PER; k++) {
+                const int t = k * 1024 + tid;
+                if (ps[k] >= 0) { ref[ps[k]] = s_hole[t]; phys[s_hole[t]] = ps[k]; }
+                if (pl[k] >= 0) {
+                    const int p = pl[k];
+                    const double mult = s_map[t] & SIDE1 ? -1.0 : 1.0;
+                    X[p] = X[p] + (dim == 0 ? mult : 0.0) * g.len[0];
+                    Y[p] = Y[p] + (dim == 1 ? mult : 0.0) * g.len[1];
+                    Z[p] = Z[p] + (dim == 2 ? mult : 0.0) * g.len[2];
+                    ref[p] = nl - n + t;
+                    phys[nl - n + t] = p;
+                }
             }
         } else {
             int o0 = 0, o1 = n0;
@@ -2376,6 +2409,7 @@ struct BorderArgs {
     int *type, *uid, *shape, *flags, *ref, *phys, *counters;
     Geom g;
     int px, py, pz, pitch, send_cap, cap;
+    int share;  // workgroups per tile (a power of two)
     int *cnt;  // [kind][tile], kinds pitch apart
     int *send_map, *send_mult;
 };
@@ -2419,7 +2453,7 @@ __global__ __launch_bounds__(BORDER_T) void k_border_count(BorderArgs A) {
 // by dimension; on overflow the counts stay as they were.  Bound by latency in
 // small systems and by the ghosts' writes in large ones; with k_border_count it
 // takes the place of a count and a scatter pass per dimension (us per rebuild:
-// 256 atoms 20 -> 15, 131072 31 -> 25, 1048576 111 -> 61).
+// 256 atoms 20 -> 12, 131072 31 -> 23, 1048576 111 -> 61).
 template <int ND>
 __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
     constexpr int NK = pow3(ND), NW = BORDER_T / 64;
@@ -2427,8 +2461,9 @@ __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
     int *c = A.counters;
     if (c[C_OVF]) return;
     const int nl = c[C_NLOCAL], ntiles = (nl + BORDER_T - 1) / BORDER_T;
-    if (blockIdx.x > 0 && (int) blockIdx.x >= ntiles) return;  // workgroup 0 always writes the counts
-    const int r = blockIdx.x * BORDER_T + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (blockIdx.x > 0 && (int) blockIdx.x >= ntiles) return;  // tile 0's first workgroup always writes the counts
+    const int tile = blockIdx.x, part = blockIdx.y;
+    const int r = tile * BORDER_T + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int p = 0, fl = 0, uid = 0, type = 0, shape = 0;
     double xs[3] = {0.0, 0.0, 0.0}, m = 0.0, v[3] = {0.0, 0.0, 0.0};
     if (r < nl) {
@@ -2457,7 +2492,7 @@ __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
             const int k = 1 + wave + NW * e;
             const int x = k < NK ? A.cnt[(size_t) k * A.pitch + u] : 0;
             t[e] += x;
-            q[e] += u < (int) blockIdx.x ? x : 0;
+            q[e] += u < tile ? x : 0;
         }
     }
 #pragma unroll
@@ -2489,7 +2524,7 @@ __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
         ovf_send = need > A.send_cap;
         ovf_part = nl + need > A.cap;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (tile == 0 && part == 0 && threadIdx.x == 0) {
         if (ovf_send) {
             c[C_OVF] = OVF_SEND;
             c[C_REQ_SEND] = max(c[C_REQ_SEND], need);
@@ -2521,7 +2556,7 @@ __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
         const int pos = at + s_pre[k][wave] + lane_rank(mask);
         at += s_total[k];
         if (k < pow3(ND - 1)) to[k] = pos;
-        if (!K.has(k)) continue;
+        if ((k & (A.share - 1)) != part || !K.has(k)) continue;
         int top = 0, digits = k, mult[3] = {0, 0, 0};
 #pragma unroll
         for (int d = 0; d < ND; d++) {
@@ -2893,7 +2928,7 @@ void launch_exchange(hipStream_t s, const DevState &d, const Geom &g, const int 
 template <int ND>
 static void borders_nd(hipStream_t s, const BorderArgs &A) {
     hipLaunchKernelGGL(k_border_count<ND>, dim3(A.pitch), dim3(BORDER_T), 0, s, A);
-    hipLaunchKernelGGL(k_border_ghosts<ND>, dim3(A.pitch), dim3(BORDER_T), 0, s, A);
+    hipLaunchKernelGGL(k_border_ghosts<ND>, dim3(A.pitch, A.share), dim3(BORDER_T), 0, s, A);
 }
 
 void launch_borders(hipStream_t s, const DevState &d, const Geom &g, const int *periodic) {
@@ -2904,9 +2939,15 @@ void launch_borders(hipStream_t s, const DevState &d, const Geom &g, const int *
         launch_set_counters(s, d.counters, C_NGHOST, 8, 0);
         return;
     }
+    // few tiles leave the chip idle while each stores its particles' ghosts, kind
+    // by kind, so their kinds are shared out.  k_border_ghosts, us, one workgroup
+    // per tile | so: 256 atoms 10.8 | 7.9, 2048 15 | 9.6, 19652 17.6 | 11.4, 131072
+    // (two) 17.2 | 16.8
+    const int tiles = (d.nlocal + BORDER_T - 1) / BORDER_T, share = tiles <= 32 ? 8 : tiles <= 256 ? 2 : 1;
     const BorderArgs A = {d.X[c], d.Y[c], d.Z[c], d.vx, d.vy, d.vz, d.mass, d.type, d.uid, d.shape, d.flags, d.ref,
                           d.phys, d.counters, g, periodic[0], periodic[1], periodic[2],
-                          (d.cap + BORDER_T - 1) / BORDER_T, d.send_cap, d.cap, d.tile_cnt, d.send_map, d.send_mult};
+                          (d.cap + BORDER_T - 1) / BORDER_T, d.send_cap, d.cap, share, d.tile_cnt, d.send_map,
+                          d.send_mult};
     if (nd == 1) borders_nd<1>(s, A);
     else if (nd == 2) borders_nd<2>(s, A);
     else borders_nd<3>(s, A);

@@ -92,7 +92,7 @@ constexpr int TILE_CAP = 1088;
 
 constexpr int IMG_MAX = 8;
 // leavers that the one-workgroup exchange takes from its list
-constexpr int LEAVE_CAP = 1024;
+constexpr int LEAVE_CAP = 4096;
 // ghost kinds: per periodic dimension none, side 0 or side 1
 constexpr int MAX_KIND = 27;
 

@@ -519,9 +519,10 @@ int pairs_hip_upload(pairs_hip_ctx *ctx, int n, const double *x, const double *v
     CHECK_LAUNCH();
     HIP_OK(hipStreamSynchronize(ctx->stream));
     d.nlocal = n;
-    // the leavers of a rebuild (some 600 at 131072 locals of the LJ fluid) fit the
-    // list of the one-workgroup exchange (200 steps of 198400 atoms 15.6 ms with
-    // the wide kernels, 15.1 with the list); with 389344 atoms they do not
+    // the leavers of a rebuild (some 600 at 131072 locals of the LJ fluid, 3900 at
+    // the start of a lattice of 186624) fit the list of the one-workgroup exchange.
+    // 200 steps of 198400 atoms 15.6 ms with the wide kernels, 15.1 with the list; at
+    // 389344 no difference was measured
     d.exch_listed = n < 200000;
     ctx->nghost = 0;
     ctx->nsend_all = 0;

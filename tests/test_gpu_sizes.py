@@ -268,13 +268,14 @@ def test_dem_exchange_and_borders_vs_oracle(pairs, periodic, dom, speed):
     assert nc.max() > 0
 
 
-# exchange and borders of a rebuild: 0 to 3 periodic dimensions; leavers that fit
-# the list of the one-workgroup exchange (1024) or do not (then, from the next
-# rebuild on, the wide kernels run); a box narrower than two cell spacings; more
+# exchange and borders of a rebuild: 0 to 3 periodic dimensions; leavers that are
+# one per thread of the one-workgroup exchange (1024), several, or do not fit its
+# list (4096; then, from the next rebuild on, the wide kernels run); a box narrower than two cell spacings; more
 # than one border tile (1024 reference indices)
 @pytest.mark.parametrize("n,periodic,edge,speed", [
     (1, (1, 1, 1), 39.0, 300.0), (1023, (1, 1, 1), 21.0, 200.0), (1025, (1, 1, 1), 22.0, 200.0),
     (6000, (1, 1, 1), 39.0, 200.0), (6000, (1, 1, 1), 39.0, 2500.0), (6000, (0, 1, 1), 39.0, 3500.0),
+    (6000, (1, 1, 1), 39.0, 7000.0),
     (6000, (1, 1, 0), 39.0, 200.0), (6000, (1, 0, 1), 39.0, 200.0), (3000, (0, 1, 0), 31.0, 200.0),
     (3000, (0, 0, 1), 31.0, 200.0), (3000, (1, 0, 0), 31.0, 200.0), (3000, (0, 0, 0), 31.0, 200.0),
     (100, (1, 1, 1), 5.04, 100.0), (3000, (1, 1, 1), 100.0, 300.0)])  # (54873 cells: several rounds of the scan)
