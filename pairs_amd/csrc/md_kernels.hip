@@ -1607,6 +1607,7 @@ __global__ __launch_bounds__(TILE_G) void k_ljt(LJArgs A, TileArgs B) {
         } else {
             // eight entries at a time from memory (a local's own record past its end)
             const uint4 *from = (const uint4 *) A.nl + (size_t) (row0 >> 2) * stride + ii;
+            const uint32_t jmax = (uint32_t) max(nlocal + A.counters[C_NGHOST] - 1, 0);
             for (int k = 0; k < nmax; k += 8) {
                 uint32_t c[8];
 #pragma unroll
@@ -1618,7 +1619,7 @@ __global__ __launch_bounds__(TILE_G) void k_ljt(LJArgs A, TileArgs B) {
                 double z[8];
 #pragma unroll
                 for (int q = 0; q < 8; q++) {
-                    const size_t at = (size_t) (k + q < cnt ? c[q] : (uint32_t) ii) << 5;
+                    const size_t at = (size_t) (k + q < cnt ? min(c[q], jmax) : (uint32_t) ii) << 5;
                     xy[q] = *(const double2 *) (P + at);
                     z[q] = *(const double *) (P + at + 16);
                 }
