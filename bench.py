@@ -441,7 +441,7 @@ def main():
             "frac_of_measured_copy": (achieved / copy_gbps) if (achieved and copy_gbps) else None,
             "traffic_source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this workload, scaled by a "
                               "1 GiB device copy (profiles/lj_fcc32_force_pmc.md)",
-            "kernel": "k_lj2<1,1,false,false,true> (LJ force + final/initial integrate + next packed positions, "
+            "kernel": "k_lj2<1,1,false,true> (LJ force + final/initial integrate + next packed positions, "
                       "fused; two lanes per local, 32 locals per wave)",
             "timing": "HIP events around every 5th force launch of a separate pass of 200 steps after the timed "
                       "steps (eager launches on the context stream)",
