@@ -598,6 +598,9 @@ __global__ __launch_bounds__(1024) void k_scan_add(const int *__restrict__ in, i
 // writing of cell_start for the passes behind.
 constexpr int SCAN_LDS = 2048;
 constexpr int CELL_PLANE = (int) 0x80000000;
+// what a half-space's ordered record holds in place of its radius (a value that
+// no sphere has, also one of negative radius)
+constexpr double PLANE_MARK = -__builtin_inf();
 template <bool ADD>
 __global__ __launch_bounds__(256) void k_cell_fill(DemPtrs p, const int *__restrict__ c, int nstart, int nblk) {
     __shared__ int s_off[ADD ? SCAN_LDS : 1];
@@ -710,7 +713,7 @@ __global__ __launch_bounds__(256) void k_cell_order(DemPtrs p, const int *__rest
         }
     auto put = [&](int q, int j, int jf, double jx, double jy, double jz, double jr, int jsh) {
         p.corder[q] = make_int2(j, cell | ((jf & DFLAG_FIXED) ? (int) 0x80000000 : 0));
-        p.crec[q] = make_double4(jx, jy, jz, jsh == DSHAPE_SPHERE ? jr : -1.0);
+        p.crec[q] = make_double4(jx, jy, jz, jsh == DSHAPE_SPHERE ? jr : PLANE_MARK);
     };
     if (!mixed) {
         put(s0 + rank, i, fl, x, y, z, r, sh);
@@ -1033,7 +1036,8 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
         }
     }
     const double xi[3] = {me.x, me.y, me.z};
-    const double ri = me.w;
+    // a half-space that is not FIXED looks for partners itself, as a point of its own radius
+    const double ri = me.w == PLANE_MARK ? p.r[i] : me.w;
     const int upto = group_scan<LPS>(len[0] + len[1]);
     const int total = __shfl(upto, LPS - 1, LPS);
     const int at[2] = {upto - len[0] - len[1], upto - len[1]};  // the runs' first candidates
@@ -1042,12 +1046,12 @@ __global__ __launch_bounds__(256) void k_contact_find(DemPtrs p, const int *__re
         double nv[3], cpt[3], delta;
         const double xj[3] = {r.x, r.y, r.z};
         if (q == qi) return 0;
-        if (r.w >= 0.0) {
+        if (r.w != PLANE_MARK) {
             // sqrt(d2) - ri - rj <= 0 without the root where d2 is below (ri +
             // rj)^2 by more than 1e-12 of it (the rounding errors are 1e-15)
             const double d0 = xi[0] - xj[0], d1 = xi[1] - xj[1], d2 = xi[2] - xj[2], rs = ri + r.w;
             const double dd = (d0 * d0 + d1 * d1) + d2 * d2, rr = rs * rs;
-            if (ri >= 0.0 && rr > 1e-280 && dd < rr * (1.0 - 1e-12)) return 1;
+            if (ri >= 0.0 && r.w >= 0.0 && rr > 1e-280 && dd < rr * (1.0 - 1e-12)) return 1;
             return sphere_contact(xi, ri, xj, r.w, nv, cpt, delta) ? 1 : 0;
         }
         return plane_contact(p, xi, ri, p.corder[q].x, xj, nv, cpt, delta) ? 2 : 0;

@@ -70,8 +70,8 @@ struct DemPtrs {
     int *send_map, *send_side, *exchg_flag, *copy_to, *blk, *scan_tmp;
     double *buf, *hbuf;
     // the particles in cell order (each cell in the reference's order): index
-    // and cell (bit 31: FIXED), (x, y, z, radius; -1 for a half-space); cmixed:
-    // scratch of cells that hold a half-space
+    // and cell (bit 31: FIXED), (x, y, z, radius; a mark for a half-space);
+    // cmixed: scratch of cells that hold a half-space
     int2 *corder;
     int *cmixed;
     double4 *crec;

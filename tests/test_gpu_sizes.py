@@ -119,6 +119,40 @@ def test_dem_contacts_vs_oracle(case):
             assert np.abs(p - q).max() <= 1e-10 * max(np.abs(q).max(), 1e-300), (b, name)
 
 
+@pytest.mark.parametrize("flags", [0, 8])
+def test_dem_unfixed_halfspaces_vs_oracle(flags):
+    """half-spaces without the FIXED flag look for contacts themselves, as points
+    of radius 0; a sphere of negative radius is a sphere all the same"""
+    from pairs_amd import dem
+    uid, r, x, v, dom, planes = _spheres("walls")
+    uid, r = np.append(uid, 500), np.append(r, -0.0004)
+    x, v = np.concatenate([x, x[:1] - [0.0, 0.0, 0.0008]]), np.concatenate([v, [[0.0, 0.01, 0.0]]])
+    g = dem.DEMSystem(dom, particle_capacity=16384, contact_capacity=48)
+    o = po.OracleDEM(dom, cap=16384, ccap=48, cellcap=256)
+    g.add_spheres(uid, r, x, v)
+    for k in range(len(r)):
+        o.add_sphere(int(uid[k]), r[k], x[k], v[k])
+    for s in (g, o):
+        for u, pos, nrm, fl in planes:
+            s.add_halfspace(u, pos, nrm, flags=fl if fl == 13 else flags)
+        s.setup()
+    for a, b in ((0, 1), (1, 4), (4, 30)):
+        g.run(a, b)
+        o.run(a, b)
+        assert np.array_equal(g.get("uid"), o.get("uid")), b
+        nc, cl, sk, _, _ = g.contacts()
+        onc, ocl, osk, _, _ = o.contacts()
+        assert np.array_equal(nc, onc), b
+        for i in range(len(nc)):
+            m = nc[i]
+            assert np.array_equal(cl[i, :m], ocl[i, :m]) and np.array_equal(sk[i, :m], osk[i, :m]), (b, i)
+        if b == 1:
+            assert (nc[g.get("shape") == 1] > 0).sum() == 2 and nc[g.get("uid") == 500] > 0
+        for name, p, q in [(k, g.get(k), o.get(k)) for k in ("position", "linear_velocity", "angular_velocity",
+                                                              "force", "torque")]:
+            assert np.abs(p - q).max() <= 1e-10 * max(np.abs(q).max(), 1e-300), (b, name)
+
+
 # k_mlp_eval takes workgroups of 4 waves below 8192 rows, of 16 from there; past
 # 65536 rows a wave walks several tiles
 @pytest.mark.parametrize("n", [1, 15, 17, 8191, 8192, 8193, 65537, 131089])
