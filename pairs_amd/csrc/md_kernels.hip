@@ -1532,9 +1532,11 @@ __global__ __launch_bounds__(TILE_G) void k_ljt(LJArgs A, TileArgs B) {
     for (int k = 0; k < PER; k++)
         sl[k] = B.slots[(size_t) blockIdx.x * TILE_CAP + min(k * TILE_G + t, TILE_CAP - 1)];
     const int4 G = B.tile[blockIdx.x];
-    if (G.y == 0) return;
-    const int size = G.z;
     const int nlocal = A.nlocal;
+    // no locals (a table never holds others outside the range: nothing below
+    // leaves the arrays whatever it holds)
+    if (G.y <= 0 || G.x < 0 || G.x >= nlocal) return;
+    const int size = min(G.z, TILE_CAP);
     const int i = G.x + t;
     const bool live = t < G.y && i < nlocal;
     const int ii = live ? i : G.x;

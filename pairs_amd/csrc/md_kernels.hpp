@@ -24,6 +24,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <vector>
+
 #include "common.hpp"
 
 namespace pk {
@@ -239,8 +242,16 @@ struct TileArgs {
     int *slots;
     int gmax;
 };
-// the most groups of a system's tiles
+// the most groups of a system's tiles: the length of its table
 int tile_groups_max(int nlocal, const Geom &g);
+// the table before a build has made tiles: every local, none with a tile (their
+// forces come from the 32-bit lists); the rest is empty, as the force kernel
+// reads all of it
+inline std::vector<int4> tiles_before_build(int nlocal, int gmax) {
+    std::vector<int4> tab(gmax, make_int4(0, 0, 0, 0));
+    for (int k = 0; k * TILE_G < nlocal; k++) tab[k] = make_int4(k * TILE_G, std::min(TILE_G, nlocal - k * TILE_G), 0, 0);
+    return tab;
+}
 // dynamic LDS of one system's build workgroup
 size_t build_lds_bytes(const DevState &d, const Geom &g, int half);
 // the builds of many systems in one launch (block b: system rep[b], its

@@ -177,10 +177,7 @@ static int setup_tiles(pairs_hip_ctx *ctx) {
         dalloc(ctx, &d.nl16, (size_t) list_rows(d.ncap) / 8 * (d.rev0 > 0 ? 2 : 1) * d.nl_stride))
         return PAIRS_HIP_ERR_HIP;
     launch_set_counters(ctx->stream, d.counters, C_NGROUPS, 2, 0);
-    // until a build has made tiles: every local, over the 32-bit lists
-    std::vector<int4> tab((d.nlocal + TILE_G - 1) / TILE_G);
-    for (size_t k = 0; k < tab.size(); k++)
-        tab[k] = make_int4((int) k * TILE_G, std::min(TILE_G, d.nlocal - (int) k * TILE_G), 0, 0);
+    const std::vector<int4> tab = tiles_before_build(d.nlocal, d.tile_gmax);
     HIP_OK(hipMemcpyAsync(d.tile_tab, tab.data(), tab.size() * sizeof(int4), hipMemcpyHostToDevice, ctx->stream));
     HIP_OK(hipStreamSynchronize(ctx->stream));
     d.tiles = 1;

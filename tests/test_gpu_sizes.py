@@ -377,6 +377,43 @@ def test_lj_tiles_vs_gathers(half, sites, spacing, every):
         assert np.array_equal(p, q)
 
 
+def test_lj_forces_before_a_build():
+    """a large system's forces where no build has made tiles yet: after an upload,
+    after another one, after the lists have grown, in a run that starts between
+    two rebuilds; two types with the same parameters take no tiles"""
+    from pairs_amd import md
+    rng = np.random.default_rng(3)
+    m, a = 59, 1.06
+    k = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    x = (k + 0.5 + rng.uniform(-0.08, 0.08, k.shape)) * a
+    v = rng.standard_normal(k.shape)
+    y = x[rng.permutation(n)]
+    out = []
+    for nt in (1, 2):
+        t = np.arange(n, dtype=np.int32) % nt
+        g = md.LJSystem([(0.0, m * a)] * 3, particle_capacity=2 * n, send_capacity=n, neighbor_capacity=120,
+                        ntypes=nt, reneighbor_every=10)
+        g.upload(x, v, types=t)
+        g.lennard_jones()
+        assert not g.forces().any()
+        g.run(1, 3, 100)
+        got = [g.positions(), g.velocities()]
+        g.run(3, 25, 100)
+        got.append(g.forces())
+        g.upload(y, v, types=t)  # (the lists are those of the run)
+        g.lennard_jones()
+        got.append(g.forces())
+        g._call("pairs_hip_reserve", 0, 200, 0)
+        g.lennard_jones()
+        assert not g.forces().any()
+        g.run(0, 12, 100)
+        got += [g.positions(True), g.velocities(), g.forces()]
+        out.append(got)
+    for p, q in zip(*out):
+        assert np.array_equal(p, q, equal_nan=True)
+
+
 # downloads come in blocks of 1 MiB: 43690 rows of three doubles, 131072 doubles, 262144 words
 @pytest.mark.parametrize("n", [1, 43690, 43691, 87381, 131073, 262145])
 def test_downloads_at_block_edges(n):

@@ -1,0 +1,35 @@
+"""Host rules of the LJ kernels' launches, compiled for the host alone and run
+without a device."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _run(tmp_path, body):
+    """the output of a host program with the LJ kernels' header and this main()"""
+    from pairs_amd import build
+    src, exe = tmp_path / "main.cpp", tmp_path / "main"
+    src.write_text('#include "%s/pairs_amd/csrc/md_kernels.hpp"\n#include <cstdio>\nusing namespace pk;\n'
+                   "int main() {\n%s\n}\n" % (ROOT, body))
+    subprocess.run([build.hipcc(), "-O1", "-std=c++17", "-x", "hip", "--offload-host-only", "--offload-arch=gfx950",
+                    "-Wno-unused-result", "-o", str(exe), str(src)], check=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+
+
+@pytest.mark.parametrize("nlocal,gmax", [(200000, 4000), (200064, 1563), (200065, 1564), (1048576, 26970)])
+def test_tile_table_before_a_build(tmp_path, nlocal, gmax):
+    """the force kernel reads every row of the table: all locals once, the rest empty"""
+    out = _run(tmp_path, "for (const int4 &t : tiles_before_build(%d, %d)) printf(\"%%d %%d %%d\\n\", t.x, t.y, t.z);"
+               % (nlocal, gmax))
+    rows = [tuple(map(int, l.split())) for l in out.splitlines()]
+    assert len(rows) == gmax
+    at = 0
+    for first, count, size in rows:
+        assert size == 0 and 0 <= count <= 128
+        if count:
+            assert first == at
+            at += count
+    assert at == nlocal
