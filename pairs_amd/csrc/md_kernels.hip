@@ -1539,7 +1539,7 @@ __global__ __launch_bounds__(TILE_G) void k_ljt(LJArgs A, TileArgs B) {
     const int size = min(G.z, TILE_CAP);
     const int i = G.x + t;
     const bool live = t < G.y && i < nlocal;
-    const int ii = live ? i : G.x;
+    const int ii = min(G.x + tile_lane_row(t, G.y), nlocal - 1);
     const char *__restrict__ P = (const char *) A.P;
     const size_t stride = A.nl_stride;
     // the first rows of the list, and what the integration needs

@@ -92,6 +92,14 @@ __host__ __device__ __forceinline__ int list_rows(int ncap) { return (ncap + LIS
 constexpr int TILE_G = 128;
 constexpr int TILE_SPAN = 8;
 constexpr int TILE_CAP = 1088;
+// the local of a group of n whose list thread t of the force kernel walks: its
+// own, or, without one, its wave's first (a local's 16-bit rows are padded to
+// the depth of its own wave, and not further)
+__host__ __device__ __forceinline__ int tile_lane_row(int t, int n) {
+    if (t < n) return t;
+    const int first = t & ~63;
+    return first < n ? first : n - 1;
+}
 
 constexpr int IMG_MAX = 8;
 // leavers that the one-workgroup exchange takes from its list

@@ -33,3 +33,14 @@ def test_tile_table_before_a_build(tmp_path, nlocal, gmax):
             assert first == at
             at += count
     assert at == nlocal
+
+
+def test_idle_lanes_of_a_tile_walk_rows_of_their_wave(tmp_path):
+    """a local's 16-bit rows are padded to the depth of the wave that it is in"""
+    out = _run(tmp_path, "for (int n = 1; n <= TILE_G; n++) for (int t = 0; t < TILE_G; t++) "
+                         "printf(\"%d %d %d\\n\", n, t, tile_lane_row(t, n));")
+    for l in out.splitlines():
+        n, t, r = map(int, l.split())
+        assert 0 <= r < n and (r == t or t >= n)
+        # (a wave without a local has no entry to walk)
+        assert r // 64 == t // 64 or n <= t // 64 * 64
