@@ -1531,11 +1531,14 @@ __global__ __launch_bounds__(TILE_G) void k_ljt(LJArgs A, TileArgs B) {
 #pragma unroll
     for (int k = 0; k < PER; k++)
         sl[k] = B.slots[(size_t) blockIdx.x * TILE_CAP + min(k * TILE_G + t, TILE_CAP - 1)];
+    const int ovf = A.counters[C_OVF];
     const int4 G = B.tile[blockIdx.x];
     const int nlocal = A.nlocal;
-    // no locals (a table never holds others outside the range: nothing below
-    // leaves the arrays whatever it holds)
-    if (G.y <= 0 || G.x < 0 || G.x >= nlocal) return;
+    // behind a rebuild that overflowed, the list lengths may be those of one build
+    // and tiles and offsets those of another: the step is thrown away, so it is
+    // left out.  No locals: an empty row (none holds locals outside the range;
+    // nothing below leaves the arrays whatever it holds).
+    if (ovf || G.y <= 0 || G.x < 0 || G.x >= nlocal) return;
     const int size = min(G.z, TILE_CAP);
     const int i = G.x + t;
     const bool live = t < G.y && i < nlocal;

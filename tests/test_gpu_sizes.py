@@ -414,6 +414,37 @@ def test_lj_forces_before_a_build():
         assert np.array_equal(p, q, equal_nan=True)
 
 
+# a large system's steps behind a rebuild that overflowed and is repeated: the
+# ghosts outgrow the send map, or a segment's tile outgrows what the build stages
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("what", ["send", "tile"])
+def test_lj_tiles_behind_failed_rebuilds(what, half):
+    from pairs_amd import md, native
+    rng = np.random.default_rng(5)
+    m, a = 59, 1.06
+    k = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    # (the third layer from each lower face straddles the ghost layer's edge)
+    x = (k + 0.64 + rng.uniform(-0.08, 0.08, k.shape)) * a
+    v = -(10.0 if what == "send" else 16.0) * np.sin(2.0 * np.pi * x / (m * a))  # towards the faces
+    out = []
+    for nt in (1, 2):
+        t = np.arange(n, dtype=np.int32) % nt
+        kw = dict(particle_capacity=3 * n, neighbor_capacity=300, half=half, ntypes=nt, reneighbor_every=10)
+        g = md.LJSystem([(0.0, m * a)] * 3, send_capacity=n, **kw)
+        g.upload(x, v, types=t)
+        g.run(0, 1, 100)
+        if what == "send":  # (room for the ghosts of the first rebuild, hardly more)
+            ghosts = g.nghost
+            g = md.LJSystem([(0.0, m * a)] * 3, send_capacity=ghosts + 64, **kw)
+            g.upload(x, v, types=t)
+        g.run(0, 37, 100)
+        assert g.count(native.REBUILD_ROLLBACKS) > 0
+        out.append([g.positions(True), g.velocities(), g.forces()])
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+
+
 # downloads come in blocks of 1 MiB: 43690 rows of three doubles, 131072 doubles, 262144 words
 @pytest.mark.parametrize("n", [1, 43690, 43691, 87381, 131073, 262145])
 def test_downloads_at_block_edges(n):
