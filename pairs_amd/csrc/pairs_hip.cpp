@@ -523,6 +523,7 @@ int pairs_hip_upload(pairs_hip_ctx *ctx, int n, const double *x, const double *v
     d.exch_listed = n < 200000;
     ctx->nghost = 0;
     ctx->nsend_all = 0;
+    d.img_on = 0;  // no ghosts, no images
     setup_segments(ctx, ctx->zc_override);
     return setup_tiles(ctx);
 }
@@ -789,7 +790,10 @@ int pairs_hip_bin_cells(pairs_hip_ctx *ctx) {
     if (!ctx) return PAIRS_HIP_ERR_ARG;
     drop_graphs(ctx);
     launch_bin_sort(ctx->stream, ctx->d, ctx->geom);
-    return finish_module(ctx);
+    const int code = finish_module(ctx);
+    // the image table was made again: not used if it does not hold every ghost
+    if (code || ctx->h_counters[C_IMG_OVF]) ctx->d.img_on = 0;
+    return code;
 }
 
 // LDS entries the neighbour build stages per segment tile: the largest tile

@@ -243,6 +243,60 @@ def test_mlp_forces_vs_oracle_at_size_edges(cells):
     assert abs(e - Ex.sum()) < 1e-3 * abs(Ex.sum())
 
 
+def test_mlp_forces_after_module_rebuild_with_many_images():
+    """a run whose locals have 7 images each, then a rebuild by modules after which
+    half of them have 11, more than the image table holds, those that the table
+    leaves out inside the cutoff of others: forces as those of a system that
+    starts there"""
+    from pairs_amd import md, mlp
+    L = 5.04  # less than two cell spacings
+    x = 1.2 + 3.7 * np.stack(np.meshgrid(*[np.arange(2)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x += np.random.default_rng(8).uniform(-0.02, 0.02, x.shape)
+    v = np.zeros((8, 3))
+    v[:4, 0] = (2.27 - x[:4, 0]) / 0.005  # within a spacing of both faces in one step
+    m = mlp.MLPModel(seed=3)
+
+    def system(x, v):
+        s = md.LJSystem([(0.0, L)] * 3, particle_capacity=4000, send_capacity=4000, neighbor_capacity=120)
+        s.upload(x, v)
+        return s
+    g = system(x, v)
+    g.run(0, 1, 0)
+    g.euler()
+    for s in (g, None):
+        s = s or system(g.positions(), g.velocities())
+        s.exchange()
+        s.borders()
+        s.build_cell_lists()
+        s.build_neighbor_lists()
+        e, w = mlp.forces(s, m)
+        out = (e, w, s.nghost, s.positions(True), s.forces())
+        if s is g:
+            got = out
+    assert got[2] == out[2] == 4 * 7 + 4 * 11
+    assert got[0] == out[0] and got[1] == out[1]
+    assert np.array_equal(got[3], out[3]) and np.array_equal(got[4], out[4])
+
+
+def test_second_upload_starts_without_images():
+    """an upload into a system that has run: the first rebuild is checked before the
+    steps behind it, as a new system's, and the run is the same"""
+    from pairs_amd import md, native
+    out = []
+    for first in (700, 0):
+        g = md.LJSystem([(0.0, 14.0)] * 3, particle_capacity=16000, send_capacity=12000, neighbor_capacity=120)
+        if first:
+            _, x, v = _fluid(first, first / 14.0 ** 3, 1)
+            g.upload(x, v)
+            g.run(0, 3, 100)
+        _, x, v = _fluid(2300, 2300 / 14.0 ** 3, 2)
+        g.upload(x, v)
+        g.run(0, 23, 100)
+        out.append((g.positions(True), g.velocities(), g.forces(), g.count(native.REBUILDS_DEFERRED)))
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+
+
 # exchange and borders: 0 to 3 periodic dimensions; the leavers of a step fit the
 # list that the integration keeps (1024) or do not; a box narrower than two
 # cell widths, whose particles have images on both sides; a cell grid whose
