@@ -174,8 +174,13 @@ static int setup_tiles(pairs_hip_ctx *ctx) {
     d.tile_gmax = tile_groups_max(d.nlocal, g);
     const size_t gm = (size_t) d.tile_gmax;
     if (dalloc(ctx, &d.tile_grp, gm) || dalloc(ctx, &d.tile_tab, gm) || dalloc(ctx, &d.tile_slots, gm * TILE_CAP) ||
-        dalloc(ctx, &d.nl16, (size_t) list_rows(d.ncap) / 8 * (d.rev0 > 0 ? 2 : 1) * d.nl_stride))
-        return PAIRS_HIP_ERR_HIP;
+        dalloc(ctx, &d.nl16, (size_t) list_rows(d.ncap) / 8 * (d.rev0 > 0 ? 2 : 1) * d.nl_stride)) {
+        // no room: the system runs without
+        (void) hipGetLastError();
+        ctx->err.clear();
+        free_tiles(d);
+        return 0;
+    }
     launch_set_counters(ctx->stream, d.counters, C_NGROUPS, 2, 0);
     const std::vector<int4> tab = tiles_before_build(d.nlocal, d.tile_gmax);
     HIP_OK(hipMemcpyAsync(d.tile_tab, tab.data(), tab.size() * sizeof(int4), hipMemcpyHostToDevice, ctx->stream));

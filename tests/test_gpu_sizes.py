@@ -468,6 +468,31 @@ def test_lj_forces_before_a_build():
         assert np.array_equal(p, q, equal_nan=True)
 
 
+def test_upload_without_room_for_tiles():
+    """lists that take three quarters of the device's memory leave no room for their
+    16-bit copies: the system is uploaded and runs all the same"""
+    import ctypes
+    from pairs_amd import md
+    rng = np.random.default_rng(6)
+    m, a = 59, 1.06
+    k = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    x = (k + 0.5 + rng.uniform(-0.08, 0.08, k.shape)) * a
+    v = rng.standard_normal(k.shape)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert md.nat.lib() and ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    out = []
+    for ncap in (120, int(0.75 * free.value / (4 * 2 * n))):
+        g = md.LJSystem([(0.0, m * a)] * 3, particle_capacity=2 * n, send_capacity=n, neighbor_capacity=ncap,
+                        reneighbor_every=10)
+        g.upload(x, v)
+        g.run(0, 12, 100)
+        out.append((g.positions(True), g.velocities(), g.forces()))
+        del g
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+
+
 # a large system's steps behind a rebuild that overflowed and is repeated: the
 # ghosts outgrow the send map, or a segment's tile outgrows what the build stages
 @pytest.mark.parametrize("half", [False, True])
