@@ -419,8 +419,6 @@ __host__ __device__ __forceinline__ CopyBackArgs copy_back_args(const DevState &
 // slots, which spares the inner loop a test and a look-up, the runs are summed
 // with DPP and the table's cell starts are loaded ahead: 119 -> 113 us at
 // 131072 atoms, 603 -> 556 at 1048576.
-constexpr int BB = 128;        // threads per build workgroup
-constexpr int BB_SMALL = 512;  // in small systems
 constexpr int NB_CAND = 2048;  // candidates of one home cell
 // half lists: mirror entries of one home particle collected in the top
 // RMAX slots of the wave's candidate buffer before they are sorted
@@ -2846,8 +2844,21 @@ BuildArgs build_args(const DevState &d, const Geom &g, int half, double rc2) {
     return A;
 }
 
-size_t build_lds_bytes(const DevState &d, const Geom &g, int half) {
-    return build_lds(d, g, half, min(d.tile_cap, build_tile_limit(d, g, half)));
+size_t build_lds_bytes(const DevState &d, const Geom &g, int half, int threads) {
+    return build_lds(d, g, half, min(d.tile_cap, build_tile_limit(d, g, half)), threads);
+}
+
+// Eight waves per segment share its cells' home particles where the segments
+// are too few to fill the chip.  Build, us, on 2 | 8 waves: 256 atoms 30 | 18,
+// 19200 40 | 35; 200 steps of 70304 atoms 6.89 | 6.84 ms; 131072 atoms 113 |
+// 122 (half lists 263 | 305).  (A larger tile leaves no room for eight
+// candidate buffers at the occupancy measured; long columns of a sparse system,
+// whose table of cells takes most of the LDS, leave none at all.)
+int build_threads(const DevState &d, const Geom &g, int half) {
+    const int tcap = min(d.tile_cap, build_tile_limit(d, g, half));
+    return d.nlocal < 80000 && tcap <= 8192 && build_lds(d, g, half, tcap, BB_SMALL) + 2048 <= (size_t) d.max_lds
+               ? BB_SMALL
+               : BB;
 }
 
 static TileArgs tile_args(const DevState &d, const Geom &g) {
@@ -2876,12 +2887,7 @@ static void build_launch(hipStream_t s, const DevState &d, const Geom &g, int ha
 
 void launch_build_neighbors(hipStream_t s, const DevState &d, const Geom &g, int half, double rc2) {
     const BuildArgs A = build_args(d, g, half, rc2);
-    // eight waves per segment share its cells' home particles where the segments
-    // are too few to fill the chip.  Build, us, on 2 | 8 waves: 256 atoms 30 | 18,
-    // 19200 40 | 35; 200 steps of 70304 atoms 6.89 | 6.84 ms; 131072 atoms 113 |
-    // 122 (half lists 263 | 305).  (A larger tile leaves no room for eight
-    // candidate buffers at the occupancy measured.)
-    if (d.nlocal < 80000 && A.tcap <= 8192) build_launch<BB_SMALL>(s, d, g, half, A);
+    if (build_threads(d, g, half) == BB_SMALL) build_launch<BB_SMALL>(s, d, g, half, A);
     else build_launch<BB>(s, d, g, half, A);
     if (!d.tiles) return;
     const TileArgs T = tile_args(d, g);

@@ -260,8 +260,12 @@ inline std::vector<int4> tiles_before_build(int nlocal, int gmax) {
     for (int k = 0; k * TILE_G < nlocal; k++) tab[k] = make_int4(k * TILE_G, std::min(TILE_G, nlocal - k * TILE_G), 0, 0);
     return tab;
 }
-// dynamic LDS of one system's build workgroup
-size_t build_lds_bytes(const DevState &d, const Geom &g, int half);
+// threads of a build workgroup: of one system (BB, or BB_SMALL in small ones),
+// of a batch (BB); and its dynamic LDS
+constexpr int BB = 128;
+constexpr int BB_SMALL = 512;
+int build_threads(const DevState &d, const Geom &g, int half);
+size_t build_lds_bytes(const DevState &d, const Geom &g, int half, int threads);
 // the builds of many systems in one launch (block b: system rep[b], its
 // segment b - seg_base[rep[b]]); lds = the largest system's need
 void launch_build_batch(hipStream_t s, const BuildArgs *desc, const int *rep, const int *seg_base, int nblocks,

@@ -1895,7 +1895,7 @@ static int batch_rebuild(pairs_hip_batch *b) {
     for (int r = 0; r < R; r++) {
         pairs_hip_ctx *c = b->rep[r];
         b->h_bdesc[r] = build_args(c->d, c->geom, 0, c->cfg.cell_spacing * c->cfg.cell_spacing);
-        lds = std::max(lds, build_lds_bytes(c->d, c->geom, 0));
+        lds = std::max(lds, build_lds_bytes(c->d, c->geom, 0, BB));
     }
     BATCH_OK(hipMemcpyAsync(b->d_bdesc, b->h_bdesc, R * sizeof(BuildArgs), hipMemcpyHostToDevice, s));
     launch_build_batch(s, b->d_bdesc, b->d_srep, b->d_sbase, b->nsblocks, lds, 0);

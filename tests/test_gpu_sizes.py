@@ -398,6 +398,31 @@ def test_lj_exchange_and_borders_vs_oracle(n, periodic, edge, speed):
         tm._compare_lists(g, o, step)
 
 
+@pytest.mark.parametrize("half", [False, True])
+def test_lj_long_columns_vs_oracle(half):
+    """a sparse system of columns of 953 cells, whose table of cells takes most of a
+    build workgroup's LDS"""
+    from pairs_amd import md
+    rng = np.random.default_rng(9)
+    n, box = 300, [(0.0, 8.4), (0.0, 8.4), (0.0, 2660.0)]
+    x = rng.uniform(0.0, 1.0, (n, 3)) * [8.4, 8.4, 1.0]
+    x[:, 2] = (np.arange(n) // 10 + 0.5) * 88.0 + 1.1 * (np.arange(n) % 10)  # strings of ten
+    v = rng.standard_normal((n, 3))
+    g = md.LJSystem(box, particle_capacity=8000, neighbor_capacity=100, send_capacity=6000, half=half)
+    o = po.OracleMD(box, 8000, ncap=100, ccap=64, send_cap=6000, half=half)
+    g.upload(x, v)
+    o.set_particles(x, v)
+    o.setup_cells()
+    for a, b in ((0, 1), (1, 23)):
+        g.run(a, b, 100)
+        o.run(a, b)
+        assert o.overflow == 0
+        for name, p, q in (("position", g.positions(True), o.positions(True)),
+                           ("velocity", g.velocities(), o.velocities()), ("force", g.forces(), o.forces())):
+            assert np.array_equal(p, q), (name, b)
+    assert g.numneighs().max() > 0
+
+
 # large systems of one type take the timestep's forces from LDS tiles; two types
 # with the same parameters do not, and give the same bits
 @pytest.mark.parametrize("half", [False, True])

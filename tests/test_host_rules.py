@@ -9,13 +9,15 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _run(tmp_path, body):
-    """the output of a host program with the LJ kernels' header and this main()"""
+    """the output of a host program with the LJ kernels' header and this main(),
+    linked with the library"""
     from pairs_amd import build
     src, exe = tmp_path / "main.cpp", tmp_path / "main"
     src.write_text('#include "%s/pairs_amd/csrc/md_kernels.hpp"\n#include <cstdio>\nusing namespace pk;\n'
                    "int main() {\n%s\n}\n" % (ROOT, body))
     subprocess.run([build.hipcc(), "-O1", "-std=c++17", "-x", "hip", "--offload-host-only", "--offload-arch=gfx950",
-                    "-Wno-unused-result", "-o", str(exe), str(src)], check=True)
+                    "-Wno-unused-result", str(src), "-o", str(exe), "-L" + build.HERE, "-lpairs_hip",
+                    "-Wl,-rpath," + build.HERE], check=True)
     return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
 
 
@@ -44,3 +46,23 @@ def test_idle_lanes_of_a_tile_walk_rows_of_their_wave(tmp_path):
         assert 0 <= r < n and (r == t or t >= n)
         # (a wave without a local has no entry to walk)
         assert r // 64 == t // 64 or n <= t // 64 * 64
+
+
+def test_build_workgroup_fits_the_lds(tmp_path):
+    """whatever the length of the columns, the tile and the list form: a build that
+    fits a workgroup of two waves is launched in one that fits"""
+    out = _run(tmp_path, """
+    for (int nz = 4; nz < 1300; nz += 7) for (int half = 0; half < 2; half++) for (int chunks = 1; chunks < 3; chunks++)
+    for (int cap : {64, 640, 4096, 8192, 8256, 30000}) for (int n : {300, 79999, 80001}) {
+        DevState d{};
+        Geom g{};
+        d.max_lds = 163840; d.nlocal = n; d.tile_cap = cap;
+        g.dim_cells[0] = g.dim_cells[1] = 7; g.dim_cells[2] = nz; g.nchunks = chunks; g.zc = nz / chunks;
+        if (build_tile_limit(d, g, half) < 64) continue;
+        const int t = build_threads(d, g, half);
+        printf("%d %zu %d\\n", t, build_lds_bytes(d, g, half, t), d.max_lds);
+    }""")
+    rows = [tuple(map(int, l.split())) for l in out.splitlines()]
+    assert {t for t, _, _ in rows} == {128, 512}
+    for threads, lds, most in rows:
+        assert lds + 512 <= most, (threads, lds)  # (less than 512 bytes of static LDS)
