@@ -30,7 +30,8 @@ struct pairs_hip_ctx {
     int ghost_grid = 1;
     int max_lds = 65536;       // shared memory a workgroup may allocate
     int zc_override = 0;
-    bool tiles_off = false;    // no force tiles: forces come from elsewhere (MLP, batch), or tiles do not fit
+    bool tiles_off = false;    // no force tiles: the batched kernels do without
+    bool tiles_big = false;    // nor for this upload: too many groups did not fit theirs
     int home_target = 40;      // home particles a segment aims at (sets zc; about 3 cells at rho 0.84)
     // graphs of n consecutive non-rebuild steps (slot n - 1, n <=
     // CHAIN_MAX), by parity of the current buffer at their first step: a run

@@ -155,9 +155,9 @@ static void free_tiles(DevState &d) {
 }
 
 // Force tiles (k_ljt) or not, and their arrays: called where the number of
-// locals or the lists' capacity changes, when no lists are valid.  The tiles
-// cost a rebuild some 40 us per 100000 locals and save each step's force pass
-// half its memory traffic.  A rebuild every 20 steps, ms without | with:
+// locals, the lists' capacity or the potential changes; until the next build
+// the forces come from the 32-bit lists.  The tiles cost a rebuild some 40 us
+// per 100000 locals and save each step's force pass half its memory traffic.  A rebuild every 20 steps, ms without | with:
 // 157216 locals (100 steps) 7.29 | 7.43, 186624 8.18 | 8.08 (half lists 11.2 |
 // 11.4), 198400 (200) 14.8 | 13.7, 389344 (100) 15.8 | 14.7 (half 24.1 | 19.9),
 // 1048576 (200) 86.0 | 65.2 (half, 60: 46.0 | 38.7); at 200000 they pay from 8
@@ -168,8 +168,8 @@ static int setup_tiles(pairs_hip_ctx *ctx) {
     const Geom &g = ctx->geom;
     free_tiles(d);
     const double per_column = d.nlocal * (g.spacing / g.len[0]) * (g.spacing / g.len[1]);
-    if (ctx->tiles_off || ctx->cfg.ntypes != 1 || d.nlocal < 200000 || ctx->cfg.reneighbor_every < 10 ||
-        per_column < 96.0)
+    if (ctx->tiles_off || ctx->tiles_big || ctx->mlp_on || ctx->cfg.ntypes != 1 || d.nlocal < 200000 ||
+        ctx->cfg.reneighbor_every < 10 || per_column < 96.0)
         return 0;
     d.tile_gmax = tile_groups_max(d.nlocal, g);
     const size_t gm = (size_t) d.tile_gmax;
@@ -273,9 +273,10 @@ static void take_counters(pairs_hip_ctx *ctx) {
     }
     if (ctx->d.tiles && ctx->h_counters[C_BIG] > ctx->h_counters[C_NGROUPS] / 16) {
         // too many groups whose tile does not fit (they walk the 32-bit lists)
-        ctx->tiles_off = true;
-        ctx->d.tiles = 0;
+        ctx->tiles_big = true;
         drop_graphs(ctx);
+        hipStreamSynchronize(ctx->stream);
+        free_tiles(ctx->d);
     }
 }
 
@@ -529,6 +530,7 @@ int pairs_hip_upload(pairs_hip_ctx *ctx, int n, const double *x, const double *v
     ctx->nghost = 0;
     ctx->nsend_all = 0;
     d.img_on = 0;  // no ghosts, no images
+    ctx->tiles_big = false;
     setup_segments(ctx, ctx->zc_override);
     return setup_tiles(ctx);
 }
@@ -1716,15 +1718,18 @@ int pairs_hip_mlp_attach(pairs_hip_ctx *ctx, pairs_hip_mlp *m, double max_rel_rm
         if (int r = pairs_hip_mlp_force_error(ctx, m, &rel)) return r;
         if (rel_rms) *rel_rms = rel;
         if (!(rel <= max_rel_rms)) {  // fallback: keep LJ (its forces are in the force array)
+            const bool was_on = ctx->mlp_on;
             ctx->mlp_on = false;
+            if (was_on)
+                if (int r = setup_tiles(ctx)) return r;
             return 1;
         }
     }
     ctx->mlp = mlp_bind(ctx, m);
     ctx->mlp_on = true;
-    ctx->tiles_off = true;
-    ctx->d.tiles = 0;
     DevState &d = ctx->d;
+    HIP_OK(hipStreamSynchronize(ctx->stream));
+    free_tiles(d);  // (until detached)
     launch_mlp_forces(ctx->stream, d, ctx->geom, ctx->mlp, d.cur, 0, ctx->ghost_grid);
     CHECK_LAUNCH();
     HIP_OK(hipStreamSynchronize(ctx->stream));
@@ -1734,8 +1739,9 @@ int pairs_hip_mlp_attach(pairs_hip_ctx *ctx, pairs_hip_mlp *m, double max_rel_rm
 int pairs_hip_mlp_detach(pairs_hip_ctx *ctx) {
     if (!ctx) return PAIRS_HIP_ERR_ARG;
     drop_graphs(ctx);
+    if (!ctx->mlp_on) return 0;
     ctx->mlp_on = false;
-    return 0;
+    return setup_tiles(ctx);
 }
 
 int pairs_hip_mlp_active(const pairs_hip_ctx *ctx) { return ctx && ctx->mlp_on ? 1 : 0; }

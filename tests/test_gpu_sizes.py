@@ -493,6 +493,61 @@ def test_lj_forces_before_a_build():
         assert np.array_equal(p, q, equal_nan=True)
 
 
+def test_tiles_come_back():
+    """the tile arrays of a large system (more than 100 MB here) are given back while
+    an MLP potential is attached and while a configuration is too dense for
+    them, and are there again after a detach and after the next upload; the
+    trajectory is that of a system that never was without"""
+    import ctypes
+    from pairs_amd import md, mlp
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value / 1e6
+    rng = np.random.default_rng(7)
+    m, a = 59, 1.06
+    k = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    x = (k + 0.5 + rng.uniform(-0.08, 0.08, k.shape)) * a
+    v = rng.standard_normal(k.shape)
+    model = mlp.MLPModel(seed=1)
+    out = []
+    for attach in (False, True):
+        g = md.LJSystem([(0.0, m * a)] * 3, particle_capacity=3 * n, send_capacity=2 * n, neighbor_capacity=256,
+                        reneighbor_every=10)
+        g.upload(x, v)
+        g.run(0, 12, 100)
+        if attach:
+            f0 = free()
+            mlp.attach(g, model, -1.0)
+            f1 = free()
+            mlp.detach(g)
+            f2 = free()
+            assert f2 < f1 - 100, (f0, f1, f2)
+            g.lennard_jones()
+        g.run(12, 33, 100)
+        out.append((g.positions(True), g.velocities(), g.forces()))
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+    # a density of 1.59: the tiles of many groups do not fit
+    f0 = free()
+    dense = (np.stack(np.meshgrid(*[np.arange(73)] * 3, indexing="ij"), -1).reshape(-1, 3) + 0.5) * (m * a / 73)
+    g.upload(dense, np.zeros(dense.shape))
+    g.exchange()
+    g.borders()
+    g.build_cell_lists()
+    g.build_neighbor_lists()
+    assert free() > f0 + 100, (f0, free())
+    g.upload(x, v)
+    assert abs(free() - f0) < 100, (f0, free())
+    g.run(0, 12, 100)
+    g.run(12, 33, 100)
+    for p, q in zip(out[0], (g.positions(True), g.velocities(), g.forces())):
+        assert np.array_equal(p, q)
+
+
 def test_upload_without_room_for_tiles():
     """lists that take three quarters of the device's memory leave no room for their
     16-bit copies: the system is uploaded and runs all the same"""
