@@ -260,6 +260,15 @@ static int setup_geometry(pairs_hip_ctx *ctx) {
     return 0;
 }
 
+// no force tiles until the next upload
+static void drop_tiles(pairs_hip_ctx *ctx) {
+    ctx->tiles_big = true;
+    if (!ctx->d.tiles) return;
+    drop_graphs(ctx);
+    hipStreamSynchronize(ctx->stream);
+    free_tiles(ctx->d);
+}
+
 // host-side bookkeeping of a counters snapshot already in ctx->h_counters
 static void take_counters(pairs_hip_ctx *ctx) {
     ctx->nghost = ctx->h_counters[C_NGHOST];
@@ -273,10 +282,7 @@ static void take_counters(pairs_hip_ctx *ctx) {
     }
     if (ctx->d.tiles && ctx->h_counters[C_BIG] > ctx->h_counters[C_NGROUPS] / 16) {
         // too many groups whose tile does not fit (they walk the 32-bit lists)
-        ctx->tiles_big = true;
-        drop_graphs(ctx);
-        hipStreamSynchronize(ctx->stream);
-        free_tiles(ctx->d);
+        drop_tiles(ctx);
     }
 }
 
@@ -841,18 +847,23 @@ static int grow_tile(pairs_hip_ctx *ctx) {
 }
 
 // the build enqueued, counters read: repeat the build while its tile grows,
-// then report the other overflows
+// then report the other overflows; a build given up leaves list lengths that are
+// not those of the force tiles
 static int finish_build(pairs_hip_ctx *ctx) {
     for (int attempt = 0; attempt < 64; attempt++) {
         if (ctx->h_counters[C_OVF] != OVF_TILE) {
             set_tile_cap(ctx);
             return take_overflow(ctx);
         }
-        if (int r = grow_tile(ctx)) return r;
+        if (int r = grow_tile(ctx)) {
+            drop_tiles(ctx);
+            return r;
+        }
         enqueue_build(ctx);
         CHECK_LAUNCH();
         if (read_counters(ctx)) return PAIRS_HIP_ERR_HIP;
     }
+    drop_tiles(ctx);
     ctx->err = "neighbour build did not converge";
     return PAIRS_HIP_ERR_STATE;
 }

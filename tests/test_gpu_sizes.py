@@ -548,6 +548,44 @@ def test_tiles_come_back():
         assert np.array_equal(p, q)
 
 
+def test_tiles_off_behind_a_build_given_up():
+    """a clump whose cells' candidates no build workgroup can hold: the build fails,
+    the forces behind it do without tiles, and the next upload starts anew"""
+    import ctypes
+    from pairs_amd import md, native
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value / 1e6
+    rng = np.random.default_rng(11)
+    m, a = 59, 1.06
+    k = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    x = (k + 0.5 + rng.uniform(-0.08, 0.08, k.shape)) * a
+    v = rng.standard_normal(k.shape)
+    y = x.copy()
+    y[:60000] = 26.0 + rng.uniform(0.0, 8.4, (60000, 3))
+    g = md.LJSystem([(0.0, m * a)] * 3, particle_capacity=3 * n, send_capacity=2 * n, neighbor_capacity=256,
+                    reneighbor_every=10)
+    g.upload(x, v)
+    g.run(0, 2, 100)
+    first = g.forces()
+    g.upload(y, v)
+    g.exchange()
+    g.borders()
+    g.build_cell_lists()
+    before = free()
+    with pytest.raises(native.PairsHipError):
+        g.build_neighbor_lists()
+    assert free() > before + 100, (before, free())
+    g.lennard_jones()
+    g.upload(x, v)
+    g.run(0, 2, 100)
+    assert np.array_equal(first, g.forces())
+
+
 def test_upload_without_room_for_tiles():
     """lists that take three quarters of the device's memory leave no room for their
     16-bit copies: the system is uploaded and runs all the same"""
