@@ -1419,8 +1419,7 @@ __global__ __launch_bounds__(TILE_G) void k_tile_build(TileArgs A) {
     __syncthreads();
     // the runs by start, empty ones left out
     if (t < NRUNS && r_off[t + 1] > r_off[t]) {
-        int rank = 0;
-        for (int k = 0; k < NRUNS; k++) rank += r_off[k + 1] > r_off[k] && r_start[k] < r_start[t] ? 1 : 0;
+        const int rank = tile_run_rank(r_start, r_off, t);
         s_from[rank] = r_start[t];
         s_delta[rank] = r_off[t] - r_start[t];
     }
@@ -1428,12 +1427,7 @@ __global__ __launch_bounds__(TILE_G) void k_tile_build(TileArgs A) {
     const int i = G.x + t;
     const bool live = t < G.y;
     const size_t stride = A.nl_stride;
-    auto place = [&](uint32_t j) {
-        int p = 0;
-#pragma unroll
-        for (int s = 16; s > 0; s >>= 1) p += s_from[p + s] <= (int) j ? s : 0;
-        return min((unsigned) ((int) j + s_delta[p]), (unsigned) CMAX - 1);
-    };
+    auto place = [&](uint32_t j) { return min((unsigned) tile_place(s_from, s_delta, (int) j), (unsigned) CMAX - 1); };
     // pass over one part of the list: rows of eight, to the wave's depth
     auto mark = [&](int n, int row0, int out0) {
         const int rows = (wave_max_uniform(n) + 7) / 8;

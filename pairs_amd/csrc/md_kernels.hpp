@@ -107,6 +107,33 @@ constexpr int LEAVE_CAP = 4096;
 // ghost kinds: per periodic dimension none, side 0 or side 1
 constexpr int MAX_KIND = 27;
 
+// The runs of a group's candidate cells as the tile build searches them: sorted
+// by first slot, so that a slot's place among the candidates is that of the last
+// run that begins at or before it.  Runs of neighbouring columns may overlap (a
+// column's range of flat cells reaches into the next column's first cell), and
+// then begin at one slot where the cells between are empty: the longer of them
+// comes last, as it holds all of the shorter.
+constexpr int NRUNS = 20;
+// run t's rank among the runs that are not empty (off: their exclusive sums)
+__host__ __device__ __forceinline__ int tile_run_rank(const int *start, const int *off, int t) {
+    const int len = off[t + 1] - off[t];
+    int rank = 0;
+    for (int k = 0; k < NRUNS; k++) {
+        const int n = off[k + 1] - off[k];
+        if (n == 0 || start[k] > start[t]) continue;
+        rank += start[k] < start[t] || n < len || (n == len && k < t) ? 1 : 0;
+    }
+    return rank;
+}
+// slot j's place (from, delta by rank: first slot, place minus slot; from is
+// the largest number behind the last)
+__host__ __device__ __forceinline__ int tile_place(const int *from, const int *delta, int j) {
+    int p = 0;
+#pragma unroll
+    for (int s = 16; s > 0; s >>= 1) p += from[p + s] <= j ? s : 0;
+    return j + delta[p];
+}
+
 // what a position-advancing kernel needs to refresh the ghost images
 struct Images {
     const int *cnt;

@@ -45,8 +45,6 @@ __device__ __forceinline__ SegInfo seg_info(int seg, const Geom &g) {
     return s;
 }
 
-constexpr int NRUNS = 20;
-
 // The 20 physical runs of a segment's tile, in the reference's candidate
 // order of cells: cell 0 (locals, ghosts), then the columns (dx, dy) of the
 // stencil (dx outer, dy inner; src/pairs/sim/cell_lists.py:70-87), each over

@@ -456,6 +456,31 @@ def test_lj_tiles_vs_gathers(half, sites, spacing, every):
         assert np.array_equal(p, q)
 
 
+def test_lj_tiles_of_a_slab_with_a_gap_vs_gathers():
+    """columns no longer than a group, particles below the open lower face, and empty
+    columns: runs of a group's candidate cells that begin at one slot"""
+    from pairs_amd import md
+    rng = np.random.default_rng(12)
+    k = np.stack(np.meshgrid(np.arange(220), np.arange(65), np.arange(14), indexing="ij"), -1).reshape(-1, 3)
+    n = len(k)
+    x = (k + 0.5 + rng.uniform(-0.06, 0.06, k.shape)) * [0.95, 0.95, 1.0]
+    x[:, 1] += 4.0
+    x[:, 2] -= 1.0
+    v = rng.standard_normal(k.shape)
+    out = []
+    for nt in (1, 2):
+        g = md.LJSystem([(0.0, 209.0), (0.0, 70.25), (0.0, 13.9)], particle_capacity=2 * n, send_capacity=n,
+                        neighbor_capacity=160, ntypes=nt, reneighbor_every=10, periodic=(1, 1, 0))
+        g.upload(x, v, types=np.arange(n, dtype=np.int32) % nt)
+        got = []
+        for a, b in ((0, 1), (1, 12)):
+            g.run(a, b, 100)
+            got += [g.positions(True), g.velocities(), g.forces()]
+        out.append(got)
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+
+
 def test_lj_forces_before_a_build():
     """a large system's forces where no build has made tiles yet: after an upload,
     after another one, after the lists have grown, in a run that starts between

@@ -66,3 +66,55 @@ def test_build_workgroup_fits_the_lds(tmp_path):
     assert {t for t, _, _ in rows} == {128, 512}
     for threads, lds, most in rows:
         assert lds + 512 <= most, (threads, lds)  # (less than 512 bytes of static LDS)
+
+
+def test_tile_places_of_overlapping_runs(tmp_path):
+    """cells with many empty ones, columns no longer than a group: a slot of any
+    candidate run has a place, and the place is the slot's"""
+    out = _run(tmp_path, """
+    unsigned seed = 1;
+    auto rnd = [&](int n) { seed = seed * 1664525u + 1013904223u; return (int) ((seed >> 8) % (unsigned) n); };
+    int equal = 0, wrong = 0, slots = 0;
+    for (int c = 0; c < 4000; c++) {
+        const int nx = 3 + rnd(3), ny = 3 + rnd(3), nz = 3 + rnd(6), ncells = nx * ny * nz + 1, fill = 1 + rnd(12);
+        std::vector<int> at[2];  // first slots of the cells: locals, ghosts
+        int n = 0;
+        for (int k = 0; k < 2; k++) {
+            at[k].resize(ncells + 1);
+            for (int i = 0; i < ncells; i++) { at[k][i] = n; n += rnd(12) < fill ? rnd(5) : 0; }
+            at[k][ncells] = n;
+        }
+        const int cx = rnd(nx), cy = rnd(ny), za = rnd(nz), zb = za + 1 + rnd(nz - za);
+        int start[NRUNS], off[NRUNS + 1] = {0};
+        for (int t = 0; t < NRUNS; t++) {
+            int lo = 0, hi = 0;
+            if (t >= 2) {
+                const int col = (t - 2) / 2, B = ((cx + col / 3 - 1) * ny + cy + col % 3 - 1) * nz + 1;
+                lo = std::max(B + za - 1, 1);
+                hi = std::min(B + zb, ncells - 1);
+            }
+            start[t] = lo <= hi ? at[t & 1][lo] : 0;
+            off[t + 1] = off[t] + (lo <= hi ? at[t & 1][hi + 1] - start[t] : 0);
+        }
+        int from[32], delta[32] = {0};
+        for (int &f : from) f = 0x7fffffff;
+        for (int t = 0; t < NRUNS; t++) {
+            if (off[t + 1] == off[t]) continue;
+            const int r = tile_run_rank(start, off, t);
+            from[r] = start[t];
+            delta[r] = off[t] - start[t];
+            for (int k = 0; k < t; k++) equal += off[k + 1] > off[k] && start[k] == start[t];
+        }
+        for (int t = 0; t < NRUNS; t++)
+            for (int j = start[t]; j < start[t] + off[t + 1] - off[t]; j++) {
+                const int p = tile_place(from, delta, j);
+                bool ok = false;
+                for (int r = 0; r < NRUNS; r++) ok = ok || (p >= off[r] && p < off[r + 1] && start[r] + p - off[r] == j);
+                wrong += !ok;
+                slots++;
+            }
+    }
+    printf("%d %d %d\\n", equal, wrong, slots);""")
+    equal, wrong, slots = map(int, out.split())
+    assert equal > 100 and slots > 10000
+    assert wrong == 0, (wrong, slots)
