@@ -1144,7 +1144,7 @@ __device__ __forceinline__ void lj_multi(const LJArgs &A, int wv) {
         constexpr int BUF = 3 * M * S;
         const uint32_t off_e = odd ? 16u : 0u, off_o = odd ? 0u : 16u;
         // half of list group h / 4 of the round, read by both lanes of a pair: entries 0, 2 or 1, 3
-        const uint32_t loff = ((uint32_t) (h >> 2) * (uint32_t) stride + (uint32_t) ii) * 16u + (h & 2) * 4u;
+        const size_t loff = ((size_t) (h >> 2) * stride + ii) * 16 + (h & 2) * 4;
         const int rounds = A.rows / L;  // rounds the allocated rows hold
         auto ldl = [&](int row0, int r, int R) {
             return *(const uint2 *) ((const char *) (A.nl + (size_t) row0 * stride) +

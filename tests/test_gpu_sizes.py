@@ -51,6 +51,22 @@ def test_lj_run_vs_oracle_at_size_edges(n, ntypes, half):
             assert np.array_equal(p, q), f"{name} after step {b}: max |diff| {np.abs(p - q).max()}"
 
 
+def test_lj_run_in_arrays_of_many_slots():
+    """a small system in arrays of 38.5 million slots: a list row's offset passes 4 GiB"""
+    from pairs_amd import md
+    L, x, v = _fluid(500, 0.8, 1)
+    out = []
+    for cap in (8000, 38500000):
+        g = md.LJSystem([(0.0, L)] * 3, particle_capacity=cap, send_capacity=8000, neighbor_capacity=128)
+        g.upload(x, v)
+        g.run(0, 30, 100)
+        out.append((g.positions(True), g.velocities(), g.forces()))
+        assert g.numneighs().min() > 28
+        del g
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+
+
 def _spheres(case):
     """uid, radius, position, velocity of a few spheres, domain, half-spaces"""
     rng = np.random.default_rng(len(case))
