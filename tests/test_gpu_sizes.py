@@ -51,6 +51,31 @@ def test_lj_run_vs_oracle_at_size_edges(n, ntypes, half):
             assert np.array_equal(p, q), f"{name} after step {b}: max |diff| {np.abs(p - q).max()}"
 
 
+@pytest.mark.parametrize("n", [100, 5000, 13000, 45000, 110000])
+def test_forces_beside_a_particle_at_infinity(n):
+    """a particle that has left for infinity, in the last slot of an open system,
+    leaves the forces of the others as they are without it"""
+    from pairs_amd import md, mlp
+    L, x, v = _fluid(n, 0.8, n)
+    m = mlp.MLPModel(seed=2)
+    out = []
+    for far in (False, True):
+        g = md.LJSystem([(0.0, L)] * 3, particle_capacity=n + 8, send_capacity=64, neighbor_capacity=120,
+                        periodic=(0, 0, 0))
+        g.upload(np.concatenate([x, np.full((1, 3), np.inf)]) if far else x,
+                 np.concatenate([v, np.zeros((1, 3))]) if far else v)
+        g.exchange()
+        g.borders()
+        g.build_cell_lists()
+        g.build_neighbor_lists()
+        g.lennard_jones()
+        got = [g.forces()[:n], g.numneighs()[:n]]
+        mlp.forces(g, m)
+        out.append(got + [g.forces()[:n]])
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
+
+
 def test_lj_run_in_arrays_of_many_slots():
     """a small system in arrays of 38.5 million slots: a list row's offset passes 4 GiB"""
     from pairs_amd import md
