@@ -2705,13 +2705,6 @@ void launch_bin_sort(hipStream_t s, DevState &d, const Geom &g, bool pack) {
     (void) g;                                        \
     (void) c
 
-// dim < 0: every system; else only systems periodic in dim
-__global__ void k_set_counters_batch(const RepDesc *__restrict__ D, int dim, int first, int count, int v) {
-    REP_ARGS;
-    if (dim >= 0 && !R.periodic[dim]) return;
-    if ((int) threadIdx.x < count) d.counters[first + threadIdx.x] = v;
-}
-
 // dim is the system's first periodic dimension
 __device__ __forceinline__ bool first_periodic(const RepDesc &R, int dim) {
     for (int k = 0; k < dim; k++)
@@ -2741,14 +2734,6 @@ __global__ __launch_bounds__(1024) void k_exchange_relabel_batch(const RepDesc *
     int *sc = d.scratch_i;
     k_exchange_relabel_body(d.X[c], d.Y[c], d.Z[c], d.ref, d.phys, d.counters[C_NSEND_ALL], d.counters[C_NLOCAL], g,
                             d.send_map, d.send_mult, d.exchg_flag, sc, sc + d.send_cap, sc + 2 * d.send_cap, sc + 3 * d.send_cap);
-}
-
-// which: 0 lcount, 1 gcount (ncells + 1 entries), 2 img_cnt (cap entries)
-__global__ __launch_bounds__(256) void k_fill_batch(const RepDesc *__restrict__ D, int which, int v) {
-    REP_ARGS;
-    int *p = which == 0 ? d.lcount : (which == 1 ? d.gcount : d.img_cnt);
-    const int n = which == 2 ? d.cap : g.ncells + 1;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) p[i] = v;
 }
 
 __global__ __launch_bounds__(256) void k_bin_count_batch(const RepDesc *__restrict__ D) {
@@ -3023,7 +3008,6 @@ LJArgs lj_args(const DevState &d, const Geom &g, const LJParams &prm, int cur, i
     A.nlocal = d.nlocal;
     A.rows = list_rows(d.ncap);
     A.g = g;
-    A.lstart = d.lstart; A.gstart = d.gstart;
     A.X = d.X[cur]; A.Y = d.Y[cur]; A.Z = d.Z[cur];
     A.P = d.P[cur];
     A.Pn = (packed && fused && do_vv1 && next != cur) ? d.P[next] : nullptr;

@@ -322,7 +322,6 @@ struct LJArgs {
     const int *counters;
     int nlocal, rows;    // locals; allocated list rows of each part
     Geom g;
-    const int *lstart, *gstart;
     const double *X, *Y, *Z;
     const double4 *P;    // packed (x, y, z, 0) of X, Y, Z
     double4 *Pn;         // packed copy of the next positions, or null
