@@ -1098,9 +1098,9 @@ __global__ __launch_bounds__(64) void k_lj2(LJArgs A) {
 // instruction (x, y on one lane, z and the type on the other, swapped by DPP);
 // the two pairs of a list group take entries 0, 2 and 1, 3, so that one
 // instruction touches consecutive entries (13.0 -> 10.1 M cache-line lookups
-// per launch at 131072 atoms).  A padded entry reads the local's own record (its
-// zero factor times the distance to another particle would be NaN where that
-// one has left for infinity).
+// per launch at 131072 atoms).  A padded entry reads the spare record behind the
+// last slot, one line for all lanes (a particle's might be at infinity, and the
+// entry's zero factor times that distance is NaN).
 // Measured (100 steps with 5 rebuilds, one lane pair per local -> this):
 // 256 atoms 2.67 -> 1.61 ms, 2048 2.63 -> 1.74, 19652 2.81 -> 2.28, 55296
 // 3.82 -> 3.39; half lists 55296 5.21 -> 4.74, 131072 (400 steps) 32.5 -> 30.9.
@@ -1158,8 +1158,8 @@ __device__ __forceinline__ void lj_multi(const LJArgs &A, int wv) {
             if (R <= 0) return;  // wave-uniform
             const int cnt_h = cnt - eh, cnt_e = cnt - (eh & ~2), cnt_o = cnt - (eh | 2);
             auto gather = [&](int r, uint2 j, Pos &q) {
-                const uint32_t je = cnt_e > r * L ? min(j.x, jmax) : (uint32_t) ii;
-                const uint32_t jo = cnt_o > r * L ? min(j.y, jmax) : (uint32_t) ii;
+                const uint32_t je = cnt_e > r * L ? min(j.x, jmax) : (uint32_t) stride;
+                const uint32_t jo = cnt_o > r * L ? min(j.y, jmax) : (uint32_t) stride;
                 q.a = *(const double2 *) (P + ((je << 5) + off_e));
                 q.b = *(const double2 *) (P + ((jo << 5) + off_o));
             };

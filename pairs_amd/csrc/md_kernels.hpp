@@ -161,7 +161,8 @@ struct DevState {
     int pstride;  // row stride of the partials array
     int max_lds;  // shared memory a workgroup may allocate
     double *X[2], *Y[2], *Z[2];
-    double4 *P[2];       // (x, y, z, 0) of each position buffer, packed for the force kernels' gathers
+    double4 *P[2];       // (x, y, z, type) of each position buffer, packed for the force kernels' gathers; one
+                         // more record, at the origin, for padded list entries
     double *vx, *vy, *vz, *fx, *fy, *fz, *mass;
     int *type, *flags, *uid, *shape, *ref;
     int *phys;    // physical slot of each reference index
@@ -323,7 +324,7 @@ struct LJArgs {
     int nlocal, rows;    // locals; allocated list rows of each part
     Geom g;
     const double *X, *Y, *Z;
-    const double4 *P;    // packed (x, y, z, 0) of X, Y, Z
+    const double4 *P;    // packed (x, y, z, type) of X, Y, Z, and the spare record
     double4 *Pn;         // packed copy of the next positions, or null
     double *Xn, *Yn, *Zn;
     const int *type;

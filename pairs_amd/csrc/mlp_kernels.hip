@@ -295,7 +295,7 @@ constexpr float MLP_PIRC = 3.14159265358979323846f / (float) MLP_RC;
 struct MLPSegArgs {
     const int *counters;
     const double *X, *Y, *Z;
-    const double4 *P;    // (x, y, z, 0) of X, Y, Z packed: one 16-byte and one 8-byte gather
+    const double4 *P;    // (x, y, z, type) of X, Y, Z packed: one 16-byte and one 8-byte gather
     const uint32_t *nl;
     int nl_stride;
     const int *numneighs;
@@ -390,8 +390,9 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
         const int chunk_in = (lane & 3) ^ ((rsub >> 2) & 3);
         for (int st = 0; st < nst; st++) {
             // groups past the lane's list re-read its last group; entries past
-            // its count read the local's own slot (zero times the distance to a
-            // particle at infinity would be NaN), entries are clamped to the last
+            // its count read the spare record behind the last slot (zero times the
+            // distance to a particle at infinity would be NaN), entries are
+            // clamped to the last particle slot
             const uint4 grp = lp[(size_t) min(st, gl) * A.nl_stride];
             uint32_t jq[U];
 #pragma unroll
@@ -399,7 +400,7 @@ __global__ __launch_bounds__(64) void k_mlp_wave(MLPSegArgs A) {
                 const int c = L * q + h;
                 // (a group holds its entries as 0, 2, 1, 3)
                 const uint32_t e = (c & 2) ? ((c & 1) ? grp.w : grp.y) : ((c & 1) ? grp.z : grp.x);
-                jq[q] = 4 * st + c < n ? min(e, jmax) : (uint32_t) ii;
+                jq[q] = 4 * st + c < n ? min(e, jmax) : (uint32_t) A.nl_stride;
             }
             struct Ent { double2 a, b; float4 d0, d1, d2, d3, rho; };
             auto gather = [&](uint32_t j, Ent &e) __attribute__((always_inline)) {

@@ -116,8 +116,9 @@ static void free_particle_arrays(DevState &d) {
 static int alloc_particle_arrays(pairs_hip_ctx *ctx, DevState &d, int cap) {
     int r = 0;
     for (int b = 0; b < 2; b++) { r |= dalloc(ctx, &d.X[b], cap); r |= dalloc(ctx, &d.Y[b], cap); r |= dalloc(ctx, &d.Z[b], cap); }
-    r |= dalloc(ctx, &d.P[0], cap);
-    r |= dalloc(ctx, &d.P[1], cap);
+    // (and one record at the origin, which padded list entries read)
+    r |= dalloc(ctx, &d.P[0], (size_t) cap + 1);
+    r |= dalloc(ctx, &d.P[1], (size_t) cap + 1);
     double **dd[] = {&d.vx, &d.vy, &d.vz, &d.fx, &d.fy, &d.fz, &d.mass, &d.alt_vx, &d.alt_vy, &d.alt_vz, &d.alt_mass};
     for (auto p : dd) r |= dalloc(ctx, p, cap);
     int **ii[] = {&d.type, &d.flags, &d.uid, &d.shape, &d.ref, &d.phys, &d.alt_type, &d.alt_flags, &d.alt_uid,
@@ -133,6 +134,7 @@ static int alloc_particle_arrays(pairs_hip_ctx *ctx, DevState &d, int cap) {
     d.pstride = (int) pstride_of(d, ctx->geom);
     r |= dalloc(ctx, &d.partials, 3 * (size_t) d.pstride);
     if (r) return PAIRS_HIP_ERR_HIP;
+    for (double4 *P : d.P) launch_fill_f64(ctx->stream, (double *) (P + cap), 0.0, 4);
     return 0;
 }
 
@@ -1007,7 +1009,7 @@ static int ensure_mlp_work(pairs_hip_ctx *ctx) {
         dfree(ctx->mlp_G); dfree(ctx->mlp_D); dfree(ctx->mlp_E); dfree(ctx->mlp_f);
         ctx->mlp_G = ctx->mlp_D = ctx->mlp_E = nullptr;
         ctx->mlp_f = nullptr;
-        if (dalloc(ctx, &ctx->mlp_G, (size_t) cap * MLP_ND) || dalloc(ctx, &ctx->mlp_D, (size_t) cap * MLP_ND) ||
+        if (dalloc(ctx, &ctx->mlp_G, (size_t) cap * MLP_ND) || dalloc(ctx, &ctx->mlp_D, ((size_t) cap + 1) * MLP_ND) ||
             dalloc(ctx, &ctx->mlp_E, cap) || dalloc(ctx, &ctx->mlp_f, (size_t) 3 * cap))
             return PAIRS_HIP_ERR_HIP;
         ctx->mlp_cap = cap;
@@ -1674,7 +1676,7 @@ int pairs_hip_mlp_config_grad(pairs_hip_ctx *ctx, pairs_hip_mlp *m, double w_ene
         dfree(ctx->mlp_rho); dfree(ctx->mlp_U);
         ctx->mlp_rho = nullptr;
         ctx->mlp_U = nullptr;
-        if (dalloc(ctx, &ctx->mlp_rho, d.cap) || dalloc(ctx, &ctx->mlp_U, (size_t) d.cap * MLP_ND))
+        if (dalloc(ctx, &ctx->mlp_rho, (size_t) d.cap + 1) || dalloc(ctx, &ctx->mlp_U, (size_t) d.cap * MLP_ND))
             return PAIRS_HIP_ERR_HIP;
         ctx->mlp_train_cap = d.cap;
     }
