@@ -38,7 +38,7 @@ struct pairs_hip_dem_ctx {
     int time_every = 0;
     // timed steps: before prepare, before the contact search, after it, after
     // the slot and the pair kernels, after the sums, after euler
-    hipEvent_t ev[7] = {};
+    hipEvent_t ev[5] = {};
     double t_phase[6] = {};
     double t_sum = 0.0;
     int t_count = 0;
@@ -526,9 +526,8 @@ static void enqueue_step(pairs_hip_dem_ctx *ctx, bool timed) {
     launch_contacts(ctx->stream, ctx->p, ctx->counters, ctx->nlocal, ctx->geom, ctx->prm,
                     timed ? ctx->ev + 2 : nullptr);
     if (!timed) return;  // integrated by the contact kernel
-    hipEventRecord(ctx->ev[5], ctx->stream);
     launch_euler(ctx->stream, ctx->p, ctx->counters, ctx->geom, ctx->prm);
-    hipEventRecord(ctx->ev[6], ctx->stream);
+    hipEventRecord(ctx->ev[4], ctx->stream);
 }
 
 static int ensure_graph(pairs_hip_dem_ctx *ctx) {
@@ -554,14 +553,15 @@ static int enqueue_steps(pairs_hip_dem_ctx *ctx, int a, int b, int t0) {
         if (timed) {
             enqueue_step(ctx, true);
             CHECK_LAUNCH();
-            HIP_OK(hipEventSynchronize(ctx->ev[6]));
-            for (int k = 0; k < 6; k++) {
-                float ms = 0.0f;
-                HIP_OK(hipEventElapsedTime(&ms, ctx->ev[k], ctx->ev[k + 1]));
-                ctx->t_phase[k] += ms;
-            }
+            HIP_OK(hipEventSynchronize(ctx->ev[4]));
+            // (slots and sums, phases 2 and 4, are part of the contact kernel)
+            const int phase[4] = {0, 1, 3, 5};
             float ms = 0.0f;
-            HIP_OK(hipEventElapsedTime(&ms, ctx->ev[1], ctx->ev[5]));
+            for (int k = 0; k < 4; k++) {
+                HIP_OK(hipEventElapsedTime(&ms, ctx->ev[k], ctx->ev[k + 1]));
+                ctx->t_phase[phase[k]] += ms;
+            }
+            HIP_OK(hipEventElapsedTime(&ms, ctx->ev[1], ctx->ev[3]));
             ctx->t_sum += ms;
             ctx->t_count++;
         } else if (ctx->use_graphs) {

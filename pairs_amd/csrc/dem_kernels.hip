@@ -1389,10 +1389,10 @@ static void launch_solve(hipStream_t s, const DemPtrs &p, int *c, int nlocal, co
 void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
                      const hipEvent_t *between) {
     hipLaunchKernelGGL(k_contact_find, dim3(grid_of(p.cap, 256 / LPS)), dim3(256), 0, s, p, c, g);
-    if (between) { hipEventRecord(between[0], s); hipEventRecord(between[1], s); }
+    if (between) hipEventRecord(between[0], s);
     if (between) launch_solve<false>(s, p, c, nlocal, g, prm);
     else launch_solve<true>(s, p, c, nlocal, g, prm);
-    if (between) hipEventRecord(between[2], s);
+    if (between) hipEventRecord(between[1], s);
 }
 
 void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, const DemParams &prm) {

@@ -97,9 +97,9 @@ void launch_mass_inertia(hipStream_t s, const DemPtrs &p, int nl);
 void launch_prepare(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g);
 // the leavers of the first of several steps (each step notes those of the next)
 void launch_find_leavers(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g);
-// nlocal: the host's count; between: three events recorded after the search
-// (two) and after the contact kernel (timed steps only); without them the
-// contact kernel integrates too, and launch_euler is not called
+// nlocal: the host's count; between: two events recorded after the search and
+// after the contact kernel (timed steps only); without them the contact kernel
+// integrates too, and launch_euler is not called
 void launch_contacts(hipStream_t s, const DemPtrs &p, int *c, int nlocal, const DemGeom &g, const DemParams &prm,
                      const hipEvent_t *between = nullptr);
 void launch_euler(hipStream_t s, const DemPtrs &p, int *c, const DemGeom &g, const DemParams &prm);

@@ -221,7 +221,8 @@ class DEMSystem:
         """Average ms of the timed steps' phases: prepare, contact search,
         history slots, spring-dashpot, sums + history clean-up, euler.  Slots,
         spring-dashpot, sums and clean-up are one kernel, timed as the
-        spring-dashpot phase; the slot and sum phases read about zero."""
+        spring-dashpot phase; the slot and sum phases read zero.  A step that
+        is not timed integrates in that kernel too."""
         ms = (_D * 6)()
         self._check(self.L.pairs_hip_dem_phase_times(self.ctx, ms), "phase_times")
         return tuple(ms)

@@ -160,6 +160,25 @@ def test_dem_contacts_vs_oracle(case):
             assert np.abs(p - q).max() <= 1e-10 * max(np.abs(q).max(), 1e-300), (b, name)
 
 
+def test_dem_phase_times_add_up():
+    """the phases that are part of the contact kernel read zero, and the others make
+    up the time of the contact kernels"""
+    from pairs_amd import dem
+    uid, r, x, v, dom, planes = _spheres("pile257")
+    s = dem.DEMSystem(dom, particle_capacity=4096)
+    s.add_spheres(uid, r, x, v)
+    for u, pos, nrm, fl in planes:
+        s.add_halfspace(u, pos, nrm, flags=fl)
+    s.setup()
+    s.set_timing(2)
+    s.run(0, 20)
+    phases, (contact, launches) = s.phase_times(), s.contact_kernel_time()
+    assert launches == 10 and phases[2] == phases[4] == 0.0
+    assert all(phases[k] > 0.0 for k in (0, 1, 3, 5))
+    # (event times are rounded to 1e-7 ms in float)
+    assert abs(phases[1] + phases[3] - contact) < 1e-5 * contact + 1e-6
+
+
 @pytest.mark.parametrize("flags", [0, 8])
 def test_dem_unfixed_halfspaces_vs_oracle(flags):
     """half-spaces without the FIXED flag look for contacts themselves, as points
