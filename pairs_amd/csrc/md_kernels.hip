@@ -755,7 +755,7 @@ __device__ __forceinline__ bool lj_pair(double xi, double yi, double zi, double 
 // locals (cell-sorted, so their neighbours are close in memory), each lane
 // walks its own list in order and adds its pair forces in list order, so the
 // sum is bit-identical to the reference's.  Neighbour positions are gathered
-// from the packed copy P (x, y, z, 0 at 32 bytes per particle): one 16-byte
+// from the packed copy P (x, y, z, type at 32 bytes per particle): one 16-byte
 // and one 8-byte load per entry at a 32-bit byte offset.
 // MODE 0: forces only (lennard_jones with reset_volatile_properties);
 // MODE 1: fused F(ts) + final_integrate(ts) + [thermo] + initial_integrate(ts+1)
@@ -1507,8 +1507,9 @@ __global__ __launch_bounds__(TILE_G) void k_tile_build(TileArgs A) {
 // (padding names a particle at 1e100, which fails the cutoff test and adds a
 // signed zero), the pairs of a row of eight computed together and added in list
 // order.  Bound by vector work (32 operations per entry, 26 of them FP64: 95 of
-// 163 us at 1048576 atoms) and by memory (11 records staged per local, 2 bytes
-// per entry: 690 MB), with 12 waves on a CU.  Against two lanes per local that
+// 163 us at 1048576 atoms) and by memory (up to 1088 records staged per group of
+// some 110 locals, 1152 slots read for them, 2 bytes per entry: 690 MB), with 12
+// waves on a CU.  Against two lanes per local that
 // gather from memory (k_lj2): 283 -> 163 us there, half lists 42.6 -> 38.8 us at
 // 131072 atoms, full lists there 31 either way (a tile's latency is not hidden
 // by other tiles).  Groups of 192 or 256 locals keep fewer waves resident: 182
@@ -2186,9 +2187,10 @@ __global__ __launch_bounds__(256) void k_find_leavers(const double *__restrict__
 // and the relabeling is that of k_exchange_relabel_body.  More leavers than the list
 // holds are found by a scan of the locals in reference order instead.  Bound by
 // the latency of its phases; with k_find_leavers it takes the place of three
-// kernels per dimension (us per rebuild: 256 atoms 27 -> 12, 131072 45 ->
-// 25; a lattice start, where 3072 leave at once, 1.82 -> 1.70 ms for 25 steps).  Beyond some 200000 locals the leavers of a rebuild no longer fit
-// and the three kernels remain (exch_listed).
+// kernels per dimension (us per rebuild: 256 atoms 27 -> 12, 131072 45 -> 29, 36
+// to 41 in the first rebuilds behind a lattice; a lattice start, where 3072 leave
+// at once, 1.82 -> 1.70 ms for 25 steps).  The three kernels remain for larger
+// systems (exch_listed) and once the list has overflowed.
 __global__ __launch_bounds__(1024) void k_exchange(double *__restrict__ X, double *__restrict__ Y,
                                                    double *__restrict__ Z, const int *__restrict__ flags,
                                                    int *__restrict__ ref, int *__restrict__ phys,
@@ -2451,7 +2453,7 @@ __global__ __launch_bounds__(BORDER_T) void k_border_count(BorderArgs A) {
 // by dimension; on overflow the counts stay as they were.  Bound by latency in
 // small systems and by the ghosts' writes in large ones; with k_border_count it
 // takes the place of a count and a scatter pass per dimension (us per rebuild:
-// 256 atoms 20 -> 12, 131072 31 -> 23, 1048576 111 -> 61).
+// 256 atoms 20 -> 12, 131072 31 -> 28, 1048576 111 -> 67).
 template <int ND>
 __global__ __launch_bounds__(BORDER_T) void k_border_ghosts(BorderArgs A) {
     constexpr int NK = pow3(ND), NW = BORDER_T / 64;

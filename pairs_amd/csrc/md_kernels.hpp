@@ -17,9 +17,11 @@
 // (cell 0 plus the 3x3 columns around it, z range widened by one) are 20
 // contiguous physical runs: the segment's tile, staged in LDS once and shared
 // by all its home particles.  Neighbour lists hold physical slots (32 bits),
-// in the reference's candidate order.  The force kernels work on "waves": 64
-// consecutive physical locals, one per lane, gathering neighbour positions
-// from a packed (x, y, z, 0) copy of the position buffer.
+// in the reference's candidate order.  The force kernels work on "waves" of 2
+// to 64 consecutive physical locals, 32 lanes to one lane per local by the size
+// of the system, gathering neighbour positions from a packed (x, y, z, type) copy
+// of the position buffer; large systems of one type stage them in LDS, a tile
+// per group of locals.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

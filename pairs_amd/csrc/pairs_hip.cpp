@@ -530,10 +530,12 @@ int pairs_hip_upload(pairs_hip_ctx *ctx, int n, const double *x, const double *v
     CHECK_LAUNCH();
     HIP_OK(hipStreamSynchronize(ctx->stream));
     d.nlocal = n;
-    // the leavers of a rebuild (some 600 at 131072 locals of the LJ fluid, 3900 at
-    // the start of a lattice of 186624) fit the list of the one-workgroup exchange.
-    // 200 steps of 198400 atoms 15.6 ms with the wide kernels, 15.1 with the list; at
-    // 389344 no difference was measured
+    // the one-workgroup exchange from a list of leavers, or the wide kernels: 200
+    // steps of 198400 atoms 15.6 ms with the wide kernels, 15.1 with the list; at
+    // 389344 no difference was measured.  (That was with a list of 1024, which
+    // overflowed there.  With room for 4096 the leavers of larger systems would
+    // fit, some 600 at 131072 locals of the LJ fluid growing with the surface, but
+    // for the start of a lattice, 3900 at 186624; not timed there since.)
     d.exch_listed = n < 200000;
     ctx->nghost = 0;
     ctx->nsend_all = 0;
@@ -1038,10 +1040,13 @@ static void enqueue_rebuild(pairs_hip_ctx *ctx, hipStream_t s) {
     enqueue_build(ctx, s, false);
 }
 
-// The rebuild's ~37 small kernels have grids that depend only on
-// capacities, and their counts live on the device: they are replayed from a
-// graph (one per position buffer, captured on the context's stream), so they
-// run back to back and cost one launch on the host.
+// The rebuild's ten kernels (three more with force tiles; seven more where the
+// wide exchange runs) take their counts from the device: they are replayed from
+// a graph (one per position buffer, captured on the context's stream), so they
+// run back to back and cost one launch on the host.  Their grids depend on the
+// capacities and, where workgroups share work in small systems (border ghosts,
+// neighbour build), on the number of locals: what changes that number drops the
+// graphs, as an upload does.
 // The first launch of an executable graph prepares its dispatch packets on
 // the host (several times the cost of a later launch, with the device idle
 // when the graph opens a run); uploading it when it is instantiated moves
