@@ -32,6 +32,7 @@ struct pairs_hip_ctx {
     int zc_override = 0;
     bool tiles_off = false;    // no force tiles: the batched kernels do without
     bool tiles_big = false;    // nor for this upload: too many groups did not fit theirs
+    size_t tile_rows16 = 0;    // entries of the 16-bit lists' allocation
     int home_target = 40;      // home particles a segment aims at (sets zc; about 3 cells at rho 0.84)
     // graphs of n consecutive non-rebuild steps (slot n - 1, n <=
     // CHAIN_MAX), by parity of the current buffer at their first step: a run
